@@ -30,7 +30,7 @@
 extern "C" {
 #endif
 
-#define TAM_ABI_VERSION 8
+#define TAM_ABI_VERSION 9
 #define TAM_BLOCK_SIZE 128 /* elements per quantisation / CoState block */
 #define TAM_TAIL_TILES 4   /* tiles per tail workgroup of an unaligned tensor */
 
@@ -100,7 +100,8 @@ typedef struct TamTensor {
   uint32_t chunk0;      /* [derived] COSTATE: first alpha-reduction chunk    */
   uint64_t ratio_off;   /* [derived] COSTATE: offset of its ratios (blocks)  */
   double inv_bc2;       /* [in] 1 / (double)bias_correction2 (correctly rounded) */
-  uint32_t slice0;      /* [derived] COSTATE: first selection slice (8192 blocks each) */
+  uint32_t slice0;      /* [derived] COSTATE: first selection slice (16384 blocks  */
+                        /*      each; none for at most TamStepInfo.sel_small)      */
   float c_lr;           /* [derived] f32(neg_lr / bias_correction1)          */
   float* ef_residual;   /* [in] EF: f32[n] error-feedback residual (in/out;  */
                         /*      written, not read, without HAS_EF)           */
@@ -127,10 +128,11 @@ typedef struct TamTensor {
                             /*      pointer): the launches test descriptor 0.   */
   uint32_t tail0;           /* [derived] first workgroup of this tensor in pass 0's */
                             /*      kernel for quarters that are not full        */
-  uint32_t tail_wgs;        /* [derived] its workgroups there: 1, or one per    */
-                            /*      TAM_TAIL_TILES tiles when param or grad is  */
-                            /*      not 16-byte aligned (every quarter is then  */
-                            /*      bounds-checked)                             */
+  uint32_t tail_wgs;        /* [derived] its workgroups there: one when a part of */
+                            /*      it lies outside full units (8 blocks), none  */
+                            /*      otherwise or with EF; one per TAM_TAIL_TILES */
+                            /*      tiles when param or grad is not 16-byte      */
+                            /*      aligned (every quarter is then bounds-checked) */
 } TamTensor;
 
 /* Launch summary and workspace layout, filled by tam_prepare(). */
@@ -139,7 +141,7 @@ typedef struct TamStepInfo {
   uint32_t total_tiles;
   uint32_t n_costate;
   uint32_t total_chunks;   /* alpha-reduction chunks (8192 partial sums each) */
-  uint32_t total_slices;   /* selection slices (8192 block ratios each) */
+  uint32_t total_slices;   /* selection slices (16384 block ratios each) of the larger CoState tensors */
   uint32_t dtype_mask;     /* bit TAM_DTYPE_x set when a tensor of that dtype without TAM_FLAG_EF is present */
   uint64_t ratio_blocks;   /* sum of nb over CoState tensors */
   uint64_t off_partials;   /* workspace byte offsets */
@@ -148,11 +150,13 @@ typedef struct TamStepInfo {
   uint64_t ws_bytes;       /* required workspace size */
   uint64_t off_chunks;
   uint64_t off_sel;
-  uint64_t off_hist;
   uint32_t n_ef;           /* tensors with error feedback (a fifth pass runs) */
   uint32_t n_device_step;  /* DEVICE_STEP tensors (pass 0 starts with their prologue) */
   uint64_t off_ef_alpha;   /* EF: previous alpha of each tensor (f32 per tensor) */
   uint32_t tail_blocks;    /* workgroups of pass 0's kernel for quarters that are not full */
+  uint32_t sel_small;      /* a CoState tensor of at most this many blocks is one workgroup's selection: */
+                           /* 32768, or 12288 when some tensor has more than 32768 (slices run then) */
+  uint32_t sel_max;        /* blocks of the largest such tensor (0: none) */
 } TamStepInfo;
 
 /* Version of this ABI (TAM_ABI_VERSION). */

@@ -28,7 +28,7 @@ TAM_FLAG_EF = 0x10
 TAM_FLAG_HAS_EF = 0x20
 TAM_FLAG_DEVICE_STEP = 0x40
 
-ABI_VERSION = 8
+ABI_VERSION = 9
 # workspace of tam_multi_tensor_step_static (include/turboadam_amd.h)
 TAM_STATIC_SCRATCH_BYTES = 64 << 20
 
@@ -101,11 +101,12 @@ class TamStepInfo(ctypes.Structure):
         ("ws_bytes", ctypes.c_uint64),
         ("off_chunks", ctypes.c_uint64),
         ("off_sel", ctypes.c_uint64),
-        ("off_hist", ctypes.c_uint64),
         ("n_ef", ctypes.c_uint32),
         ("n_device_step", ctypes.c_uint32),
         ("off_ef_alpha", ctypes.c_uint64),
         ("tail_blocks", ctypes.c_uint32),
+        ("sel_small", ctypes.c_uint32),
+        ("sel_max", ctypes.c_uint32),
     ]
 
 

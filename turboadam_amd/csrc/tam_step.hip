@@ -974,6 +974,31 @@ __device__ __forceinline__ void tam_update(const TamTensor& d, float* p, const f
   }
 }
 
+// First index i in [0, nT) whose test is true, for a test that is false up to
+// some index and true after (true for nT - 1 at the latest); uniform over the
+// wave, every lane of which must be active.  The 64 lanes probe 64 positions at
+// once, so up to 64 tensors take one round of loads and up to 4096 two, where a
+// binary search takes log2(nT) dependent ones: for the small kernels, whose time
+// is such a chain.  (The tile loops of passes 0 and 2 search by scalar loads
+// below: tens of thousands of workgroups probing 64 descriptors each cost the
+// GPT-2-sized fp32 step 28 us of 412.)
+template <typename F>
+__device__ __forceinline__ int tam_wave_first(int nT, F&& test) {
+  const int lane = (int)(threadIdx.x & 63u);
+  int lo = 0, n = nT;
+  while (n > 1) {
+    const int step = (n + 63) >> 6;
+    const int last = lo + (lane + 1) * step - 1;  // the lane's group ends here
+    const int i = last < lo + n ? last : lo + n - 1;
+    const uint64_t hit = __ballot(test(i));  // the last group's end tests true
+    const int f = hit ? (int)__builtin_ctzll(hit) : 63;
+    const int left = n - f * step;
+    lo += f * step;
+    n = left < step ? left : step;
+  }
+  return lo;
+}
+
 // Tensor owning global tile `tile` (binary search over tile0).
 __device__ __forceinline__ int tam_find_tensor(const TamTensor* __restrict__ T, int nT, uint32_t tile) {
   int lo = 0, hi = nT - 1;
@@ -1616,61 +1641,16 @@ TAM_K1_FULL_KERNEL(tam_k1_main_bf16, TAM_DTYPE_BF16, TAM_K1_WAVES_BF16)
 TAM_K1_FULL_KERNEL(tam_k1_main_f16, TAM_DTYPE_F16, TAM_K1_WAVES_F16)
 TAM_K1_FULL_KERNEL(tam_k1_main_f32, TAM_DTYPE_F32, TAM_K1_WAVES_F32)
 
-// ---------------------------------------------------------------------------
-// Selection state of a CoState tensor (workspace), set afresh every step by
-// pass 0's tail kernel
-// ---------------------------------------------------------------------------
-struct TamSel {
-  uint32_t kmin, kmax;  // key range (tam_k_sel_minmax)
-  uint32_t prefix[2];   // bits fixed so far of the k_lo-th and k_hi-th smallest ratio
-  uint32_t k[2];        // rank within the ratios sharing that prefix
-  uint32_t mask;        // bits fixed so far
-  int32_t top;          // highest bit not yet fixed (-1: done; 32: no round run yet)
-};
-
-// Every thread of one workgroup: tensor d's selection state before the key
-// range is known and its cleared histogram (4096 counts).
-__device__ __forceinline__ void tam_sel_reset_wg(const TamTensor& d, TamSel* __restrict__ sel,
-                                                 uint32_t* __restrict__ hist) {
-  for (uint32_t i = threadIdx.x; i < 4096u; i += blockDim.x) tam_g(hist)[i] = 0u;
-  if (threadIdx.x == 0) {
-    TamSel z;
-    z.kmin = 0xffffffffu;
-    z.kmax = 0u;
-    z.prefix[0] = z.prefix[1] = 0u;
-    z.k[0] = d.k_lo;
-    z.k[1] = d.k_hi;
-    z.mask = 0u;
-    z.top = 32;
-    *sel = z;
-  }
-}
-
 // The quarters outside full units: the last (at most five) quarters of each
 // tensor, or every quarter of a tensor whose parameter or gradient is not
 // 16-byte aligned.  An aligned tensor has one workgroup; an unaligned one has
 // one per TAM_TAIL_TILES tiles (tam_prepare: tail0, tail_wgs), so a large
 // unaligned tensor spreads over the GPU.  Wave w takes every fourth quarter of
 // the workgroup's range.
-__device__ __forceinline__ int tam_tail_tensor(const TamTensor* __restrict__ T, int nT, uint32_t wg) {
-  int lo = 0, hi = nT - 1;  // the last tensor whose first tail workgroup is at or before wg
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (T[mid].tail0 <= wg) lo = mid; else hi = mid - 1;
-  }
-  return lo;
-}
-
 __global__ __launch_bounds__(TAM_WG) void tam_k1_tail(const TamTensor* __restrict__ T, int nT, uint32_t seed_lo,
-                                                      uint32_t seed_hi, double2* __restrict__ partials,
-                                                      TamSel* __restrict__ sel, uint32_t* __restrict__ hist) {
+                                                      uint32_t seed_hi, double2* __restrict__ partials) {
   if (tam_step_skipped(T)) return;
-  const int ti = tam_tail_tensor(T, nT, blockIdx.x);
-  const TamTensor& d = T[ti];
-  // the tensor's first tail workgroup sets its selection state
-  if ((d.flags & TAM_FLAG_COSTATE) && blockIdx.x == d.tail0)
-    tam_sel_reset_wg(d, sel + ti, hist + (uint64_t)ti * 4096u);
-  if (d.flags & TAM_FLAG_EF) return;  // the whole workgroup: tam_k1_ef covers the tensor
+  const TamTensor& d = T[tam_wave_first(nT, [&](int i) { return T[i].tail0 + T[i].tail_wgs > blockIdx.x; })];
   __shared__ float lut[TAM_WG / 64][4 * 64];
   __shared__ TamLdsTabs tabs;
   tam_lds_tabs_fill(&tabs);
@@ -1744,18 +1724,21 @@ __global__ __launch_bounds__(TAM_WG) void tam_k1_ef(const TamTensor* __restrict_
 // partials zero-padded to a power of two P.  The padded array is cut into
 // aligned chunks of 8192 (one chunk of P when P <= 8192); chunk sums are
 // subtrees of the same tree.  tam_k_alpha_chunks sums every chunk of every
-// tensor (one workgroup per chunk: 32 consecutive values per thread, then a
-// tree in LDS); tam_k_alpha sums each tensor's chunk sums (at most 2048, a
-// power of two) and forms alpha.  Zero padding does not change the sum:
-// x + 0 == x, and +0.0 added to the result settles the sign of an exact zero.
-#define TAM_PAIR_PER_THREAD 32
-#define TAM_CHUNK (TAM_WG * TAM_PAIR_PER_THREAD)
+// tensor (one workgroup per chunk); a tensor of one chunk (up to 4.2M elements)
+// gets its alpha there, and tam_k_alpha, launched only when some tensor has
+// more, sums the others' chunk sums (at most 2048, a power of two).  Zero
+// padding does not change the sum: x + 0 == x, and +0.0 added to the result
+// settles the sign of an exact zero.
+//
+// Leaf 1024 j + 4 t + i of a chunk is loaded by thread t (i < 4: 64 consecutive
+// bytes per lane, so a wave reads 4 KB at a time; 32 consecutive leaves per
+// thread, as before, touched 64 lines per load: 81 us for the 251 MB of an
+// 8B-parameter set).  The tree goes over i in the thread, over t across the
+// wave's lanes (the first three levels also spread the eight values of j over
+// the lanes: each halves the values a lane holds) and the four waves, then over j.
+#define TAM_CHUNK 8192
+#define TAM_ALPHA_STRIDE (4 * TAM_WG)  // leaves per j
 
-__device__ __forceinline__ uint32_t tam_pow2_at_least(uint32_t x) {
-  uint32_t p = 1;
-  while (p < x) p <<= 1;
-  return p;
-}
 // Chunks of a tensor's padded partial array (0 for tensors without CoState).
 __host__ __device__ __forceinline__ uint32_t tam_alpha_chunks(uint32_t flags, uint32_t ntiles) {
   if (!(flags & TAM_FLAG_COSTATE)) return 0;
@@ -1781,44 +1764,100 @@ __device__ double2 tam_wg_tree(double2* sh, uint32_t n) {
   return sh[0];
 }
 
+// alpha from the dot products: they round to fp32 once; +0.0 makes an
+// exact-zero sum +0.
+__device__ __forceinline__ float tam_alpha_of(double2 s) {
+  const float gg = (float)(s.x + 0.0);
+  const float mg = (float)(s.y + 0.0);
+  return gg > 0.0f ? mg / gg : 0.0f;
+}
+
+__device__ __forceinline__ double2 tam_add2(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
+template <int X>
+__device__ __forceinline__ double2 tam_xor2(double2 v) {
+  return make_double2(__shfl_xor(v.x, X), __shfl_xor(v.y, X));
+}
+
+// Selection state (pass 3); a tensor of several slices keeps one per round in the
+// workspace, the first reset in pass 1.
+struct TamSel {
+  uint32_t kmin, kmax;  // key range (tam_k_sel_minmax)
+  uint32_t prefix[2];   // bits fixed so far of the k_lo-th and k_hi-th smallest ratio
+  uint32_t k[2];        // rank within the ratios sharing that prefix
+  uint32_t mask;        // bits fixed so far
+  int32_t top;          // highest bit not yet fixed (-1: done; 32: no round run yet)
+};
+
+__device__ __forceinline__ TamSel tam_sel_fresh(uint32_t kmin, uint32_t kmax, uint32_t k_lo, uint32_t k_hi) {
+  TamSel z;
+  z.kmin = kmin;
+  z.kmax = kmax;
+  z.prefix[0] = z.prefix[1] = 0u;
+  z.k[0] = k_lo;
+  z.k[1] = k_hi;
+  z.mask = 0u;
+  z.top = 32;
+  return z;
+}
+__device__ void tam_sel_reset(const TamTensor& d, TamSel* sel) {
+  *sel = tam_sel_fresh(0xffffffffu, 0u, d.k_lo, d.k_hi);
+}
+
 __global__ __launch_bounds__(TAM_WG) void tam_k_alpha_chunks(const TamTensor* __restrict__ T, int nT,
                                                              const double2* __restrict__ partials,
-                                                             double2* __restrict__ chunk_sums) {
+                                                             double2* __restrict__ chunk_sums,
+                                                             float* __restrict__ alpha_new,
+                                                             TamSel* __restrict__ sel) {
   if (tam_step_skipped(T)) return;
-  __shared__ double2 sh[TAM_WG];
+  __shared__ double2 sh[TAM_WG / 64][8];
   const uint32_t c = blockIdx.x;
   // tensor owning chunk c: the first whose chunk range ends after c
-  int lo = 0, hi = nT - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (T[mid].chunk0 + tam_alpha_chunks(T[mid].flags, T[mid].ntiles) > c) hi = mid; else lo = mid + 1;
-  }
-  const TamTensor& d = T[lo];
-  const uint32_t count = d.ntiles * 4u;                 // quarter-tile partials of the tensor
-  const uint32_t P = tam_pow2_at_least(count);
-  const uint32_t lim = P > TAM_CHUNK ? TAM_CHUNK : P;   // leaves of this chunk's subtree
+  const int ti =
+      tam_wave_first(nT, [&](int i) { return T[i].chunk0 + tam_alpha_chunks(T[i].flags, T[i].ntiles) > c; });
+  const TamTensor& d = T[ti];
   const uint32_t base = (c - d.chunk0) * TAM_CHUNK;
-  const double2* x = partials + (uint64_t)d.tile0 * 4u;
-  const uint32_t tid = threadIdx.x;
-  double sa[4], sq[4];
+  const uint32_t left = d.ntiles * 4u - base;  // partials from here on (chunks start inside the tensor's
+  const uint32_t count = d.ntiles * 4u > base ? (left < TAM_CHUNK ? left : TAM_CHUNK) : 0u;  // padded array)
+  const double2* x = partials + (uint64_t)d.tile0 * 4u + base;
+  const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
+  double2 s[8];
 #pragma unroll
-  for (int h = 0; h < 4; ++h) {
-    double a[8], q[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const uint32_t local = tid * TAM_PAIR_PER_THREAD + h * 8 + i;
-      const uint32_t k = base + local;
-      const double2 v = (local < lim && k < count) ? x[k] : make_double2(0.0, 0.0);
-      a[i] = v.x;
-      q[i] = v.y;
-    }
-    sa[h] = tam_pair8(a);
-    sq[h] = tam_pair8(q);
+  for (uint32_t j = 0; j < 8u; ++j) {
+    const uint32_t k = TAM_ALPHA_STRIDE * j + 4u * t;  // count is a multiple of 4
+    s[j] = make_double2(0.0, 0.0);
+    if (k < count) s[j] = tam_add2(tam_add2(x[k], x[k + 1u]), tam_add2(x[k + 2u], x[k + 3u]));
   }
-  sh[tid] = make_double2((sa[0] + sa[1]) + (sa[2] + sa[3]), (sq[0] + sq[1]) + (sq[2] + sq[3]));
+  // lanes l and l ^ 1, l ^ 2, l ^ 4: each keeps half of its values of j
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const bool odd = (lane & 1u) != 0;
+    const double2 keep = odd ? s[2 * j + 1] : s[2 * j], give = odd ? s[2 * j] : s[2 * j + 1];
+    s[j] = tam_add2(keep, tam_xor2<1>(give));
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const bool odd = (lane & 2u) != 0;
+    const double2 keep = odd ? s[2 * j + 1] : s[2 * j], give = odd ? s[2 * j] : s[2 * j + 1];
+    s[j] = tam_add2(keep, tam_xor2<2>(give));
+  }
+  const bool odd = (lane & 4u) != 0;
+  double2 v = tam_add2(odd ? s[1] : s[0], tam_xor2<4>(odd ? s[0] : s[1]));
+  v = tam_add2(v, tam_xor2<8>(v));
+  v = tam_add2(v, tam_xor2<16>(v));
+  v = tam_add2(v, tam_xor2<32>(v));
+  if (lane < 8u) sh[wave][lane] = v;  // lane l: the sum over the wave's t of j = l
   __syncthreads();
-  const double2 r = tam_wg_tree(sh, TAM_WG);
-  if (tid == 0) chunk_sums[c] = r;
+  if (t < 64u) {  // over the four waves, then over j
+    v = tam_add2(tam_add2(sh[0][t & 7u], sh[1][t & 7u]), tam_add2(sh[2][t & 7u], sh[3][t & 7u]));
+    v = tam_add2(v, tam_xor2<1>(v));
+    v = tam_add2(v, tam_xor2<2>(v));
+    v = tam_add2(v, tam_xor2<4>(v));
+    if (t == 0u) {
+      if (tam_alpha_chunks(d.flags, d.ntiles) == 1u) alpha_new[ti] = tam_alpha_of(v);
+      else chunk_sums[c] = v;
+      if (c == d.chunk0) tam_sel_reset(d, sel + 3 * ti);
+    }
+  }
 }
 
 __global__ __launch_bounds__(TAM_WG) void tam_k_alpha(const TamTensor* __restrict__ T,
@@ -1828,7 +1867,7 @@ __global__ __launch_bounds__(TAM_WG) void tam_k_alpha(const TamTensor* __restric
   __shared__ double2 sh[2048];
   const TamTensor& d = T[blockIdx.x];
   const uint32_t nch = tam_alpha_chunks(d.flags, d.ntiles);
-  if (nch == 0) return;
+  if (nch <= 1) return;  // no CoState, or done by tam_k_alpha_chunks
   for (uint32_t i = threadIdx.x; i < nch; i += TAM_WG) sh[i] = chunk_sums[d.chunk0 + i];
   __syncthreads();
   // nch is a power of two <= 2048: fold it to at most 2 * TAM_WG with pairwise steps first
@@ -1851,12 +1890,7 @@ __global__ __launch_bounds__(TAM_WG) void tam_k_alpha(const TamTensor* __restric
     n = w;
   }
   const double2 s = tam_wg_tree(sh, n);
-  if (threadIdx.x == 0) {
-    // dot products round to fp32 once; +0.0 makes an exact-zero sum +0
-    const float gg = (float)(s.x + 0.0);
-    const float mg = (float)(s.y + 0.0);
-    alpha_new[blockIdx.x] = gg > 0.0f ? mg / gg : 0.0f;
-  }
+  if (threadIdx.x == 0) alpha_new[blockIdx.x] = tam_alpha_of(s);
 }
 
 // ---------------------------------------------------------------------------
@@ -2133,54 +2167,51 @@ tam_k2_encode_f32(const TamTensor* __restrict__ T, int nT, uint32_t total_tiles,
 // (costate.py:146-148), alpha write-back (costate.py:443-454)
 // ---------------------------------------------------------------------------
 // Ratios are >= +0 or NaN, so their fp32 bit patterns order like torch.sort
-// (NaN last).  The selection is an MSD radix select on those patterns, spread
-// over slices of 8192 keys so that large tensors use many workgroups (the
-// state and histogram of each tensor are set by pass 0's tail kernel):
+// (NaN last).  The selection is an MSD radix select on those patterns.  The
+// bits all keys share need no round: the first digit starts at the highest bit
+// that differs.  A few outliers (blocks whose ratio is near zero) push that bit
+// up and pile the other keys into a few bins of the first digit, where LDS
+// atomics serialise, so the first digit is short and its LDS histogram is held
+// in several copies, one per residue of the lane (a 32768-key selection with one
+// key at zero: 30 us with one copy of 11 bits).  Later digits have 11 bits.
+//
+// A small tensor is one workgroup's: tam_k_sel_one keeps its keys in LDS, runs the
+// rounds there until few keys are left for each rank, ranks those directly and
+// writes the labels, one launch for all such tensors.  A larger one is cut into
+// slices of TAM_SLICE keys, and kernel boundaries order its rounds:
 //   tam_k_sel_minmax  per slice: min / max of the keys (atomic min / max per
-//                     tensor) -- the bits all keys share need no round, and
-//                     the first digit starts at the highest bit that differs,
-//                     so keys of similar magnitude spread over its bins
-//                     instead of piling into a few (LDS atomics on one bin
-//                     serialise);
-//   tam_k_sel_hist    per slice, three times: LDS histogram of the next 11-bit
-//                     digit below the bits already fixed, for the keys that
-//                     match the prefix of each of the two ranks, added into
-//                     the tensor's histogram;
-//   tam_k_sel_pick    per tensor, after each histogram: prefix sums of the
-//                     histogram pick the digit holding each rank; the
-//                     histogram is cleared for the next round;
-//   tam_k_sel_labels  per slice: labels from the two thresholds; alpha
-//                     write-back.
-#define TAM_SLICE 8192u
+//                     tensor); clears the tensor's histograms;
+//   tam_k_sel_hist    per slice, three times: LDS histogram of the next digit
+//                     below the bits already fixed, for the keys that match the
+//                     prefix of each of the two ranks, added into the round's
+//                     histogram of the tensor.  Every workgroup first picks the
+//                     previous round's digits itself (prefix sums of that
+//                     round's histogram); the first slice's keeps the result;
+//   tam_k_sel_labels  per slice: the last pick, labels from the two thresholds,
+//                     alpha write-back.
+// Small is at most TAM_SEL_SMALL blocks (128 KB of keys beside the histograms
+// fill LDS; 1024 threads) when no tensor of the step is larger, else at most
+// TAM_SEL_TINY (256 threads, two workgroups to a CU): the slices' five launches
+// (about 6 us each) run anyway then, and take the tensors between at no cost,
+// where one CU needs 13 us for 18432 keys and 20 for 32768 (6 for 32).
+// The three histograms of a tensor (48 KB) lie in its partial sums, which
+// pass 1 has used up and which are at least 128 KB for a tensor of several
+// slices.
+#define TAM_SEL_WG 1024
+#define TAM_SEL_SMALL 32768u
+#define TAM_SEL_TINY 12288u
+#define TAM_SLICE 16384u
+#define TAM_SEL_HIST_WORDS (3u * 4096u)
+static_assert((TAM_SEL_TINY / 4u + 1u) * sizeof(double2) >= TAM_SEL_HIST_WORDS * sizeof(uint32_t),
+              "the histograms fit a sliced tensor's partials (one per 4 blocks)");
+#define TAM_SEL_FEW 256u  // keys left for a rank that are ranked directly
+#define TAM_SEL_W0 8        // bits of the first digit in one workgroup (16 copies of 256 bins) and
+#define TAM_SEL_W0_SLICE 10 // in slices (4 copies of 1024): three rounds of 10 + 11 + 11 bits fix all 32
+#define TAM_SEL_W 11        // bits of the later digits (2048 bins for each rank)
 
-__host__ __device__ __forceinline__ uint32_t tam_sel_slices(uint32_t flags, uint32_t nb) {
-  return (flags & TAM_FLAG_COSTATE) ? (nb + TAM_SLICE - 1u) / TAM_SLICE : 0u;
-}
-
-// Tensor owning selection slice j: the first whose slice range ends after j.
-__device__ __forceinline__ int tam_slice_tensor(const TamTensor* __restrict__ T, int nT, uint32_t j) {
-  int lo = 0, hi = nT - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (T[mid].slice0 + tam_sel_slices(T[mid].flags, T[mid].nb) > j) hi = mid; else lo = mid + 1;
-  }
-  return lo;
-}
-
-// Keys [k0, k1) of a tensor's ratios, visited by the 256 threads of a
-// workgroup, 8 keys per thread per round (two 16-byte loads; k0 is a
-// multiple of 4 and the ratio array 16-byte aligned).
-template <typename F>
-__device__ __forceinline__ void tam_slice_keys(const uint32_t* __restrict__ keys, uint32_t k0, uint32_t k1, F&& f) {
-  for (uint32_t i = k0 + threadIdx.x * 8u; i < k1; i += TAM_WG * 8u) {
-    if (i + 8u <= k1) {
-      const TamW4 a = tam_g((const TamW4*)(keys + i))[0], b = tam_g((const TamW4*)(keys + i))[1];
-      f(a.x); f(a.y); f(a.z); f(a.w);
-      f(b.x); f(b.y); f(b.z); f(b.w);
-    } else {
-      for (uint32_t j = i; j < k1; ++j) f(tam_g(keys)[j]);
-    }
-  }
+// Slices of a tensor in a step whose small tensors have at most `small` blocks.
+__host__ __device__ __forceinline__ uint32_t tam_sel_slices(uint32_t flags, uint32_t nb, uint32_t small) {
+  return (flags & TAM_FLAG_COSTATE) && nb > small ? (nb + TAM_SLICE - 1u) / TAM_SLICE : 0u;
 }
 
 // The state a round starts from: before the first round, the bits above the
@@ -2195,177 +2226,387 @@ __device__ __forceinline__ TamSel tam_sel_begin(TamSel s) {
   return s;
 }
 
-// Digit window below the fixed bits: bits [sh, top].
-__device__ __forceinline__ void tam_sel_window(int top, int& sh, uint32_t& dmask) {
-  sh = top >= 10 ? top - 10 : 0;
+// Digit window of at most `width` bits below the fixed ones: bits [sh, top].
+__device__ __forceinline__ void tam_sel_window(int top, int width, int& sh, uint32_t& dmask) {
+  sh = top >= width ? top - width + 1 : 0;
   dmask = (1u << (top - sh + 1)) - 1u;
 }
 
-__global__ __launch_bounds__(TAM_WG) void tam_k_sel_minmax(const TamTensor* __restrict__ T, int nT,
-                                                           const float* __restrict__ ratios, TamSel* __restrict__ sel) {
-  if (tam_step_skipped(T)) return;
-  __shared__ uint32_t red[2][TAM_WG / 64];
-  const int t = tam_slice_tensor(T, nT, blockIdx.x);
-  const TamTensor& d = T[t];
-  const uint32_t k0 = (blockIdx.x - d.slice0) * TAM_SLICE;
-  const uint32_t k1 = k0 + TAM_SLICE < d.nb ? k0 + TAM_SLICE : d.nb;
-  uint32_t kmin = 0xffffffffu, kmax = 0u;
-  tam_slice_keys((const uint32_t*)(ratios + d.ratio_off), k0, k1, [&](uint32_t k) {
-    kmin = k < kmin ? k : kmin;
-    kmax = k > kmax ? k : kmax;
-  });
+struct TamPickLds {
+  uint32_t wsum[2][16];  // per wave
+  uint32_t prefix[2], k[2], count[2];
+};
+
+// After a round's histogram (two of 2048 bins; ranks with equal prefixes share
+// the first) of digits of `width` bits: the digit holding each rank, as the state the next round starts
+// from.  st is the state the round started from (tam_sel_begin applied or not).
+// Every thread of a workgroup of WG calls it; the result is uniform.  pk.count
+// holds the number of keys sharing each new prefix afterwards.
+template <int WG = TAM_SEL_WG>
+__device__ __forceinline__ TamSel tam_sel_pick(TamSel st, const uint32_t* hist, int width, TamPickLds& pk) {
+  st = tam_sel_begin(st);
+  if (st.top < 0) return st;  // every bit fixed (or every key equal): the prefixes are the keys
+  int sh;
+  uint32_t dmask;
+  tam_sel_window(st.top, width, sh, dmask);
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
+  const bool same = st.prefix[0] == st.prefix[1];
+  constexpr int BINS = 2048 / WG;  // consecutive bins of a thread
+  uint32_t c[2][BINS], tot[2], inc[2];
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const uint32_t* h = hist + (same ? 0u : (uint32_t)r) * 2048u + BINS * tid;
+    tot[r] = 0u;
+#pragma unroll
+    for (int i = 0; i < BINS; i += 2) {
+      const TamW2 x = *(const TamW2*)(h + i);
+      c[r][i] = x.x;
+      c[r][i + 1] = x.y;
+      tot[r] += x.x + x.y;
+    }
+    inc[r] = tot[r];
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t t = __shfl_up(inc[r], off);
+      if (lane >= (uint32_t)off) inc[r] += t;
+    }
+    if (lane == 63u) pk.wsum[r][w] = inc[r];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    // sum of the waves before: each lane adds one wave's total
+    uint32_t before = lane < w ? pk.wsum[r][lane] : 0u;
+#pragma unroll
+    for (int off = 8; off >= 1; off >>= 1) before += __shfl_xor(before, off);
+    before = __builtin_amdgcn_readfirstlane(before);
+    uint32_t pre = before + inc[r] - tot[r];  // keys in the bins before
+    const uint32_t k = st.k[r];
+    if (k >= pre && k - pre < tot[r]) {  // one thread: its bins hold rank k
+#pragma unroll
+      for (int i = 0; i < BINS; ++i) {
+        if (k >= pre && k - pre < c[r][i]) {
+          pk.k[r] = k - pre;
+          pk.count[r] = c[r][i];
+          pk.prefix[r] = st.prefix[r] | ((BINS * tid + (uint32_t)i) << sh);
+        }
+        pre += c[r][i];
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    st.prefix[r] = pk.prefix[r];
+    st.k[r] = pk.k[r];
+  }
+  st.mask |= dmask << sh;
+  st.top = sh - 1;
+  return st;
+}
+
+// Minimum and maximum over a workgroup of WG threads (uniform).
+template <int WG = TAM_SEL_WG>
+__device__ __forceinline__ void tam_wg_minmax(uint32_t& kmin, uint32_t& kmax, uint32_t (*red)[16]) {
+  constexpr int WAVES = WG / 64;
+  const uint32_t lane = threadIdx.x & 63u;
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
     const uint32_t a = __shfl_xor(kmin, off), b = __shfl_xor(kmax, off);
     kmin = a < kmin ? a : kmin;
     kmax = b > kmax ? b : kmax;
   }
-  if ((threadIdx.x & 63u) == 0) {
+  if (lane == 0u) {
     red[0][threadIdx.x >> 6] = kmin;
     red[1][threadIdx.x >> 6] = kmax;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < TAM_WG / 64; ++w) {
-      kmin = red[0][w] < kmin ? red[0][w] : kmin;
-      kmax = red[1][w] > kmax ? red[1][w] : kmax;
-    }
-    atomicMin(&sel[t].kmin, kmin);
-    atomicMax(&sel[t].kmax, kmax);
-  }
-}
-
-// Exclusive prefix sum over the TAM_WG threads of the workgroup.
-__device__ uint32_t tam_wg_excl_scan(uint32_t v, uint32_t* wsum) {
-  const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
-  uint32_t inc = v;
+  kmin = red[0][lane & (WAVES - 1)];
+  kmax = red[1][lane & (WAVES - 1)];
 #pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t t = __shfl_up(inc, off);
-    if (lane >= (uint32_t)off) inc += t;
+  for (int off = WAVES / 2; off >= 1; off >>= 1) {
+    const uint32_t a = __shfl_xor(kmin, off), b = __shfl_xor(kmax, off);
+    kmin = a < kmin ? a : kmin;
+    kmax = b > kmax ? b : kmax;
   }
-  if (lane == 63u) wsum[w] = inc;
-  __syncthreads();
-  uint32_t before = 0u;
-  for (uint32_t i = 0; i < w; ++i) before += wsum[i];
-  __syncthreads();  // wsum may be reused once every wave has read it
-  return before + inc - v;
 }
 
-// One round of the selection (three launches, in order; a tensor whose bits
-// are all fixed returns at once).
-__global__ __launch_bounds__(TAM_WG) void tam_k_sel_hist(const TamTensor* __restrict__ T, int nT,
-                                                         const float* __restrict__ ratios,
-                                                         const TamSel* __restrict__ sel, uint32_t* __restrict__ hist) {
+// Adds one key's digit to the histograms of the ranks whose prefix it shares.
+__device__ __forceinline__ void tam_sel_count(uint32_t key, const TamSel& st, int sh, uint32_t dmask, uint32_t* h) {
+  const uint32_t dg = (key >> sh) & dmask, km = key & st.mask;
+  if (km == st.prefix[0]) atomicAdd(&h[dg], 1u);
+  if (st.prefix[0] != st.prefix[1] && km == st.prefix[1]) atomicAdd(&h[2048u + dg], 1u);
+}
+
+template <uint32_t CAP>
+struct TamSelLds {
+  __attribute__((aligned(16))) uint32_t key[CAP];
+  __attribute__((aligned(16))) uint32_t hist[4096];
+  TamPickLds pk;
+  uint32_t red[2][16];
+  uint32_t tau[2];
+  uint32_t left[2];
+};
+
+// Calls f(key) for the keys of the workgroup's LDS copy, four per thread and
+// round.
+template <int WG, uint32_t CAP, typename F>
+__device__ __forceinline__ void tam_lds_keys(const TamSelLds<CAP>& sh, uint32_t nb, F&& f) {
+  const uint32_t nv = nb & ~3u;
+#pragma unroll 2
+  for (uint32_t i = 4u * threadIdx.x; i < nv; i += 4u * WG) {
+    const TamW4 k = *(const TamW4*)(sh.key + i);
+    f(k.x);
+    f(k.y);
+    f(k.z);
+    f(k.w);
+  }
+  if (threadIdx.x < nb - nv) f(sh.key[nv + threadIdx.x]);
+}
+
+// The whole selection of one tensor of nb <= CAP ratios by a workgroup of WG
+// threads; the thresholds' bit patterns (uniform) in tau, the keys left in LDS.
+template <int WG, uint32_t CAP>
+__device__ __forceinline__ void tam_sel_small(const uint32_t* __restrict__ keys, uint32_t nb, uint32_t k_lo,
+                                              uint32_t k_hi, uint32_t* tau, TamSelLds<CAP>& sh) {
+  const uint32_t tid = threadIdx.x;
+  uint32_t kmin = 0xffffffffu, kmax = 0u;
+  const auto see = [&](uint32_t k) {
+    kmin = k < kmin ? k : kmin;
+    kmax = k > kmax ? k : kmax;
+  };
+  const uint32_t nv = nb & ~3u;  // the array is 16-byte aligned
+#pragma unroll 4
+  for (uint32_t i = 4u * tid; i < nv; i += 4u * WG) {
+    const TamW4 k = tam_g((const TamW4*)(keys + i))[0];
+    *(TamW4*)(sh.key + i) = k;
+    see(k.x);
+    see(k.y);
+    see(k.z);
+    see(k.w);
+  }
+  if (tid < nb - nv) {
+    const uint32_t k = tam_g(keys)[nv + tid];
+    sh.key[nv + tid] = k;
+    see(k);
+  }
+  if (tid < 2u) sh.left[tid] = 0u;
+  tam_wg_minmax<WG>(kmin, kmax, sh.red);  // its barrier also orders the keys
+  TamSel st = tam_sel_begin(tam_sel_fresh(kmin, kmax, k_lo, k_hi));
+  for (bool first = true; st.top >= 0; first = false) {  // uniform
+    for (uint32_t i = 4u * tid; i < 4096u; i += 4u * WG) *(TamW4*)(sh.hist + i) = TamW4{0u, 0u, 0u, 0u};
+    const int width = first ? TAM_SEL_W0 : TAM_SEL_W;
+    int s;
+    uint32_t dmask;
+    tam_sel_window(st.top, width, s, dmask);
+    __syncthreads();
+    if (first) {  // every key has the prefix
+      tam_lds_keys<WG>(sh, nb, [&](uint32_t k) { atomicAdd(&sh.hist[((k >> s) & dmask) * 16u + (tid & 15u)], 1u); });
+      __syncthreads();
+      uint32_t sum = 0u;  // of bin tid's copies
+      if (tid < 256u) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const TamW4 x = *(const TamW4*)(sh.hist + 16u * tid + 4 * c);
+          sum += (x.x + x.y) + (x.z + x.w);
+        }
+      }
+      __syncthreads();
+      for (uint32_t i = tid; i < 2048u; i += WG) sh.hist[i] = i < 256u ? sum : 0u;
+    } else {
+      tam_lds_keys<WG>(sh, nb, [&](uint32_t k) { tam_sel_count(k, st, s, dmask, sh.hist); });
+    }
+    __syncthreads();
+    st = tam_sel_pick<WG>(st, sh.hist, width, sh.pk);
+    if (st.top >= 0 && sh.pk.count[0] <= TAM_SEL_FEW && sh.pk.count[1] <= TAM_SEL_FEW) {
+      // gather the keys left for each rank (in the histogram, read by now); the
+      // one with k smaller keys among them is the threshold
+      const bool same = st.prefix[0] == st.prefix[1];
+      tam_lds_keys<WG>(sh, nb, [&](uint32_t k) {
+        const uint32_t km = k & st.mask;
+        if (km == st.prefix[0]) sh.hist[atomicAdd(&sh.left[0], 1u)] = k;
+        else if (km == st.prefix[1]) sh.hist[2048u + atomicAdd(&sh.left[1], 1u)] = k;
+      });
+      __syncthreads();
+      // thread 256 r + i takes key i of rank r
+      for (uint32_t u = tid; u < 2u * TAM_SEL_FEW; u += WG) {
+        const uint32_t r = u / TAM_SEL_FEW, i = u % TAM_SEL_FEW, c = sh.pk.count[r];
+        const uint32_t* list = sh.hist + (same ? 0u : 2048u * r);
+        const uint32_t k = list[i];
+        uint32_t less = 0u, equal = 0u;
+#pragma unroll 4
+        for (uint32_t j = 0; j < c; j += 4u) {
+          const TamW4 x = *(const TamW4*)(list + j);
+          const uint32_t xs[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+          for (uint32_t e = 0; e < 4u; ++e) {
+            const bool in = j + e < c;
+            less += in && xs[e] < k ? 1u : 0u;
+            equal += in && xs[e] == k ? 1u : 0u;
+          }
+        }
+        // equal keys write the same
+        const uint32_t rank = r ? st.k[1] : st.k[0];
+        if (i < c && less <= rank && rank < less + equal) sh.tau[r] = k;
+      }
+      __syncthreads();
+      tau[0] = sh.tau[0];
+      tau[1] = sh.tau[1];
+      return;
+    }
+  }
+  tau[0] = st.prefix[0];
+  tau[1] = st.prefix[1];
+}
+
+// Label of a block (costate.py:146-148).
+__device__ __forceinline__ uint8_t tam_label_of(uint32_t key, float tau0, float tau1) {
+  const float x = tam_u2f(key);
+  return x >= tau1 ? (uint8_t)2 : (x >= tau0 ? (uint8_t)1 : (uint8_t)0);
+}
+
+// One workgroup per tensor of at most `small` <= CAP blocks.
+template <int WG, uint32_t CAP>
+__global__ __launch_bounds__(WG) void tam_k_sel_one(const TamTensor* __restrict__ T,
+                                                    const float* __restrict__ alpha_new,
+                                                    const float* __restrict__ ratios, char* __restrict__ ws,
+                                                    float* __restrict__ alpha_old, uint32_t small) {
   if (tam_step_skipped(T)) return;
-  __shared__ uint32_t h[2][2048];
-  const int t = tam_slice_tensor(T, nT, blockIdx.x);
+  const uint32_t t = blockIdx.x;
   const TamTensor& d = T[t];
-  const TamSel st = tam_sel_begin(sel[t]);
+  const uint32_t nb = d.nb;
+  if (!(d.flags & TAM_FLAG_COSTATE) || nb > small) return;
+  __shared__ TamSelLds<CAP> sh;
+  uint32_t tau[2];
+  tam_sel_small<WG>((const uint32_t*)(ratios + d.ratio_off), nb, d.k_lo, d.k_hi, tau, sh);
+  const float tau0 = tam_u2f(tau[0]), tau1 = tam_u2f(tau[1]);
+  const bool ef = (d.flags & TAM_FLAG_EF) != 0;  // error feedback: labels to the staging area
+  uint8_t* labels = ef ? tam_stage(d, ws).labels : d.labels;
+  for (uint32_t i = threadIdx.x; i < nb; i += WG) tam_g(labels)[i] = tam_label_of(sh.key[i], tau0, tau1);
+  if (threadIdx.x == 0) {
+    if (ef) alpha_old[t] = tam_g(d.alpha)[0];  // pass 4 decodes the previous encoding
+    tam_g(d.alpha)[0] = alpha_new[t];
+  }
+}
+
+// Tensor owning selection slice j: the first whose slice range ends after j.
+__device__ __forceinline__ int tam_slice_tensor(const TamTensor* __restrict__ T, int nT, uint32_t j, uint32_t small) {
+  return tam_wave_first(nT, [&](int i) { return T[i].slice0 + tam_sel_slices(T[i].flags, T[i].nb, small) > j; });
+}
+
+// Keys [k0, k1) of a tensor's ratios, visited by the threads of a workgroup, 8
+// keys per thread per round (two 16-byte loads; k0 is a multiple of 4 and the
+// ratio array 16-byte aligned).
+template <typename F>
+__device__ __forceinline__ void tam_slice_keys(const uint32_t* __restrict__ keys, uint32_t k0, uint32_t k1, F&& f) {
+  for (uint32_t i = k0 + threadIdx.x * 8u; i < k1; i += TAM_SEL_WG * 8u) {
+    if (i + 8u <= k1) {
+      const TamW4 a = tam_g((const TamW4*)(keys + i))[0], b = tam_g((const TamW4*)(keys + i))[1];
+      f(a.x); f(a.y); f(a.z); f(a.w);
+      f(b.x); f(b.y); f(b.z); f(b.w);
+    } else {
+      for (uint32_t j = i; j < k1; ++j) f(tam_g(keys)[j]);
+    }
+  }
+}
+
+// The histograms of a sliced tensor (three of 4096 counts), in its partials.
+__device__ __forceinline__ uint32_t* tam_sel_hists(const TamTensor& d, double2* partials) {
+  return (uint32_t*)(partials + (uint64_t)d.tile0 * 4u);
+}
+
+__global__ __launch_bounds__(TAM_SEL_WG) void tam_k_sel_minmax(const TamTensor* __restrict__ T, int nT,
+                                                               const float* __restrict__ ratios,
+                                                               TamSel* __restrict__ sel,
+                                                               double2* __restrict__ partials, uint32_t small) {
+  if (tam_step_skipped(T)) return;
+  __shared__ uint32_t red[2][16];
+  const int t = tam_slice_tensor(T, nT, blockIdx.x, small);
+  const TamTensor& d = T[t];
+  const uint32_t slice = blockIdx.x - d.slice0, k0 = slice * TAM_SLICE;
+  const uint32_t k1 = k0 + TAM_SLICE < d.nb ? k0 + TAM_SLICE : d.nb;
+  // pass 1 has read the partials: its slices clear the tensor's histograms
+  uint32_t* hist = tam_sel_hists(d, partials);
+  for (uint32_t i = slice * TAM_SEL_WG + threadIdx.x; i < TAM_SEL_HIST_WORDS;
+       i += tam_sel_slices(d.flags, d.nb, small) * TAM_SEL_WG)
+    tam_g(hist)[i] = 0u;
+  uint32_t kmin = 0xffffffffu, kmax = 0u;
+  tam_slice_keys((const uint32_t*)(ratios + d.ratio_off), k0, k1, [&](uint32_t k) {
+    kmin = k < kmin ? k : kmin;
+    kmax = k > kmax ? k : kmax;
+  });
+  tam_wg_minmax(kmin, kmax, red);
+  if (threadIdx.x == 0) {
+    atomicMin(&sel[3 * t].kmin, kmin);
+    atomicMax(&sel[3 * t].kmax, kmax);
+  }
+}
+
+// Round `round` of a sliced tensor's selection (a tensor whose bits are all
+// fixed adds nothing).
+__global__ __launch_bounds__(TAM_SEL_WG) void tam_k_sel_hist(const TamTensor* __restrict__ T, int nT,
+                                                             const float* __restrict__ ratios,
+                                                             TamSel* __restrict__ sel,
+                                                             double2* __restrict__ partials, int round,
+                                                             uint32_t small) {
+  if (tam_step_skipped(T)) return;
+  __shared__ __attribute__((aligned(16))) uint32_t h[4096];
+  __shared__ TamPickLds pk;
+  const int t = tam_slice_tensor(T, nT, blockIdx.x, small);
+  const TamTensor& d = T[t];
+  uint32_t* hist = tam_sel_hists(d, partials) + (uint32_t)round * 4096u;
+  TamSel st;
+  if (round == 0) {
+    st = tam_sel_begin(sel[3 * t]);
+  } else {
+    st = tam_sel_pick(sel[3 * t + round - 1], hist - 4096, round == 1 ? TAM_SEL_W0_SLICE : TAM_SEL_W, pk);
+    if (blockIdx.x == d.slice0 && threadIdx.x == 0) sel[3 * t + round] = st;
+  }
   if (st.top < 0) return;  // uniform over the workgroup
   int sh;
   uint32_t dmask;
-  tam_sel_window(st.top, sh, dmask);
-  for (uint32_t i = threadIdx.x; i < 4096u; i += TAM_WG) (&h[0][0])[i] = 0u;
+  tam_sel_window(st.top, round == 0 ? TAM_SEL_W0_SLICE : TAM_SEL_W, sh, dmask);
+  for (uint32_t i = threadIdx.x; i < 4096u; i += TAM_SEL_WG) h[i] = 0u;
   __syncthreads();
-  const uint32_t p0 = st.prefix[0], p1 = st.prefix[1], mask = st.mask;
-  const bool same = p0 == p1;
   const uint32_t k0 = (blockIdx.x - d.slice0) * TAM_SLICE;
   const uint32_t k1 = k0 + TAM_SLICE < d.nb ? k0 + TAM_SLICE : d.nb;
-  tam_slice_keys((const uint32_t*)(ratios + d.ratio_off), k0, k1, [&](uint32_t key) {
-    const uint32_t dg = (key >> sh) & dmask;
-    const uint32_t km = key & mask;
-    if (km == p0) atomicAdd(&h[0][dg], 1u);
-    if (!same && km == p1) atomicAdd(&h[1][dg], 1u);
-  });
-  __syncthreads();
-  uint32_t* gh = hist + (uint64_t)t * 4096u;
-  for (uint32_t i = threadIdx.x; i < 4096u; i += TAM_WG) {
-    const uint32_t c = (&h[0][0])[i];
-    if (c) atomicAdd(&gh[i], c);
-  }
-}
-
-// After a round's histogram: the digit holding each of a tensor's two ranks
-// (ranks with equal prefixes share the first half of the histogram), the new
-// state, and the histogram cleared for the next round.  One workgroup per
-// tensor.
-__global__ __launch_bounds__(TAM_WG) void tam_k_sel_pick(const TamTensor* __restrict__ T, TamSel* __restrict__ sel,
-                                                         uint32_t* __restrict__ hist) {
-  if (tam_step_skipped(T)) return;
-  if (!(T[blockIdx.x].flags & TAM_FLAG_COSTATE)) return;
-  __shared__ uint32_t wsum[TAM_WG / 64];
-  __shared__ uint32_t new_prefix[2], new_k[2];
-  const TamSel st = tam_sel_begin(sel[blockIdx.x]);
-  const uint32_t tid = threadIdx.x;
-  if (st.top < 0) {  // every bit fixed (or every key equal): the prefixes are the keys
-    if (tid == 0) sel[blockIdx.x] = st;
+  const uint32_t* keys = (const uint32_t*)(ratios + d.ratio_off);
+  if (round == 0) {  // every key has the prefix
+    tam_slice_keys(keys, k0, k1,
+                   [&](uint32_t key) { atomicAdd(&h[((key >> sh) & dmask) * 4u + (threadIdx.x & 3u)], 1u); });
+    __syncthreads();
+    const TamW4 x = *(const TamW4*)(h + 4u * threadIdx.x);
+    const uint32_t c = (x.x + x.y) + (x.z + x.w);
+    if (c) atomicAdd(&hist[threadIdx.x], c);
     return;
   }
-  int sh;
-  uint32_t dmask;
-  tam_sel_window(st.top, sh, dmask);
-  uint32_t* gh = hist + (uint64_t)blockIdx.x * 4096u;
-  const bool same = st.prefix[0] == st.prefix[1];
-  if (tid < 2) {
-    new_prefix[tid] = st.prefix[tid];
-    new_k[tid] = st.k[tid];
-  }
+  tam_slice_keys(keys, k0, k1, [&](uint32_t key) { tam_sel_count(key, st, sh, dmask, h); });
   __syncthreads();
-  for (int r = 0; r < 2; ++r) {
-    // bins 8 tid .. 8 tid + 7 of rank r's histogram
-    const uint32_t* hr = gh + (same ? 0u : (uint32_t)r) * 2048u + 8u * tid;
-    const TamW4 a = tam_g((const TamW4*)hr)[0], b = tam_g((const TamW4*)hr)[1];
-    const uint32_t c[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-    uint32_t tot = 0u;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) tot += c[i];
-    uint32_t pre = tam_wg_excl_scan(tot, wsum);
-    const uint32_t k = st.k[r];
-    if (k >= pre && k - pre < tot) {  // one thread: its bins hold rank k
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        if (k >= pre && k - pre < c[i]) {
-          new_k[r] = k - pre;
-          new_prefix[r] = st.prefix[r] | ((8u * tid + (uint32_t)i) << sh);
-        }
-        pre += c[i];
-      }
-    }
-  }
-  __syncthreads();
-  for (uint32_t i = tid; i < 4096u; i += TAM_WG) tam_g(gh)[i] = 0u;  // for the next round
-  if (tid == 0) {
-    TamSel o = st;
-    o.prefix[0] = new_prefix[0];
-    o.prefix[1] = new_prefix[1];
-    o.k[0] = new_k[0];
-    o.k[1] = new_k[1];
-    o.mask = st.mask | (dmask << sh);
-    o.top = sh - 1;
-    sel[blockIdx.x] = o;
+  for (uint32_t i = threadIdx.x; i < 4096u; i += TAM_SEL_WG) {
+    const uint32_t c = h[i];
+    if (c) atomicAdd(&hist[i], c);
   }
 }
 
-__global__ __launch_bounds__(TAM_WG) void tam_k_sel_labels(const TamTensor* __restrict__ T, int nT,
-                                                           const float* __restrict__ alpha_new,
-                                                           const float* __restrict__ ratios,
-                                                           const TamSel* __restrict__ sel, char* __restrict__ ws,
-                                                           float* __restrict__ alpha_old) {
+__global__ __launch_bounds__(TAM_SEL_WG) void tam_k_sel_labels(const TamTensor* __restrict__ T, int nT,
+                                                               const float* __restrict__ alpha_new,
+                                                               const float* __restrict__ ratios,
+                                                               const TamSel* __restrict__ sel,
+                                                               double2* __restrict__ partials, char* __restrict__ ws,
+                                                               float* __restrict__ alpha_old, uint32_t small) {
   if (tam_step_skipped(T)) return;
-  const int t = tam_slice_tensor(T, nT, blockIdx.x);
+  __shared__ TamPickLds pk;
+  const int t = tam_slice_tensor(T, nT, blockIdx.x, small);
   const TamTensor& d = T[t];
-  const float tau0 = tam_u2f(sel[t].prefix[0]);
-  const float tau1 = tam_u2f(sel[t].prefix[1]);
+  const TamSel st = tam_sel_pick(sel[3 * t + 2], tam_sel_hists(d, partials) + 2u * 4096u, TAM_SEL_W, pk);
+  const float tau0 = tam_u2f(st.prefix[0]), tau1 = tam_u2f(st.prefix[1]);
   const uint32_t k0 = (blockIdx.x - d.slice0) * TAM_SLICE;
   const uint32_t k1 = k0 + TAM_SLICE < d.nb ? k0 + TAM_SLICE : d.nb;
-  const float* r = ratios + d.ratio_off;
+  const uint32_t* r = (const uint32_t*)(ratios + d.ratio_off);
   const bool ef = (d.flags & TAM_FLAG_EF) != 0;  // error feedback: labels to the staging area
   uint8_t* labels = ef ? tam_stage(d, ws).labels : d.labels;
-  for (uint32_t i = k0 + threadIdx.x; i < k1; i += TAM_WG) {
-    const float x = tam_g(r)[i];
-    tam_g(labels)[i] = x >= tau1 ? (uint8_t)2 : (x >= tau0 ? (uint8_t)1 : (uint8_t)0);
-  }
+  for (uint32_t i = k0 + threadIdx.x; i < k1; i += TAM_SEL_WG)
+    tam_g(labels)[i] = tam_label_of(tam_g(r)[i], tau0, tau1);
   if (blockIdx.x == d.slice0 && threadIdx.x == 0) {
     if (ef) alpha_old[t] = tam_g(d.alpha)[0];  // pass 4 decodes the previous encoding
     tam_g(d.alpha)[0] = alpha_new[t];
@@ -2555,10 +2796,9 @@ __global__ void tam_k_make_desc(TamTensor* __restrict__ out, uint64_t n, uint32_
   *out = d;
 }
 
-// Fresh selection state of the one tensor of desc and its cleared histogram.
-__global__ __launch_bounds__(TAM_WG) void tam_k_sel_reset(const TamTensor* __restrict__ desc, TamSel* __restrict__ sel,
-                                                          uint32_t* __restrict__ hist) {
-  tam_sel_reset_wg(desc[0], sel, hist);
+// Fresh selection state of the one tensor of desc.
+__global__ void tam_k_sel_reset(const TamTensor* __restrict__ desc, TamSel* __restrict__ sel) {
+  tam_sel_reset(desc[0], sel);
 }
 
 // delta = fl(m - fl(alpha*g)) (costate.py:42)
@@ -2621,10 +2861,29 @@ __global__ void tam_k_classify(const float* __restrict__ ratios, uint64_t nb, co
   labels[i] = x >= tau1 ? (uint8_t)2 : (x >= tau0 ? (uint8_t)1 : (uint8_t)0);
 }
 
-// The two thresholds of a finished selection.
-__global__ void tam_k_sel_taus(const TamSel* __restrict__ sel, float* __restrict__ taus) {
-  taus[0] = tam_u2f(sel[0].prefix[0]);
-  taus[1] = tam_u2f(sel[0].prefix[1]);
+// The two thresholds of one tensor of at most TAM_SEL_SMALL ratios.
+__global__ __launch_bounds__(TAM_SEL_WG) void tam_k_taus_small(const float* __restrict__ ratios, uint32_t nb,
+                                                               uint32_t k_lo, uint32_t k_hi,
+                                                               float* __restrict__ taus) {
+  __shared__ TamSelLds<TAM_SEL_SMALL> sh;
+  uint32_t tau[2];
+  tam_sel_small<TAM_SEL_WG>((const uint32_t*)ratios, nb, k_lo, k_hi, tau, sh);
+  if (threadIdx.x == 0) {
+    taus[0] = tam_u2f(tau[0]);
+    taus[1] = tam_u2f(tau[1]);
+  }
+}
+
+// The two thresholds of a larger tensor after its last histogram.
+__global__ __launch_bounds__(TAM_SEL_WG) void tam_k_sel_taus(const TamSel* __restrict__ sel,
+                                                             const uint32_t* __restrict__ hist,
+                                                             float* __restrict__ taus) {
+  __shared__ TamPickLds pk;
+  const TamSel st = tam_sel_pick(sel[2], hist + 2u * 4096u, TAM_SEL_W, pk);
+  if (threadIdx.x == 0) {
+    taus[0] = tam_u2f(st.prefix[0]);
+    taus[1] = tam_u2f(st.prefix[1]);
+  }
 }
 
 // fused_v_update (quantize.py:222-299) for one tensor: the 1Q half of pass 1
@@ -2866,7 +3125,11 @@ int tam_prepare(TamTensor* tensors, int n_tensors, TamStepInfo* info) {
   if (!info || n_tensors < 0 || (n_tensors > 0 && !tensors)) return tam_fail(TAM_E_INVALID, "%snull argument", "");
   uint64_t tiles = 0, ratio_blocks = 0, chunks = 0, slices = 0, ef_bytes = 0, tail_blocks = 0;
   uint32_t dtype_mask = 0;
-  uint32_t ncs = 0, nef = 0, ndev = 0;
+  uint32_t ncs = 0, nef = 0, ndev = 0, nsmall = 0, sel_max = 0;
+  uint32_t sel_small = TAM_SEL_SMALL;  // blocks of the largest tensor whose selection is one workgroup's
+  for (int i = 0; i < n_tensors; ++i)
+    if ((tensors[i].flags & TAM_FLAG_COSTATE) && tensors[i].n > (uint64_t)TAM_SEL_SMALL * TAM_BLOCK_SIZE)
+      sel_small = TAM_SEL_TINY;
   for (int i = 0; i < n_tensors; ++i) {
     TamTensor& t = tensors[i];
     if (t.n == 0) return tam_fail(TAM_E_INVALID, "%stensor %ld has no elements", "", i);
@@ -2909,6 +3172,10 @@ int tam_prepare(TamTensor* tensors, int n_tensors, TamStepInfo* info) {
       t.ratio_off = ratio_blocks;
       ratio_blocks += (nb + 3) & ~3ull;  // 16-byte aligned per tensor
       ++ncs;
+      if (nb <= sel_small) {
+        ++nsmall;
+        sel_max = nb > sel_max ? (uint32_t)nb : sel_max;
+      }
       if (t.flags & TAM_FLAG_EF) {
         if (!t.ef_residual || ((uintptr_t)t.ef_residual & 15u))
           return tam_fail(TAM_E_INVALID, "%stensor %ld: ef_residual null or misaligned", "", i);
@@ -2927,7 +3194,9 @@ int tam_prepare(TamTensor* tensors, int n_tensors, TamStepInfo* info) {
     t.tile0 = (uint32_t)tiles;
     const bool aligned = (((uintptr_t)t.param | (uintptr_t)t.grad) & 15u) == 0;
     t.tail0 = (uint32_t)tail_blocks;
-    t.tail_wgs = (aligned || (t.flags & TAM_FLAG_EF)) ? 1u : (uint32_t)((nt + TAM_TAIL_TILES - 1) / TAM_TAIL_TILES);
+    if (t.flags & TAM_FLAG_EF) t.tail_wgs = 0u;  // tam_k1_ef covers the tensor
+    else if (aligned) t.tail_wgs = t.n % (8u * TAM_BLOCK_SIZE) ? 1u : 0u;  // whole units only: nothing left
+    else t.tail_wgs = (uint32_t)((nt + TAM_TAIL_TILES - 1) / TAM_TAIL_TILES);
     tail_blocks += t.tail_wgs;
     if (!(t.flags & TAM_FLAG_EF)) dtype_mask |= 1u << t.dtype;  // pass 0's per-dtype kernels skip EF tensors
     t.chunk0 = (uint32_t)chunks;
@@ -2936,7 +3205,7 @@ int tam_prepare(TamTensor* tensors, int n_tensors, TamStepInfo* info) {
     t.k_abs = tam_abs_term(t.bias_correction1, t.eps);
     tiles += nt;
     chunks += tam_alpha_chunks(t.flags, t.ntiles);
-    slices += tam_sel_slices(t.flags, t.nb);
+    slices += tam_sel_slices(t.flags, t.nb, sel_small);
     // below 2^31, so that a tile index plus a grid stride cannot wrap
     if (tiles > (1ull << 31)) return tam_fail(TAM_E_INVALID, "%stoo many tiles", "", 0);
   }
@@ -2947,6 +3216,8 @@ int tam_prepare(TamTensor* tensors, int n_tensors, TamStepInfo* info) {
   info->n_costate = ncs;
   info->total_chunks = (uint32_t)chunks;
   info->total_slices = (uint32_t)slices;
+  info->sel_small = sel_small;
+  info->sel_max = nsmall ? sel_max : 0u;
   info->dtype_mask = dtype_mask;
   info->ratio_blocks = ratio_blocks;
   uint64_t off = 0;
@@ -2959,9 +3230,7 @@ int tam_prepare(TamTensor* tensors, int n_tensors, TamStepInfo* info) {
   info->off_chunks = off;
   off = tam_align_up(off + chunks * sizeof(double2), 256);
   info->off_sel = off;
-  off = tam_align_up(off + (uint64_t)n_tensors * sizeof(TamSel), 256);
-  info->off_hist = off;
-  off = tam_align_up(off + (uint64_t)n_tensors * 4096u * sizeof(uint32_t), 256);
+  off = tam_align_up(off + (uint64_t)n_tensors * 3u * sizeof(TamSel), 256);
   info->n_ef = nef;
   info->n_device_step = ndev;
   info->off_ef_alpha = off;
@@ -2988,7 +3257,6 @@ static int tam_launch_pass(int pass, const TamTensor* d_tensors, const TamStepIn
   float* ratios = (float*)(ws + info->off_ratios);
   double2* chunk_sums = (double2*)(ws + info->off_chunks);
   TamSel* sel = (TamSel*)(ws + info->off_sel);
-  uint32_t* hist = (uint32_t*)(ws + info->off_hist);
   float* alpha_old = (float*)(ws + info->off_ef_alpha);
   // vwg: virtual workgroups (each striding over the tiles on its own) per workgroup
   auto grid_of = [&](int which, const void* kernel, int block = TAM_WG, uint32_t vwg = 1u) {
@@ -3023,14 +3291,16 @@ static int tam_launch_pass(int pass, const TamTensor* d_tensors, const TamStepIn
                            d_tensors, info->n_tensors, info->total_tiles, (uint32_t)seed, (uint32_t)(seed >> 32),
                            partials);
       TAM_HIP_CHECK(hipGetLastError());
-      hipLaunchKernelGGL(tam_k1_tail, dim3(info->tail_blocks), dim3(TAM_WG), 0, s, d_tensors, info->n_tensors,
-                         (uint32_t)seed, (uint32_t)(seed >> 32), partials, sel, hist);
+      if (info->tail_blocks)
+        hipLaunchKernelGGL(tam_k1_tail, dim3(info->tail_blocks), dim3(TAM_WG), 0, s, d_tensors, info->n_tensors,
+                           (uint32_t)seed, (uint32_t)(seed >> 32), partials);
       break;
     case 1:
       hipLaunchKernelGGL(tam_k_alpha_chunks, dim3(info->total_chunks), dim3(TAM_WG), 0, s, d_tensors,
-                         info->n_tensors, partials, chunk_sums);
+                         info->n_tensors, partials, chunk_sums, alpha_new, sel);
       TAM_HIP_CHECK(hipGetLastError());
-      hipLaunchKernelGGL(tam_k_alpha, dim3(info->n_tensors), dim3(TAM_WG), 0, s, d_tensors, chunk_sums, alpha_new);
+      if (info->total_chunks > info->n_costate)  // some tensor has several chunks
+        hipLaunchKernelGGL(tam_k_alpha, dim3(info->n_tensors), dim3(TAM_WG), 0, s, d_tensors, chunk_sums, alpha_new);
       break;
     case 2: {
       // full units by dtype class; the other units' quarters go to the 16-bit
@@ -3051,19 +3321,27 @@ static int tam_launch_pass(int pass, const TamTensor* d_tensors, const TamStepIn
       break;
     }
     default:
-      // the state and histograms were set by pass 0's tail kernel
-      hipLaunchKernelGGL(tam_k_sel_minmax, dim3(info->total_slices), dim3(TAM_WG), 0, s, d_tensors,
-                         info->n_tensors, ratios, sel);
+      // one launch for every small tensor, by the largest: two (by size) took 34 us
+      // where one takes 18 (148 tensors of a GPT-2-sized set)
+      if (info->sel_max > TAM_SEL_TINY)
+        hipLaunchKernelGGL((tam_k_sel_one<TAM_SEL_WG, TAM_SEL_SMALL>), dim3(info->n_tensors), dim3(TAM_SEL_WG), 0, s,
+                           d_tensors, alpha_new, ratios, ws, alpha_old, info->sel_small);
+      else if (info->sel_max)
+        hipLaunchKernelGGL((tam_k_sel_one<256, TAM_SEL_TINY>), dim3(info->n_tensors), dim3(256), 0, s, d_tensors,
+                           alpha_new, ratios, ws, alpha_old, info->sel_small);
       TAM_HIP_CHECK(hipGetLastError());
-      for (int r = 0; r < 3; ++r) {  // 11-bit digits: at most three rounds fix all 32 bits
-        hipLaunchKernelGGL(tam_k_sel_hist, dim3(info->total_slices), dim3(TAM_WG), 0, s, d_tensors,
-                           info->n_tensors, ratios, sel, hist);
+      if (info->total_slices) {
+        hipLaunchKernelGGL(tam_k_sel_minmax, dim3(info->total_slices), dim3(TAM_SEL_WG), 0, s, d_tensors,
+                           info->n_tensors, ratios, sel, partials, info->sel_small);
         TAM_HIP_CHECK(hipGetLastError());
-        hipLaunchKernelGGL(tam_k_sel_pick, dim3(info->n_tensors), dim3(TAM_WG), 0, s, d_tensors, sel, hist);
-        TAM_HIP_CHECK(hipGetLastError());
+        for (int r = 0; r < 3; ++r) {  // 11-bit digits: at most three rounds fix all 32 bits
+          hipLaunchKernelGGL(tam_k_sel_hist, dim3(info->total_slices), dim3(TAM_SEL_WG), 0, s, d_tensors,
+                             info->n_tensors, ratios, sel, partials, r, info->sel_small);
+          TAM_HIP_CHECK(hipGetLastError());
+        }
+        hipLaunchKernelGGL(tam_k_sel_labels, dim3(info->total_slices), dim3(TAM_SEL_WG), 0, s, d_tensors,
+                           info->n_tensors, alpha_new, ratios, sel, partials, ws, alpha_old, info->sel_small);
       }
-      hipLaunchKernelGGL(tam_k_sel_labels, dim3(info->total_slices), dim3(TAM_WG), 0, s, d_tensors,
-                         info->n_tensors, alpha_new, ratios, sel, ws, alpha_old);
       break;
     case 4:
       hipLaunchKernelGGL(tam_k4_ef, dim3(grid_of(TAM_KS_K4_EF, (const void*)tam_k4_ef)), dim3(TAM_WG), 0, s, d_tensors,
@@ -3209,7 +3487,7 @@ int tam_costate_decode(const uint8_t* labels, const uint8_t* signs, const float*
   return TAM_OK;
 }
 
-static uint64_t tam_decompose_layout(uint64_t n, uint64_t* off_part, uint64_t* off_chunks, uint64_t* off_alpha) {
+static uint64_t tam_decompose_layout(uint64_t n, uint64_t* off_part, uint64_t* off_chunks, uint64_t* off_sel) {
   const uint64_t nt = tam_tiles_of(n);
   const uint32_t nch = tam_alpha_chunks(TAM_FLAG_COSTATE, (uint32_t)nt);
   uint64_t off = tam_align_up(sizeof(TamTensor), 256);
@@ -3217,8 +3495,8 @@ static uint64_t tam_decompose_layout(uint64_t n, uint64_t* off_part, uint64_t* o
   off = tam_align_up(off + nt * 4u * sizeof(double2), 256);
   *off_chunks = off;
   off = tam_align_up(off + (uint64_t)nch * sizeof(double2), 256);
-  *off_alpha = off;
-  return tam_align_up(off + sizeof(float), 256);
+  *off_sel = off;
+  return tam_align_up(off + 3u * sizeof(TamSel), 256);
 }
 
 size_t tam_decompose_workspace(uint64_t n) {
@@ -3232,8 +3510,8 @@ int tam_decompose(const float* m, const float* g, uint64_t n, float* alpha, floa
   if (!m || !g || !alpha || !delta || !workspace) return tam_fail(TAM_E_INVALID, "%snull argument", "");
   if (n == 0 || (n + TAM_BLOCK_SIZE - 1) / TAM_BLOCK_SIZE > (1ull << 31))
     return tam_fail(TAM_E_INVALID, "%selement count out of range", "");
-  uint64_t off_part, off_chunks, off_alpha;
-  const uint64_t need = tam_decompose_layout(n, &off_part, &off_chunks, &off_alpha);
+  uint64_t off_part, off_chunks, off_sel;
+  const uint64_t need = tam_decompose_layout(n, &off_part, &off_chunks, &off_sel);
   if (ws_bytes < need) return tam_fail(TAM_E_WORKSPACE, "%sworkspace too small: need %ld bytes", "", (long)need);
   hipStream_t s = (hipStream_t)stream;
   char* ws = (char*)workspace;
@@ -3244,11 +3522,14 @@ int tam_decompose(const float* m, const float* g, uint64_t n, float* alpha, floa
   TAM_HIP_CHECK(hipGetLastError());
   hipLaunchKernelGGL(tam_k_dot_quarters, dim3(nt), dim3(TAM_WG), 0, s, m, g, n, (double2*)(ws + off_part));
   TAM_HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(tam_k_alpha_chunks, dim3(tam_alpha_chunks(TAM_FLAG_COSTATE, nt)), dim3(TAM_WG), 0, s, desc, 1,
-                     (const double2*)(ws + off_part), (double2*)(ws + off_chunks));
+  const uint32_t chunks = tam_alpha_chunks(TAM_FLAG_COSTATE, nt);
+  hipLaunchKernelGGL(tam_k_alpha_chunks, dim3(chunks), dim3(TAM_WG), 0, s, desc, 1, (const double2*)(ws + off_part),
+                     (double2*)(ws + off_chunks), alpha, (TamSel*)(ws + off_sel));
   TAM_HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(tam_k_alpha, dim3(1), dim3(TAM_WG), 0, s, desc, (const double2*)(ws + off_chunks), alpha);
-  TAM_HIP_CHECK(hipGetLastError());
+  if (chunks > 1) {
+    hipLaunchKernelGGL(tam_k_alpha, dim3(1), dim3(TAM_WG), 0, s, desc, (const double2*)(ws + off_chunks), alpha);
+    TAM_HIP_CHECK(hipGetLastError());
+  }
   hipLaunchKernelGGL(tam_k_delta, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, m, g, n, alpha, delta);
   TAM_HIP_CHECK(hipGetLastError());
   return TAM_OK;
@@ -3266,9 +3547,9 @@ int tam_block_ratios(const float* delta, const float* m, uint64_t n, float* rati
 static uint64_t tam_thresholds_layout(uint64_t* off_sel, uint64_t* off_hist) {
   uint64_t off = tam_align_up(sizeof(TamTensor), 256);
   *off_sel = off;
-  off = tam_align_up(off + sizeof(TamSel), 256);
+  off = tam_align_up(off + 3u * sizeof(TamSel), 256);
   *off_hist = off;
-  return tam_align_up(off + 4096u * sizeof(uint32_t), 256);
+  return tam_align_up(off + TAM_SEL_HIST_WORDS * sizeof(uint32_t), 256);
 }
 
 size_t tam_thresholds_workspace(uint64_t nb) {
@@ -3288,24 +3569,29 @@ int tam_thresholds(const float* ratios, uint64_t nb, uint32_t k_lo, uint32_t k_h
   const uint64_t need = tam_thresholds_layout(&off_sel, &off_hist);
   if (ws_bytes < need) return tam_fail(TAM_E_WORKSPACE, "%sworkspace too small: need %ld bytes", "", (long)need);
   hipStream_t s = (hipStream_t)stream;
+  if (nb <= TAM_SEL_SMALL) {
+    hipLaunchKernelGGL(tam_k_taus_small, dim3(1), dim3(TAM_SEL_WG), 0, s, ratios, (uint32_t)nb, k_lo, k_hi, taus);
+    TAM_HIP_CHECK(hipGetLastError());
+    return TAM_OK;
+  }
   char* ws = (char*)workspace;
   TamTensor* desc = (TamTensor*)ws;
   TamSel* sel = (TamSel*)(ws + off_sel);
-  uint32_t* hist = (uint32_t*)(ws + off_hist);
-  const uint32_t slices = tam_sel_slices(TAM_FLAG_COSTATE, (uint32_t)nb);
+  double2* hist = (double2*)(ws + off_hist);  // stands for the tensor's partials
+  const uint32_t slices = tam_sel_slices(TAM_FLAG_COSTATE, (uint32_t)nb, TAM_SEL_SMALL);
   hipLaunchKernelGGL(tam_k_make_desc, dim3(1), dim3(1), 0, s, desc, nb * TAM_BLOCK_SIZE, (uint32_t)nb, k_lo, k_hi);
   TAM_HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(tam_k_sel_reset, dim3(1), dim3(TAM_WG), 0, s, desc, sel, hist);
+  hipLaunchKernelGGL(tam_k_sel_reset, dim3(1), dim3(1), 0, s, desc, sel);
   TAM_HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(tam_k_sel_minmax, dim3(slices), dim3(TAM_WG), 0, s, desc, 1, ratios, sel);
+  hipLaunchKernelGGL(tam_k_sel_minmax, dim3(slices), dim3(TAM_SEL_WG), 0, s, desc, 1, ratios, sel, hist,
+                     TAM_SEL_SMALL);
   TAM_HIP_CHECK(hipGetLastError());
   for (int r = 0; r < 3; ++r) {
-    hipLaunchKernelGGL(tam_k_sel_hist, dim3(slices), dim3(TAM_WG), 0, s, desc, 1, ratios, sel, hist);
-    TAM_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(tam_k_sel_pick, dim3(1), dim3(TAM_WG), 0, s, desc, sel, hist);
+    hipLaunchKernelGGL(tam_k_sel_hist, dim3(slices), dim3(TAM_SEL_WG), 0, s, desc, 1, ratios, sel, hist, r,
+                       TAM_SEL_SMALL);
     TAM_HIP_CHECK(hipGetLastError());
   }
-  hipLaunchKernelGGL(tam_k_sel_taus, dim3(1), dim3(1), 0, s, sel, taus);
+  hipLaunchKernelGGL(tam_k_sel_taus, dim3(1), dim3(TAM_SEL_WG), 0, s, sel, (const uint32_t*)hist, taus);
   TAM_HIP_CHECK(hipGetLastError());
   return TAM_OK;
 }
