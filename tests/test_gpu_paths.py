@@ -54,3 +54,24 @@ def test_alpha_at_the_chunk_sizes(n):
     alpha, delta = C.decompose(_t(m), _t(g))
     assert np.float32(alpha.item()) == np.float32(alpha_o)
     assert np.array_equal(delta.cpu().numpy().view(np.uint32), delta_o.view(np.uint32))
+
+
+# a tensor's last tile may hold quarters past its end, whose partial sums no kernel writes
+@pytest.mark.parametrize("dt", [O.DT_F32, O.DT_BF16])
+def test_step_reads_no_workspace_it_did_not_write(dt, monkeypatch):
+    from tests.helpers import run_side_by_side
+    from turboadam_amd import optimizer
+
+    sizes = [1024 * 5, 1024 * 9, 4096 + 77, 512 * 9, 512 * 11 + 3, 2048 * 3, 128 * 33, 700]
+    log(f"step on a workspace of NaN bytes, dtype {dt}")
+    plain = optimizer._DeviceBuffers.workspace
+
+    def poisoned(self, nbytes):
+        ws = plain(self, nbytes)
+        ws.fill_(255)
+        return ws
+
+    monkeypatch.setattr(optimizer._DeviceBuffers, "workspace", poisoned)
+    for ef in (False, True):
+        bad = run_side_by_side(sizes, [dt] * len(sizes), steps=3, error_feedback=ef)
+        assert not bad, "\n".join(bad[:10])

@@ -1816,16 +1816,23 @@ __global__ __launch_bounds__(TAM_WG) void tam_k_alpha_chunks(const TamTensor* __
       tam_wave_first(nT, [&](int i) { return T[i].chunk0 + tam_alpha_chunks(T[i].flags, T[i].ntiles) > c; });
   const TamTensor& d = T[ti];
   const uint32_t base = (c - d.chunk0) * TAM_CHUNK;
-  const uint32_t left = d.ntiles * 4u - base;  // partials from here on (chunks start inside the tensor's
-  const uint32_t count = d.ntiles * 4u > base ? (left < TAM_CHUNK ? left : TAM_CHUNK) : 0u;  // padded array)
+  // partials from here on (a chunk of the padded array may start past the
+  // tensor's quarters; no kernel writes the slots past its last quarter)
+  const uint32_t nq = (d.nb + 3u) / 4u;
+  const uint32_t count = nq > base ? nq - base : 0u;
   const double2* x = partials + (uint64_t)d.tile0 * 4u + base;
   const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
   double2 s[8];
 #pragma unroll
   for (uint32_t j = 0; j < 8u; ++j) {
-    const uint32_t k = TAM_ALPHA_STRIDE * j + 4u * t;  // count is a multiple of 4
-    s[j] = make_double2(0.0, 0.0);
-    if (k < count) s[j] = tam_add2(tam_add2(x[k], x[k + 1u]), tam_add2(x[k + 2u], x[k + 3u]));
+    const uint32_t k = TAM_ALPHA_STRIDE * j + 4u * t;
+    double2 y[4];
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; ++i) {
+      y[i] = make_double2(0.0, 0.0);
+      if (k + i < count) y[i] = x[k + i];
+    }
+    s[j] = tam_add2(tam_add2(y[0], y[1]), tam_add2(y[2], y[3]));
   }
   // lanes l and l ^ 1, l ^ 2, l ^ 4: each keeps half of its values of j
 #pragma unroll
