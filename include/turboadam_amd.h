@@ -277,6 +277,16 @@ int tam_fused_v_update(const uint8_t* idx_in, const uint16_t* scales_in, const v
 int tam_v_quantize(const float* v, uint64_t n_padded, uint32_t v_bits, int stochastic, uint32_t tensor_id,
                    uint32_t step, uint64_t seed, uint8_t* idx, uint16_t* scales, void* stream);
 
+/* compress_v_logscale (reference oneq.py:13-48) of v (n elements): the whole
+ * blocks as tam_v_quantize, and a last partial block filled up with
+ * max(min(v), 1e-38) (NaN when v holds one), formed on the device.  idx
+ * receives ceil(n/128)*128 indices.  Workspace: tam_v_compress_workspace(n)
+ * bytes of device memory (not used when n is a multiple of 128). */
+size_t tam_v_compress_workspace(uint64_t n);
+int tam_v_compress(const float* v, uint64_t n, uint32_t v_bits, int stochastic, uint32_t tensor_id,
+                   uint32_t step, uint64_t seed, uint8_t* idx, uint16_t* scales, void* workspace,
+                   size_t ws_bytes, void* stream);
+
 /* Self-check of the device arithmetic: out[i] = f(in[i]) with f selected by
  * `fn` (0 log, 1 exp, 2 f32->f16->f32, 3 f32->bf16->f32 in software, 4 sqrt,
  * 5 f32->bf16->f32 by the hardware conversion; the raw hardware instructions

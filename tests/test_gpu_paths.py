@@ -56,6 +56,120 @@ def test_alpha_at_the_chunk_sizes(n):
     assert np.array_equal(delta.cpu().numpy().view(np.uint32), delta_o.view(np.uint32))
 
 
+def _np(t):
+    t = t.detach().cpu()
+    return t.view(torch.int16).numpy().view(np.uint16) if t.dtype == torch.float16 else t.numpy()
+
+
+def _values(n, seed):
+    """A positive v with what the certified index must hand to the exact path:
+    values on a block's index boundaries, zeros, negatives, NaN and infinities."""
+    rng = np.random.default_rng(seed)
+    v = np.exp(rng.uniform(-30, -12, n)).astype(np.float32)
+    nb = n // 128
+    for b in range(0, nb, 3):  # log-equidistant: every index boundary of 16 levels is hit
+        v[128 * b:128 * (b + 1)] = np.exp(np.linspace(-20, -12, 129)[:128]).astype(np.float32)
+        v[128 * b + 127] = np.float32(np.exp(-12.0))
+    for b in range(1, nb, 5):
+        v[128 * b + 3] = 0.0
+    if nb > 6:
+        v[128 * 2 + 7] = -1.0
+        v[128 * 4 + 9] = np.nan
+        v[128 * 5 + 1] = np.inf
+        v[128 * 6:128 * 7] = np.float32(0.25)  # no span
+    return v
+
+
+# a unit is 8 blocks (1024 elements) of one wave
+@pytest.mark.parametrize("stochastic", [False, True])
+@pytest.mark.parametrize("bits", [2, 3, 4, 6, 8])
+@pytest.mark.parametrize("n", [128, 128 * 7, 1024, 1024 * 4 + 128, 1024 * 40])
+def test_quantize_units(n, bits, stochastic):
+    from turboadam_amd import quantize as Q
+
+    log(f"quantize n={n} bits={bits} stochastic={stochastic}")
+    v = _values(n, n + bits)
+    idx_o, sc_o = np.empty(n, np.uint8), np.empty(n // 64, np.uint16)
+    O.lib().or_quantize_logscale(O.ptr(v), n, bits, int(stochastic), 3, 4, 99, O.ptr(idx_o), O.ptr(sc_o))
+    idx, sc, _ = Q.quantize_logscale_nbits(_t(v), bits, stochastic_round=stochastic, tensor_id=3, step=4, seed=99)
+    assert np.array_equal(_np(idx), idx_o)
+    nan = np.isnan(sc_o.view(np.float16))
+    got = _np(sc).reshape(-1)
+    assert np.array_equal(np.isnan(got.view(np.float16)), nan) and np.array_equal(got[~nan], sc_o[~nan])
+    # a view that is aligned to its elements only
+    base = torch.zeros(n + 1, device=DEV)
+    base[1:] = _t(v)
+    idx2, _, _ = Q.quantize_logscale_nbits(base[1:], bits, stochastic_round=stochastic, tensor_id=3, step=4, seed=99)
+    assert torch.equal(idx, idx2)
+
+
+@pytest.mark.parametrize("stochastic", [False, True])
+@pytest.mark.parametrize("what", ["plain", "zero", "nan"])
+@pytest.mark.parametrize("n", [1, 64, 127, 129, 1024 + 5, 128 * 33 + 90])
+def test_compress_partial_block(n, what, stochastic):
+    """The last block's missing elements take max(min(v), 1e-38) of the whole
+    tensor, NaN when it holds one."""
+    from turboadam_amd import oneq
+
+    log(f"compress n={n} {what} stochastic={stochastic}")
+    v = np.exp(np.random.default_rng(n).uniform(-30, -12, n)).astype(np.float32)
+    if what != "plain":
+        v[n // 3] = 0.0 if what == "zero" else np.nan
+    nb = (n + 127) // 128
+    pad = np.full(nb * 128, np.nan if what == "nan" else max(v.min(), np.float32(1e-38)), np.float32)
+    pad[:n] = v
+    idx_o, sc_o = np.empty(nb * 128, np.uint8), np.empty(nb * 2, np.uint16)
+    O.lib().or_quantize_logscale(O.ptr(pad), nb * 128, 4, int(stochastic), 0, 1, 7, O.ptr(idx_o), O.ptr(sc_o))
+    c = oneq.compress_v_logscale(_t(v), 4, stochastic_round=stochastic, seed=7)
+    assert np.array_equal(_np(c["indices"]), idx_o)
+    nan = np.isnan(sc_o.view(np.float16))
+    got = _np(c["scales"]).reshape(-1)
+    assert np.array_equal(np.isnan(got.view(np.float16)), nan) and np.array_equal(got[~nan], sc_o[~nan])
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, 6, 8])
+@pytest.mark.parametrize("n", [1, 128, 1023, 1024, 1025, 1024 * 5 + 77])
+def test_dequantize_units(n, bits):
+    from turboadam_amd import quantize as Q
+
+    log(f"dequantize n={n} bits={bits}")
+    rng = np.random.default_rng(n + bits)
+    nb = (n + 127) // 128
+    lo = rng.uniform(-60, 10, nb).astype(np.float32)
+    sc = np.stack([lo, lo + rng.uniform(0, 9, nb).astype(np.float32)], 1).astype(np.float16)
+    for top in (1 << bits, 256):  # in range, and beyond it (decoded by the same formula)
+        idx = rng.integers(0, top, nb * 128).astype(np.uint8)
+        want = O.dequantize(idx, sc.view(np.uint16).reshape(-1), n, bits)
+        got = Q.dequantize_logscale_nbits(_t(idx), _t(sc), bits, original_numel=n)
+        assert np.array_equal(_np(got).view(np.uint32), want.view(np.uint32)), top
+        base = torch.zeros(nb * 128 + 1, dtype=torch.uint8, device=DEV)
+        base[1:] = _t(idx)
+        assert torch.equal(Q.dequantize_logscale_nbits(base[1:], _t(sc), bits, original_numel=n), got)
+
+
+@pytest.mark.parametrize("bits,dt", [(4, torch.float32), (2, torch.bfloat16), (8, torch.float16), (6, torch.bfloat16)])
+@pytest.mark.parametrize("n", [1, 513, 1024, 1025, 1024 * 4 + 640])
+def test_fused_v_units(n, bits, dt):
+    from turboadam_amd import quantize as Q
+
+    log(f"fused_v_update n={n} bits={bits} {dt}")
+    rng = np.random.default_rng(n + bits)
+    nb = (n + 127) // 128
+    idx = rng.integers(0, 1 << bits, nb * 128).astype(np.uint8)
+    lo = rng.uniform(-25, -15, nb).astype(np.float32)
+    sc = np.stack([lo, lo + rng.uniform(0, 6, nb).astype(np.float32)], 1).astype(np.float16).view(np.uint16)
+    base = torch.zeros(n + 1, dtype=dt)  # the gradient is a view one element into it
+    base[1:] = (torch.from_numpy(rng.standard_normal(n).astype(np.float32)) * 1e-3).to(dt)
+    g32 = base[1:].float().numpy().copy()
+    idx_o, sc_o, v_o = idx.copy(), sc.reshape(-1).copy(), np.empty(n, np.float32)
+    O.lib().or_fused_v_update(O.ptr(idx_o), O.ptr(sc_o), O.ptr(g32), n, bits, O.f32(0.999), O.f32(1.0 - 0.999),
+                              5, 9, 1234, O.ptr(v_o))
+    ni, ns, v = Q.fused_v_update(_t(idx), _t(sc.view(np.float16)), base.to(DEV)[1:], 0.999, bits, tensor_id=5, step=9,
+                                 seed=1234)
+    assert np.array_equal(_np(ni), idx_o) and np.array_equal(_np(ns).reshape(-1), sc_o)
+    assert np.array_equal(_np(v).view(np.uint32), v_o.view(np.uint32))
+
+
 # a tensor's last tile may hold quarters past its end, whose partial sums no kernel writes
 @pytest.mark.parametrize("dt", [O.DT_F32, O.DT_BF16])
 def test_step_reads_no_workspace_it_did_not_write(dt, monkeypatch):

@@ -160,6 +160,12 @@ SIGNATURES = {
         [_VP, ctypes.c_uint64, ctypes.c_uint32, ctypes.c_int, ctypes.c_uint32, ctypes.c_uint32, ctypes.c_uint64, _VP,
          _VP, _VP],
     ),
+    "tam_v_compress_workspace": (ctypes.c_size_t, [ctypes.c_uint64]),
+    "tam_v_compress": (
+        ctypes.c_int,
+        [_VP, ctypes.c_uint64, ctypes.c_uint32, ctypes.c_int, ctypes.c_uint32, ctypes.c_uint32, ctypes.c_uint64, _VP,
+         _VP, _VP, ctypes.c_size_t, _VP],
+    ),
 }
 
 _lib = None

@@ -122,6 +122,38 @@ __device__ __forceinline__ void tam_unpack8(TamW4 w, float* out) {
   }
 }
 
+// The same vectors at element alignment: gfx950 loads and stores global memory at
+// any address, so one instruction moves 16 bytes of a caller's array that is
+// only aligned to its elements.
+typedef float TamF4E __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t TamW4E __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t TamW4B __attribute__((ext_vector_type(4), aligned(1)));
+typedef uint32_t TamW2B __attribute__((ext_vector_type(2), aligned(1)));
+typedef uint32_t TamW1B __attribute__((aligned(1)));
+
+// 16 consecutive elements of an array of dtype DT as fp32 (all exist).
+template <uint32_t DT>
+__device__ __forceinline__ void tam_ld16(const void* base, uint64_t e0, float* out) {
+  if constexpr (DT == TAM_DTYPE_F32) {
+    const TAM_GLOBAL TamF4E* b = tam_g((const TamF4E*)((const float*)base + e0));
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const TamF4 x = b[k];
+      out[4 * k] = x.x; out[4 * k + 1] = x.y; out[4 * k + 2] = x.z; out[4 * k + 3] = x.w;
+    }
+  } else {
+    const TAM_GLOBAL TamW4E* b = tam_g((const TamW4E*)((const uint16_t*)base + e0));
+    const TamW4 x = b[0], y = b[1];
+    tam_unpack8<DT>(x, out);
+    tam_unpack8<DT>(y, out + 8);
+  }
+}
+__device__ __forceinline__ void tam_st16_f32(float* base, uint64_t e0, const float* v) {
+  TAM_GLOBAL TamF4E* b = tam_g((TamF4E*)(base + e0));
+#pragma unroll
+  for (int k = 0; k < 4; ++k) b[k] = TamF4{v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]};
+}
+
 // Elements [e0, e0+8) of a parameter or gradient.  FULL: all 8 exist and the
 // array is 16-byte aligned; otherwise only the first nv exist (the rest read 0).
 template <uint32_t DT, bool FULL>
@@ -1327,44 +1359,59 @@ __device__ __forceinline__ TamVExt tam_vunit_a(const TamTensor& d, uint32_t lane
   return x;
 }
 
-// Logs of the block extremes, scales, certified stochastic re-quantisation of
-// a lane's 16 elements; as tam_vpath_b for a full quarter (same bound, same
-// fast path, same exact fallback).  Every v of a block that passes the block
-// test lies in [vmin, vmax] with vmin >= 2^-126, where the clamp to 1e-38
-// (quantize.py:275) leaves it unchanged, so the fast path reads v itself; the
-// exact path clamps.
-__device__ __forceinline__ void tam_vunit_b(const TamTensor& d, uint32_t lane, uint32_t b, uint64_t e0,
-                                            const float* v, TamVExt x, const TamLdsTabs* tabs, uint32_t seed_lo,
-                                            uint32_t seed_hi) {
-  const float fnb = (float)(1u << d.v_bits);
+// Logs of a block's extremes, its scales (stored by the first lane of each block
+// when `store`), and the constants of the certified index c~ = K log2(v rmin):
+// |c~ - c| <= Bb on a block with ok (the bound of tam_vpath_b, full blocks).
+struct TamVBlk {
+  float lmn, lmx, sp, K, rmin, Bb;
+  bool ok;
+};
+__device__ __forceinline__ TamVBlk tam_vunit_blk(uint32_t v_bits, uint16_t* v_scales, uint32_t lane, uint32_t b,
+                                                 TamVExt x, const TamLdsTabs* tabs, bool store) {
+  const float fnb = (float)(1u << v_bits);
   const uint32_t l8 = lane & 7u;
   const uint32_t kmn = __builtin_elementwise_max(x.kmn, TAM_BITS_1EM38);
   const uint32_t kmx = __builtin_elementwise_max(x.kmx, TAM_BITS_1EM38);
   const bool nan_seen = (x.nan_seen & TAM_VEXT_NAN) != 0u;
+  TamVBlk r;
   // correctly rounded logs of the extremes: even lanes log(vmin), odd lanes log(vmax)
   const float lx = tam_logf_lds(tam_u2f((l8 & 1u) ? kmx : kmn), tabs);
   const float ly = tam_dppf<TAM_DPP_XOR1>(lx);
-  float lmn = (l8 & 1u) ? ly : lx;
-  float lmx = (l8 & 1u) ? lx : ly;
-  if (nan_seen) lmn = lmx = tam_qnan();  // torch.min / torch.max propagate NaN
-  float sp = lmx - lmn;  // quantize.py:283
-  sp = sp < 1e-10f ? 1e-10f : sp;
-  if (l8 == 0u)
-    tam_g((uint32_t*)d.v_scales)[b] = (uint32_t)tam_f32_to_f16(lmn) | ((uint32_t)tam_f32_to_f16(lmx) << 16);
-  const float rsp = __builtin_amdgcn_rcpf(sp);
-  const float K = (0x1.62e430p-1f * fnb) * rsp;
-  // the block bound of tam_vpath_b (full blocks)
-  const float rmin = __builtin_amdgcn_rcpf(tam_u2f(kmn));
-  const float Lm = __builtin_fmaxf(__builtin_fabsf(lmn), __builtin_fabsf(lmx));
-  const float per_sp = __builtin_fmaf(Lm + __builtin_fabsf(lmn), 0x1p-24f, 0x1p-22f);
+  r.lmn = (l8 & 1u) ? ly : lx;
+  r.lmx = (l8 & 1u) ? lx : ly;
+  if (nan_seen) r.lmn = r.lmx = tam_qnan();  // torch.min / torch.max propagate NaN
+  r.sp = r.lmx - r.lmn;  // quantize.py:283
+  r.sp = r.sp < 1e-10f ? 1e-10f : r.sp;
+  if (l8 == 0u && store)
+    tam_g((uint32_t*)v_scales)[b] = (uint32_t)tam_f32_to_f16(r.lmn) | ((uint32_t)tam_f32_to_f16(r.lmx) << 16);
+  const float rsp = __builtin_amdgcn_rcpf(r.sp);
+  r.K = (0x1.62e430p-1f * fnb) * rsp;
+  r.rmin = __builtin_amdgcn_rcpf(tam_u2f(kmn));
+  const float Lm = __builtin_fmaxf(__builtin_fabsf(r.lmn), __builtin_fabsf(r.lmx));
+  const float per_sp = __builtin_fmaf(Lm + __builtin_fabsf(r.lmn), 0x1p-24f, 0x1p-22f);
   const float flat = __builtin_fmaf(fnb, 0x1p-21f + 0x1p-20f, (fnb + 2.0f) * 0x1p-21f);
-  const float Bb = __builtin_fmaf(fnb * rsp, per_sp, flat) * (1.0f + 0x1p-16f);
-  const bool blk_ok = (tam_u2f(kmn) >= 0x1p-126f) && (tam_u2f(kmx) < 0x1p100f) && !nan_seen && (sp <= 64.0f) &&
-                      (Bb < 0.25f);
+  r.Bb = __builtin_fmaf(fnb * rsp, per_sp, flat) * (1.0f + 0x1p-16f);
+  r.ok = (tam_u2f(kmn) >= 0x1p-126f) && (tam_u2f(kmx) < 0x1p100f) && !nan_seen && (r.sp <= 64.0f) && (r.Bb < 0.25f);
+  return r;
+}
+
+// Scales and certified stochastic re-quantisation of a lane's 16 elements; as
+// tam_vpath_b for a full quarter (same bound, same fast path, same exact
+// fallback).  Every v of a block that passes the block test lies in
+// [vmin, vmax] with vmin >= 2^-126, where the clamp to 1e-38 (quantize.py:275)
+// leaves it unchanged, so the fast path reads v itself; the exact path clamps.
+// W8: type of the 8-byte index stores (their alignment); with store false
+// (uniform over a block's lanes) nothing is written.
+template <typename W8 = TamW2>
+__device__ __forceinline__ void tam_vunit_b(const TamTensor& d, uint32_t lane, uint32_t b, uint64_t e0,
+                                            const float* v, TamVExt x, const TamLdsTabs* tabs, uint32_t seed_lo,
+                                            uint32_t seed_hi, bool store = true) {
+  const TamVBlk q_ = tam_vunit_blk(d.v_bits, d.v_scales, lane, b, x, tabs, store);
+  const float fnb = (float)(1u << d.v_bits), lmn = q_.lmn, sp = q_.sp, K = q_.K, rmin = q_.rmin;
   // The fast path subtracts u' = hi 2^-16 + 2^-17 from c~ + 1, hi the high 16
   // bits of the draw: |u - u'| <= 2^-17.  The quarter path's bound plus 2^-17
   // covers that, plus 2^-21 the rounding of the larger c~ + 1.
-  const float H = blk_ok ? 0.5f - (Bb + (0x1p-17f + 0x1p-21f)) : -1.0f;
+  const float H = q_.ok ? 0.5f - (q_.Bb + (0x1p-17f + 0x1p-21f)) : -1.0f;
   const uint32_t byte_lsb = d.v_bits < 8u ? 0x01010101u : 0u;  // uniform
   const uint32_t m16 = tam_vconst(0x7fff80u), one = tam_vconst(0x3f800040u);  // 1 + 2^-17
   // the lane's 16 elements are one group of draws (tam_draws8): half h of 8
@@ -1428,7 +1475,7 @@ __device__ __forceinline__ void tam_vunit_b(const TamTensor& d, uint32_t lane, u
         }
       }
     }
-    tam_g((TamW2*)(d.v_idx + e0 + TAM_EPL * h))[0] = TamW2{ow[0], ow[1]};
+    if (store) tam_g((W8*)(d.v_idx + e0 + TAM_EPL * h))[0] = TamW2{ow[0], ow[1]};
   }
 }
 
@@ -2893,124 +2940,323 @@ __global__ __launch_bounds__(TAM_SEL_WG) void tam_k_sel_taus(const TamSel* __res
   }
 }
 
-// fused_v_update (quantize.py:222-299) for one tensor: the 1Q half of pass 1
+// fused_v_update (quantize.py:222-299) for one tensor: the 1Q half of pass 0
 // without the first moment and the parameter update; v (fp32, n values) is
-// written out.  idx_out / scales_out may equal idx_in / scales_in.
-__global__ __launch_bounds__(TAM_WG) void tam_k_fused_v(const uint8_t* idx_in, const uint16_t* scales_in,
-                                                        const void* __restrict__ g, uint32_t g_dtype, uint64_t n,
-                                                        uint32_t bits, float beta2, float one_minus_beta2,
-                                                        uint32_t tensor_id, uint32_t step, uint32_t seed_lo,
-                                                        uint32_t seed_hi, uint8_t* idx_out, uint16_t* scales_out,
-                                                        float* __restrict__ v_out) {
-  __shared__ float lut[TAM_WG / 64][4 * 64];
+// written out.  idx_out / scales_out may equal idx_in / scales_in.  Bound by
+// memory (a 16-bit gradient, the indices in and out and fp32 v: 8 bytes per
+// element): each wave takes whole units (1024 elements) with 16-byte loads and
+// stores and pass 0's certified arithmetic, and the last partial unit by
+// bounds-checked quarters.  Quarters alone, loaded element by element, took
+// 64 us for 2^24 bf16 elements.
+template <uint32_t DT>
+__global__ __launch_bounds__(TAM_WG) __attribute__((amdgpu_waves_per_eu(4, 4))) void tam_k_fused_v(
+    const uint8_t* idx_in, const uint16_t* scales_in, const void* __restrict__ g, uint64_t n, uint32_t bits,
+    float beta2, float one_minus_beta2, uint32_t tensor_id, uint32_t step, uint32_t seed_lo, uint32_t seed_hi,
+    uint8_t* idx_out, uint16_t* scales_out, float* __restrict__ v_out) {
+  __shared__ __attribute__((aligned(256))) float lut[TAM_WG / 64][8 * 64];
   __shared__ TamLdsTabs tabs;
   tam_lds_tabs_fill(&tabs);
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
   TamTensor d = tam_local_desc(n);
-  d.v_idx = (uint8_t*)idx_in;
-  d.v_scales = (uint16_t*)scales_in;
   d.v_bits = bits;
   d.beta2 = beta2;
   d.one_minus_beta2 = one_minus_beta2;
   d.tensor_id = tensor_id;
   d.step = step;
-  const TamWave W = tam_wave(d, blockIdx.x * 4u + wave, lane, false);
-  float gv[TAM_EPL], v[TAM_EPL], vc[TAM_EPL];
-  switch (g_dtype) {
-    case TAM_DTYPE_BF16: tam_ld8<TAM_DTYPE_BF16, false>(g, W.e0, W.nv, gv); break;
-    case TAM_DTYPE_F16: tam_ld8<TAM_DTYPE_F16, false>(g, W.e0, W.nv, gv); break;
-    default: tam_ld8<TAM_DTYPE_F32, false>(g, W.e0, W.nv, gv); break;
+  // work items: the full units, then the (at most two) quarters left
+  const uint32_t nfull = (uint32_t)(n / (8u * TAM_BLOCK_SIZE)), items = nfull + (d.nb + 3u) / 4u - 2u * nfull;
+  for (uint32_t w = blockIdx.x * (TAM_WG / 64) + wave; w < items; w += gridDim.x * (TAM_WG / 64)) {
+    if (w < nfull) {
+      const uint32_t b = w * 8u + (lane >> 3);
+      const uint64_t e0 = (uint64_t)b * TAM_BLOCK_SIZE + (lane & 7u) * TAM_EPU;
+      float gv[TAM_EPU], v[TAM_EPU];
+      uint32_t sc = tam_g((const uint32_t*)scales_in)[b];
+      TamW4 iw = tam_g((const TamW4B*)(idx_in + e0))[0];
+      tam_ld16<DT>(g, e0, gv);
+      tam_compiler_fence();
+      tam_pin(sc);
+      tam_pin(iw);
+      const TamVExt x = tam_vunit_a(d, lane, sc, iw, gv, v, lut[wave], &tabs);
+      tam_st16_f32(v_out, e0, v);
+      d.v_idx = idx_out;
+      d.v_scales = scales_out;
+      tam_vunit_b(d, lane, b, e0, v, x, &tabs, seed_lo, seed_hi);
+    } else {
+      const TamWave W = tam_wave(d, 2u * nfull + (w - nfull), lane, false);
+      float gv[TAM_EPL], v[TAM_EPL], vc[TAM_EPL];
+      tam_ld8<DT, false>(g, W.e0, W.nv, gv);
+      d.v_idx = (uint8_t*)idx_in;
+      d.v_scales = (uint16_t*)scales_in;
+      const TamVIn vin = tam_v_load<false>(d, W);
+      const TamVExt x = tam_vpath_a<false>(d, W, vin, gv, v, vc, lut[wave], &tabs);
+      if (W.bvalid) tam_st8_f32<false>(v_out, W.e0, W.nv, v);
+      d.v_idx = idx_out;
+      d.v_scales = scales_out;
+      tam_vpath_b<false>(d, W, vc, x, &tabs, seed_lo, seed_hi);
+    }
   }
-  const TamVIn vin = tam_v_load<false>(d, W);
-  const TamVExt x = tam_vpath_a<false>(d, W, vin, gv, v, vc, lut[wave], &tabs);
-  if (W.bvalid) tam_st8_f32<false>(v_out, W.e0, W.nv, v);
-  d.v_idx = idx_out;
-  d.v_scales = scales_out;
-  tam_vpath_b<false>(d, W, vc, x, &tabs, seed_lo, seed_hi);
 }
 
-// quantize_logscale_nbits (quantize.py:126-180) of a padded positive tensor:
-// per-block fp16 (log_min, log_max) over all of the block's values, and
-// indices trunc(clamp(c, 0, 2^bits - 0.001)) (deterministic) or
-// floor(c) + (u < frac(c)) clamped (stochastic, Philox draws as in the step),
-// c = fl(fl(log v - log_min) / max(span, 1e-10)) * 2^bits.
-__global__ __launch_bounds__(TAM_WG) void tam_k_quantize(const float* __restrict__ v, uint64_t npad, uint32_t bits,
-                                                         int stochastic, uint32_t tensor_id, uint32_t step,
-                                                         uint32_t seed_lo, uint32_t seed_hi,
-                                                         uint8_t* __restrict__ idx, uint16_t* __restrict__ scales) {
-  __shared__ TamLdsTabs tabs;
-  tam_lds_tabs_fill(&tabs);
-  const TamTensor d = tam_local_desc(npad);
-  const TamWave W = tam_wave(d, blockIdx.x * 4u + (threadIdx.x >> 6), threadIdx.x & 63u, false);
-  const float fnb = (float)(1u << bits);
-  float x[TAM_EPL], l[TAM_EPL];
-  tam_ld8<TAM_DTYPE_F32, false>(v, W.e0, W.nv, x);
-  float lmn = tam_inf(), lmx = -tam_inf();
-  uint32_t nan_seen = 0;
+// The exact index of one value from its correctly rounded log l
+// (quantize.py:160-178): trunc(clamp(c, 0, 2^bits - 0.001)), or with a draw rw
+// floor(c) + (u < frac(c)) clamped, c = fl(fl(l - log_min) / span) * 2^bits.
+template <bool STO>
+__device__ __forceinline__ uint32_t tam_quantize_exact(float l, float lmn, float sp, float fnb, uint32_t rw) {
+  const float c = ((l - lmn) / sp) * fnb;
+  float q;
+  if (STO) {
+    const float f = __builtin_floorf(c);
+    const float u = (float)rw * 0x1p-24f;
+    q = f + (u < c - f ? 1.0f : 0.0f);
+    q = q < 0.0f ? 0.0f : q;
+    q = q > fnb - 1.0f ? fnb - 1.0f : q;
+  } else {
+    const float top = fnb - 0.001f;  // f32(2^bits - 0.001)
+    q = c < 0.0f ? 0.0f : c;
+    q = q > top ? top : q;
+  }
+  return tam_isnan(q) ? 0u : (uint32_t)q;
+}
+
+// The indices of a lane's 16 elements, rounded down.  As in the stochastic
+// re-quantisation, c~ = K log2(v rmin) lies within Bb < 1/4 of the exact path's
+// c on a block with q.ok; c lies in [0, F] (l is monotone in v), so any c~ below
+// 1/4 means index 0 and any above F - 1/4 index F - 1, and between them floor(c~)
+// is the index when c~ lies farther than Bb (plus 2^-21 for the test's own
+// roundings) from every integer.  A lane with a closer element takes the exact
+// path for those elements (correctly rounded log and division).
+__device__ __forceinline__ void tam_vunit_floor(uint32_t v_bits, uint64_t e0, const float* v, const TamVBlk& q,
+                                                const TamLdsTabs* tabs, uint8_t* idx, bool store) {
+  const float fnb = (float)(1u << v_bits);
+  const float H = q.ok ? 0.5f - (q.Bb + 0x1p-21f) : -1.0f;
+  const auto dev_of = [&](float x, float& f) {
+    const float t = __builtin_amdgcn_fmed3f(__builtin_amdgcn_logf(x * q.rmin) * q.K, 0.25f, fnb - 0.25f);
+    f = __builtin_floorf(t);
+    return __builtin_fabsf((t - f) - 0.5f);
+  };
+  uint32_t ow[4] = {0u, 0u, 0u, 0u};
+  float dev = 0.0f;
 #pragma unroll
-  for (int i = 0; i < TAM_EPL; ++i) {
-    const float c = x[i] < 1e-38f ? 1e-38f : x[i];  // clamp(min=1e-38), NaN stays
-    l[i] = tam_logf_lds(c, &tabs);
-    if ((uint32_t)i < W.nv) {
-      nan_seen |= tam_isnan(l[i]) ? 1u : 0u;
-      lmn = __builtin_fminf(lmn, l[i]);
-      lmx = __builtin_fmaxf(lmx, l[i]);
+  for (int i = 0; i < TAM_EPU; ++i) {
+    float f;
+    dev = __builtin_fmaxf(dev, dev_of(v[i], f));
+    ow[i >> 2] = __builtin_amdgcn_cvt_pk_u8_f32(f, i & 3, ow[i >> 2]);
+  }
+  if (!(dev < H)) {
+#pragma unroll
+    for (int i = 0; i < TAM_EPU; ++i) {
+      float f;
+      if (!(dev_of(v[i], f) < H)) {
+        const uint32_t qi = tam_quantize_exact<false>(tam_logf_lds(v[i], tabs), q.lmn, q.sp, fnb, 0u);
+        const uint32_t sh = 8u * (uint32_t)(i & 3);
+        ow[i >> 2] = (ow[i >> 2] & ~(0xffu << sh)) | (qi << sh);
+      }
     }
   }
+  if (store) tam_g((TamW4B*)(idx + e0))[0] = TamW4{ow[0], ow[1], ow[2], ow[3]};
+}
+
+// quantize_logscale_nbits (quantize.py:126-180) of nb blocks of v: per-block fp16
+// (log_min, log_max) over all of the block's values, and their indices
+// (tam_quantize_exact).  One unit (8 blocks, 16 elements per lane) per wave and
+// round, in pass 0's layout: two correctly rounded logs per block and the
+// certified index instead of a correctly rounded log per element (103 us for
+// 38.6M elements).  wgmin, if given, receives each workgroup's smallest clamped
+// v (bit pattern; 0 when one is a NaN), for the fill of a partial last block.
+template <bool STO>
+__global__ __launch_bounds__(TAM_WG) void tam_k_quantize(const float* __restrict__ v, uint32_t nb, uint32_t bits,
+                                                         uint32_t tensor_id, uint32_t step, uint32_t seed_lo,
+                                                         uint32_t seed_hi, uint8_t* __restrict__ idx,
+                                                         uint16_t* __restrict__ scales,
+                                                         uint32_t* __restrict__ wgmin) {
+  __shared__ TamLdsTabs tabs;
+  __shared__ uint32_t least[TAM_WG / 64];
+  tam_lds_tabs_fill(&tabs);
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+  const uint32_t units = (nb + 7u) / 8u;
+  TamTensor d = tam_local_desc((uint64_t)nb * TAM_BLOCK_SIZE);
+  d.v_bits = bits;
+  d.v_idx = idx;
+  d.v_scales = scales;
+  d.tensor_id = tensor_id;
+  d.step = step;
+  uint32_t mn = 0xffffffffu;
+  for (uint32_t u = blockIdx.x * (TAM_WG / 64) + wave; u < units; u += gridDim.x * (TAM_WG / 64)) {
+    const uint32_t b = u * 8u + (lane >> 3);
+    const uint64_t e0 = (uint64_t)b * TAM_BLOCK_SIZE + (lane & 7u) * TAM_EPU;
+    const bool ok = b < nb;  // uniform over a block's lanes
+    float x[TAM_EPU];
+    if (ok) {
+      tam_ld16<TAM_DTYPE_F32>(v, e0, x);
+    } else {
 #pragma unroll
-  for (int s = 0; s < 4; ++s) {  // block min / max over the 16 lanes (minNum / maxNum; NaN tracked apart)
-    const float a = s == 0 ? tam_dppf<TAM_DPP_XOR1>(lmn) : s == 1 ? tam_dppf<TAM_DPP_XOR2>(lmn)
-                  : s == 2 ? tam_dppf<TAM_DPP_HALF_MIRROR>(lmn) : tam_dppf<TAM_DPP_MIRROR>(lmn);
-    const float b = s == 0 ? tam_dppf<TAM_DPP_XOR1>(lmx) : s == 1 ? tam_dppf<TAM_DPP_XOR2>(lmx)
-                  : s == 2 ? tam_dppf<TAM_DPP_HALF_MIRROR>(lmx) : tam_dppf<TAM_DPP_MIRROR>(lmx);
-    lmn = __builtin_fminf(lmn, a);
-    lmx = __builtin_fmaxf(lmx, b);
+      for (int i = 0; i < TAM_EPU; ++i) x[i] = 1.0f;
+    }
+    uint32_t kmn = 0xffffffffu, kmx = 0u;
+#pragma unroll
+    for (int i = 0; i < TAM_EPU; ++i) {
+      x[i] = x[i] < 1e-38f ? 1e-38f : x[i];  // clamp(min=1e-38), NaN stays (its pattern lies above +inf's)
+      kmn = __builtin_elementwise_min(kmn, tam_f2u(x[i]));
+      kmx = __builtin_elementwise_max(kmx, tam_f2u(x[i]));
+    }
+    TamVExt e;
+    e.kmn = tam_half_umin(kmn);
+    e.kmx = tam_half_umax(kmx);
+    e.nan_seen = e.kmx > 0x7f800000u ? TAM_VEXT_NAN : 0u;
+    if (ok) mn = __builtin_elementwise_min(mn, e.nan_seen ? 0u : e.kmn);
+    if (STO) {
+      tam_vunit_b<TamW2B>(d, lane, b, e0, x, e, &tabs, seed_lo, seed_hi, ok);
+    } else {
+      const TamVBlk q = tam_vunit_blk(bits, scales, lane, b, e, &tabs, ok);
+      tam_vunit_floor(bits, e0, x, q, &tabs, idx, ok);
+    }
   }
-  nan_seen = tam_block_or(nan_seen);
-  if (nan_seen) lmn = lmx = tam_qnan();
-  if (!W.bvalid) return;
-  if (W.l16 == 0)
-    tam_g((uint32_t*)scales)[W.b] = (uint32_t)tam_f32_to_f16(lmn) | ((uint32_t)tam_f32_to_f16(lmx) << 16);
+  if (wgmin) {  // uniform
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) mn = __builtin_elementwise_min(mn, (uint32_t)__shfl_xor((int)mn, off));
+    if (lane == 0u) least[wave] = mn;
+    __syncthreads();
+    if (threadIdx.x == 0)
+      wgmin[blockIdx.x] = __builtin_elementwise_min(__builtin_elementwise_min(least[0], least[1]),
+                                                    __builtin_elementwise_min(least[2], least[3]));
+  }
+}
+
+// The last, partial block of compress_v_logscale (oneq.py:13-48): its missing
+// elements take max(min(v), 1e-38), the smallest clamped v of the whole tensor
+// (NaN when it holds a NaN), from the n_wg workgroup minima of the whole blocks
+// and the block's own elements.  One wave; lane l holds elements l and l + 64.
+__global__ __launch_bounds__(64) void tam_k_quantize_last(const float* __restrict__ v, uint64_t n,
+                                                          const uint32_t* __restrict__ wgmin, uint32_t n_wg,
+                                                          uint32_t bits, int stochastic, uint32_t tensor_id,
+                                                          uint32_t step, uint32_t seed_lo, uint32_t seed_hi,
+                                                          uint8_t* __restrict__ idx, uint16_t* __restrict__ scales) {
+  const uint32_t lane = threadIdx.x;
+  const uint64_t b = n / TAM_BLOCK_SIZE, first = b * TAM_BLOCK_SIZE;
+  const auto min_all = [](uint32_t k) {
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) k = __builtin_elementwise_min(k, (uint32_t)__shfl_xor((int)k, off));
+    return k;
+  };
+  uint32_t least = 0xffffffffu;
+  for (uint32_t i = lane; i < n_wg; i += 64u) least = __builtin_elementwise_min(least, wgmin[i]);
+  float x[2];
+  bool in[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const uint64_t e = first + lane + 64u * (uint32_t)j;
+    in[j] = e < n;
+    x[j] = in[j] ? v[e] : 0.0f;
+    x[j] = x[j] < 1e-38f ? 1e-38f : x[j];
+    if (in[j]) least = __builtin_elementwise_min(least, tam_isnan(x[j]) ? 0u : tam_f2u(x[j]));
+  }
+  least = min_all(least);
+  const float fill = least == 0u ? tam_qnan() : tam_u2f(least);
+  float l[2];
+  uint32_t kmn = 0xffffffffu, kmx = 0u;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    if (!in[j]) x[j] = fill;
+    kmn = __builtin_elementwise_min(kmn, tam_f2u(x[j]));
+    kmx = __builtin_elementwise_max(kmx, tam_f2u(x[j]));
+    l[j] = tam_logf(x[j]);
+  }
+  kmn = min_all(kmn);
+  kmx = ~min_all(~kmx);
+  // log is monotone: the logs of the extremes are the extremes of the logs
+  float lmn = tam_logf(tam_u2f(kmn)), lmx = tam_logf(tam_u2f(kmx));
+  if (kmx > 0x7f800000u) lmn = lmx = tam_qnan();
+  if (lane == 0u) ((uint32_t*)scales)[b] = (uint32_t)tam_f32_to_f16(lmn) | ((uint32_t)tam_f32_to_f16(lmx) << 16);
   float sp = lmx - lmn;
   sp = sp < 1e-10f ? 1e-10f : sp;
-  uint32_t rw[TAM_EPL] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
-  if (stochastic) {
-    tam_draws8(W.e0, tensor_id, step, seed_lo, seed_hi, rw);
-  }
-  const float top = fnb - 0.001f;  // f32(2^bits - 0.001)
+  const float fnb = (float)(1u << bits);
 #pragma unroll
-  for (int i = 0; i < TAM_EPL; ++i) {
-    const float c = ((l[i] - lmn) / sp) * fnb;
-    float q;
+  for (int j = 0; j < 2; ++j) {
+    const uint64_t e = first + lane + 64u * (uint32_t)j;
+    uint32_t qi;
     if (stochastic) {
-      const float f = __builtin_floorf(c);
-      const float u = (float)rw[i] * 0x1p-24f;
-      q = f + (u < c - f ? 1.0f : 0.0f);
-      q = q < 0.0f ? 0.0f : q;
-      q = q > fnb - 1.0f ? fnb - 1.0f : q;
+      uint32_t rw[TAM_EPL], mine = 0u;
+      tam_draws8(e & ~7ull, tensor_id, step, seed_lo, seed_hi, rw);
+#pragma unroll
+      for (uint32_t k = 0; k < TAM_EPL; ++k) mine = (e & 7u) == k ? rw[k] : mine;
+      qi = tam_quantize_exact<true>(l[j], lmn, sp, fnb, mine);
     } else {
-      q = c < 0.0f ? 0.0f : c;
-      q = q > top ? top : q;
+      qi = tam_quantize_exact<false>(l[j], lmn, sp, fnb, 0u);
     }
-    if ((uint32_t)i < W.nv) idx[W.e0 + i] = tam_isnan(q) ? (uint8_t)0 : (uint8_t)(uint32_t)q;
+    idx[e] = (uint8_t)qi;
+  }
+}
+
+// Decode of 1Q indices (quantize.py:183-214).  A unit (8 blocks) per wave and
+// round: the 2^bits values of each block once (correctly rounded exps, in LDS,
+// by the 8 lanes whose share of the unit the block is), then four passes of 4
+// consecutive elements per lane, so that every store instruction writes 1 KB in
+// a row.  8-bit indices (more levels than a block has elements), indices out of
+// range and the last partial unit evaluate per element.  One exp per element,
+// one element per thread, took 117 us for 38.6M elements.
+__global__ __launch_bounds__(TAM_WG) void tam_k_v_dequantize(const uint8_t* __restrict__ idx,
+                                                             const uint16_t* __restrict__ scales, uint64_t n,
+                                                             uint32_t bits, float* __restrict__ out) {
+  __shared__ float lut[TAM_WG / 64][8 * 64];
+  __shared__ TamLdsTabs tabs;
+  tam_lds_tabs_fill(&tabs);
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+  const uint32_t nbk = 1u << bits;
+  const float inv_nbk = 1.0f / (float)nbk;
+  const uint64_t units = (n + 1023u) / 1024u, nfull = n / 1024u;
+  const auto value = [&](float lmin, float span, uint32_t k) {
+    return tam_expf_lds(lmin + ((float)k + 0.5f) * inv_nbk * span, &tabs);
+  };
+  const auto scale = [&](uint64_t b, float& lmin, float& span) {
+    lmin = tam_f16_to_f32(tam_g(scales)[2u * b]);
+    span = tam_f16_to_f32(tam_g(scales)[2u * b + 1u]) - lmin;
+  };
+  for (uint64_t u = (uint64_t)blockIdx.x * (TAM_WG / 64) + wave; u < units; u += gridDim.x * (TAM_WG / 64)) {
+    if (u >= nfull) {
+      for (uint64_t e = 1024u * u + lane; e < n; e += 64u) {
+        float lmin, span;
+        scale(e / TAM_BLOCK_SIZE, lmin, span);
+        tam_g(out)[e] = value(lmin, span, tam_g(idx)[e]);
+      }
+      continue;
+    }
+    const uint64_t e0 = 1024u * u + 4u * lane;  // pass j: elements e0 + 256 j .. + 3, of block 2 j + lane / 32
+    uint32_t w[4], high = 0u;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      w[j] = tam_g((const TamW1B*)(idx + e0 + 256u * (uint32_t)j))[0];
+      high |= w[j];
+    }
+    const bool table = bits < 8u && !__any((high & ~((nbk - 1u) * 0x01010101u)) != 0u);
+    float* tab = lut[wave];
+    if (table) {
+      float lmin, span;
+      scale(8u * u + (lane >> 3), lmin, span);
+      for (uint32_t k = lane & 7u; k < nbk; k += 8u) tab[(lane >> 3) * 64u + k] = value(lmin, span, k);
+      tam_wave_lds_sync();
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float* t = tab + (2u * (uint32_t)j + (lane >> 5)) * 64u;
+        tam_g((TamF4E*)(out + e0 + 256u * (uint32_t)j))[0] =
+            TamF4{t[w[j] & 0xffu], t[(w[j] >> 8) & 0xffu], t[(w[j] >> 16) & 0xffu], t[w[j] >> 24]};
+      }
+      tam_wave_lds_sync();  // the next unit rewrites the table
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float lmin, span;
+        scale(8u * u + 2u * (uint32_t)j + (lane >> 5), lmin, span);
+        tam_g((TamF4E*)(out + e0 + 256u * (uint32_t)j))[0] =
+            TamF4{value(lmin, span, w[j] & 0xffu), value(lmin, span, (w[j] >> 8) & 0xffu),
+                  value(lmin, span, (w[j] >> 16) & 0xffu), value(lmin, span, w[j] >> 24)};
+      }
+    }
   }
 }
 
 // ---------------------------------------------------------------------------
 // utility kernels
 // ---------------------------------------------------------------------------
-__global__ void tam_k_v_dequantize(const uint8_t* __restrict__ idx, const uint16_t* __restrict__ scales,
-                                   uint64_t n, uint32_t bits, float* __restrict__ out) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint64_t b = i / TAM_BLOCK_SIZE;
-  const float lmin = tam_f16_to_f32(scales[2 * b]);
-  const float lmax = tam_f16_to_f32(scales[2 * b + 1]);
-  const float span = lmax - lmin;
-  const float inv_nbk = 1.0f / (float)(1u << bits);
-  out[i] = tam_expf(lmin + ((float)idx[i] + 0.5f) * inv_nbk * span);
-}
-
 // One thread per 8 elements (half a group of draws).
 __global__ void tam_k_philox_uniforms(uint32_t tid, uint32_t step, uint32_t seed_lo, uint32_t seed_hi,
                                       uint64_t count, float* __restrict__ out) {
@@ -3113,6 +3359,15 @@ static uint32_t tam_resident_grid(int which, const void* kernel, int block) {
     cache[dev][which].store(g, std::memory_order_relaxed);
   }
   return g;
+}
+
+// Workgroups of a standalone codec kernel over `units` of 1024 elements, four
+// waves each, one unit per wave and round: at most eight rounds of what a GPU
+// holds at four workgroups per CU (the tables a workgroup copies to LDS are then
+// shared by up to 2^25 elements' units).
+static uint32_t tam_codec_grid(uint64_t units) {
+  const uint64_t wgs = (units + 3) / 4, most = (uint64_t)tam_device_cus() * 32u;
+  return (uint32_t)(wgs < 1 ? 1 : (wgs < most ? wgs : most));
 }
 
 extern "C" {
@@ -3439,9 +3694,8 @@ int tam_v_dequantize(const uint8_t* v_idx, const uint16_t* v_scales, uint64_t n,
   if (!(v_bits == 2 || v_bits == 3 || v_bits == 4 || v_bits == 6 || v_bits == 8))
     return tam_fail(TAM_E_INVALID, "%sv_bits must be 2, 3, 4, 6 or 8", "");
   if (n == 0) return TAM_OK;
-  const uint64_t blocks = (n + 255) / 256;
-  hipLaunchKernelGGL(tam_k_v_dequantize, dim3((uint32_t)blocks), dim3(256), 0, (hipStream_t)stream, v_idx,
-                     v_scales, n, v_bits, out);
+  hipLaunchKernelGGL(tam_k_v_dequantize, dim3(tam_codec_grid((n + 1023) / 1024)), dim3(TAM_WG), 0,
+                     (hipStream_t)stream, v_idx, v_scales, n, v_bits, out);
   TAM_HIP_CHECK(hipGetLastError());
   return TAM_OK;
 }
@@ -3636,8 +3890,11 @@ int tam_fused_v_update(const uint8_t* idx_in, const uint16_t* scales_in, const v
   if (((uintptr_t)idx_in | (uintptr_t)idx_out) & 7u || ((uintptr_t)scales_in | (uintptr_t)scales_out) & 3u)
     return tam_fail(TAM_E_INVALID, "%smisaligned v state", "");
   if (n == 0) return TAM_OK;
-  hipLaunchKernelGGL(tam_k_fused_v, dim3(tam_tiles_of(n)), dim3(TAM_WG), 0, (hipStream_t)stream, idx_in, scales_in, g,
-                     g_dtype, n, v_bits, beta2, one_minus_beta2, tensor_id, step, (uint32_t)seed,
+  const auto kernel = g_dtype == TAM_DTYPE_BF16 ? tam_k_fused_v<TAM_DTYPE_BF16>
+                      : g_dtype == TAM_DTYPE_F16 ? tam_k_fused_v<TAM_DTYPE_F16>
+                                                 : tam_k_fused_v<TAM_DTYPE_F32>;
+  hipLaunchKernelGGL(kernel, dim3(tam_codec_grid((n + 1023) / 1024 + 1)), dim3(TAM_WG), 0, (hipStream_t)stream,
+                     idx_in, scales_in, g, n, v_bits, beta2, one_minus_beta2, tensor_id, step, (uint32_t)seed,
                      (uint32_t)(seed >> 32), idx_out, scales_out, v_out);
   TAM_HIP_CHECK(hipGetLastError());
   return TAM_OK;
@@ -3652,8 +3909,40 @@ int tam_v_quantize(const float* v, uint64_t n_padded, uint32_t v_bits, int stoch
     return tam_fail(TAM_E_INVALID, "%sv_bits must be 2, 3, 4, 6 or 8", "");
   if ((uintptr_t)scales & 3u) return tam_fail(TAM_E_INVALID, "%smisaligned scales", "");
   if (n_padded == 0) return TAM_OK;
-  hipLaunchKernelGGL(tam_k_quantize, dim3(tam_tiles_of(n_padded)), dim3(TAM_WG), 0, (hipStream_t)stream, v, n_padded,
-                     v_bits, stochastic, tensor_id, step, (uint32_t)seed, (uint32_t)(seed >> 32), idx, scales);
+  const uint32_t nb = (uint32_t)(n_padded / TAM_BLOCK_SIZE);
+  hipLaunchKernelGGL(stochastic ? tam_k_quantize<true> : tam_k_quantize<false>, dim3(tam_codec_grid((nb + 7u) / 8u)),
+                     dim3(TAM_WG), 0, (hipStream_t)stream, v, nb, v_bits, tensor_id, step, (uint32_t)seed,
+                     (uint32_t)(seed >> 32), idx, scales, (uint32_t*)nullptr);
+  TAM_HIP_CHECK(hipGetLastError());
+  return TAM_OK;
+}
+
+size_t tam_v_compress_workspace(uint64_t n) {
+  return (size_t)tam_codec_grid((n / TAM_BLOCK_SIZE + 7) / 8) * sizeof(uint32_t);
+}
+
+int tam_v_compress(const float* v, uint64_t n, uint32_t v_bits, int stochastic, uint32_t tensor_id, uint32_t step,
+                   uint64_t seed, uint8_t* idx, uint16_t* scales, void* workspace, size_t ws_bytes, void* stream) {
+  tam_err_buf[0] = 0;
+  if (n % TAM_BLOCK_SIZE == 0)
+    return tam_v_quantize(v, n, v_bits, stochastic, tensor_id, step, seed, idx, scales, stream);
+  if (!v || !idx || !scales || !workspace) return tam_fail(TAM_E_INVALID, "%snull argument", "");
+  if (!(v_bits == 2 || v_bits == 3 || v_bits == 4 || v_bits == 6 || v_bits == 8))
+    return tam_fail(TAM_E_INVALID, "%sv_bits must be 2, 3, 4, 6 or 8", "");
+  if ((uintptr_t)scales & 3u) return tam_fail(TAM_E_INVALID, "%smisaligned scales", "");
+  const size_t need = tam_v_compress_workspace(n);
+  if (ws_bytes < need) return tam_fail(TAM_E_WORKSPACE, "%sworkspace too small: need %ld bytes", "", (long)need);
+  hipStream_t s = (hipStream_t)stream;
+  const uint32_t nb = (uint32_t)(n / TAM_BLOCK_SIZE);  // whole blocks
+  uint32_t* wgmin = (uint32_t*)workspace;
+  const uint32_t grid = tam_codec_grid((nb + 7u) / 8u);
+  if (nb) {
+    hipLaunchKernelGGL(stochastic ? tam_k_quantize<true> : tam_k_quantize<false>, dim3(grid), dim3(TAM_WG), 0, s, v,
+                       nb, v_bits, tensor_id, step, (uint32_t)seed, (uint32_t)(seed >> 32), idx, scales, wgmin);
+    TAM_HIP_CHECK(hipGetLastError());
+  }
+  hipLaunchKernelGGL(tam_k_quantize_last, dim3(1), dim3(64), 0, s, v, n, wgmin, nb ? grid : 0u, v_bits,
+                     stochastic ? 1 : 0, tensor_id, step, (uint32_t)seed, (uint32_t)(seed >> 32), idx, scales);
   TAM_HIP_CHECK(hipGetLastError());
   return TAM_OK;
 }

@@ -9,7 +9,7 @@ State dict layout (reference src/turboadam/oneq.py:41-48):
 import torch
 
 from . import _lib
-from .quantize import DEFAULT_SEED, _dequantize_operands, quantize_logscale_nbits
+from .quantize import DEFAULT_SEED, _check, _dequantize_operands, quantize_logscale_nbits
 from .utils import BLOCK_SIZE, num_blocks
 
 # TurboAdam starts v from full(1e-30) quantised deterministically
@@ -43,17 +43,27 @@ def compress_v_logscale(v: torch.Tensor, n_bits: int = 3, block_size: int = BLOC
     The last block is filled up to block_size elements with the fp32 value
     max(min(v), 1e-38): padding can then neither lower the block's minimum
     nor (a log of zero) make it infinite.  That value is formed on the device
-    (the reference reads min(v) back to the host first); the blocks then go
-    through quantize_logscale_nbits."""
+    (the reference reads min(v) back to the host first), by the pass that
+    quantises the whole blocks; a v of whole blocks is read in place."""
     flat = v.reshape(-1).to(torch.float32)
     count = flat.numel()
-    blocks = torch.empty(num_blocks(count, block_size) * block_size, dtype=torch.float32, device=flat.device)
-    blocks[:count] = flat
-    if blocks.numel() > count:
-        blocks[count:] = flat.min().clamp(min=1e-38)  # NaN stays NaN, as Python's max(nan, 1e-38)
-    indices, scales, _ = quantize_logscale_nbits(blocks, n_bits=n_bits, block_size=block_size,
-                                                 stochastic_round=stochastic_round, tensor_id=tensor_id,
-                                                 step=step, seed=seed)
+    if count % BLOCK_SIZE == 0 or block_size != BLOCK_SIZE:
+        indices, scales, _ = quantize_logscale_nbits(flat, n_bits=n_bits, block_size=block_size,
+                                                     stochastic_round=stochastic_round, tensor_id=tensor_id,
+                                                     step=step, seed=seed)
+    else:
+        _check(n_bits, block_size, flat, "compress_v_logscale")
+        lib = _lib.load()
+        flat = flat.contiguous()
+        dev = flat.device
+        nb = num_blocks(count, block_size)
+        indices = torch.empty(nb * block_size, dtype=torch.uint8, device=dev)
+        scales = torch.empty((nb, 2), dtype=torch.float16, device=dev)
+        with torch.cuda.device(dev):
+            ws = torch.empty(lib.tam_v_compress_workspace(count), dtype=torch.uint8, device=dev)
+            _lib.check(lib.tam_v_compress(flat.data_ptr(), count, n_bits, int(bool(stochastic_round)), tensor_id, step,
+                                          seed, indices.data_ptr(), scales.data_ptr(), ws.data_ptr(), ws.numel(),
+                                          _lib.stream_of(dev)), "tam_v_compress")
     return dict(indices=indices, scales=scales, n_bits=n_bits, original_shape=v.shape, original_length=count,
                 block_size=block_size)
 
