@@ -32,7 +32,6 @@ extern "C" {
 
 #define TAM_ABI_VERSION 9
 #define TAM_BLOCK_SIZE 128 /* elements per quantisation / CoState block */
-#define TAM_TAIL_TILES 4   /* tiles per tail workgroup of an unaligned tensor */
 
 /* error codes */
 #define TAM_OK 0
@@ -130,9 +129,7 @@ typedef struct TamTensor {
                             /*      kernel for quarters that are not full        */
   uint32_t tail_wgs;        /* [derived] its workgroups there: one when a part of */
                             /*      it lies outside full units (8 blocks), none  */
-                            /*      otherwise or with EF; one per TAM_TAIL_TILES */
-                            /*      tiles when param or grad is not 16-byte      */
-                            /*      aligned (every quarter is then bounds-checked) */
+                            /*      otherwise or with EF                         */
 } TamTensor;
 
 /* Launch summary and workspace layout, filled by tam_prepare(). */

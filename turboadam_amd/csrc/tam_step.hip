@@ -154,14 +154,14 @@ __device__ __forceinline__ void tam_st16_f32(float* base, uint64_t e0, const flo
   for (int k = 0; k < 4; ++k) b[k] = TamF4{v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]};
 }
 
-// Elements [e0, e0+8) of a parameter or gradient.  FULL: all 8 exist and the
-// array is 16-byte aligned; otherwise only the first nv exist (the rest read 0).
+// Elements [e0, e0+8) of a parameter or gradient.  FULL: all 8 exist;
+// otherwise only the first nv exist (the rest read 0).
 template <uint32_t DT, bool FULL>
 __device__ __forceinline__ void tam_ld8(const void* base, uint64_t e0, uint32_t nv, float* out) {
   if (DT == TAM_DTYPE_F32) {
     const float* b = (const float*)base + e0;
     if (FULL) {
-      const TamF4 a = tam_g((const TamF4*)b)[0], c = tam_g((const TamF4*)b)[1];
+      const TamF4 a = tam_g((const TamF4E*)b)[0], c = tam_g((const TamF4E*)b)[1];
       out[0] = a.x; out[1] = a.y; out[2] = a.z; out[3] = a.w;
       out[4] = c.x; out[5] = c.y; out[6] = c.z; out[7] = c.w;
     } else {
@@ -171,7 +171,7 @@ __device__ __forceinline__ void tam_ld8(const void* base, uint64_t e0, uint32_t 
   } else {
     const uint16_t* b = (const uint16_t*)base + e0;
     if (FULL) {
-      tam_unpack8<DT>(tam_g((const TamW4*)b)[0], out);
+      tam_unpack8<DT>(tam_g((const TamW4E*)b)[0], out);
     } else {
 #pragma unroll
       for (int i = 0; i < TAM_EPL; ++i) out[i] = (uint32_t)i < nv ? tam_h2f<DT>(tam_g(b)[i]) : 0.0f;
@@ -179,7 +179,7 @@ __device__ __forceinline__ void tam_ld8(const void* base, uint64_t e0, uint32_t 
   }
 }
 
-// fp32 state arrays (exp_avg / exp_avg_sq, 16-byte aligned)
+// fp32 arrays (the moments and residuals, an fp32 parameter)
 template <bool FULL>
 __device__ __forceinline__ void tam_ld8_f32(const float* base, uint64_t e0, uint32_t nv, float* out) {
   tam_ld8<TAM_DTYPE_F32, FULL>(base, e0, nv, out);
@@ -188,8 +188,8 @@ template <bool FULL>
 __device__ __forceinline__ void tam_st8_f32(float* base, uint64_t e0, uint32_t nv, const float* v) {
   float* b = base + e0;
   if (FULL) {
-    tam_g((TamF4*)b)[0] = TamF4{v[0], v[1], v[2], v[3]};
-    tam_g((TamF4*)b)[1] = TamF4{v[4], v[5], v[6], v[7]};
+    tam_g((TamF4E*)b)[0] = TamF4{v[0], v[1], v[2], v[3]};
+    tam_g((TamF4E*)b)[1] = TamF4{v[4], v[5], v[6], v[7]};
   } else {
 #pragma unroll
     for (int i = 0; i < TAM_EPL; ++i)
@@ -203,7 +203,7 @@ template <bool FULL>
 __device__ __forceinline__ void tam_st8_bits(void* base, uint64_t e0, uint32_t nv, const uint32_t* pw2) {
   uint16_t* b = (uint16_t*)base + e0;
   if (FULL) {
-    tam_g((TamW4*)b)[0] = TamW4{pw2[0], pw2[1], pw2[2], pw2[3]};
+    tam_g((TamW4E*)b)[0] = TamW4{pw2[0], pw2[1], pw2[2], pw2[3]};
   } else {
 #pragma unroll
     for (int i = 0; i < TAM_EPL; ++i)
@@ -1076,10 +1076,9 @@ __device__ __forceinline__ int tam_advance_tensor(const TamTensor* __restrict__ 
   return lo;
 }
 
-// Whether a wave's quarter of tile `wq` lies inside the tensor with aligned arrays.
+// Whether a wave's quarter of tile `wq` lies inside the tensor.
 __device__ __forceinline__ bool tam_quarter_full(const TamTensor& d, uint32_t wq) {
-  const bool aligned = (((uintptr_t)d.param | (uintptr_t)d.grad) & 15u) == 0;
-  return aligned && (uint64_t)(wq + 1u) * (4u * TAM_BLOCK_SIZE) <= d.n;
+  return (uint64_t)(wq + 1u) * (4u * TAM_BLOCK_SIZE) <= d.n;
 }
 
 // ---------------------------------------------------------------------------
@@ -1272,10 +1271,9 @@ __device__ __forceinline__ double tam_unit_sum2(double a, double b, uint32_t lan
   return tam_swap_add<1>(x);
 }
 
-// Whether unit u lies inside the tensor with aligned arrays.
+// Whether unit u lies inside the tensor.
 __device__ __forceinline__ bool tam_unit_full(const TamTensor& d, uint32_t u) {
-  const bool aligned = (((uintptr_t)d.param | (uintptr_t)d.grad) & 15u) == 0;
-  return aligned && (uint64_t)(u + 1u) * (8u * TAM_BLOCK_SIZE) <= d.n;
+  return (uint64_t)(u + 1u) * (8u * TAM_BLOCK_SIZE) <= d.n;
 }
 
 // 1Q decode (quantize.py:252-256), EMA (:259-270) and block extremes of a
@@ -1498,12 +1496,12 @@ __device__ __forceinline__ void tam_k1_unit(const TamTensor& d, uint32_t u, uint
   const uint64_t off = e0 * (DT == TAM_DTYPE_F32 ? 4u : 2u);
   TamW4 gw[NW], pw[NW];
 #pragma unroll
-  for (int k = 0; k < NW; ++k) gw[k] = tam_g((const TamW4*)((const char*)d.grad + off))[k];
+  for (int k = 0; k < NW; ++k) gw[k] = tam_g((const TamW4E*)((const char*)d.grad + off))[k];
   // an fp32 parameter (16 registers) is loaded just before the update: held
   // from here it would make the kernel spill at 4 waves per SIMD
   if constexpr (DT != TAM_DTYPE_F32) {
 #pragma unroll
-    for (int k = 0; k < NW; ++k) pw[k] = tam_g((const TamW4*)((const char*)d.param + off))[k];
+    for (int k = 0; k < NW; ++k) pw[k] = tam_g((const TamW4E*)((const char*)d.param + off))[k];
   }
   uint32_t label = 0u, amp = 0u, sbytes = 0u;  // sbytes: sign bytes of elements e0..e0+7 (low) and e0+8..e0+15
   float nrm = 0.0f, alpha_prev = 0.0f;
@@ -1596,7 +1594,7 @@ __device__ __forceinline__ void tam_k1_unit(const TamTensor& d, uint32_t u, uint
     if constexpr (DT == TAM_DTYPE_F32) {
 #pragma unroll
       for (int k = 0; k < NW; ++k) {
-        const TamF4 pk = __builtin_bit_cast(TamF4, tam_g((const TamW4*)((const char*)d.param + off))[k]);
+        const TamF4 pk = tam_g((const TamF4E*)((const char*)d.param + off))[k];
         p[4 * k] = pk.x; p[4 * k + 1] = pk.y; p[4 * k + 2] = pk.z; p[4 * k + 3] = pk.w;
       }
     }
@@ -1627,7 +1625,7 @@ __device__ __forceinline__ void tam_k1_unit(const TamTensor& d, uint32_t u, uint
   if (compress_v) tam_vunit_b(d, lane, b, e0, v, vx, tabs, seed_lo, seed_hi);
 }
 
-// Full units (inside the tensor, aligned arrays) of one parameter dtype:
+// Full units (inside the tensor) of one parameter dtype:
 // persistent workgroups of two waves stride over the tiles; wave w takes unit
 // 2(tile - tile0) + w of the tile's tensor (quarters 4(tile - tile0) + 2w and
 // + 2w + 1), and the waves never synchronise with each other.  One kernel per
@@ -1654,10 +1652,9 @@ __device__ __forceinline__ void tam_k1_full_body(const TamTensor* __restrict__ T
     const TamTensor& d = T[ti];
     const uint32_t end = d.tile0 + d.ntiles;  // the tensor's tiles end here
     if (d.dtype == DT && !(d.flags & TAM_FLAG_EF)) {  // uniform; EF: tam_k1_ef
-      // units u < nfull are full (inside the tensor, aligned arrays); the
-      // rest are tam_k1_tail's, and u grows with the tile
-      const bool aligned = (((uintptr_t)d.param | (uintptr_t)d.grad) & 15u) == 0;
-      const uint64_t nfull = aligned ? d.n / (8u * TAM_BLOCK_SIZE) : 0u;
+      // units u < nfull are full; the rest is tam_k1_tail's, and u grows with
+      // the tile
+      const uint64_t nfull = d.n / (8u * TAM_BLOCK_SIZE);
       for (; tile < end; tile += stride) {
         const uint32_t u = (tile - d.tile0) * 2u + wave;  // unit within the tensor
         if (u >= nfull) break;
@@ -1688,32 +1685,19 @@ TAM_K1_FULL_KERNEL(tam_k1_main_bf16, TAM_DTYPE_BF16, TAM_K1_WAVES_BF16)
 TAM_K1_FULL_KERNEL(tam_k1_main_f16, TAM_DTYPE_F16, TAM_K1_WAVES_F16)
 TAM_K1_FULL_KERNEL(tam_k1_main_f32, TAM_DTYPE_F32, TAM_K1_WAVES_F32)
 
-// The quarters outside full units: the last (at most five) quarters of each
-// tensor, or every quarter of a tensor whose parameter or gradient is not
-// 16-byte aligned.  An aligned tensor has one workgroup; an unaligned one has
-// one per TAM_TAIL_TILES tiles (tam_prepare: tail0, tail_wgs), so a large
-// unaligned tensor spreads over the GPU.  Wave w takes every fourth quarter of
-// the workgroup's range.
-__global__ __launch_bounds__(TAM_WG) void tam_k1_tail(const TamTensor* __restrict__ T, int nT, uint32_t seed_lo,
+// The at most two quarters of each tensor outside full units, one workgroup per
+// tensor that has any (tam_prepare: tail0, tail_wgs), a wave per quarter.
+__global__ __launch_bounds__(TAM_K1U_WG) void tam_k1_tail(const TamTensor* __restrict__ T, int nT, uint32_t seed_lo,
                                                       uint32_t seed_hi, double2* __restrict__ partials) {
   if (tam_step_skipped(T)) return;
   const TamTensor& d = T[tam_wave_first(nT, [&](int i) { return T[i].tail0 + T[i].tail_wgs > blockIdx.x; })];
-  __shared__ float lut[TAM_WG / 64][4 * 64];
+  __shared__ float lut[TAM_K1U_WG / 64][4 * 64];
   __shared__ TamLdsTabs tabs;
   tam_lds_tabs_fill(&tabs);
   const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-  const bool aligned = (((uintptr_t)d.param | (uintptr_t)d.grad) & 15u) == 0;
-  const uint32_t nq = d.ntiles * 4u;
-  uint32_t first, last;
-  if (aligned) {  // full units precede: tam_k1_main_<dtype> takes them
-    first = 2u * (uint32_t)(d.n / (8u * TAM_BLOCK_SIZE));
-    last = nq;
-  } else {
-    const uint32_t local = blockIdx.x - d.tail0;
-    first = local * (4u * TAM_TAIL_TILES);
-    last = first + 4u * TAM_TAIL_TILES < nq ? first + 4u * TAM_TAIL_TILES : nq;
-  }
-  for (uint32_t wq = first + wave; wq < last; wq += 4u) {
+  // full units precede: tam_k1_main_<dtype> takes them
+  const uint32_t first = 2u * (uint32_t)(d.n / (8u * TAM_BLOCK_SIZE)), last = (d.nb + 3u) / 4u;
+  for (uint32_t wq = first + wave; wq < last; wq += TAM_K1U_WG / 64) {
     double2* part = partials + (uint64_t)d.tile0 * 4u + wq;
     switch (d.dtype) {
       case TAM_DTYPE_BF16:
@@ -2059,7 +2043,7 @@ template <bool F32>
 __device__ __forceinline__ TamK2U<F32> tam_k2u_load(const TamTensor& d, uint32_t u, uint32_t lane) {
   const uint32_t b = u * 8u + (lane >> 3);
   const uint64_t e0 = (uint64_t)b * TAM_BLOCK_SIZE + (lane & 7u) * TAM_EPU;
-  const TAM_GLOBAL TamW4* gp = tam_g((const TamW4*)((const char*)d.grad + e0 * (F32 ? 4u : 2u)));
+  const TAM_GLOBAL TamW4E* gp = tam_g((const TamW4E*)((const char*)d.grad + e0 * (F32 ? 4u : 2u)));
   TamK2U<F32> r;
 #pragma unroll
   for (int k = 0; k < (F32 ? 4 : 2); ++k) r.g[k] = gp[k];
@@ -3454,11 +3438,9 @@ int tam_prepare(TamTensor* tensors, int n_tensors, TamStepInfo* info) {
     t.nb = (uint32_t)nb;
     t.ntiles = (uint32_t)nt;
     t.tile0 = (uint32_t)tiles;
-    const bool aligned = (((uintptr_t)t.param | (uintptr_t)t.grad) & 15u) == 0;
     t.tail0 = (uint32_t)tail_blocks;
-    if (t.flags & TAM_FLAG_EF) t.tail_wgs = 0u;  // tam_k1_ef covers the tensor
-    else if (aligned) t.tail_wgs = t.n % (8u * TAM_BLOCK_SIZE) ? 1u : 0u;  // whole units only: nothing left
-    else t.tail_wgs = (uint32_t)((nt + TAM_TAIL_TILES - 1) / TAM_TAIL_TILES);
+    // tam_k1_ef covers an error-feedback tensor
+    t.tail_wgs = !(t.flags & TAM_FLAG_EF) && t.n % (8u * TAM_BLOCK_SIZE) ? 1u : 0u;
     tail_blocks += t.tail_wgs;
     if (!(t.flags & TAM_FLAG_EF)) dtype_mask |= 1u << t.dtype;  // pass 0's per-dtype kernels skip EF tensors
     t.chunk0 = (uint32_t)chunks;
@@ -3554,7 +3536,7 @@ static int tam_launch_pass(int pass, const TamTensor* d_tensors, const TamStepIn
                            partials);
       TAM_HIP_CHECK(hipGetLastError());
       if (info->tail_blocks)
-        hipLaunchKernelGGL(tam_k1_tail, dim3(info->tail_blocks), dim3(TAM_WG), 0, s, d_tensors, info->n_tensors,
+        hipLaunchKernelGGL(tam_k1_tail, dim3(info->tail_blocks), dim3(TAM_K1U_WG), 0, s, d_tensors, info->n_tensors,
                            (uint32_t)seed, (uint32_t)(seed >> 32), partials);
       break;
     case 1:
