@@ -235,6 +235,20 @@ int tam_costate_decode(const uint8_t* labels, const uint8_t* signs, const float*
                        const float* alpha, const void* g, uint32_t g_dtype, uint64_t n, int has_state, int ema,
                        float beta1, float one_minus_beta1, float* m_out, void* stream);
 
+/* CoStateManager.update (reference costate.py:367-464) on one tensor, in the
+ * step's launches: m_out (fp32[n]) = the EMA of the decoded previous state (0
+ * without has_state) and g; alpha, labels, signs, norms and amp (aligned as in
+ * TamTensor) then hold the new encoding, with the thresholds at ranks k_lo and
+ * k_hi.  ef_residual (or NULL: no error feedback) is fp32[n], 16-byte aligned:
+ * added to g in the EMA with has_residual, and updated (written, not read,
+ * without).  Workspace: tam_costate_update_workspace bytes (0: n is out of
+ * range), 256-byte aligned. */
+size_t tam_costate_update_workspace(uint64_t n, int error_feedback);
+int tam_costate_update(const void* g, uint32_t g_dtype, uint64_t n, uint8_t* labels, uint8_t* signs, float* norms,
+                       uint16_t* amp, float* alpha, int has_state, float beta1, float one_minus_beta1,
+                       uint32_t k_lo, uint32_t k_hi, float* ef_residual, int has_residual, float* m_out,
+                       void* workspace, size_t ws_bytes, void* stream);
+
 /* decompose (reference costate.py:22-43): *alpha (device float) = fl(mg)/fl(gg)
  * with the step's dot products (the contract above; 0 when gg == 0), delta =
  * fl(m - fl(alpha*g)).  m, g fp32[n].  Workspace: tam_decompose_workspace(n)

@@ -189,3 +189,46 @@ def test_step_reads_no_workspace_it_did_not_write(dt, monkeypatch):
     for ef in (False, True):
         bad = run_side_by_side(sizes, [dt] * len(sizes), steps=3, error_feedback=ef)
         assert not bad, "\n".join(bad[:10])
+
+
+# units of 1024 elements, then quarters of 512; one dot-product chunk up to 4194304
+@pytest.mark.parametrize("ef", [False, True])
+@pytest.mark.parametrize("n,dt", [(1, torch.float32), (513, torch.bfloat16), (1024, torch.float16),
+                                  (1025, torch.float32), (1024 * 9 + 640, torch.bfloat16),
+                                  (512 * 8192 + 1000, torch.float32)])
+def test_costate_update_units(n, dt, ef):
+    from turboadam_amd import costate as C
+
+    log(f"CoStateManager.update n={n} {dt} ef={ef}, 3 steps")
+    rng = np.random.default_rng(n)
+    nb = (n + 127) // 128
+    labels, signs = np.zeros(nb, np.uint8), np.zeros((n + 7) // 8, np.uint8)
+    norms, amp, alpha, res = (np.zeros(nb, np.float32), np.zeros(nb, np.uint16), np.zeros(1, np.float32),
+                              np.zeros(n, np.float32))
+    mgr = C.CoStateManager(error_feedback=ef)
+    # state arrays that the kernels cannot take as they are are updated through copies
+    mgr.allocate(n, DEV)
+    mgr._encoded["block_norms"] = torch.zeros(nb, dtype=torch.float64, device=DEV)
+    mgr._encoded["sign_packed"] = torch.zeros(signs.size + 1, dtype=torch.uint8, device=DEV)[1:]
+    k_lo, k_hi = O.ranks(nb, 0.10, 0.90)
+    kept = None
+    for s in range(3):
+        g = (torch.from_numpy(rng.standard_normal(n).astype(np.float32)) * 1e-3).to(dt)
+        g32, m_o = g.float().numpy().copy(), np.empty(n, np.float32)
+        O.lib().or_costate_update_ef(O.ptr(g32), n, O.f32(0.9), O.f32(1.0 - 0.9), float(np.float32(np.sqrt(128.0))),
+                                     k_lo, k_hi, int(s > 0), O.ptr(labels), O.ptr(signs), O.ptr(norms), O.ptr(amp),
+                                     O.ptr(alpha), int(ef), int(ef and s > 0), O.ptr(res), O.ptr(m_o))
+        before = (kept, kept.clone()) if kept is not None else None
+        m = mgr.update(g.to(DEV), 0.9)
+        enc = mgr._encoded
+        got = {"m": m, "labels": enc["labels"], "signs": enc["sign_packed"], "norms": enc["block_norms"].float(),
+               "amp": enc["scales"], "alpha": mgr._alpha.reshape(1)}
+        want = {"m": m_o, "labels": labels, "signs": signs, "norms": norms, "amp": amp, "alpha": alpha}
+        if ef:
+            got["residual"], want["residual"] = mgr._ef_residual, res
+            if before is not None:  # the previous residual tensor is left as it was
+                assert torch.equal(*before)
+            kept = mgr._ef_residual
+        for k, t in got.items():
+            a, b = np.ascontiguousarray(_np(t)), want[k]
+            assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), f"step {s}: {k}"

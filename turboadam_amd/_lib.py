@@ -140,6 +140,12 @@ SIGNATURES = {
         [_VP, _VP, _VP, _VP, _VP, _VP, ctypes.c_uint32, ctypes.c_uint64, ctypes.c_int, ctypes.c_int, ctypes.c_float,
          ctypes.c_float, _VP, _VP],
     ),
+    "tam_costate_update_workspace": (ctypes.c_size_t, [ctypes.c_uint64, ctypes.c_int]),
+    "tam_costate_update": (
+        ctypes.c_int,
+        [_VP, ctypes.c_uint32, ctypes.c_uint64, _VP, _VP, _VP, _VP, _VP, ctypes.c_int, ctypes.c_float, ctypes.c_float,
+         ctypes.c_uint32, ctypes.c_uint32, _VP, ctypes.c_int, _VP, _VP, ctypes.c_size_t, _VP],
+    ),
     "tam_decompose_workspace": (ctypes.c_size_t, [ctypes.c_uint64]),
     "tam_decompose": (ctypes.c_int, [_VP, _VP, ctypes.c_uint64, _VP, _VP, _VP, ctypes.c_size_t, _VP]),
     "tam_block_ratios": (ctypes.c_int, [_VP, _VP, ctypes.c_uint64, _VP, _VP]),

@@ -12,6 +12,8 @@ products and block norms, exact radix selection).  Inputs must be on an
 MI355X (HIP) device.
 """
 
+import ctypes
+
 import torch
 
 from . import _lib
@@ -126,6 +128,24 @@ def encode_blocks(delta: torch.Tensor, labels: torch.Tensor, block_size: int = B
     return {"labels": labels, "sign_packed": signs, "block_norms": norms, "scales": amp}
 
 
+_ENCODED_DTYPES = {"labels": torch.uint8, "sign_packed": torch.uint8, "block_norms": torch.float32,
+                   "scales": torch.float16}
+
+
+def _check_covers(encoded: dict, n: int) -> None:
+    nb = num_blocks(n)
+    if (encoded["labels"].numel() != nb or encoded["block_norms"].numel() != nb
+            or encoded["scales"].numel() != nb or encoded["sign_packed"].numel() < (n + 7) // 8):
+        raise ValueError(f"decode_blocks: the encoding does not cover {n} elements ({nb} blocks)")
+
+
+def _in_form(t: torch.Tensor, dtype, device) -> torch.Tensor:
+    """t itself when it is a contiguous array of dtype on device, aligned as the
+    kernels need (4 bytes at most), else a copy that is."""
+    c = t.to(device=device, dtype=dtype).contiguous()
+    return c if c.data_ptr() % 4 == 0 else c.clone()
+
+
 def _decode(encoded: dict, alpha, g: torch.Tensor, n: int, has_state: bool, ema: bool, beta1: float = 0.0):
     lib = _lib.load()
     dev = g.device
@@ -139,10 +159,7 @@ def _decode(encoded: dict, alpha, g: torch.Tensor, n: int, has_state: bool, ema:
     ptrs = [0, 0, 0, 0, 0]
     keep = []
     if has_state:
-        nb = num_blocks(n)
-        if (encoded["labels"].numel() != nb or encoded["block_norms"].numel() != nb
-                or encoded["scales"].numel() != nb or encoded["sign_packed"].numel() < (n + 7) // 8):
-            raise ValueError(f"decode_blocks: the encoding does not cover {n} elements ({nb} blocks)")
+        _check_covers(encoded, n)
         labels = encoded["labels"].to(device=dev, dtype=torch.uint8).contiguous()
         signs = encoded["sign_packed"].to(device=dev, dtype=torch.uint8).contiguous()
         norms = encoded["block_norms"].to(device=dev, dtype=torch.float32).contiguous()
@@ -208,42 +225,59 @@ class CoStateManager:
         """One CoState step for gradient g (reference costate.py:367-464): decode
         the previous state (or zeros), m = beta1*m_hat + (1-beta1)*g, then
         decompose, ratios, thresholds, labels and encode into the persistent
-        buffers.  With error feedback (:409-437) the EMA takes g + residual and
-        the residual then takes the encoding loss delta - decode(new, alpha=0)
-        (its EMA after the first step), in fp32 elementwise ops in the
-        reference's order.  Returns m (fp32, shape of g)."""
+        buffers, in the optimizer step's launches.  With error feedback
+        (:409-437) the EMA takes g + residual and the residual then takes the
+        encoding loss delta - decode(new, alpha=0) (its EMA after the first
+        step).  Returns m (fp32, shape of g)."""
         _require_gpu(g, "CoStateManager.update")
         _require_block_size(self.block_size)
         n = g.numel()
-        if self._encoded is None or self._encoded["labels"].device != g.device:
-            self.allocate(n, g.device)
-        g32 = _f32_flat(g)
-        if self._error_feedback and self._ef_residual is not None:
-            m_hat = (_decode(self._encoded, self._alpha, g, n, True, False) if self._has_state
-                     else torch.zeros(n, dtype=torch.float32, device=g.device))
-            g_corrected = g32 + self._ef_residual.reshape(-1).float()
-            m = beta1 * m_hat + (1.0 - beta1) * g_corrected
-        else:
-            m = _decode(self._encoded, self._alpha, g, n, self._has_state, True, beta1)
-        alpha_new, delta = decompose(m, g32)
-        ratios = compute_block_ratios(delta, m)
-        tau0, tau1 = compute_thresholds(ratios, self._null_pct, self._amp_pct)
-        labels = classify_blocks(ratios, tau0, tau1)
-        enc = encode_blocks(delta, labels)
-        if self._error_feedback:
-            zero = torch.zeros(1, dtype=torch.float32, device=g.device)
-            ef_error = delta.reshape(-1) - _decode(enc, zero, g, n, True, False)
-            if self._ef_residual is None:
-                self._ef_residual = ef_error.reshape(g.shape)
+        dev = g.device
+        if self._encoded is None or self._encoded["labels"].device != dev:
+            self.allocate(n, dev)
+        lib = _lib.load()
+        gf = g.reshape(-1)
+        if gf.dtype not in _lib.DTYPES:
+            gf = gf.float()
+        gf = gf.contiguous()
+        nb = num_blocks(n)
+        if self._has_state:
+            _check_covers(self._encoded, n)
+        # the arrays the kernels update in place; a copy where one is not in
+        # their form, written back after
+        held = {k: _in_form(self._encoded[k], dt, dev) for k, dt in _ENCODED_DTYPES.items()}
+        sizes = {"labels": nb, "sign_packed": (n + 7) // 8, "block_norms": nb, "scales": nb}
+        if any(held[k].numel() != c for k, c in sizes.items()):
+            raise RuntimeError(f"CoStateManager.update: the state arrays do not match {n} elements ({nb} blocks)")
+        alpha = _scalar_on(self._alpha, dev)
+        res = None
+        if self._error_feedback:  # a new tensor each update, as the reference rebinds it
+            old = self._ef_residual
+            if old is None:
+                res = torch.empty(n, dtype=torch.float32, device=dev)
             else:
-                self._ef_residual = (beta1 * self._ef_residual.reshape(-1).float()
-                                     + (1.0 - beta1) * ef_error).reshape(g.shape)
-        for k in ("labels", "sign_packed", "block_norms", "scales"):
-            self._encoded[k].copy_(enc[k])
-        if isinstance(self._alpha, torch.Tensor):
-            self._alpha.copy_(alpha_new)
-        else:
-            self._alpha = alpha_new.clone()
+                if old.numel() != n or old.device != dev:
+                    raise RuntimeError("CoStateManager.update: the residual does not match the gradient")
+                res = old.detach().reshape(-1).to(torch.float32, copy=True).contiguous()
+        m = torch.empty(n, dtype=torch.float32, device=dev)
+        ws = torch.empty(lib.tam_costate_update_workspace(n, int(res is not None)), dtype=torch.uint8, device=dev)
+        k_lo, k_hi = self.ranks(nb)
+        b1, ob1 = ctypes.c_float(beta1).value, ctypes.c_float(1.0 - beta1).value
+        with torch.cuda.device(dev):
+            _lib.check(lib.tam_costate_update(
+                gf.data_ptr(), _lib.DTYPES[gf.dtype], n, held["labels"].data_ptr(), held["sign_packed"].data_ptr(),
+                held["block_norms"].data_ptr(), held["scales"].data_ptr(), alpha.data_ptr(), int(self._has_state), b1,
+                ob1, k_lo, k_hi, 0 if res is None else res.data_ptr(), int(self._ef_residual is not None),
+                m.data_ptr(), ws.data_ptr(), ws.numel(), _lib.stream_of(dev)), "tam_costate_update")
+        for k, t in held.items():
+            if t is not self._encoded[k]:
+                self._encoded[k].copy_(t.reshape(self._encoded[k].shape))
+        if not isinstance(self._alpha, torch.Tensor):
+            self._alpha = alpha.reshape(())
+        elif alpha.data_ptr() != self._alpha.data_ptr():
+            self._alpha.copy_(alpha.reshape(self._alpha.shape))
+        if res is not None:
+            self._ef_residual = res.reshape(g.shape)
         self._original_numel = n
         self._has_state = True
         return m.reshape(g.shape)

@@ -2805,6 +2805,76 @@ __global__ __launch_bounds__(TAM_WG) void tam_k_decode(const uint8_t* __restrict
   tam_st8_f32<false>(out, W.e0, W.nv, m);
 }
 
+// The first launch of CoStateManager.update (costate.py:367-416) on one tensor:
+// the EMA m of the decoded previous state, written out, and the quarter partials
+// of g.g and m.g, in pass 0's units (last quarters bounds-checked).  d comes as a
+// kernel argument; *desc receives it for the step's passes 1 to 4, which do the
+// rest of the update (pass 2 recomputes m: g and the encoding are fewer bytes
+// than m).
+template <uint32_t DT>
+__global__ __launch_bounds__(TAM_WG) void tam_k_costate_m(const TamTensor d, TamTensor* __restrict__ desc,
+                                                          float* __restrict__ m_out, double2* __restrict__ partials) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *desc = d;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+  const bool has_state = (d.flags & TAM_FLAG_HAS_STATE) != 0, has_ef = (d.flags & TAM_FLAG_HAS_EF) != 0;
+  const uint32_t nfull = (uint32_t)(d.n / (8u * TAM_BLOCK_SIZE)), items = nfull + (d.nb + 3u) / 4u - 2u * nfull;
+  for (uint32_t w = blockIdx.x * (TAM_WG / 64) + wave; w < items; w += gridDim.x * (TAM_WG / 64)) {
+    if (w < nfull) {
+      const uint32_t b = w * 8u + (lane >> 3);
+      const uint64_t e0 = (uint64_t)b * TAM_BLOCK_SIZE + (lane & 7u) * TAM_EPU;
+      float g[TAM_EPU], ge[TAM_EPU], m[TAM_EPU];
+      tam_ld16<DT>(d.grad, e0, g);
+      TamCsIn cs = {0u, 0u, 0u, 0.0f};
+      uint32_t sbytes = 0u;
+      float alpha_prev = 0.0f;
+      if (has_state) {
+        cs.label = tam_g(d.labels)[b];
+        cs.nrm = tam_g(d.norms)[b];
+        cs.amp = tam_g(d.amp)[b];
+        sbytes = tam_g((const uint16_t*)(d.signs + (e0 >> 3)))[0];
+        alpha_prev = tam_g(d.alpha)[0];
+      }
+      if (has_ef) {  // costate.py:410-413
+        tam_ld16<TAM_DTYPE_F32>(d.ef_residual, e0, ge);
+#pragma unroll
+        for (int i = 0; i < TAM_EPU; ++i) ge[i] = g[i] + ge[i];
+      } else {
+#pragma unroll
+        for (int i = 0; i < TAM_EPU; ++i) ge[i] = g[i];
+      }
+      if (has_state) {
+        const uint32_t sabs = tam_cs_sabs(cs);
+        tam_cs_decode_m<true>(d, sabs, sbytes & 0xffu, alpha_prev, g, ge, m);
+        tam_cs_decode_m<true>(d, sabs, sbytes >> 8, alpha_prev, g + TAM_EPL, ge + TAM_EPL, m + TAM_EPL);
+      } else {
+#pragma unroll
+        for (int i = 0; i < TAM_EPU; ++i) m[i] = d.beta1 * 0.0f + d.one_minus_beta1 * ge[i];
+      }
+      const double t = tam_unit_sum2((double)tam_lane_dot(g, g) + (double)tam_lane_dot(g + TAM_EPL, g + TAM_EPL),
+                                     (double)tam_lane_dot(m, g) + (double)tam_lane_dot(m + TAM_EPL, g + TAM_EPL),
+                                     lane);
+      double* part = (double*)(partials + 2u * (uint64_t)w);
+      if ((lane & 31u) - 12u < 2u) tam_g(part)[(lane >> 5) * 2u + (lane & 1u)] = t;
+      tam_st16_f32(m_out, e0, m);
+    } else {
+      const uint32_t wq = 2u * nfull + (w - nfull);
+      const TamWave W = tam_wave(d, wq, lane, false);
+      float g[TAM_EPL], ge[TAM_EPL], m[TAM_EPL];
+      tam_ld8<DT, false>(d.grad, W.e0, W.nv, g);  // elements past n read 0
+      const TamCsIn cs = tam_cs_load<false>(d, W);
+      const float alpha_prev = has_state ? tam_g(d.alpha)[0] : 0.0f;
+      tam_ef_grad<false>(d, W, g, ge);
+      tam_costate_m<false>(d, W, cs, alpha_prev, g, ge, m);
+      tam_st8_f32<false>(m_out, W.e0, W.nv, m);
+#pragma unroll
+      for (int i = 0; i < TAM_EPL; ++i)
+        if ((uint32_t)i >= W.nv) m[i] = 0.0f;
+      const double t = tam_quarter_sum2((double)tam_lane_dot(g, g), (double)tam_lane_dot(m, g), lane);
+      if (lane - 12u < 2u) tam_g((double*)(partials + wq))[lane - 12u] = t;
+    }
+  }
+}
+
 // Quarter partials of g.g and m.g (fp32 inputs), as pass 1 forms them.
 __global__ __launch_bounds__(TAM_WG) void tam_k_dot_quarters(const float* __restrict__ m, const float* __restrict__ g,
                                                              uint64_t n, double2* __restrict__ partials) {
@@ -3775,6 +3845,78 @@ int tam_decompose(const float* m, const float* g, uint64_t n, float* alpha, floa
   }
   hipLaunchKernelGGL(tam_k_delta, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, m, g, n, alpha, delta);
   TAM_HIP_CHECK(hipGetLastError());
+  return TAM_OK;
+}
+
+// One tensor's descriptor at the start of the workspace of tam_costate_update,
+// the step's workspace after it.
+#define TAM_COSTATE_DESC_BYTES 512
+static_assert(sizeof(TamTensor) <= TAM_COSTATE_DESC_BYTES, "the descriptor fits its share of the workspace");
+
+// The descriptor of a CoState update without a parameter or second moment
+// (passes 1 to 4 read neither).
+static int tam_costate_prepare(TamTensor* t, TamStepInfo* info) {
+  t->param = (void*)t->grad;
+  t->exp_avg_sq = (float*)(uintptr_t)16;  // not read
+  t->bias_correction1 = 1.0f;
+  t->sqrt_block = TAM_SQRT_BLOCK_F;
+  return tam_prepare(t, 1, info);
+}
+
+size_t tam_costate_update_workspace(uint64_t n, int error_feedback) {
+  TamTensor t;
+  TamStepInfo info;
+  memset(&t, 0, sizeof(t));
+  t.grad = t.labels = t.signs = (uint8_t*)(uintptr_t)16;
+  t.norms = t.alpha = t.ef_residual = (float*)(uintptr_t)16;
+  t.amp = (uint16_t*)(uintptr_t)16;
+  t.n = n;
+  t.flags = TAM_FLAG_COSTATE | (error_feedback ? TAM_FLAG_EF : 0u);
+  if (tam_costate_prepare(&t, &info) != TAM_OK) return 0;
+  return (size_t)info.ws_bytes + TAM_COSTATE_DESC_BYTES;
+}
+
+int tam_costate_update(const void* g, uint32_t g_dtype, uint64_t n, uint8_t* labels, uint8_t* signs, float* norms,
+                       uint16_t* amp, float* alpha, int has_state, float beta1, float one_minus_beta1, uint32_t k_lo,
+                       uint32_t k_hi, float* ef_residual, int has_residual, float* m_out, void* workspace,
+                       size_t ws_bytes, void* stream) {
+  tam_err_buf[0] = 0;
+  if (!g || !m_out || !workspace) return tam_fail(TAM_E_INVALID, "%snull argument", "");
+  TamTensor t;
+  TamStepInfo info;
+  memset(&t, 0, sizeof(t));
+  t.grad = g;
+  t.labels = labels;
+  t.signs = signs;
+  t.norms = norms;
+  t.amp = amp;
+  t.alpha = alpha;
+  t.n = n;
+  t.dtype = g_dtype;
+  t.k_lo = k_lo;
+  t.k_hi = k_hi;
+  t.beta1 = beta1;
+  t.one_minus_beta1 = one_minus_beta1;
+  t.ef_residual = ef_residual;
+  t.flags = TAM_FLAG_COSTATE | (has_state ? TAM_FLAG_HAS_STATE : 0u);
+  if (ef_residual) t.flags |= TAM_FLAG_EF | (has_residual ? TAM_FLAG_HAS_EF : 0u);
+  int rc = tam_costate_prepare(&t, &info);
+  if (rc != TAM_OK) return rc;
+  if (ws_bytes < info.ws_bytes + TAM_COSTATE_DESC_BYTES)
+    return tam_fail(TAM_E_WORKSPACE, "%sworkspace too small: need %ld bytes", "",
+                    (long)(info.ws_bytes + TAM_COSTATE_DESC_BYTES));
+  TamTensor* desc = (TamTensor*)workspace;
+  char* ws = (char*)workspace + TAM_COSTATE_DESC_BYTES;
+  const auto kernel = g_dtype == TAM_DTYPE_BF16 ? tam_k_costate_m<TAM_DTYPE_BF16>
+                      : g_dtype == TAM_DTYPE_F16 ? tam_k_costate_m<TAM_DTYPE_F16>
+                                                 : tam_k_costate_m<TAM_DTYPE_F32>;
+  hipLaunchKernelGGL(kernel, dim3(tam_codec_grid((n + 1023) / 1024 + 1)), dim3(TAM_WG), 0, (hipStream_t)stream, t, desc,
+                     m_out, (double2*)(ws + info.off_partials));
+  TAM_HIP_CHECK(hipGetLastError());
+  for (int pass = 1; pass < 5; ++pass) {
+    rc = tam_launch_pass(pass, desc, &info, 0, ws, info.ws_bytes, (hipStream_t)stream);
+    if (rc != TAM_OK) return rc;
+  }
   return TAM_OK;
 }
 
