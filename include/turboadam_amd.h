@@ -154,6 +154,9 @@ typedef struct TamStepInfo {
   uint32_t sel_small;      /* a CoState tensor of at most this many blocks is one workgroup's selection: */
                            /* 32768, or 12288 when some tensor has more than 32768 (slices run then) */
   uint32_t sel_max;        /* blocks of the largest such tensor (0: none) */
+  uint32_t ef_mask;        /* bit TAM_DTYPE_x set when a tensor of that dtype with TAM_FLAG_EF is present */
+  uint32_t v_f32_mask;     /* dtype_mask's bits whose tensors without EF all lack TAM_FLAG_COMPRESS_V, */
+  uint32_t m_f32_mask;     /* and whose all have it and lack TAM_FLAG_COSTATE */
 } TamStepInfo;
 
 /* Version of this ABI (TAM_ABI_VERSION). */
@@ -302,7 +305,8 @@ int tam_v_compress(const float* v, uint64_t n, uint32_t v_bits, int stochastic, 
  * `fn` (0 log, 1 exp, 2 f32->f16->f32, 3 f32->bf16->f32 in software, 4 sqrt,
  * 5 f32->bf16->f32 by the hardware conversion; the raw hardware instructions
  * whose error bounds the certified fast paths assume: 6 v_sqrt_f32,
- * 7 v_rcp_f32, 8 v_log_f32 (log2)).  No counterpart in the reference: it lets
+ * 7 v_rcp_f32, 8 v_log_f32 (log2); and the fp32 update's own operations: 9
+ * square root (inputs from 2^-62), 10 reciprocal (inputs up to 2^126)).  No counterpart in the reference: it lets
  * a caller confirm the device math equals the host. */
 int tam_math_eval(int fn, const float* in, float* out, uint64_t n, void* stream);
 

@@ -232,3 +232,19 @@ def test_costate_update_units(n, dt, ef):
         for k, t in got.items():
             a, b = np.ascontiguousarray(_np(t)), want[k]
             assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), f"step {s}: {k}"
+
+
+# pass 0 has a kernel for each mode (fp32 first moment, fp32 second moment, error feedback, any), pass 2 for
+# error feedback; mixed: tensors of two modes in one dtype
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("dt", [O.DT_F32, O.DT_BF16, O.DT_F16])
+@pytest.mark.parametrize("kw", [dict(compress_m=False), dict(compress_v=False), dict(compress_m=False, compress_v=False),
+                                dict(error_feedback=True), dict(error_feedback=True, compress_v=False),
+                                dict(error_feedback=True, v_bits=8), dict(min_m_compress_elements=6000)])
+def test_step_modes(kw, dt, offset):
+    from tests.helpers import run_side_by_side
+
+    log(f"step {kw} dtype {dt} offset {offset}")
+    sizes = [1024 * 5 + 300, 4096, 1024 * 2, 700, 9000, 512 * 17]
+    bad = run_side_by_side(sizes, [dt] * len(sizes), steps=3, offset=offset, **kw)
+    assert not bad, "\n".join(bad[:10])

@@ -107,6 +107,9 @@ class TamStepInfo(ctypes.Structure):
         ("tail_blocks", ctypes.c_uint32),
         ("sel_small", ctypes.c_uint32),
         ("sel_max", ctypes.c_uint32),
+        ("ef_mask", ctypes.c_uint32),
+        ("v_f32_mask", ctypes.c_uint32),
+        ("m_f32_mask", ctypes.c_uint32),
     ]
 
 

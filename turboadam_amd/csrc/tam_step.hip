@@ -130,28 +130,15 @@ typedef uint32_t TamW4E __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t TamW4B __attribute__((ext_vector_type(4), aligned(1)));
 typedef uint32_t TamW2B __attribute__((ext_vector_type(2), aligned(1)));
 typedef uint32_t TamW1B __attribute__((aligned(1)));
+typedef uint16_t TamH1B __attribute__((aligned(1)));
 
-// 16 consecutive elements of an array of dtype DT as fp32 (all exist).
+// 16 consecutive elements of an array of a 16-bit dtype DT as fp32 (all exist).
 template <uint32_t DT>
 __device__ __forceinline__ void tam_ld16(const void* base, uint64_t e0, float* out) {
-  if constexpr (DT == TAM_DTYPE_F32) {
-    const TAM_GLOBAL TamF4E* b = tam_g((const TamF4E*)((const float*)base + e0));
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const TamF4 x = b[k];
-      out[4 * k] = x.x; out[4 * k + 1] = x.y; out[4 * k + 2] = x.z; out[4 * k + 3] = x.w;
-    }
-  } else {
-    const TAM_GLOBAL TamW4E* b = tam_g((const TamW4E*)((const uint16_t*)base + e0));
-    const TamW4 x = b[0], y = b[1];
-    tam_unpack8<DT>(x, out);
-    tam_unpack8<DT>(y, out + 8);
-  }
-}
-__device__ __forceinline__ void tam_st16_f32(float* base, uint64_t e0, const float* v) {
-  TAM_GLOBAL TamF4E* b = tam_g((TamF4E*)(base + e0));
-#pragma unroll
-  for (int k = 0; k < 4; ++k) b[k] = TamF4{v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]};
+  const TAM_GLOBAL TamW4E* b = tam_g((const TamW4E*)((const uint16_t*)base + e0));
+  const TamW4 x = b[0], y = b[1];
+  tam_unpack8<DT>(x, out);
+  tam_unpack8<DT>(y, out + 8);
 }
 
 // Elements [e0, e0+8) of a parameter or gradient.  FULL: all 8 exist;
@@ -357,6 +344,7 @@ __device__ __forceinline__ void tam_compiler_fence() { asm volatile("" ::: "memo
 __device__ __forceinline__ void tam_pin(uint32_t& x) { asm volatile("" : "+v"(x)); }
 __device__ __forceinline__ void tam_pin(float& x) { asm volatile("" : "+v"(x)); }
 __device__ __forceinline__ void tam_pin(TamW4& x) { asm volatile("" : "+v"(x)); }
+__device__ __forceinline__ void tam_pin(TamF4& x) { asm volatile("" : "+v"(x)); }
 
 // Instruction choices the compiler would not make by itself.  On gfx950 a
 // shift or v_and_or_b32 issues at half the rate of v_add_u32 or of a
@@ -391,6 +379,92 @@ __device__ __forceinline__ void tam_wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// ---------------------------------------------------------------------------
+// a unit's fp32 arrays
+// ---------------------------------------------------------------------------
+// A lane of a unit owns 16 consecutive elements: 64 bytes of an fp32 array.
+// Loaded or stored in place, each of its four 16-byte accesses leaves a 64-byte
+// stride between lanes, and a wave touches every 128-byte line four times: such
+// a stream reads 4.9 and writes 3.8 TB/s where whole lines at a time give 6.1
+// (4 GiB arrays).  So the wave moves 1 KB per instruction, lane after lane, and
+// turns the rows in LDS.  The unit's 256 16-byte chunks q (element 4 q) lie at
+// slot q ^ ((q >> 4) & 3): a wave's 16-byte accesses, by chunk 64 k + lane or by
+// chunk 4 lane + j, then touch every bank once per 16 lanes.
+struct TamTurn {
+  TamW4 slot[256];
+};
+struct TamTurnAt {  // byte addresses of a lane's slots
+  uint32_t col, row;
+};
+__device__ __forceinline__ TamTurnAt tam_turn_at(TamTurn* t, uint32_t lane) {
+  // opaque: formed where they are used rather than held across the unit loop
+  // (two registers that the kernels do not have)
+  asm volatile("" : "+v"(lane));
+  const uint32_t base = (uint32_t)(uintptr_t)(TAM_LDS TamTurn*)t;
+  TamTurnAt at;
+  at.col = base + 16u * (lane ^ ((lane >> 4) & 3u));         // chunk 64 k + lane: + 1024 k
+  at.row = base + 64u * lane + 16u * ((lane >> 2) & 3u);     // chunk 4 lane + j: ^ 16 j
+  return at;
+}
+__device__ __forceinline__ TAM_LDS TamF4* tam_lds_f4(uint32_t addr) { return (TAM_LDS TamF4*)(uintptr_t)addr; }
+
+// Chunk 64 k + lane of the unit at element e of an fp32 array, k = 0..3.  NT:
+// nontemporal, for what no later pass reads again (the parameter and the
+// moments, the gradient in pass 2): 1127 -> 1053 us for 2^28 elements with an
+// fp32 first moment; a gradient that pass 2 still reads is left to the caches.
+template <bool NT = false>
+__device__ __forceinline__ void tam_unit_ld(const float* base, uint64_t e, uint32_t lane, TamF4* w) {
+  const TAM_GLOBAL TamF4E* b = tam_g((const TamF4E*)(base + e)) + lane;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) w[k] = NT ? __builtin_nontemporal_load(b + 64 * k) : b[64 * k];
+}
+__device__ __forceinline__ void tam_unit_st(float* base, uint64_t e, uint32_t lane, const TamF4* w) {
+  TAM_GLOBAL TamF4E* b = tam_g((TamF4E*)(base + e)) + lane;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) b[64 * k] = w[k];
+}
+// From chunks 64 k + lane to the lane's own 16 elements, and back.  Every lane of
+// the wave takes part.
+__device__ __forceinline__ void tam_turn_in(TamTurn* t, uint32_t lane, const TamF4* w, float* x) {
+  const TamTurnAt at = tam_turn_at(t, lane);
+#pragma unroll
+  for (uint32_t k = 0; k < 4u; ++k) *tam_lds_f4(at.col + 1024u * k) = w[k];
+  tam_wave_lds_sync();
+#pragma unroll
+  for (uint32_t j = 0; j < 4u; ++j) {
+    const TamF4 y = *tam_lds_f4(at.row ^ (16u * j));
+    x[4 * j] = y.x; x[4 * j + 1] = y.y; x[4 * j + 2] = y.z; x[4 * j + 3] = y.w;
+  }
+  tam_wave_lds_sync();
+}
+__device__ __forceinline__ void tam_turn_out(TamTurn* t, uint32_t lane, const float* x, TamF4* w) {
+  const TamTurnAt at = tam_turn_at(t, lane);
+#pragma unroll
+  for (uint32_t j = 0; j < 4u; ++j)
+    *tam_lds_f4(at.row ^ (16u * j)) = TamF4{x[4 * j], x[4 * j + 1], x[4 * j + 2], x[4 * j + 3]};
+  tam_wave_lds_sync();
+#pragma unroll
+  for (uint32_t k = 0; k < 4u; ++k) w[k] = *tam_lds_f4(at.col + 1024u * k);
+  tam_wave_lds_sync();
+}
+// A lane's 16 elements of the unit at element e of an array of dtype DT.
+template <uint32_t DT>
+__device__ __forceinline__ void tam_unit_load(TamTurn* t, const void* base, uint64_t e, uint32_t lane, float* x) {
+  if constexpr (DT == TAM_DTYPE_F32) {
+    TamF4 w[4];
+    tam_unit_ld((const float*)base, e, lane, w);
+    tam_turn_in(t, lane, w, x);
+  } else {
+    tam_ld16<DT>(base, e + 16u * lane, x);
+  }
+}
+__device__ __forceinline__ void tam_unit_store(TamTurn* t, float* base, uint64_t e, uint32_t lane,
+                                               const float* x) {
+  TamF4 w[4];
+  tam_turn_out(t, lane, x, w);
+  tam_unit_st(base, e, lane, w);
 }
 
 // ---------------------------------------------------------------------------
@@ -1135,7 +1209,7 @@ __device__ __forceinline__ bool tam_step_skipped(const TamTensor* __restrict__ T
 // Per quarter tile: loads, first moment (CoState or fp32), second moment (1Q or
 // fp32), update, store; for CoState tensors the fp64 partial sums of g.g and
 // m.g over the quarter's 4 blocks (pairwise: blocks, then pairs of blocks).
-template <uint32_t DT, bool FULL, bool EF = false>
+template <uint32_t DT, bool FULL>
 __device__ __forceinline__ void tam_k1_quarter(const TamTensor& d, uint32_t wq, uint32_t lane, float* lutw,
                                                const TamLdsTabs* tabs, uint32_t seed_lo, uint32_t seed_hi,
                                                double2* __restrict__ part) {
@@ -1160,13 +1234,9 @@ __device__ __forceinline__ void tam_k1_quarter(const TamTensor& d, uint32_t wq, 
 
   // ---- first moment ---------------------------------------------------
   if (costate) {
-    if (EF) {  // error feedback: the EMA takes g + residual (costate.py:410-416)
-      float ge[TAM_EPL];
-      tam_ef_grad<FULL>(d, W, g, ge);
-      if (FULL || W.bvalid) tam_costate_m<FULL>(d, W, cs, alpha_prev, g, ge, m);
-    } else if (FULL || W.bvalid) {
-      tam_costate_m<FULL>(d, W, cs, alpha_prev, g, g, m);
-    }
+    float ge[TAM_EPL];  // error feedback: the EMA takes g + residual (costate.py:410-416)
+    tam_ef_grad<FULL>(d, W, g, ge);
+    if (FULL || W.bvalid) tam_costate_m<FULL>(d, W, cs, alpha_prev, g, ge, m);
     float gz[TAM_EPL], mz[TAM_EPL];
 #pragma unroll
     for (int i = 0; i < TAM_EPL; ++i) {
@@ -1482,21 +1552,36 @@ __device__ __forceinline__ void tam_vunit_b(const TamTensor& d, uint32_t lane, u
 // the unit's two quarters (part: quarter 2u's {g.g, m.g}, then 2u + 1's).
 // Every load of the unit (but an fp32 parameter's) is issued first and its
 // value pinned, so the unit waits on memory once.
-template <uint32_t DT>
+//
+// MODE fixes what a kernel's tensors have in common, so that its registers and
+// its first loads are theirs:
+//   TAM_K1_ANY     flags decide (fp32 moments are loaded when they are needed:
+//                  up front their registers would count against every unit)
+//   TAM_K1_V_F32   fp32 second moment (loaded up front, no 1Q code), either first
+//   TAM_K1_M_F32   fp32 first moment (loaded up front), 1Q second
+//   TAM_K1_EF      CoState with error feedback (the residual is loaded up front)
+enum { TAM_K1_ANY, TAM_K1_V_F32, TAM_K1_M_F32, TAM_K1_EF };
+template <uint32_t DT, int MODE>
 __device__ __forceinline__ void tam_k1_unit(const TamTensor& d, uint32_t u, uint32_t lane, float* lutw,
-                                            const TamLdsTabs* tabs, uint32_t seed_lo, uint32_t seed_hi,
-                                            double* __restrict__ part) {
+                                            const TamLdsTabs* tabs, TamTurn* turn, uint32_t seed_lo,
+                                            uint32_t seed_hi, double* __restrict__ part) {
   constexpr int NW = DT == TAM_DTYPE_F32 ? 4 : 2;  // 16-byte words per lane of a parameter-dtype array
   const uint32_t l8 = lane & 7u;
   const uint32_t b = u * 8u + (lane >> 3);
   const uint64_t e0 = (uint64_t)b * TAM_BLOCK_SIZE + l8 * TAM_EPU;
-  const bool costate = (d.flags & TAM_FLAG_COSTATE) != 0;
-  const bool compress_v = (d.flags & TAM_FLAG_COMPRESS_V) != 0;
+  const bool costate = MODE == TAM_K1_EF || (MODE != TAM_K1_M_F32 && (d.flags & TAM_FLAG_COSTATE) != 0);
+  const bool compress_v = MODE == TAM_K1_M_F32 || (MODE != TAM_K1_V_F32 && (d.flags & TAM_FLAG_COMPRESS_V) != 0);
   const bool has_state = costate && (d.flags & TAM_FLAG_HAS_STATE);
   const uint64_t off = e0 * (DT == TAM_DTYPE_F32 ? 4u : 2u);
+  const uint64_t eu = (uint64_t)u * (8u * TAM_BLOCK_SIZE);  // the unit's first element
   TamW4 gw[NW], pw[NW];
+  TamF4 gf[4];
+  if constexpr (DT == TAM_DTYPE_F32) {
+    tam_unit_ld((const float*)d.grad, eu, lane, gf);
+  } else {
 #pragma unroll
-  for (int k = 0; k < NW; ++k) gw[k] = tam_g((const TamW4E*)((const char*)d.grad + off))[k];
+    for (int k = 0; k < NW; ++k) gw[k] = tam_g((const TamW4E*)((const char*)d.grad + off))[k];
+  }
   // an fp32 parameter (16 registers) is loaded just before the update: held
   // from here it would make the kernel spill at 4 waves per SIMD
   if constexpr (DT != TAM_DTYPE_F32) {
@@ -1518,11 +1603,23 @@ __device__ __forceinline__ void tam_k1_unit(const TamTensor& d, uint32_t u, uint
     sc = tam_g((const uint32_t*)d.v_scales)[b];
     iw = tam_g((const TamW4*)(d.v_idx + e0))[0];
   }
+  TamF4 early[4] = {};  // the mode's fp32 array
+  const bool has_ef = MODE == TAM_K1_EF && (d.flags & TAM_FLAG_HAS_EF) != 0;
+  if constexpr (MODE == TAM_K1_V_F32) tam_unit_ld<true>(d.exp_avg_sq, eu, lane, early);
+  if constexpr (MODE == TAM_K1_M_F32) tam_unit_ld<true>(d.exp_avg, eu, lane, early);
+  if constexpr (MODE == TAM_K1_EF) {
+    if (has_ef) tam_unit_ld(d.ef_residual, eu, lane, early);
+  }
   tam_compiler_fence();
+  if constexpr (DT == TAM_DTYPE_F32) {
 #pragma unroll
-  for (int k = 0; k < NW; ++k) {
-    tam_pin(gw[k]);
-    if constexpr (DT != TAM_DTYPE_F32) tam_pin(pw[k]);
+    for (int k = 0; k < 4; ++k) tam_pin(gf[k]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < NW; ++k) {
+      tam_pin(gw[k]);
+      tam_pin(pw[k]);
+    }
   }
   tam_pin(label);
   tam_pin(nrm);
@@ -1531,13 +1628,13 @@ __device__ __forceinline__ void tam_k1_unit(const TamTensor& d, uint32_t u, uint
   tam_pin(alpha_prev);
   tam_pin(sc);
   tam_pin(iw);
+  if constexpr (MODE != TAM_K1_ANY) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) tam_pin(early[k]);
+  }
   float g[TAM_EPU], p[TAM_EPU], m[TAM_EPU], v[TAM_EPU];
   if constexpr (DT == TAM_DTYPE_F32) {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const TamF4 gk = __builtin_bit_cast(TamF4, gw[k]);
-      g[4 * k] = gk.x; g[4 * k + 1] = gk.y; g[4 * k + 2] = gk.z; g[4 * k + 3] = gk.w;
-    }
+    tam_turn_in(turn, lane, gf, g);
   } else {
     tam_unpack8<DT>(gw[0], g);
     tam_unpack8<DT>(gw[1], g + TAM_EPL);
@@ -1548,13 +1645,23 @@ __device__ __forceinline__ void tam_k1_unit(const TamTensor& d, uint32_t u, uint
 
   // ---- first moment ---------------------------------------------------
   if (costate) {
-    if (has_state) {
-      const uint32_t sabs = tam_cs_sabs(cs);  // shared by the lane's two sign bytes
-      tam_cs_decode_m<true>(d, sabs, sbytes & 0xffu, alpha_prev, g, g, m);
-      tam_cs_decode_m<true>(d, sabs, sbytes >> 8, alpha_prev, g + TAM_EPL, g + TAM_EPL, m + TAM_EPL);
+    // error feedback: the EMA takes g + residual (costate.py:410-416)
+    float ge[TAM_EPU];
+    if (MODE == TAM_K1_EF && has_ef) {
+      tam_turn_in(turn, lane, early, ge);
+#pragma unroll
+      for (int i = 0; i < TAM_EPU; ++i) ge[i] = g[i] + ge[i];
     } else {
 #pragma unroll
-      for (int i = 0; i < TAM_EPU; ++i) m[i] = d.beta1 * 0.0f + d.one_minus_beta1 * g[i];
+      for (int i = 0; i < TAM_EPU; ++i) ge[i] = g[i];
+    }
+    if (has_state) {
+      const uint32_t sabs = tam_cs_sabs(cs);  // shared by the lane's two sign bytes
+      tam_cs_decode_m<true>(d, sabs, sbytes & 0xffu, alpha_prev, g, ge, m);
+      tam_cs_decode_m<true>(d, sabs, sbytes >> 8, alpha_prev, g + TAM_EPL, ge + TAM_EPL, m + TAM_EPL);
+    } else {
+#pragma unroll
+      for (int i = 0; i < TAM_EPU; ++i) m[i] = d.beta1 * 0.0f + d.one_minus_beta1 * ge[i];
     }
     // lane partials in fp32, their fp64 sum, then per block and quarter in fp64
     const double t = tam_unit_sum2((double)tam_lane_dot(g, g) + (double)tam_lane_dot(g + TAM_EPL, g + TAM_EPL),
@@ -1563,15 +1670,17 @@ __device__ __forceinline__ void tam_k1_unit(const TamTensor& d, uint32_t u, uint
     if ((lane & 31u) - 12u < 2u) tam_g(part)[(lane >> 5) * 2u + (lane & 1u)] = t;
   } else {
     // fp32 exp_avg (optimizer.py:113): m = fma(1-b1, g, fl(m*b1))
-    // (fp32 moments are loaded here, not with the unit's other loads: their
-    // registers would otherwise count against every unit of the kernel)
     float ea[TAM_EPU];
-    tam_ld8_f32<true>(d.exp_avg, e0, TAM_EPL, ea);
-    tam_ld8_f32<true>(d.exp_avg, e0 + TAM_EPL, TAM_EPL, ea + TAM_EPL);
+    if constexpr (MODE == TAM_K1_M_F32) {
+      tam_turn_in(turn, lane, early, ea);
+    } else {
+      TamF4 w[4];
+      tam_unit_ld<true>(d.exp_avg, eu, lane, w);
+      tam_turn_in(turn, lane, w, ea);
+    }
 #pragma unroll
     for (int i = 0; i < TAM_EPU; ++i) m[i] = __builtin_fmaf(d.one_minus_beta1, g[i], ea[i] * d.beta1);
-    tam_st8_f32<true>(d.exp_avg, e0, TAM_EPL, m);
-    tam_st8_f32<true>(d.exp_avg, e0 + TAM_EPL, TAM_EPL, m + TAM_EPL);
+    tam_unit_store(turn, d.exp_avg, eu, lane, m);
   }
 
   // ---- second moment --------------------------------------------------
@@ -1581,22 +1690,24 @@ __device__ __forceinline__ void tam_k1_unit(const TamTensor& d, uint32_t u, uint
   } else {
     // fp32 exp_avg_sq (optimizer.py:166): v = fma(fl((1-b2)*g), g, fl(v*b2))
     float es[TAM_EPU];
-    tam_ld8_f32<true>(d.exp_avg_sq, e0, TAM_EPL, es);
-    tam_ld8_f32<true>(d.exp_avg_sq, e0 + TAM_EPL, TAM_EPL, es + TAM_EPL);
+    if constexpr (MODE == TAM_K1_V_F32) {
+      tam_turn_in(turn, lane, early, es);
+    } else {
+      TamF4 w[4];
+      tam_unit_ld<true>(d.exp_avg_sq, eu, lane, w);
+      tam_turn_in(turn, lane, w, es);
+    }
 #pragma unroll
     for (int i = 0; i < TAM_EPU; ++i) v[i] = __builtin_fmaf(d.one_minus_beta2 * g[i], g[i], es[i] * d.beta2);
-    tam_st8_f32<true>(d.exp_avg_sq, e0, TAM_EPL, v);
-    tam_st8_f32<true>(d.exp_avg_sq, e0 + TAM_EPL, TAM_EPL, v + TAM_EPL);
+    tam_unit_store(turn, d.exp_avg_sq, eu, lane, v);
   }
 
   // ---- parameter update -----------------------------------------------
   {
     if constexpr (DT == TAM_DTYPE_F32) {
-#pragma unroll
-      for (int k = 0; k < NW; ++k) {
-        const TamF4 pk = tam_g((const TamF4E*)((const char*)d.param + off))[k];
-        p[4 * k] = pk.x; p[4 * k + 1] = pk.y; p[4 * k + 2] = pk.z; p[4 * k + 3] = pk.w;
-      }
+      TamF4 pf[4];
+      tam_unit_ld<true>((const float*)d.param, eu, lane, pf);
+      tam_turn_in(turn, lane, pf, p);
     }
     uint32_t pw2[TAM_EPU / 2];
     bool q_ok = false;
@@ -1613,8 +1724,7 @@ __device__ __forceinline__ void tam_k1_unit(const TamTensor& d, uint32_t u, uint
     tam_update<DT>(d, p, m, v, pw2, q_ok);
     tam_update<DT>(d, p + TAM_EPL, m + TAM_EPL, v + TAM_EPL, pw2 + TAM_EPL / 2, q_ok);
     if (DT == TAM_DTYPE_F32) {
-      tam_st8_f32<true>((float*)d.param, e0, TAM_EPL, p);
-      tam_st8_f32<true>((float*)d.param, e0 + TAM_EPL, TAM_EPL, p + TAM_EPL);
+      tam_unit_store(turn, (float*)d.param, eu, lane, p);
     } else {
       tam_st8_bits<true>(d.param, e0, TAM_EPL, pw2);
       tam_st8_bits<true>(d.param, e0 + TAM_EPL, TAM_EPL, pw2 + TAM_EPL / 2);
@@ -1628,9 +1738,9 @@ __device__ __forceinline__ void tam_k1_unit(const TamTensor& d, uint32_t u, uint
 // Full units (inside the tensor) of one parameter dtype:
 // persistent workgroups of two waves stride over the tiles; wave w takes unit
 // 2(tile - tile0) + w of the tile's tensor (quarters 4(tile - tile0) + 2w and
-// + 2w + 1), and the waves never synchronise with each other.  One kernel per
-// dtype holds only that dtype's code, so each gets its own register budget.
-template <uint32_t DT>
+// + 1), and the waves never synchronise with each other.  One kernel per
+// dtype and mode holds only that code, so each gets its own register budget.
+template <uint32_t DT, int MODE>
 __device__ __forceinline__ void tam_k1_full_body(const TamTensor* __restrict__ T, int nT, uint32_t total_tiles,
                                                  uint32_t seed_lo, uint32_t seed_hi,
                                                  double2* __restrict__ partials) {
@@ -1638,7 +1748,8 @@ __device__ __forceinline__ void tam_k1_full_body(const TamTensor* __restrict__ T
   // rows of 64 levels, 256-byte aligned (tam_vunit_a forms addresses by or)
   __shared__ __attribute__((aligned(256))) float lut[TAM_K1_BLOCK / 64][8 * 64];
   __shared__ TamLdsTabs tabs;
-  tam_lds_tabs_fill(&tabs);
+  __shared__ TamTurn turn[TAM_K1_BLOCK / 64];
+  if constexpr (MODE != TAM_K1_V_F32) tam_lds_tabs_fill(&tabs);
   const uint32_t hw_wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
   const uint32_t wave = hw_wave & 1u;  // within the virtual workgroup
   const uint32_t stride = gridDim.x * TAM_K1_VWG;
@@ -1651,7 +1762,7 @@ __device__ __forceinline__ void tam_k1_full_body(const TamTensor* __restrict__ T
     ti = tam_advance_tensor(T, nT, ti, tile);
     const TamTensor& d = T[ti];
     const uint32_t end = d.tile0 + d.ntiles;  // the tensor's tiles end here
-    if (d.dtype == DT && !(d.flags & TAM_FLAG_EF)) {  // uniform; EF: tam_k1_ef
+    if (d.dtype == DT && ((d.flags & TAM_FLAG_EF) != 0) == (MODE == TAM_K1_EF)) {  // uniform
       // units u < nfull are full; the rest is tam_k1_tail's, and u grows with
       // the tile
       const uint64_t nfull = d.n / (8u * TAM_BLOCK_SIZE);
@@ -1659,18 +1770,18 @@ __device__ __forceinline__ void tam_k1_full_body(const TamTensor* __restrict__ T
         const uint32_t u = (tile - d.tile0) * 2u + wave;  // unit within the tensor
         if (u >= nfull) break;
         double* part = (double*)(partials + (uint64_t)tile * 4u + 2u * wave);
-        tam_k1_unit<DT>(d, u, lane, lutw, &tabs, seed_lo, seed_hi, part);
+        tam_k1_unit<DT, MODE>(d, u, lane, lutw, &tabs, &turn[hw_wave], seed_lo, seed_hi, part);
       }
     }
     while (tile < end) tile += stride;  // this workgroup's first tile past the tensor
   }
 }
 
-#define TAM_K1_FULL_KERNEL(NAME, DT, WAVES)                                                                     \
+#define TAM_K1_FULL_KERNEL(NAME, DT, MODE, WAVES)                                                               \
   __global__ __launch_bounds__(TAM_K1_BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES))) void NAME(    \
       const TamTensor* __restrict__ T, int nT, uint32_t total_tiles, uint32_t seed_lo, uint32_t seed_hi,      \
       double2* __restrict__ partials) {                                                                       \
-    tam_k1_full_body<DT>(T, nT, total_tiles, seed_lo, seed_hi, partials);                                     \
+    tam_k1_full_body<DT, MODE>(T, nT, total_tiles, seed_lo, seed_hi, partials);                               \
   }
 #ifndef TAM_K1_WAVES_BF16
 #define TAM_K1_WAVES_BF16 4
@@ -1681,9 +1792,24 @@ __device__ __forceinline__ void tam_k1_full_body(const TamTensor* __restrict__ T
 #ifndef TAM_K1_WAVES_F32
 #define TAM_K1_WAVES_F32 4
 #endif
-TAM_K1_FULL_KERNEL(tam_k1_main_bf16, TAM_DTYPE_BF16, TAM_K1_WAVES_BF16)
-TAM_K1_FULL_KERNEL(tam_k1_main_f16, TAM_DTYPE_F16, TAM_K1_WAVES_F16)
-TAM_K1_FULL_KERNEL(tam_k1_main_f32, TAM_DTYPE_F32, TAM_K1_WAVES_F32)
+#ifndef TAM_K1_WAVES_V_F32
+#define TAM_K1_WAVES_V_F32 5
+#endif
+#ifndef TAM_K1_WAVES_V_16
+#define TAM_K1_WAVES_V_16 5
+#endif
+TAM_K1_FULL_KERNEL(tam_k1_main_bf16, TAM_DTYPE_BF16, TAM_K1_ANY, TAM_K1_WAVES_BF16)
+TAM_K1_FULL_KERNEL(tam_k1_main_f16, TAM_DTYPE_F16, TAM_K1_ANY, TAM_K1_WAVES_F16)
+TAM_K1_FULL_KERNEL(tam_k1_main_f32, TAM_DTYPE_F32, TAM_K1_ANY, TAM_K1_WAVES_F32)
+TAM_K1_FULL_KERNEL(tam_k1_vf32_bf16, TAM_DTYPE_BF16, TAM_K1_V_F32, TAM_K1_WAVES_V_16)
+TAM_K1_FULL_KERNEL(tam_k1_vf32_f16, TAM_DTYPE_F16, TAM_K1_V_F32, TAM_K1_WAVES_V_16)
+TAM_K1_FULL_KERNEL(tam_k1_vf32_f32, TAM_DTYPE_F32, TAM_K1_V_F32, TAM_K1_WAVES_V_F32)
+TAM_K1_FULL_KERNEL(tam_k1_mf32_bf16, TAM_DTYPE_BF16, TAM_K1_M_F32, TAM_K1_WAVES_BF16)
+TAM_K1_FULL_KERNEL(tam_k1_mf32_f16, TAM_DTYPE_F16, TAM_K1_M_F32, TAM_K1_WAVES_F16)
+TAM_K1_FULL_KERNEL(tam_k1_mf32_f32, TAM_DTYPE_F32, TAM_K1_M_F32, TAM_K1_WAVES_F32)
+TAM_K1_FULL_KERNEL(tam_k1_ef_bf16, TAM_DTYPE_BF16, TAM_K1_EF, TAM_K1_WAVES_BF16)
+TAM_K1_FULL_KERNEL(tam_k1_ef_f16, TAM_DTYPE_F16, TAM_K1_EF, TAM_K1_WAVES_F16)
+TAM_K1_FULL_KERNEL(tam_k1_ef_f32, TAM_DTYPE_F32, TAM_K1_EF, TAM_K1_WAVES_F32)
 
 // The at most two quarters of each tensor outside full units, one workgroup per
 // tensor that has any (tam_prepare: tail0, tail_wgs), a wave per quarter.
@@ -1708,41 +1834,6 @@ __global__ __launch_bounds__(TAM_K1U_WG) void tam_k1_tail(const TamTensor* __res
         break;
       default:
         tam_k1_quarter<TAM_DTYPE_F32, false>(d, wq, lane, lut[wave], &tabs, seed_lo, seed_hi, part);
-        break;
-    }
-  }
-}
-
-// Every quarter of the tensors with error feedback (full or not, any dtype):
-// persistent workgroups stride over the tiles as the main kernels do.
-__global__ __launch_bounds__(TAM_WG) void tam_k1_ef(const TamTensor* __restrict__ T, int nT, uint32_t total_tiles,
-                                                    uint32_t seed_lo, uint32_t seed_hi,
-                                                    double2* __restrict__ partials) {
-  if (tam_step_skipped(T)) return;
-  __shared__ float lut[TAM_WG / 64][4 * 64];
-  __shared__ TamLdsTabs tabs;
-  tam_lds_tabs_fill(&tabs);
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-  int ti = tam_find_tensor(T, nT, blockIdx.x);
-  for (uint32_t tile = blockIdx.x; tile < total_tiles; tile += gridDim.x) {
-    ti = tam_advance_tensor(T, nT, ti, tile);
-    const TamTensor& d = T[ti];
-    if (!(d.flags & TAM_FLAG_EF)) continue;  // uniform over the workgroup
-    const uint32_t wq = (tile - d.tile0) * 4u + wave;
-    double2* part = partials + (uint64_t)tile * 4u + wave;
-    const bool full = tam_quarter_full(d, wq);
-    switch (d.dtype) {
-      case TAM_DTYPE_BF16:
-        if (full) tam_k1_quarter<TAM_DTYPE_BF16, true, true>(d, wq, lane, lut[wave], &tabs, seed_lo, seed_hi, part);
-        else tam_k1_quarter<TAM_DTYPE_BF16, false, true>(d, wq, lane, lut[wave], &tabs, seed_lo, seed_hi, part);
-        break;
-      case TAM_DTYPE_F16:
-        if (full) tam_k1_quarter<TAM_DTYPE_F16, true, true>(d, wq, lane, lut[wave], &tabs, seed_lo, seed_hi, part);
-        else tam_k1_quarter<TAM_DTYPE_F16, false, true>(d, wq, lane, lut[wave], &tabs, seed_lo, seed_hi, part);
-        break;
-      default:
-        if (full) tam_k1_quarter<TAM_DTYPE_F32, true, true>(d, wq, lane, lut[wave], &tabs, seed_lo, seed_hi, part);
-        else tam_k1_quarter<TAM_DTYPE_F32, false, true>(d, wq, lane, lut[wave], &tabs, seed_lo, seed_hi, part);
         break;
     }
   }
@@ -2031,8 +2122,15 @@ __device__ __forceinline__ void tam_k2_any(const TamTensor& d, uint32_t wq, uint
 // CoState state and its two sign bytes.  tam_k2_encode takes the units of
 // 16-bit tensors, tam_k2_encode_f32 those of fp32 tensors (when it runs).
 template <bool F32>
-struct TamK2U {
-  TamW4 g[F32 ? 4 : 2];
+struct TamK2U;
+template <>
+struct TamK2U<false> {
+  TamW4 g[2];
+  TamCsIn cs;  // byte: the sign bytes of elements e0..e0+7 (low) and e0+8..e0+15
+};
+template <>
+struct TamK2U<true> {
+  TamF4 g[4];  // chunks 64 k + lane of the unit (tam_unit_ld)
   TamCsIn cs;  // byte: the sign bytes of elements e0..e0+7 (low) and e0+8..e0+15
 };
 template <bool F32>
@@ -2043,10 +2141,14 @@ template <bool F32>
 __device__ __forceinline__ TamK2U<F32> tam_k2u_load(const TamTensor& d, uint32_t u, uint32_t lane) {
   const uint32_t b = u * 8u + (lane >> 3);
   const uint64_t e0 = (uint64_t)b * TAM_BLOCK_SIZE + (lane & 7u) * TAM_EPU;
-  const TAM_GLOBAL TamW4E* gp = tam_g((const TamW4E*)((const char*)d.grad + e0 * (F32 ? 4u : 2u)));
   TamK2U<F32> r;
+  if constexpr (F32) {
+    tam_unit_ld<true>((const float*)d.grad, (uint64_t)u * (8u * TAM_BLOCK_SIZE), lane, r.g);
+  } else {
+    const TAM_GLOBAL TamW4E* gp = tam_g((const TamW4E*)((const uint16_t*)d.grad + e0));
 #pragma unroll
-  for (int k = 0; k < (F32 ? 4 : 2); ++k) r.g[k] = gp[k];
+    for (int k = 0; k < 2; ++k) r.g[k] = gp[k];
+  }
   r.cs = TamCsIn{0u, 0u, 0u, 0.0f};
   if (d.flags & TAM_FLAG_HAS_STATE) {
     r.cs.label = tam_g(d.labels)[b];
@@ -2062,20 +2164,19 @@ __device__ __forceinline__ TamK2U<F32> tam_k2u_load(const TamTensor& d, uint32_t
 // delta and m from fp32 lane partials and an fp64 tree over the block's 8
 // lanes (the parity split of tam_unit_sum2: after row_ror:4 the sum of
 // delta^2 is in lanes 4 and 6 of the half-row, of m^2 in lanes 5 and 7), the
-// fp16 amplitude (lane 4) and the ratio (lane 5).
-template <uint32_t DT>
+// fp16 amplitude (lane 4) and the ratio (lane 5).  EF: the EMA takes g + residual
+// (ge) and the encoding goes to the tensor's staging area.
+template <uint32_t DT, bool EF = false>
 __device__ __forceinline__ void tam_k2_unit(const TamTensor& d, uint32_t u, uint32_t lane, float a,
-                                            float* __restrict__ ratios, const TamK2U<DT == TAM_DTYPE_F32>& in) {
+                                            float* __restrict__ ratios, const TamK2U<DT == TAM_DTYPE_F32>& in,
+                                            TamTurn* turn, const TamF4* residual = nullptr,
+                                            char* __restrict__ ws = nullptr) {
   const uint32_t l8 = lane & 7u;
   const uint32_t b = u * 8u + (lane >> 3);
   const uint64_t e0 = (uint64_t)b * TAM_BLOCK_SIZE + l8 * TAM_EPU;
   float g[TAM_EPU], m[TAM_EPU], dl[TAM_EPU];
   if constexpr (DT == TAM_DTYPE_F32) {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const TamF4 gk = __builtin_bit_cast(TamF4, in.g[k]);
-      g[4 * k] = gk.x; g[4 * k + 1] = gk.y; g[4 * k + 2] = gk.z; g[4 * k + 3] = gk.w;
-    }
+    tam_turn_in(turn, lane, in.g, g);
   } else {
     tam_unpack8<DT>(in.g[0], g);
     tam_unpack8<DT>(in.g[1], g + TAM_EPL);
@@ -2083,13 +2184,22 @@ __device__ __forceinline__ void tam_k2_unit(const TamTensor& d, uint32_t u, uint
   // a scalar load (alpha is not written in this pass): no vector-memory wait
   // covers the next unit's loads
   const float alpha_prev = (d.flags & TAM_FLAG_HAS_STATE) ? *(const TAM_CONST float*)d.alpha : 0.0f;
+  float ge[TAM_EPU];
+  if (EF && (d.flags & TAM_FLAG_HAS_EF)) {
+    tam_turn_in(turn, lane, residual, ge);
+#pragma unroll
+    for (int i = 0; i < TAM_EPU; ++i) ge[i] = g[i] + ge[i];
+  } else {
+#pragma unroll
+    for (int i = 0; i < TAM_EPU; ++i) ge[i] = g[i];
+  }
   TamWave W;  // only its bvalid is read (full unit)
   W.bvalid = true;
   TamCsIn c0 = in.cs, c1 = in.cs;
   c0.byte = in.cs.byte & 0xffu;
   c1.byte = in.cs.byte >> 8;
-  tam_costate_m<true, false>(d, W, c0, alpha_prev, g, g, m);
-  tam_costate_m<true, false>(d, W, c1, alpha_prev, g + TAM_EPL, g + TAM_EPL, m + TAM_EPL);
+  tam_costate_m<true, false>(d, W, c0, alpha_prev, g, ge, m);
+  tam_costate_m<true, false>(d, W, c1, alpha_prev, g + TAM_EPL, ge + TAM_EPL, m + TAM_EPL);
   uint32_t sb0 = 0u, sb1 = 0u;
 #pragma unroll
   for (int i = 0; i < TAM_EPU; ++i) {
@@ -2109,10 +2219,19 @@ __device__ __forceinline__ void tam_k2_unit(const TamTensor& d, uint32_t u, uint
   const float nd = odd ? ny : nx;  // costate.py:241
   const float nm = odd ? nx : ny;
   const float qv = nd / (odd ? nm : d.sqrt_block);  // costate.py:248 / :81-84
-  tam_g((uint16_t*)(d.signs + (e0 >> 3)))[0] = (uint16_t)(sb0 | (sb1 << 8));
+  float* norms = d.norms;
+  uint16_t* amp = d.amp;
+  if constexpr (EF) {
+    const TamStage st = tam_stage(d, ws);
+    norms = st.norms;
+    amp = st.amp;
+    tam_g((TamH1B*)(st.signs + (e0 >> 3)))[0] = (uint16_t)(sb0 | (sb1 << 8));
+  } else {
+    tam_g((uint16_t*)(d.signs + (e0 >> 3)))[0] = (uint16_t)(sb0 | (sb1 << 8));
+  }
   if (l8 == 4u) {
-    tam_g(d.norms)[b] = nd;
-    tam_g(d.amp)[b] = tam_f32_to_f16(qv);
+    tam_g(norms)[b] = nd;
+    tam_g(amp)[b] = tam_f32_to_f16(qv);
   } else if (l8 == 5u) {
     tam_g(ratios)[d.ratio_off + b] = nm == 0.0f ? 0.0f : qv;
   }
@@ -2125,10 +2244,10 @@ __device__ __forceinline__ void tam_k2_unit(const TamTensor& d, uint32_t u, uint
 // loads in flight.  Workgroups of two waves stride over the tiles; wave w takes
 // unit 2(tile - tile0) + w.  tam_k2_encode takes the full units of 16-bit
 // tensors, tam_k2_encode_f32 those of fp32 tensors (both: without error
-// feedback).  The kernel given `quarters` also takes, quarter by quarter
-// (tam_k2_any), every other unit of a CoState tensor: error feedback, not
-// full, or of the other kernel's dtype when that kernel does not run
-// (`other_units` false).
+// feedback, tam_k2_ef).  The kernel given `quarters` also takes, quarter by
+// quarter (tam_k2_any), every other unit of such a CoState tensor: not full, or
+// of the other kernel's dtype when that kernel does not run (`other_units`
+// false).
 #ifndef TAM_K2_WAVES
 #define TAM_K2_WAVES 7
 #endif
@@ -2141,6 +2260,11 @@ __device__ __forceinline__ void tam_k2_body(const TamTensor* __restrict__ T, int
                                             char* __restrict__ ws, bool quarters, bool other_units) {
   if (tam_step_skipped(T)) return;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+  TamTurn* turn = nullptr;
+  if constexpr (F32) {
+    __shared__ TamTurn turns[TAM_K1U_WG / 64];
+    turn = &turns[wave];
+  }
   const auto desc = [&](int i) -> const TamTensor& { return T[__builtin_amdgcn_readfirstlane(i)]; };
   const auto unit_of = [&](uint32_t tile, int ti) { return (tile - desc(ti).tile0) * 2u + wave; };
   // the next tile at or after `tile` with work for this wave (uniform)
@@ -2148,7 +2272,7 @@ __device__ __forceinline__ void tam_k2_body(const TamTensor* __restrict__ T, int
     for (; tile < total_tiles; tile += gridDim.x) {
       ti = tam_advance_tensor(T, nT, ti, tile);
       const TamTensor& dd = desc(ti);
-      if ((dd.flags & TAM_FLAG_COSTATE) && (quarters || tam_k2u_prefetchable<F32>(dd, unit_of(tile, ti))))
+      if ((dd.flags & (TAM_FLAG_COSTATE | TAM_FLAG_EF)) == TAM_FLAG_COSTATE && (quarters || tam_k2u_prefetchable<F32>(dd, unit_of(tile, ti))))
         return true;
     }
     return false;
@@ -2171,10 +2295,10 @@ __device__ __forceinline__ void tam_k2_body(const TamTensor* __restrict__ T, int
     if (npre_ok) npre = tam_k2u_load<F32>(desc(nti), unit_of(ntile, nti), lane);
     bool done = pre_ok;
     if constexpr (F32) {
-      if (pre_ok) tam_k2_unit<TAM_DTYPE_F32>(d, u, lane, a, ratios, pre);
+      if (pre_ok) tam_k2_unit<TAM_DTYPE_F32>(d, u, lane, a, ratios, pre, turn);
     } else {
-      if (pre_ok && d.dtype == TAM_DTYPE_BF16) tam_k2_unit<TAM_DTYPE_BF16>(d, u, lane, a, ratios, pre);
-      else if (pre_ok) tam_k2_unit<TAM_DTYPE_F16>(d, u, lane, a, ratios, pre);
+      if (pre_ok && d.dtype == TAM_DTYPE_BF16) tam_k2_unit<TAM_DTYPE_BF16>(d, u, lane, a, ratios, pre, turn);
+      else if (pre_ok) tam_k2_unit<TAM_DTYPE_F16>(d, u, lane, a, ratios, pre, turn);
     }
     if (!done && quarters && !(other_units && tam_k2u_prefetchable<!F32>(d, u))) {
       tam_k2_any(d, 2u * u, lane, a, ratios, ws);
@@ -2198,6 +2322,39 @@ __global__ __launch_bounds__(TAM_K1U_WG) __attribute__((amdgpu_waves_per_eu(TAM_
 tam_k2_encode_f32(const TamTensor* __restrict__ T, int nT, uint32_t total_tiles, const float* __restrict__ alpha_new,
                   float* __restrict__ ratios, char* __restrict__ ws, int quarters, int other_units) {
   tam_k2_body<true>(T, nT, total_tiles, alpha_new, ratios, ws, quarters != 0, other_units != 0);
+}
+
+// Pass 2 of the error-feedback tensors of one dtype: units of 16 elements per
+// lane as above (quarters, 8 per lane and loaded one after the other, took
+// 298 us for 218M bf16 elements), the residual loaded with the unit's other
+// inputs instead of a unit ahead (its 16 registers beside theirs would halve the
+// waves); the last quarters bounds-checked.
+template <uint32_t DT>
+__global__ __launch_bounds__(TAM_K1U_WG) void tam_k2_ef(const TamTensor* __restrict__ T, int nT, uint32_t total_tiles,
+                                                        const float* __restrict__ alpha_new,
+                                                        float* __restrict__ ratios, char* __restrict__ ws) {
+  if (tam_step_skipped(T)) return;
+  __shared__ TamTurn turn[TAM_K1U_WG / 64];
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+  uint32_t tile = tam_tile_slot(blockIdx.x, gridDim.x);
+  int ti = tam_find_tensor(T, nT, tile < total_tiles ? tile : total_tiles - 1u);
+  for (; tile < total_tiles; tile += gridDim.x) {
+    ti = __builtin_amdgcn_readfirstlane(tam_advance_tensor(T, nT, ti, tile));
+    const TamTensor& d = T[ti];
+    if (!(d.flags & TAM_FLAG_EF) || d.dtype != DT) continue;  // uniform
+    const uint32_t u = (tile - d.tile0) * 2u + wave;
+    const float a = *(const TAM_CONST float*)(alpha_new + ti);
+    if (tam_unit_full(d, u)) {
+      const TamK2U<DT == TAM_DTYPE_F32> in = tam_k2u_load<DT == TAM_DTYPE_F32>(d, u, lane);
+      TamF4 r[4] = {};
+      if (d.flags & TAM_FLAG_HAS_EF) tam_unit_ld(d.ef_residual, (uint64_t)u * (8u * TAM_BLOCK_SIZE), lane, r);
+      tam_compiler_fence();
+      tam_k2_unit<DT, true>(d, u, lane, a, ratios, in, &turn[wave], r, ws);
+    } else {
+      tam_k2_quarter<DT, false>(d, 2u * u, lane, a, ratios, ws);
+      tam_k2_quarter<DT, false>(d, 2u * u + 1u, lane, a, ratios, ws);
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -2815,7 +2972,9 @@ template <uint32_t DT>
 __global__ __launch_bounds__(TAM_WG) void tam_k_costate_m(const TamTensor d, TamTensor* __restrict__ desc,
                                                           float* __restrict__ m_out, double2* __restrict__ partials) {
   if (blockIdx.x == 0 && threadIdx.x == 0) *desc = d;
+  __shared__ TamTurn turns[TAM_WG / 64];
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+  TamTurn* turn = &turns[wave];
   const bool has_state = (d.flags & TAM_FLAG_HAS_STATE) != 0, has_ef = (d.flags & TAM_FLAG_HAS_EF) != 0;
   const uint32_t nfull = (uint32_t)(d.n / (8u * TAM_BLOCK_SIZE)), items = nfull + (d.nb + 3u) / 4u - 2u * nfull;
   for (uint32_t w = blockIdx.x * (TAM_WG / 64) + wave; w < items; w += gridDim.x * (TAM_WG / 64)) {
@@ -2823,7 +2982,8 @@ __global__ __launch_bounds__(TAM_WG) void tam_k_costate_m(const TamTensor d, Tam
       const uint32_t b = w * 8u + (lane >> 3);
       const uint64_t e0 = (uint64_t)b * TAM_BLOCK_SIZE + (lane & 7u) * TAM_EPU;
       float g[TAM_EPU], ge[TAM_EPU], m[TAM_EPU];
-      tam_ld16<DT>(d.grad, e0, g);
+      const uint64_t eu = (uint64_t)w * (8u * TAM_BLOCK_SIZE);
+      tam_unit_load<DT>(turn, d.grad, eu, lane, g);
       TamCsIn cs = {0u, 0u, 0u, 0.0f};
       uint32_t sbytes = 0u;
       float alpha_prev = 0.0f;
@@ -2835,7 +2995,7 @@ __global__ __launch_bounds__(TAM_WG) void tam_k_costate_m(const TamTensor d, Tam
         alpha_prev = tam_g(d.alpha)[0];
       }
       if (has_ef) {  // costate.py:410-413
-        tam_ld16<TAM_DTYPE_F32>(d.ef_residual, e0, ge);
+        tam_unit_load<TAM_DTYPE_F32>(turn, d.ef_residual, eu, lane, ge);
 #pragma unroll
         for (int i = 0; i < TAM_EPU; ++i) ge[i] = g[i] + ge[i];
       } else {
@@ -2855,7 +3015,7 @@ __global__ __launch_bounds__(TAM_WG) void tam_k_costate_m(const TamTensor d, Tam
                                      lane);
       double* part = (double*)(partials + 2u * (uint64_t)w);
       if ((lane & 31u) - 12u < 2u) tam_g(part)[(lane >> 5) * 2u + (lane & 1u)] = t;
-      tam_st16_f32(m_out, e0, m);
+      tam_unit_store(turn, m_out, eu, lane, m);
     } else {
       const uint32_t wq = 2u * nfull + (w - nfull);
       const TamWave W = tam_wave(d, wq, lane, false);
@@ -3009,6 +3169,7 @@ __global__ __launch_bounds__(TAM_WG) __attribute__((amdgpu_waves_per_eu(4, 4))) 
     uint8_t* idx_out, uint16_t* scales_out, float* __restrict__ v_out) {
   __shared__ __attribute__((aligned(256))) float lut[TAM_WG / 64][8 * 64];
   __shared__ TamLdsTabs tabs;
+  __shared__ TamTurn turn[TAM_WG / 64];
   tam_lds_tabs_fill(&tabs);
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
   TamTensor d = tam_local_desc(n);
@@ -3026,12 +3187,12 @@ __global__ __launch_bounds__(TAM_WG) __attribute__((amdgpu_waves_per_eu(4, 4))) 
       float gv[TAM_EPU], v[TAM_EPU];
       uint32_t sc = tam_g((const uint32_t*)scales_in)[b];
       TamW4 iw = tam_g((const TamW4B*)(idx_in + e0))[0];
-      tam_ld16<DT>(g, e0, gv);
+      tam_unit_load<DT>(&turn[wave], g, (uint64_t)w * (8u * TAM_BLOCK_SIZE), lane, gv);
       tam_compiler_fence();
       tam_pin(sc);
       tam_pin(iw);
       const TamVExt x = tam_vunit_a(d, lane, sc, iw, gv, v, lut[wave], &tabs);
-      tam_st16_f32(v_out, e0, v);
+      tam_unit_store(&turn[wave], v_out, (uint64_t)w * (8u * TAM_BLOCK_SIZE), lane, v);
       d.v_idx = idx_out;
       d.v_scales = scales_out;
       tam_vunit_b(d, lane, b, e0, v, x, &tabs, seed_lo, seed_hi);
@@ -3125,6 +3286,7 @@ __global__ __launch_bounds__(TAM_WG) void tam_k_quantize(const float* __restrict
                                                          uint32_t* __restrict__ wgmin) {
   __shared__ TamLdsTabs tabs;
   __shared__ uint32_t least[TAM_WG / 64];
+  __shared__ TamTurn turn[TAM_WG / 64];
   tam_lds_tabs_fill(&tabs);
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
   const uint32_t units = (nb + 7u) / 8u;
@@ -3140,11 +3302,11 @@ __global__ __launch_bounds__(TAM_WG) void tam_k_quantize(const float* __restrict
     const uint64_t e0 = (uint64_t)b * TAM_BLOCK_SIZE + (lane & 7u) * TAM_EPU;
     const bool ok = b < nb;  // uniform over a block's lanes
     float x[TAM_EPU];
-    if (ok) {
-      tam_ld16<TAM_DTYPE_F32>(v, e0, x);
+    if ((u + 1u) * 8u <= nb) {  // uniform
+      tam_unit_load<TAM_DTYPE_F32>(&turn[wave], v, (uint64_t)u * (8u * TAM_BLOCK_SIZE), lane, x);
     } else {
 #pragma unroll
-      for (int i = 0; i < TAM_EPU; ++i) x[i] = 1.0f;
+      for (int i = 0; i < TAM_EPU; ++i) x[i] = ok ? tam_g(v)[e0 + (uint32_t)i] : 1.0f;
     }
     uint32_t kmn = 0xffffffffu, kmx = 0u;
 #pragma unroll
@@ -3387,18 +3549,22 @@ static bool tam_wd_keeps_16bit(uint32_t dtype, float c_wd) {
 
 // Workgroups of a kernel that fit on the device at once (CUs times the
 // occupancy its registers and LDS allow), cached per device and kernel.  The
-// tile loops launch TAM_GRID_ROUNDS times that many workgroups, pass 2
-// TAM_K2_GRID_ROUNDS times.  Measured on MI355X (Llama-shaped bf16 set): pass 0
-// is 14% faster with 32 rounds than with one resident round of persistent
-// workgroups (8 rounds: 1% slower than 32); pass 2, which loads each quarter
-// one ahead, is fastest with 8 rounds (7% faster than 32, 15% than 1).
-enum { TAM_KS_K1_BF16, TAM_KS_K1_F16, TAM_KS_K1_F32, TAM_KS_K2, TAM_KS_K2_F32, TAM_KS_K1_EF, TAM_KS_K4_EF,
-       TAM_KS_COUNT };
+// tile loops launch at most TAM_GRID_ROUNDS times that many workgroups (pass 2
+// TAM_K2_GRID_ROUNDS times), evenly loaded: every workgroup gets the same number
+// of tiles but for the last ones, and the grid is a multiple of the 8 XCDs
+// (tam_tile_slot).  Measured on MI355X: 106496 tiles (218M bf16 elements, fp32
+// second moment) over 81920 workgroups, a quarter of them with a second tile,
+// took 884 us a step, over 53248 with two each 700, over 106496 with one 757.
+// With 3.9M tiles (an 8B-parameter set) 128 rounds are 1.7% faster than 32 and 4%
+// than one tile each; pass 2, which loads each unit one ahead, is fastest with 8
+// (7% faster than 32 on that set).
+enum { TAM_KS_K1, TAM_KS_K2 = TAM_KS_K1 + 12, TAM_KS_K2_F32, TAM_KS_K2_EF, TAM_KS_K4_EF = TAM_KS_K2_EF + 3,
+       TAM_KS_COUNT };  // TAM_KS_K1 + 3 * mode + dtype, TAM_KS_K2_EF + dtype
 #ifndef TAM_K2_GRID_ROUNDS
 #define TAM_K2_GRID_ROUNDS 8
 #endif
 #ifndef TAM_GRID_ROUNDS
-#define TAM_GRID_ROUNDS 32
+#define TAM_GRID_ROUNDS 128
 #endif
 static uint32_t tam_resident_grid(int which, const void* kernel, int block) {
   static std::atomic<uint32_t> cache[64][TAM_KS_COUNT];
@@ -3440,7 +3606,7 @@ int tam_prepare(TamTensor* tensors, int n_tensors, TamStepInfo* info) {
   tam_err_buf[0] = 0;
   if (!info || n_tensors < 0 || (n_tensors > 0 && !tensors)) return tam_fail(TAM_E_INVALID, "%snull argument", "");
   uint64_t tiles = 0, ratio_blocks = 0, chunks = 0, slices = 0, ef_bytes = 0, tail_blocks = 0;
-  uint32_t dtype_mask = 0;
+  uint32_t dtype_mask = 0, ef_mask = 0, any_1q = 0, not_m_f32 = 0;
   uint32_t ncs = 0, nef = 0, ndev = 0, nsmall = 0, sel_max = 0;
   uint32_t sel_small = TAM_SEL_SMALL;  // blocks of the largest tensor whose selection is one workgroup's
   for (int i = 0; i < n_tensors; ++i)
@@ -3509,10 +3675,16 @@ int tam_prepare(TamTensor* tensors, int n_tensors, TamStepInfo* info) {
     t.ntiles = (uint32_t)nt;
     t.tile0 = (uint32_t)tiles;
     t.tail0 = (uint32_t)tail_blocks;
-    // tam_k1_ef covers an error-feedback tensor
-    t.tail_wgs = !(t.flags & TAM_FLAG_EF) && t.n % (8u * TAM_BLOCK_SIZE) ? 1u : 0u;
+    t.tail_wgs = t.n % (8u * TAM_BLOCK_SIZE) ? 1u : 0u;
     tail_blocks += t.tail_wgs;
-    if (!(t.flags & TAM_FLAG_EF)) dtype_mask |= 1u << t.dtype;  // pass 0's per-dtype kernels skip EF tensors
+    // pass 0's kernels: error feedback apart; the others of a dtype by what all
+    // of them lack
+    if (t.flags & TAM_FLAG_EF) ef_mask |= 1u << t.dtype;
+    else dtype_mask |= 1u << t.dtype;
+    if (!(t.flags & TAM_FLAG_EF)) {
+      if (t.flags & TAM_FLAG_COMPRESS_V) any_1q |= 1u << t.dtype;
+      if (!(t.flags & TAM_FLAG_COMPRESS_V) || (t.flags & TAM_FLAG_COSTATE)) not_m_f32 |= 1u << t.dtype;
+    }
     t.chunk0 = (uint32_t)chunks;
     t.slice0 = (uint32_t)slices;
     t.c_lr = t.neg_lr / t.bias_correction1;  // fp32 division, correctly rounded
@@ -3533,6 +3705,9 @@ int tam_prepare(TamTensor* tensors, int n_tensors, TamStepInfo* info) {
   info->sel_small = sel_small;
   info->sel_max = nsmall ? sel_max : 0u;
   info->dtype_mask = dtype_mask;
+  info->ef_mask = ef_mask;
+  info->v_f32_mask = dtype_mask & ~any_1q;
+  info->m_f32_mask = dtype_mask & ~not_m_f32;
   info->ratio_blocks = ratio_blocks;
   uint64_t off = 0;
   info->off_partials = off;
@@ -3575,9 +3750,24 @@ static int tam_launch_pass(int pass, const TamTensor* d_tensors, const TamStepIn
   // vwg: virtual workgroups (each striding over the tiles on its own) per workgroup
   auto grid_of = [&](int which, const void* kernel, int block = TAM_WG, uint32_t vwg = 1u) {
     const uint32_t rounds = (which == TAM_KS_K2 || which == TAM_KS_K2_F32) ? TAM_K2_GRID_ROUNDS : TAM_GRID_ROUNDS;
-    const uint32_t g = tam_resident_grid(which, kernel, block) * rounds;
+    const uint32_t most = tam_resident_grid(which, kernel, block) * rounds;
     const uint32_t need = (info->total_tiles + vwg - 1u) / vwg;
-    return need < g ? need : g;
+    const uint32_t each = (need + most - 1u) / most;  // tiles of a workgroup
+    return ((need + each - 1u) / each + 7u) & ~7u;
+  };
+  // pass 0's kernel of a mode and dtype
+  const auto k1_launch = [&](int mode, uint32_t dt) -> int {
+    typedef void (*Kernel)(const TamTensor*, int, uint32_t, uint32_t, uint32_t, double2*);
+    static const Kernel kernels[4][3] = {{tam_k1_main_f32, tam_k1_main_bf16, tam_k1_main_f16},
+                                         {tam_k1_vf32_f32, tam_k1_vf32_bf16, tam_k1_vf32_f16},
+                                         {tam_k1_mf32_f32, tam_k1_mf32_bf16, tam_k1_mf32_f16},
+                                         {tam_k1_ef_f32, tam_k1_ef_bf16, tam_k1_ef_f16}};
+    const Kernel k = kernels[mode][dt];
+    hipLaunchKernelGGL(k, dim3(grid_of(TAM_KS_K1 + 3 * mode + (int)dt, (const void*)k, TAM_K1_BLOCK, TAM_K1_VWG)),
+                       dim3(TAM_K1_BLOCK), 0, s, d_tensors, info->n_tensors, info->total_tiles, (uint32_t)seed,
+                       (uint32_t)(seed >> 32), partials);
+    TAM_HIP_CHECK(hipGetLastError());
+    return TAM_OK;
   };
   switch (pass) {
     case 0:
@@ -3585,26 +3775,18 @@ static int tam_launch_pass(int pass, const TamTensor* d_tensors, const TamStepIn
         hipLaunchKernelGGL(tam_k_device_step, dim3(1), dim3(1024), 0, s, (TamTensor*)d_tensors, info->n_tensors);
         TAM_HIP_CHECK(hipGetLastError());
       }
-      if (info->dtype_mask & (1u << TAM_DTYPE_BF16))
-        hipLaunchKernelGGL(tam_k1_main_bf16,
-                           dim3(grid_of(TAM_KS_K1_BF16, (const void*)tam_k1_main_bf16, TAM_K1_BLOCK, TAM_K1_VWG)),
-                           dim3(TAM_K1_BLOCK), 0, s, d_tensors, info->n_tensors, info->total_tiles, (uint32_t)seed,
-                           (uint32_t)(seed >> 32), partials);
-      if (info->dtype_mask & (1u << TAM_DTYPE_F16))
-        hipLaunchKernelGGL(tam_k1_main_f16,
-                           dim3(grid_of(TAM_KS_K1_F16, (const void*)tam_k1_main_f16, TAM_K1_BLOCK, TAM_K1_VWG)),
-                           dim3(TAM_K1_BLOCK), 0, s, d_tensors, info->n_tensors, info->total_tiles, (uint32_t)seed,
-                           (uint32_t)(seed >> 32), partials);
-      if (info->dtype_mask & (1u << TAM_DTYPE_F32))
-        hipLaunchKernelGGL(tam_k1_main_f32,
-                           dim3(grid_of(TAM_KS_K1_F32, (const void*)tam_k1_main_f32, TAM_K1_BLOCK, TAM_K1_VWG)),
-                           dim3(TAM_K1_BLOCK), 0, s, d_tensors, info->n_tensors, info->total_tiles, (uint32_t)seed,
-                           (uint32_t)(seed >> 32), partials);
-      if (info->n_ef)
-        hipLaunchKernelGGL(tam_k1_ef, dim3(grid_of(TAM_KS_K1_EF, (const void*)tam_k1_ef)), dim3(TAM_WG), 0, s,
-                           d_tensors, info->n_tensors, info->total_tiles, (uint32_t)seed, (uint32_t)(seed >> 32),
-                           partials);
-      TAM_HIP_CHECK(hipGetLastError());
+      for (uint32_t dt = TAM_DTYPE_F32; dt <= TAM_DTYPE_F16; ++dt) {
+        const uint32_t bit = 1u << dt;
+        if (info->dtype_mask & bit) {
+          const int mode = info->v_f32_mask & bit ? TAM_K1_V_F32 : info->m_f32_mask & bit ? TAM_K1_M_F32 : TAM_K1_ANY;
+          const int rc = k1_launch(mode, dt);
+          if (rc != TAM_OK) return rc;
+        }
+        if (info->ef_mask & bit) {
+          const int rc = k1_launch(TAM_K1_EF, dt);
+          if (rc != TAM_OK) return rc;
+        }
+      }
       if (info->tail_blocks)
         hipLaunchKernelGGL(tam_k1_tail, dim3(info->tail_blocks), dim3(TAM_K1U_WG), 0, s, d_tensors, info->n_tensors,
                            (uint32_t)seed, (uint32_t)(seed >> 32), partials);
@@ -3621,16 +3803,25 @@ static int tam_launch_pass(int pass, const TamTensor* d_tensors, const TamStepIn
       // kernel when it runs, else to the fp32 one
       const bool has16 = (info->dtype_mask & ((1u << TAM_DTYPE_BF16) | (1u << TAM_DTYPE_F16))) != 0;
       const bool has32 = (info->dtype_mask & (1u << TAM_DTYPE_F32)) != 0;
-      if (has16 || !has32)
+      if (has16)
         hipLaunchKernelGGL(tam_k2_encode, dim3(grid_of(TAM_KS_K2, (const void*)tam_k2_encode, TAM_K1U_WG)),
                            dim3(TAM_K1U_WG), 0, s, d_tensors, info->n_tensors, info->total_tiles, alpha_new, ratios,
                            ws, 1, has32 ? 1 : 0);
-      if (has32) {
-        TAM_HIP_CHECK(hipGetLastError());
+      TAM_HIP_CHECK(hipGetLastError());
+      if (has32)
         hipLaunchKernelGGL(tam_k2_encode_f32,
                            dim3(grid_of(TAM_KS_K2_F32, (const void*)tam_k2_encode_f32, TAM_K1U_WG)),
                            dim3(TAM_K1U_WG), 0, s, d_tensors, info->n_tensors, info->total_tiles, alpha_new, ratios,
                            ws, has16 ? 0 : 1, 0);
+      TAM_HIP_CHECK(hipGetLastError());
+      for (uint32_t dt = TAM_DTYPE_F32; dt <= TAM_DTYPE_F16; ++dt) {
+        if (!(info->ef_mask & (1u << dt))) continue;
+        const auto k = dt == TAM_DTYPE_BF16 ? tam_k2_ef<TAM_DTYPE_BF16>
+                       : dt == TAM_DTYPE_F16 ? tam_k2_ef<TAM_DTYPE_F16>
+                                             : tam_k2_ef<TAM_DTYPE_F32>;
+        hipLaunchKernelGGL(k, dim3(grid_of(TAM_KS_K2_EF + (int)dt, (const void*)k, TAM_K1U_WG)), dim3(TAM_K1U_WG), 0, s,
+                           d_tensors, info->n_tensors, info->total_tiles, alpha_new, ratios, ws);
+        TAM_HIP_CHECK(hipGetLastError());
       }
       break;
     }
