@@ -234,6 +234,71 @@ def test_costate_update_units(n, dt, ef):
             assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), f"step {s}: {k}"
 
 
+def test_fp32_update_square_root_and_reciprocal_on_every_input():
+    """The fp32 update's own square root and reciprocal equal the correctly
+    rounded ones on every input of the ranges it uses them on."""
+    from turboadam_amd import _lib
+
+    lib, chunk = _lib.load(), 1 << 27
+    out = torch.empty(chunk, dtype=torch.float32, device=DEV)
+    # (function, first and last bit pattern): sqrt on [2^-62, 2^127], 1/x on [2^-126, 2^126]
+    for fn, lo, hi in ((9, 0x20800000, 0x7F000001), (10, 0x00800000, 0x7E800001)):
+        wrong = 0
+        for start in range(lo, hi, chunk):
+            n = min(chunk, hi - start)
+            x = torch.arange(start, start + n, dtype=torch.int64, device=DEV).to(torch.int32).view(torch.float32)
+            _lib.check(lib.tam_math_eval(fn, x.data_ptr(), out.data_ptr(), n, _lib.stream_of(DEV)), "tam_math_eval")
+            # rounding fp64's correctly rounded result once more gives the fp32 one (sqrt and 1/x of
+            # 24-bit values stay 2^-50 away from a rounding boundary)
+            want = (x.double().sqrt() if fn == 9 else 1.0 / x.double()).float()
+            wrong += int((out[:n] != want).sum())
+        log(f"function {fn}: {hi - lo} inputs, {wrong} wrong")
+        assert wrong == 0
+
+
+@pytest.mark.parametrize("kw", [dict(eps=1e-8), dict(eps=0.0), dict(eps=1e-30), dict(eps=1e4), dict(lr=0.0),
+                                dict(betas=(0.9, 0.5)), dict(betas=(0.0, 0.999), weight_decay=0.1)])
+def test_fp32_update_ranges(kw):
+    """Parameters around 2^-40, zeros, huge and infinite ones, gradients from
+    subnormal to overflowing: lanes of the fast update and of the other one."""
+    from turboadam_amd import TurboAdam
+
+    log(f"fp32 update ranges {kw}")
+    rng = np.random.default_rng(3)
+    sizes = [1024 * 6, 3000, 1024 * 2 + 77]
+    for compress_v in (True, False):
+        init = [(rng.standard_normal(n) * 0.02).astype(np.float32) for n in sizes]
+        for p in init:
+            p[64:128] *= np.float32(2.0 ** -34)
+            p[130:140] = 0.0
+            p[300:310] = np.float32(1e38)
+            p[320] = np.inf
+            p[330] = -np.nan
+            p[340:360] = np.float32(2.0 ** -40)
+        o_params = [a.copy() for a in init]
+        params = [torch.nn.Parameter(_t(a)) for a in init]
+        opt = TurboAdam(params, compress_v=compress_v, philox_seed=5, **kw)
+        orc = O.OracleTurboAdam(o_params, dtypes=[O.DT_F32] * len(sizes), seed=5, compress_v=compress_v, **kw)
+        for s in range(3):
+            grads = [(rng.standard_normal(n) * np.exp(rng.uniform(-60, 2, n))).astype(np.float32) for n in sizes]
+            for g in grads:
+                g[200:260] = 0.0
+                g[256:384] = 0.0
+                g[400:404] = np.float32(1e-42)
+                g[410] = np.float32(1e25)
+            if s == 2:
+                grads[0][500] = np.inf
+            for p, g in zip(params, grads):
+                p.grad = _t(g)
+            opt.step()
+            orc.step(grads)
+            for i, p in enumerate(params):
+                a, b = p.detach().cpu().numpy(), o_params[i].reshape(-1)
+                assert np.array_equal(np.isnan(a), np.isnan(b)), (s, i)
+                k = ~np.isnan(b)
+                assert np.array_equal(a[k].view(np.uint32), b[k].view(np.uint32)), (s, i, compress_v)
+
+
 # pass 0 has a kernel for each mode (fp32 first moment, fp32 second moment, error feedback, any), pass 2 for
 # error feedback; mixed: tensors of two modes in one dtype
 @pytest.mark.parametrize("offset", [0, 1])

@@ -805,9 +805,13 @@ __device__ __forceinline__ TamVExt tam_lane_extremes(const float* v, uint32_t nv
 // block (the certified 16-bit update's input range): q is monotone in v, so
 // the block's smallest and largest v decide.  False when the extremes bound
 // only the clamped v or a v is NaN.
+// For an fp32 parameter: whether every q1 = fl(v/bc2) is a normal below 2^62, with
+// a margin of a factor 2 for this product's own rounding.
+template <uint32_t DT>
 __device__ __forceinline__ bool tam_q_in_range(const TamTensor& d, const TamVExt& x) {
-  return x.nan_seen == 0u && tam_u2f(x.kmn) * d.inv_bc2_f32 >= 0x1p-126f &&
-         tam_u2f(x.kmx) * d.inv_bc2_f32 <= 0x1.fffffep127f;
+  constexpr float lo = DT == TAM_DTYPE_F32 ? 0x1p-125f : 0x1p-126f;
+  constexpr float hi = DT == TAM_DTYPE_F32 ? 0x1p61f : 0x1.fffffep127f;
+  return x.nan_seen == 0u && tam_u2f(x.kmn) * d.inv_bc2_f32 >= lo && tam_u2f(x.kmx) * d.inv_bc2_f32 <= hi;
 }
 
 // Second half: logs of the extremes, scales, stochastic re-quantisation.
@@ -941,8 +945,31 @@ __device__ __forceinline__ void tam_vpath_b(const TamTensor& d, const TamWave& W
 // ---------------------------------------------------------------------------
 // Exact sequence: q1 = fl(v/bc2), s = fl(sqrt(q1)), den = fl(s + eps),
 // t2 = fl(den*bc1), a = fl(-lr*m), upd = fl(a/t2), p = R_p(fl(p + upd)).
-// fp32 parameters: q1 comes from the fp64 reciprocal of bc2 when a rounding
-// test proves the fp32 rounding, else from the division.
+// fp32 parameters: the exact sequence, its correctly rounded operations written
+// out where the operands' range allows (the compiler's expansions of sqrt and
+// division scale their operands for every range: about 45 cycles of issue each):
+//  * q1 = fl(v/bc2) is the fp32 rounding of v times the fp64 reciprocal of bc2:
+//    the product errs by less than 2^-51 relative, and a quotient of two 24-bit
+//    significands never lies within 2^-49 of an fp32 rounding boundary.  The
+//    reciprocal comes scaled by 2^64 (exact), so q = 2^64 q1 wherever q1 is a
+//    normal below 2^63.
+//  * s = fl(sqrt(q)) from y = v_rsq_f32(q): g = fl(q y), then one residual step
+//    s = fma(fma(-g, g, q), y/2, g) (Markstein 1990).  Equal to the correctly
+//    rounded root on every normal input from 2^-62 up (tests, exhaustively);
+//    den = fl(2^-32 s + eps) in one fma.
+//  * upd = fl(a/t2): y = fl(1/t2) from v_rcp_f32 and one Newton step (equal to the
+//    correctly rounded reciprocal on every normal input up to 2^126: tests,
+//    exhaustively), u0 = fl(a y) within 1.5 ulp of a/t2, u1 = fma(r0, y, u0)
+//    within one, upd = fma(r1, y, u1) with the exact residual r1: with y the
+//    correctly rounded reciprocal and u1 within one ulp, that is the correctly
+//    rounded quotient (Markstein 1990, theorem 5.3 ff.).  r1 is exact for
+//    |a| >= 2^-100.  A smaller a gives |upd| < 2^-68 (t2 >= eps bc1 >= 2^-32),
+//    which leaves any |p| >= 2^-40 unchanged whatever its last bits.
+// A lane takes these when its q1 are normal (q_ok) and below 2^62, every |p| of
+// its elements is at least 2^-40 and every |u0| below 2^100 (an infinite m or a
+// overflowing quotient fails that); bc1 and eps decide uniformly.  Any other lane
+// takes the compiler's division and square root, and q1 from the reciprocal only
+// when a rounding test proves it (an out-of-range bc2 may put q1 on a tie).
 //
 // bf16 / fp16 parameters: a fast sequence u~ = fl(fl(c*m) * r) with
 // r = rcp(fl(s~ + eps)), s~ = sqrt(q) (v_sqrt_f32), q = fl(v * fl(1/bc2)),
@@ -994,20 +1021,64 @@ __device__ __forceinline__ uint32_t tam_pack16(float x, float y) {
   if (DT == TAM_DTYPE_BF16) return __builtin_bit_cast(uint32_t, __builtin_convertvector((TamF2){x, y}, TamBf2));
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((TamF2){x, y}, TamH2));
 }
+// fl(sqrt(x)) for normal x >= 2^-62, fl(1/x) for normal x with a normal reciprocal
+// (see above).
+__device__ __forceinline__ float tam_sqrt_normal(float x) {
+  const float y = __builtin_amdgcn_rsqf(x);
+  const float g = x * y;
+  return __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * y, g);
+}
+__device__ __forceinline__ float tam_rcp_normal(float x) {
+  const float y = __builtin_amdgcn_rcpf(x);
+  return __builtin_fmaf(__builtin_fmaf(-x, y, 1.0f), y, y);
+}
+
 template <uint32_t DT>
 __device__ __forceinline__ void tam_update(const TamTensor& d, float* p, const float* m, const float* v,
                                            uint32_t* pw2, bool q_ok) {
   const bool wd = (d.flags & TAM_FLAG_WD) != 0;
   if (DT == TAM_DTYPE_F32) {
+    const float edge = d.eps * d.bias_correction1;
+    const bool fast = q_ok && edge >= 0x1p-32f && d.eps > 0.0f && d.eps < 0x1p60f && d.bias_correction1 < 0x1p20f;
+    // four elements at a time: their results wait in registers beside the inputs
 #pragma unroll
-    for (int i = 0; i < TAM_EPL; ++i) {
-      const double y = (double)v[i] * d.inv_bc2;
-      const double e = __builtin_fabs(y) * 0x1p-51;
-      float q1 = (float)(y - e);
-      if (!(q1 == (float)(y + e))) q1 = v[i] / d.bias_correction2;
-      const float den = __builtin_sqrtf(q1) + d.eps;
-      const float pv = wd ? p[i] * d.c_wd : p[i];
-      p[i] = pv + (d.neg_lr * m[i]) / (den * d.bias_correction1);
+    for (int h = 0; h < TAM_EPL; h += 4) {
+      float pn[4];
+      bool ok = false;
+      if (__any(fast)) {
+        const double inv = d.inv_bc2 * 0x1p64;
+        float pmin = tam_inf(), umax = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int i = h + j;
+          const float s = tam_sqrt_normal((float)((double)v[i] * inv));
+          const float t2 = __builtin_fmaf(s, 0x1p-32f, d.eps) * d.bias_correction1;
+          const float a = d.neg_lr * m[i], y = tam_rcp_normal(t2);
+          const float u0 = a * y;
+          const float u1 = __builtin_fmaf(__builtin_fmaf(-t2, u0, a), y, u0);
+          const float u = __builtin_fmaf(__builtin_fmaf(-t2, u1, a), y, u1);
+          const float pv = wd ? p[i] * d.c_wd : p[i];
+          pmin = __builtin_fminf(pmin, __builtin_fabsf(pv));
+          umax = __builtin_fmaxf(umax, __builtin_fabsf(u0));  // a NaN stays in u
+          pn[j] = pv + u;
+        }
+        ok = fast && pmin >= 0x1p-40f && umax < 0x1p100f;
+      }
+      if (!ok) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int i = h + j;
+          const double y = (double)v[i] * d.inv_bc2;
+          const double e = __builtin_fabs(y) * 0x1p-51;
+          float q1 = (float)(y - e);
+          if (!(q1 == (float)(y + e))) q1 = v[i] / d.bias_correction2;
+          const float den = __builtin_sqrtf(q1) + d.eps;
+          const float pv = wd ? p[i] * d.c_wd : p[i];
+          pn[j] = pv + (d.neg_lr * m[i]) / (den * d.bias_correction1);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) p[h + j] = pn[j];
     }
     return;
   }
@@ -1275,8 +1346,7 @@ __device__ __forceinline__ void tam_k1_quarter(const TamTensor& d, uint32_t wq, 
   // ---- parameter update -----------------------------------------------
   if (FULL || W.bvalid) {
     uint32_t pw2[TAM_EPL / 2];
-    bool q_ok = false;
-    if (DT != TAM_DTYPE_F32) q_ok = tam_q_in_range(d, compress_v ? vx : tam_lane_extremes<FULL>(v, W.nv));
+    const bool q_ok = tam_q_in_range<DT>(d, compress_v ? vx : tam_lane_extremes<FULL>(v, W.nv));
     tam_update<DT>(d, p, m, v, pw2, q_ok);
     if (DT == TAM_DTYPE_F32) tam_st8_f32<FULL>((float*)d.param, W.e0, W.nv, p);
     else tam_st8_bits<FULL>(d.param, W.e0, W.nv, pw2);
@@ -1710,17 +1780,14 @@ __device__ __forceinline__ void tam_k1_unit(const TamTensor& d, uint32_t u, uint
       tam_turn_in(turn, lane, pf, p);
     }
     uint32_t pw2[TAM_EPU / 2];
-    bool q_ok = false;
-    if (DT != TAM_DTYPE_F32) {
-      TamVExt e = vx;
-      if (!compress_v) {
-        const TamVExt e1 = tam_lane_extremes<true>(v, TAM_EPL), e2 = tam_lane_extremes<true>(v + TAM_EPL, TAM_EPL);
-        e.kmn = __builtin_elementwise_min(e1.kmn, e2.kmn);
-        e.kmx = __builtin_elementwise_max(e1.kmx, e2.kmx);
-        e.nan_seen = e1.nan_seen | e2.nan_seen;
-      }
-      q_ok = tam_q_in_range(d, e);
+    TamVExt e = vx;
+    if (!compress_v) {
+      const TamVExt e1 = tam_lane_extremes<true>(v, TAM_EPL), e2 = tam_lane_extremes<true>(v + TAM_EPL, TAM_EPL);
+      e.kmn = __builtin_elementwise_min(e1.kmn, e2.kmn);
+      e.kmx = __builtin_elementwise_max(e1.kmx, e2.kmx);
+      e.nan_seen = e1.nan_seen | e2.nan_seen;
     }
+    const bool q_ok = tam_q_in_range<DT>(d, e);
     tam_update<DT>(d, p, m, v, pw2, q_ok);
     tam_update<DT>(d, p + TAM_EPL, m + TAM_EPL, v + TAM_EPL, pw2 + TAM_EPL / 2, q_ok);
     if (DT == TAM_DTYPE_F32) {
@@ -3500,6 +3567,8 @@ __global__ void tam_k_math_eval(int fn, const float* __restrict__ in, float* __r
     case 6: y = __builtin_amdgcn_sqrtf(x); break;
     case 7: y = __builtin_amdgcn_rcpf(x); break;
     case 8: y = __builtin_amdgcn_logf(x); break;
+    case 9: y = tam_sqrt_normal(x); break;
+    case 10: y = tam_rcp_normal(x); break;
     default: y = x; break;
   }
   out[i] = y;
@@ -3959,7 +4028,7 @@ int tam_philox_uniforms(uint32_t tensor_id, uint32_t step, uint64_t seed, uint64
 int tam_math_eval(int fn, const float* in, float* out, uint64_t n, void* stream) {
   tam_err_buf[0] = 0;
   if (!in || !out) return tam_fail(TAM_E_INVALID, "%snull argument", "");
-  if (fn < 0 || fn > 8) return tam_fail(TAM_E_INVALID, "%sunknown function %ld", "", fn);
+  if (fn < 0 || fn > 10) return tam_fail(TAM_E_INVALID, "%sunknown function %ld", "", fn);
   if (n == 0) return TAM_OK;
   const uint64_t blocks = (n + 255) / 256;
   hipLaunchKernelGGL(tam_k_math_eval, dim3((uint32_t)blocks), dim3(256), 0, (hipStream_t)stream, fn, in, out, n);
