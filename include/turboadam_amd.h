@@ -174,6 +174,14 @@ const char* tam_last_error(void);
  * (reference optimizer.py:232-286) for one step's tensor list. */
 int tam_prepare(TamTensor* tensors, int n_tensors, TamStepInfo* info);
 
+/* Write n_tensors descriptors to d_tensors and values[i] to *ptrs[i] (device
+ * floats) on the stream, by launches that carry them as arguments (12
+ * descriptors and 8 values each): for small tensor lists, instead of a copy from
+ * a host buffer that must stay alive.  The host arrays are read before the call
+ * returns.  No counterpart in the reference. */
+int tam_put(const TamTensor* h_tensors, int n_tensors, TamTensor* d_tensors, float* const* ptrs,
+            const float* values, int n_values, void* stream);
+
 /* One fused optimizer step over every tensor of `d_tensors` (device copy of
  * the array prepared by tam_prepare) in four passes: the fused update
  * (decode, EMA, 1Q re-quantisation, AdamW update, dot partials), alpha,

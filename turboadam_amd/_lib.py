@@ -120,6 +120,7 @@ SIGNATURES = {
     "tam_struct_size": (ctypes.c_size_t, [ctypes.c_int]),
     "tam_last_error": (ctypes.c_char_p, []),
     "tam_prepare": (ctypes.c_int, [ctypes.POINTER(TamTensor), ctypes.c_int, ctypes.POINTER(TamStepInfo)]),
+    "tam_put": (ctypes.c_int, [_VP, ctypes.c_int, _VP, _VP, _VP, ctypes.c_int, _VP]),
     "tam_multi_tensor_step": (
         ctypes.c_int,
         [_VP, ctypes.POINTER(TamTensor), ctypes.POINTER(TamStepInfo), ctypes.c_uint64, _VP, ctypes.c_size_t, _VP],

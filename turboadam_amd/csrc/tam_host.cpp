@@ -13,12 +13,16 @@
 //
 // steady_rows() returns False, with nothing written, when any check fails
 // (the optimizer then takes its full path, which validates and raises where
-// something is wrong); advance_steps() adds 1 to each state's step counter
-// once the step has been launched.
+// something is wrong); steady_groups() writes the fields the parameter groups
+// set (numpy column writes took 20 us a step); advance_steps() adds 1 to each
+// state's step counter once the step has been launched.
 #include <torch/extension.h>
 
+#include <cmath>
 #include <cstdint>
 #include <cstring>
+
+#include "../../include/turboadam_amd.h"
 
 namespace py = pybind11;
 
@@ -32,7 +36,7 @@ PyObject* item(PyObject* d, PyObject* key) {
 
 struct Keys {
   PyObject *grad, *compressed_v, *indices, *scales, *exp_avg_sq, *exp_avg, *compress_m, *m_mgr, *encoded,
-      *sign_packed, *labels, *block_norms, *alpha, *ef_residual, *step;
+      *sign_packed, *labels, *block_norms, *alpha, *ef_residual, *step, *lr, *betas, *eps, *weight_decay;
   Keys() {
     grad = PyUnicode_InternFromString("grad");
     compressed_v = PyUnicode_InternFromString("compressed_v");
@@ -49,6 +53,10 @@ struct Keys {
     alpha = PyUnicode_InternFromString("_alpha");
     ef_residual = PyUnicode_InternFromString("_ef_residual");
     step = PyUnicode_InternFromString("step");
+    lr = PyUnicode_InternFromString("lr");
+    betas = PyUnicode_InternFromString("betas");
+    eps = PyUnicode_InternFromString("eps");
+    weight_decay = PyUnicode_InternFromString("weight_decay");
   }
 };
 
@@ -247,6 +255,124 @@ bool steady_rows(py::handle f, uint64_t table_addr, int64_t stride, int64_t grad
   return ok;
 }
 
+// Whether the dict holds exactly the kept values, in order, by identity.
+bool values_kept(py::handle map, py::handle kept) {
+  PyObject *D = map.ptr(), *L = kept.ptr(), *key = nullptr, *value = nullptr;
+  if (!PyDict_Check(D) || !PyList_Check(L) || PyDict_Size(D) != PyList_GET_SIZE(L)) return false;
+  Py_ssize_t pos = 0;
+  for (Py_ssize_t i = 0; PyDict_Next(D, &pos, &key, &value); ++i)
+    if (i >= PyList_GET_SIZE(L) || PyList_GET_ITEM(L, i) != value) return false;
+  return true;
+}
+
+namespace {
+
+// A Python float or int as a double; false for anything else.
+bool number(PyObject* o, double* out) {
+  if (!o || !(PyFloat_Check(o) || PyLong_Check(o))) return false;
+  *out = PyFloat_AsDouble(o);
+  if (*out == -1.0 && PyErr_Occurred()) {
+    PyErr_Clear();
+    return false;
+  }
+  return true;
+}
+
+// betas of a parameter group.
+bool betas_of(PyObject* group, double* b1, double* b2) {
+  PyObject* t = item(group, keys().betas);
+  if (!t || !(PyTuple_Check(t) || PyList_Check(t)) || PySequence_Fast_GET_SIZE(t) != 2) return false;
+  return number(PySequence_Fast_GET_ITEM(t, 0), b1) && number(PySequence_Fast_GET_ITEM(t, 1), b2);
+}
+
+}  // namespace
+
+// The fields that parameter groups set in the descriptor rows of a steady step
+// (optimizer.TurboAdam._group_fields, _set_group_fields: each scalar a double
+// rounded to fp32 once) and the rows' flags, given the kept _FastStep f: its
+// `bc` list of (group, state dict whose step sets the group's bias corrections),
+// `groups` list of (group, index into bc or -1) and the addresses of the table,
+// of the rows' group numbers (intp) and static flags (uint32), and of 2 floats
+// per bc entry that receive the bias corrections.  False, with nothing written,
+// for a hyperparameter that is no plain number or gives no finite correction.
+bool steady_groups(py::handle f, uint64_t table_addr, int64_t rows, uint64_t gsel_addr, uint64_t flags_addr,
+                   uint64_t bc_addr) {
+  const Keys& K = keys();
+  py::object groups = f.attr("groups"), bc = f.attr("bc");
+  PyObject *G = groups.ptr(), *B = bc.ptr();
+  if (!PyList_Check(G) || !PyList_Check(B)) return false;
+  std::vector<double> corr;  // (1 - beta1^t, 1 - beta2^t) of each bc entry (reference optimizer.py:172-188)
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(B); ++i) {
+    PyObject* e = PyList_GET_ITEM(B, i);
+    double b1, b2;
+    PyObject* step = item(PyTuple_GET_ITEM(e, 1), K.step);
+    if (!step || !PyLong_Check(step) || !betas_of(PyTuple_GET_ITEM(e, 0), &b1, &b2)) return false;
+    const long long s = PyLong_AsLongLong(step);
+    if (s < 0) {
+      PyErr_Clear();
+      return false;
+    }
+    const double t = (double)(s + 1), c1 = 1.0 - std::pow(b1, t), c2 = 1.0 - std::pow(b2, t);
+    if (!std::isfinite(c1) || !std::isfinite(c2)) return false;
+    corr.push_back(c1);
+    corr.push_back(c2);
+  }
+  std::vector<TamTensor> vals;  // the group fields of each group
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(G); ++i) {
+    PyObject* e = PyList_GET_ITEM(G, i);
+    PyObject* g = PyTuple_GET_ITEM(e, 0);
+    const Py_ssize_t k = PyLong_AsSsize_t(PyTuple_GET_ITEM(e, 1));
+    double lr, b1, b2, eps, wd;
+    if (!number(item(g, K.lr), &lr) || !number(item(g, K.eps), &eps) || !number(item(g, K.weight_decay), &wd) ||
+        !betas_of(g, &b1, &b2) || (size_t)(2 * (k + 1)) > corr.size()) {
+      PyErr_Clear();
+      return false;
+    }
+    TamTensor v;
+    std::memset(&v, 0, sizeof(v));
+    v.c_wd = (float)(1.0 - lr * wd);
+    v.beta1 = (float)b1;
+    v.one_minus_beta1 = (float)(1.0 - b1);
+    v.beta2 = (float)b2;
+    v.one_minus_beta2 = (float)(1.0 - b2);
+    v.bias_correction1 = (float)(k < 0 ? 1.0 : corr[2 * k]);
+    v.bias_correction2 = (float)(k < 0 ? 1.0 : corr[2 * k + 1]);
+    if (v.bias_correction2 == 0.0f) return false;
+    v.inv_bc2 = 1.0 / (double)v.bias_correction2;
+    v.inv_bc2_f32 = (float)v.inv_bc2;
+    v.eps = (float)eps;
+    v.neg_lr = (float)-lr;
+    v.flags = wd != 0.0 ? TAM_FLAG_WD : 0u;
+    vals.push_back(v);
+  }
+  TamTensor* T = (TamTensor*)(uintptr_t)table_addr;
+  const intptr_t* gsel = (const intptr_t*)(uintptr_t)gsel_addr;
+  const uint32_t* flags = (const uint32_t*)(uintptr_t)flags_addr;
+  for (int64_t j = 0; j < rows; ++j)
+    if (gsel[j] < 0 || (size_t)gsel[j] >= vals.size()) return false;
+  for (int64_t j = 0; j < rows; ++j) {
+    const TamTensor& v = vals[(size_t)gsel[j]];
+    TamTensor& t = T[j];
+    t.c_wd = v.c_wd;
+    t.beta1 = v.beta1;
+    t.one_minus_beta1 = v.one_minus_beta1;
+    t.beta2 = v.beta2;
+    t.one_minus_beta2 = v.one_minus_beta2;
+    t.bias_correction1 = v.bias_correction1;
+    t.bias_correction2 = v.bias_correction2;
+    t.inv_bc2 = v.inv_bc2;
+    t.inv_bc2_f32 = v.inv_bc2_f32;
+    t.eps = v.eps;
+    t.neg_lr = v.neg_lr;
+    t.flags = flags[j] | v.flags;  // a steady step has every encoding and residual (_keep_fast)
+    if (flags[j] & TAM_FLAG_COSTATE) t.flags |= TAM_FLAG_HAS_STATE;
+    if (flags[j] & TAM_FLAG_EF) t.flags |= TAM_FLAG_HAS_EF;
+  }
+  float* out = (float*)(uintptr_t)bc_addr;
+  for (size_t i = 0; i < corr.size(); ++i) out[i] = (float)corr[i];
+  return true;
+}
+
 // state["step"] += 1 for each state dict (once the step has been launched).
 void advance_steps(py::list states) {
   const Keys& K = keys();
@@ -269,5 +395,8 @@ PYBIND11_MODULE(_tam_host, m) {
   m.def("steady_rows", &steady_rows, py::arg("f"), py::arg("table_addr"), py::arg("stride"), py::arg("grad_off"),
         py::arg("step_off"));
   m.def("advance_steps", &advance_steps, py::arg("states"));
+  m.def("values_kept", &values_kept, py::arg("map"), py::arg("kept"));
+  m.def("steady_groups", &steady_groups, py::arg("f"), py::arg("table_addr"), py::arg("rows"), py::arg("gsel_addr"),
+        py::arg("flags_addr"), py::arg("bc_addr"));
   m.def("states_kept", &states_kept, py::arg("f"));
 }

@@ -3552,6 +3552,26 @@ __global__ void tam_k_philox_uniforms(uint32_t tid, uint32_t step, uint32_t seed
     if (e0 + k < count) out[e0 + k] = tam_u24f(rw[k]);
 }
 
+// Descriptors and single floats written to device memory from the kernel's own
+// arguments: a small step needs no host buffer that stays alive, no copy and no
+// event (a 12-tensor step's pinned copy with its event and two fills took 20 of
+// the host's 71 us).  12 descriptors and 8 floats fit the 4 KB of an argument
+// block.
+#define TAM_PUT_TENSORS 12
+#define TAM_PUT_VALUES 8
+struct TamPut {
+  TamTensor t[TAM_PUT_TENSORS];
+  float* ptr[TAM_PUT_VALUES];
+  float value[TAM_PUT_VALUES];
+};
+static_assert(sizeof(TamPut) + 16 <= 4096, "one argument block");
+__global__ __launch_bounds__(256) void tam_k_put(const TamPut a, int n_tensors, int n_values,
+                                                 TamTensor* __restrict__ out) {
+  const uint32_t words = (uint32_t)n_tensors * (uint32_t)(sizeof(TamTensor) / 4);
+  for (uint32_t i = threadIdx.x; i < words; i += 256u) ((uint32_t*)out)[i] = ((const uint32_t*)a.t)[i];
+  if ((int)threadIdx.x < n_values) *a.ptr[threadIdx.x] = a.value[threadIdx.x];
+}
+
 __global__ void tam_k_math_eval(int fn, const float* __restrict__ in, float* __restrict__ out, uint64_t n) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -3930,6 +3950,33 @@ int tam_step_pass(int pass, const TamTensor* d_tensors, const TamStepInfo* info,
                   size_t ws_bytes, void* stream) {
   tam_err_buf[0] = 0;
   return tam_launch_pass(pass, d_tensors, info, seed, workspace, ws_bytes, (hipStream_t)stream);
+}
+
+int tam_put(const TamTensor* h_tensors, int n_tensors, TamTensor* d_tensors, float* const* ptrs, const float* values,
+            int n_values, void* stream) {
+  tam_err_buf[0] = 0;
+  if (n_tensors < 0 || n_values < 0 || (n_tensors && (!h_tensors || !d_tensors)) || (n_values && (!ptrs || !values)))
+    return tam_fail(TAM_E_INVALID, "%sbad arguments", "");
+  while (n_tensors || n_values) {
+    TamPut a;
+    const int nt = n_tensors < TAM_PUT_TENSORS ? n_tensors : TAM_PUT_TENSORS;
+    const int nv = n_values < TAM_PUT_VALUES ? n_values : TAM_PUT_VALUES;
+    if (nt) memcpy(a.t, h_tensors, (size_t)nt * sizeof(TamTensor));
+    for (int i = 0; i < nv; ++i) {
+      if (!ptrs[i]) return tam_fail(TAM_E_INVALID, "%snull pointer", "");
+      a.ptr[i] = ptrs[i];
+      a.value[i] = values[i];
+    }
+    hipLaunchKernelGGL(tam_k_put, dim3(1), dim3(256), 0, (hipStream_t)stream, a, nt, nv, d_tensors);
+    TAM_HIP_CHECK(hipGetLastError());
+    h_tensors += nt;
+    d_tensors += nt;
+    n_tensors -= nt;
+    ptrs += nv;
+    values += nv;
+    n_values -= nv;
+  }
+  return TAM_OK;
 }
 
 int tam_multi_tensor_step(const TamTensor* d_tensors, const TamTensor* h_tensors, const TamStepInfo* info,

@@ -12,7 +12,6 @@ loop.  Parameters must live on a HIP device; there is no CPU path.
 
 import ctypes
 import math
-import operator
 import os
 
 import numpy as np
@@ -251,6 +250,23 @@ class _FastStep:
         self.plan = plan
         self.row_params = [params[i] for i in rows]
         self.ptrs = [p.data_ptr() for p in self.row_params]  # parameter storage the descriptor rows point at
+
+    def bind(self, group_step_tensors) -> None:
+        """What the C++ and library calls of a steady step take: the table as a
+        ctypes array, addresses, and the groups' bias-correction sources."""
+        plan = self.plan
+        n = len(plan.table)
+        self.arr = (_lib.TamTensor * n).from_buffer(plan.table)
+        self.info = _lib.TamStepInfo()
+        self.nbytes = ctypes.sizeof(self.arr)
+        self.addrs = (plan.table.ctypes.data, n, plan.gsel.ctypes.data, plan.static_flags.ctypes.data)
+        index = {key: i for i, (key, _, _) in enumerate(self.bc_src)}
+        self.bc = [(group, src) for _, group, src in self.bc_src]
+        self.groups = [(g, index.get((gi, self.device.type, self.device.index), -1)) for g, gi in plan.groups]
+        self.bc_values = (ctypes.c_float * max(1, 2 * len(self.bc)))()
+        # the shared bias-correction tensors, kept alive with their addresses
+        self.bc_tensors = [group_step_tensors[key][k] for key, _, _ in self.bc_src for k in ("bc1", "bc2")]
+        self.bc_ptrs = (ctypes.c_void_p * max(1, len(self.bc_tensors)))(*[t.data_ptr() for t in self.bc_tensors])
 
 
 class TurboAdam(Optimizer):
@@ -881,62 +897,70 @@ class TurboAdam(Optimizer):
                     src = st
             if src is not None:
                 bc_src.append(((group_idx, device.type, device.index), group, src))
+        if any(key not in self._group_step_tensors for key, _, _ in bc_src):
+            return
         self._fast = _FastStep(self._layout_version, device, params, [p.grad is None for p in params], rows,
                                [it[1] for it in items], [it[0].grad for it in items], [it[0].dtype for it in items],
                                bc_src, plan, self.state)
+        self._fast.bind(self._group_step_tensors)
 
     def _fast_state_kept(self, f) -> bool:
         """Whether opt.state still holds f's per-parameter dicts, in order, and
         each descriptor row's state tensors are the objects f kept."""
-        st = self.state
-        if st is not f.state_map or len(st) != len(f.state_values) or \
-                not all(map(operator.is_, st.values(), f.state_values)):
-            return False
-        return _host().states_kept(f)
+        return self.state is f.state_map and _host().values_kept(self.state, f.state_values) \
+            and _host().states_kept(f)
 
     def _fast_step(self) -> bool:
         """A steady step (_FastStep) if this one is; False (nothing done) otherwise."""
         f = self._fast
         if f is None or f.version != self._layout_version:
             return False
-        st = self.state
-        if st is not f.state_map or len(st) != len(f.state_values) or \
-                not all(map(operator.is_, st.values(), f.state_values)):
+        host = _host()
+        if self.state is not f.state_map or not host.values_kept(self.state, f.state_values):
             return False
-        plan = f.plan
-        if self._plans.get(f.device) is not plan:
+        if self._plans.get(f.device) is not f.plan:
             return False
-        t = plan.table
-        # per row, in C++: the same parameters with gradients, their dtypes and
-        # storage, each new gradient's checks, the state tensors; then the
-        # rows' gradient pointers and step numbers are written into t
-        if not _host().steady_rows(f, t.ctypes.data, t.itemsize, _GRAD_OFF, _STEP_OFF):
+        # in C++.  Per row: the same parameters with gradients, their dtypes and
+        # storage, each new gradient's checks, the state tensors; then the rows'
+        # gradient pointers and step numbers are written.  Per group: the scalars.
+        table, n, gsel, flags = f.addrs
+        if not host.steady_rows(f, table, f.plan.table.itemsize, _GRAD_OFF, _STEP_OFF):
             return False
-        device = f.device
-        self._bc_values = {}
-        for key, group, src in f.bc_src:
-            beta1, beta2 = group["betas"]
-            next_step = src["step"] + 1
-            bc = (1.0 - beta1**next_step, 1.0 - beta2**next_step)
-            self._bc_values[key] = bc
-            tb = self._group_step_tensors.get(key)
-            if tb is not None:
-                tb["bc1"].fill_(bc[0])
-                tb["bc2"].fill_(bc[1])
-        flags = plan.static_flags.copy()
-        if plan.cost_rows.size:
-            flags[plan.cost_rows] |= np.uint32(_lib.TAM_FLAG_HAS_STATE)
-        if plan.ef_rows.size:
-            flags[plan.ef_rows] |= np.uint32(_lib.TAM_FLAG_HAS_EF)
-        t["flags"] = flags
-        self._set_group_fields(plan, device)
+        if not host.steady_groups(f, table, n, gsel, flags, ctypes.addressof(f.bc_values)):
+            return False
         lib = _lib.load()
-        bufs = self._device_buffers(device, False)
-        with torch.cuda.device(device):
-            bufs.order_on(torch.cuda.current_stream(device))
-        self._submit(lib, device, plan, bufs, False)
-        _host().advance_steps(f.states)
+        if torch.cuda.current_device() == f.dev_index:
+            self._submit_fast(lib, f)
+        else:
+            with torch.cuda.device(f.device):
+                self._submit_fast(lib, f)
+        host.advance_steps(f.states)
         return True
+
+    # descriptor lists up to this long go up as kernel arguments (tam_put, 12 to
+    # a launch); longer ones are copied from pinned memory
+    _PUT_MAX = 36
+
+    def _submit_fast(self, lib, f) -> None:
+        """The derived fields, the descriptor upload, the shared bias-correction
+        tensors and the step's launches, on the current stream."""
+        _lib.check(lib.tam_prepare(f.arr, len(f.arr), ctypes.byref(f.info)), "tam_prepare")
+        bufs = self._prepare_buffers(f.device, self._device_buffers(f.device, False), f.nbytes, f.info.ws_bytes, None,
+                                     False)
+        stream = torch.cuda.current_stream(f.device)
+        raw = stream.cuda_stream
+        bufs.order_on(stream)
+        desc, ws = bufs.desc_buffer(f.nbytes), bufs.workspace(f.info.ws_bytes)
+        put = len(f.arr) if len(f.arr) <= self._PUT_MAX else 0
+        _lib.check(lib.tam_put(f.addrs[0], put, desc.data_ptr(), f.bc_ptrs, f.bc_values, len(f.bc_tensors), raw),
+                   "tam_put")
+        if not put:
+            upload = self._uploads.get(f.device)
+            if upload is None:
+                upload = self._uploads[f.device] = _PinnedUpload()
+            desc[:f.nbytes].copy_(upload.stage(f.arr, f.nbytes), non_blocking=True)
+            upload.copied(stream)
+        self._issue(lib, desc.data_ptr(), f.arr, f.info, ws, raw)
 
     def _issue(self, lib, desc_ptr: int, arr, info, ws: torch.Tensor, stream: int) -> None:
         """The step's launches: one tam_multi_tensor_step call, or the passes one
