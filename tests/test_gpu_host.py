@@ -192,3 +192,40 @@ def test_replaced_or_reset_state_is_followed():
     for s in (4, 6, 8, 11):  # the step after each change takes the full path
         assert s not in steady
     assert taken[-1]
+
+
+@pytest.mark.parametrize("lr", [np.float32(1e-3), torch.tensor(1e-3, dtype=torch.float64)], ids=["np_f32", "tensor"])
+def test_steady_step_takes_any_number_and_moved_bias_tensors(lr):
+    """Hyperparameters that are no Python floats keep the steady path, with the
+    results of the full one; the shared bias corrections are written where the
+    state's tensors are now, not where they were."""
+    from turboadam_amd import TurboAdam
+
+    dev = torch.device("cuda:0")
+    rng = np.random.default_rng(7)
+    sizes = [5000, 300]
+    init = [torch.from_numpy((rng.standard_normal(n) * 0.02).astype(np.float32)) for n in sizes]
+    grads = [torch.from_numpy((rng.standard_normal(n) * 1e-3).astype(np.float32)).to(dev) for n in sizes]
+    finals = []
+    for steady in (True, False):
+        params = [torch.nn.Parameter(t.to(dev)) for t in init]
+        opt = TurboAdam(params, lr=1e-3, weight_decay=0.05, philox_seed=3)
+        opt.param_groups[0]["lr"] = lr
+        for p, g in zip(params, grads):
+            p.grad = g
+        taken, fast_step = [], opt._fast_step
+        opt._fast_step = (lambda: taken.append(fast_step()) or taken[-1]) if steady else (lambda: False)
+        for step in range(5):
+            if step == 3:
+                st = opt.state[params[0]]
+                old = st["_bc1"].data
+                old_value = old.clone()
+                st["_bc1"].data = torch.zeros_like(old)
+            opt.step()
+        assert not steady or taken == [False, True, True, True, True]
+        assert torch.equal(old, old_value)
+        st = opt.state[params[0]]
+        assert st["_bc1"].item() == np.float32(1.0 - 0.9**5) and st["_bc2"].item() == np.float32(1.0 - 0.999**5)
+        finals.append([p.detach().cpu() for p in params] + [st["compressed_v"]["indices"].cpu()])
+    for a, b in zip(*finals):
+        assert torch.equal(a, b)

@@ -264,9 +264,9 @@ class _FastStep:
         self.bc = [(group, src) for _, group, src in self.bc_src]
         self.groups = [(g, index.get((gi, self.device.type, self.device.index), -1)) for g, gi in plan.groups]
         self.bc_values = (ctypes.c_float * max(1, 2 * len(self.bc)))()
-        # the shared bias-correction tensors, kept alive with their addresses
+        # the shared bias-correction tensors; their addresses are read at each step
         self.bc_tensors = [group_step_tensors[key][k] for key, _, _ in self.bc_src for k in ("bc1", "bc2")]
-        self.bc_ptrs = (ctypes.c_void_p * max(1, len(self.bc_tensors)))(*[t.data_ptr() for t in self.bc_tensors])
+        self.bc_ptrs = (ctypes.c_void_p * max(1, len(self.bc_tensors)))()
 
 
 class TurboAdam(Optimizer):
@@ -927,7 +927,7 @@ class TurboAdam(Optimizer):
         if not host.steady_rows(f, table, f.plan.table.itemsize, _GRAD_OFF, _STEP_OFF):
             return False
         if not host.steady_groups(f, table, n, gsel, flags, ctypes.addressof(f.bc_values)):
-            return False
+            self._steady_groups(f)
         lib = _lib.load()
         if torch.cuda.current_device() == f.dev_index:
             self._submit_fast(lib, f)
@@ -936,6 +936,23 @@ class TurboAdam(Optimizer):
                 self._submit_fast(lib, f)
         host.advance_steps(f.states)
         return True
+
+    def _steady_groups(self, f) -> None:
+        """steady_groups for hyperparameters that are no plain Python numbers (a
+        tensor lr): the operators and __float__ they bring decide."""
+        self._bc_values = {}
+        for i, (key, group, src) in enumerate(f.bc_src):
+            beta1, beta2 = group["betas"]
+            next_step = src["step"] + 1
+            bc = self._bc_values[key] = (1.0 - beta1**next_step, 1.0 - beta2**next_step)
+            f.bc_values[2 * i], f.bc_values[2 * i + 1] = float(bc[0]), float(bc[1])
+        flags = f.plan.static_flags.copy()
+        if f.plan.cost_rows.size:
+            flags[f.plan.cost_rows] |= np.uint32(_lib.TAM_FLAG_HAS_STATE)
+        if f.plan.ef_rows.size:
+            flags[f.plan.ef_rows] |= np.uint32(_lib.TAM_FLAG_HAS_EF)
+        f.plan.table["flags"] = flags
+        self._set_group_fields(f.plan, f.device)
 
     # descriptor lists up to this long go up as kernel arguments (tam_put, 12 to
     # a launch); longer ones are copied from pinned memory
@@ -952,6 +969,8 @@ class TurboAdam(Optimizer):
         bufs.order_on(stream)
         desc, ws = bufs.desc_buffer(f.nbytes), bufs.workspace(f.info.ws_bytes)
         put = len(f.arr) if len(f.arr) <= self._PUT_MAX else 0
+        for i, t in enumerate(f.bc_tensors):
+            f.bc_ptrs[i] = t.data_ptr()
         _lib.check(lib.tam_put(f.addrs[0], put, desc.data_ptr(), f.bc_ptrs, f.bc_values, len(f.bc_tensors), raw),
                    "tam_put")
         if not put:
