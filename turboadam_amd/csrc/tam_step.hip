@@ -13,19 +13,23 @@
 // so one launch covers the whole parameter list.
 //
 // Per step (tam_multi_tensor_step), four passes:
-//   pass 0  tam_k1_main_<dtype> (full quarters; one kernel per parameter dtype
-//           present) and tam_k1_tail (the other quarters): CoState decode + EMA
-//           (or fp32 exp_avg EMA), 1Q decode + EMA + stochastic
+//   pass 0  tam_k1_main_<dtype>, or tam_k1_vf32_ / tam_k1_mf32_ (no tensor of the
+//           dtype has 1Q v / every one has 1Q v and fp32 m) and tam_k1_ef_ (error
+//           feedback): full units; tam_k1_tail: the other quarters.  CoState
+//           decode + EMA (or fp32 exp_avg EMA), 1Q decode + EMA + stochastic
 //           re-quantisation (or fp32 exp_avg_sq), denominator, decoupled
 //           weight decay, parameter update; per-quarter-tile partials of
 //           g.g and m.g (fp32 per lane, fp64 across lanes and blocks).
-//   pass 1  tam_k_alpha_chunks, tam_k_alpha: alpha = m.g / g.g per CoState
-//           tensor (pairwise trees over the partials).
-//   pass 2  tam_k2_encode: CoState tiles: recompute m, delta = m - alpha*g,
-//           sign bits, block norms, fp16 amplitudes, block ratios.
-//   pass 3  tam_k_sel_minmax, tam_k_sel_hist and tam_k_sel_pick (three
-//           rounds), tam_k_sel_labels: radix selection of the two order
-//           statistics over slices of the ratios, labels, alpha write-back.
+//   pass 1  tam_k_alpha_chunks (and tam_k_alpha for tensors of several chunks):
+//           alpha = m.g / g.g per CoState tensor (pairwise trees over the
+//           partials).
+//   pass 2  tam_k2_encode, tam_k2_encode_f32, tam_k2_ef: CoState tiles:
+//           recompute m, delta = m - alpha*g, sign bits, block norms, fp16
+//           amplitudes, block ratios.
+//   pass 3  tam_k_sel_one (small tensors, one workgroup each); tam_k_sel_minmax,
+//           three tam_k_sel_hist and tam_k_sel_labels (the others): radix
+//           selection of the two order statistics of the ratios, labels, alpha
+//           write-back.
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -2931,32 +2935,83 @@ __device__ __forceinline__ void tam_k4_quarter(const TamTensor& d, uint32_t wq, 
   if (FULL || W.nv > 0) tam_g(d.signs)[W.e0 >> 3] = (uint8_t)cn.byte;
 }
 
-__global__ __launch_bounds__(TAM_WG) void tam_k4_ef(const TamTensor* __restrict__ T, int nT, uint32_t total_tiles,
-                                                    const float* __restrict__ alpha_new,
-                                                    const float* __restrict__ alpha_old, char* __restrict__ ws) {
+// A full unit of pass 4, 16 elements per lane as in tam_k2_ef: the residual (and
+// an fp32 gradient) in whole lines.
+template <uint32_t DT>
+__device__ __forceinline__ void tam_k4_unit(const TamTensor& d, uint32_t u, uint32_t lane, float a_old, float a_new,
+                                            char* __restrict__ ws, TamTurn* turn) {
+  const uint32_t l8 = lane & 7u;
+  const uint32_t b = u * 8u + (lane >> 3);
+  const uint64_t eu = (uint64_t)u * (8u * TAM_BLOCK_SIZE), e0 = eu + lane * TAM_EPU;
+  const bool has_ef = (d.flags & TAM_FLAG_HAS_EF) != 0;
+  const TamStage st = tam_stage(d, ws);
+  const TamK2U<DT == TAM_DTYPE_F32> in = tam_k2u_load<DT == TAM_DTYPE_F32>(d, u, lane);
+  TamF4 w[4] = {};
+  if (has_ef) tam_unit_ld<true>(d.ef_residual, eu, lane, w);
+  const uint32_t label = tam_g(st.labels)[b], amp = tam_g(st.amp)[b];  // the staged new encoding
+  const float nrm = tam_g(st.norms)[b];
+  const uint32_t bytes = tam_g((const TamH1B*)(st.signs + (e0 >> 3)))[0];
+  tam_compiler_fence();
+  float g[TAM_EPU], r[TAM_EPU], ge[TAM_EPU], m[TAM_EPU];
+  if constexpr (DT == TAM_DTYPE_F32) {
+    tam_turn_in(turn, lane, in.g, g);
+  } else {
+    tam_unpack8<DT>(in.g[0], g);
+    tam_unpack8<DT>(in.g[1], g + TAM_EPL);
+  }
+  tam_turn_in(turn, lane, w, r);
+#pragma unroll
+  for (int i = 0; i < TAM_EPU; ++i) ge[i] = has_ef ? g[i] + r[i] : g[i];
+  TamWave W;  // only its bvalid is read (full unit)
+  W.bvalid = true;
+  TamCsIn c0 = in.cs, c1 = in.cs;
+  c0.byte = in.cs.byte & 0xffu;
+  c1.byte = in.cs.byte >> 8;
+  tam_costate_m<true, false>(d, W, c0, a_old, g, ge, m);
+  tam_costate_m<true, false>(d, W, c1, a_old, g + TAM_EPL, ge + TAM_EPL, m + TAM_EPL);
+  const float sph = tam_div_sqrt_block(nrm);
+  const float s = label == 1u ? sph : (label == 2u ? tam_f16_to_f32((uint16_t)amp) : 0.0f);
+  // element 8j + k is bit 7 - k of byte j
+  const uint32_t sh = (bytes << 24) | ((bytes << 8) & 0x00ff0000u);
+#pragma unroll
+  for (int i = 0; i < TAM_EPU; ++i) {
+    const float delta = m[i] - a_new * g[i];  // costate.py:42
+    const float sd = tam_u2f((tam_f2u(s) & 0x7fffffffu) | ((sh << i) & 0x80000000u));
+    const float dh = 0.0f * g[i] + sd;        // decode with alpha = 0 (costate.py:428-432)
+    const float e = delta - dh;
+    r[i] = has_ef ? d.beta1 * r[i] + d.one_minus_beta1 * e : e;
+  }
+  tam_unit_store(turn, d.ef_residual, eu, lane, r);
+  tam_compiler_fence();
+  if (l8 == 0u) {
+    tam_g(d.labels)[b] = (uint8_t)label;
+    tam_g(d.norms)[b] = nrm;
+    tam_g(d.amp)[b] = (uint16_t)amp;
+  }
+  tam_g((uint16_t*)(d.signs + (e0 >> 3)))[0] = (uint16_t)bytes;
+}
+
+// Pass 4 of the tensors of one dtype, its tiles dealt out as in tam_k2_ef.
+template <uint32_t DT>
+__global__ __launch_bounds__(TAM_K1U_WG) void tam_k4_ef(const TamTensor* __restrict__ T, int nT, uint32_t total_tiles,
+                                                        const float* __restrict__ alpha_new,
+                                                        const float* __restrict__ alpha_old, char* __restrict__ ws) {
   if (tam_step_skipped(T)) return;
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-  int ti = tam_find_tensor(T, nT, blockIdx.x);
-  for (uint32_t tile = blockIdx.x; tile < total_tiles; tile += gridDim.x) {
-    ti = tam_advance_tensor(T, nT, ti, tile);
+  __shared__ TamTurn turn[TAM_K1U_WG / 64];
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+  uint32_t tile = tam_tile_slot(blockIdx.x, gridDim.x);
+  int ti = tam_find_tensor(T, nT, tile < total_tiles ? tile : total_tiles - 1u);
+  for (; tile < total_tiles; tile += gridDim.x) {
+    ti = __builtin_amdgcn_readfirstlane(tam_advance_tensor(T, nT, ti, tile));
     const TamTensor& d = T[ti];
-    if (!(d.flags & TAM_FLAG_EF)) continue;  // uniform over the workgroup
-    const uint32_t wq = (tile - d.tile0) * 4u + wave;
-    const float ao = alpha_old[ti], an = alpha_new[ti];
-    const bool full = tam_quarter_full(d, wq);
-    switch (d.dtype) {
-      case TAM_DTYPE_BF16:
-        if (full) tam_k4_quarter<TAM_DTYPE_BF16, true>(d, wq, lane, ao, an, ws);
-        else tam_k4_quarter<TAM_DTYPE_BF16, false>(d, wq, lane, ao, an, ws);
-        break;
-      case TAM_DTYPE_F16:
-        if (full) tam_k4_quarter<TAM_DTYPE_F16, true>(d, wq, lane, ao, an, ws);
-        else tam_k4_quarter<TAM_DTYPE_F16, false>(d, wq, lane, ao, an, ws);
-        break;
-      default:
-        if (full) tam_k4_quarter<TAM_DTYPE_F32, true>(d, wq, lane, ao, an, ws);
-        else tam_k4_quarter<TAM_DTYPE_F32, false>(d, wq, lane, ao, an, ws);
-        break;
+    if (!(d.flags & TAM_FLAG_EF) || d.dtype != DT) continue;  // uniform
+    const uint32_t u = (tile - d.tile0) * 2u + wave;
+    const float ao = *(const TAM_CONST float*)(alpha_old + ti), an = *(const TAM_CONST float*)(alpha_new + ti);
+    if (tam_unit_full(d, u)) {
+      tam_k4_unit<DT>(d, u, lane, ao, an, ws, &turn[wave]);
+    } else {
+      tam_k4_quarter<DT, false>(d, 2u * u, lane, ao, an, ws);
+      tam_k4_quarter<DT, false>(d, 2u * u + 1u, lane, ao, an, ws);
     }
   }
 }
@@ -3648,7 +3703,7 @@ static bool tam_wd_keeps_16bit(uint32_t dtype, float c_wd) {
 // than one tile each; pass 2, which loads each unit one ahead, is fastest with 8
 // (7% faster than 32 on that set).
 enum { TAM_KS_K1, TAM_KS_K2 = TAM_KS_K1 + 12, TAM_KS_K2_F32, TAM_KS_K2_EF, TAM_KS_K4_EF = TAM_KS_K2_EF + 3,
-       TAM_KS_COUNT };  // TAM_KS_K1 + 3 * mode + dtype, TAM_KS_K2_EF + dtype
+       TAM_KS_COUNT = TAM_KS_K4_EF + 3 };  // TAM_KS_K1 + 3 * mode + dtype, TAM_KS_K2_EF + dtype, TAM_KS_K4_EF + dtype
 #ifndef TAM_K2_GRID_ROUNDS
 #define TAM_K2_GRID_ROUNDS 8
 #endif
@@ -3938,8 +3993,15 @@ static int tam_launch_pass(int pass, const TamTensor* d_tensors, const TamStepIn
       }
       break;
     case 4:
-      hipLaunchKernelGGL(tam_k4_ef, dim3(grid_of(TAM_KS_K4_EF, (const void*)tam_k4_ef)), dim3(TAM_WG), 0, s, d_tensors,
-                         info->n_tensors, info->total_tiles, alpha_new, alpha_old, ws);
+      for (uint32_t dt = TAM_DTYPE_F32; dt <= TAM_DTYPE_F16; ++dt) {
+        if (!(info->ef_mask & (1u << dt))) continue;
+        const auto k = dt == TAM_DTYPE_BF16 ? tam_k4_ef<TAM_DTYPE_BF16>
+                       : dt == TAM_DTYPE_F16 ? tam_k4_ef<TAM_DTYPE_F16>
+                                             : tam_k4_ef<TAM_DTYPE_F32>;
+        hipLaunchKernelGGL(k, dim3(grid_of(TAM_KS_K4_EF + (int)dt, (const void*)k, TAM_K1U_WG)), dim3(TAM_K1U_WG), 0, s,
+                           d_tensors, info->n_tensors, info->total_tiles, alpha_new, alpha_old, ws);
+        TAM_HIP_CHECK(hipGetLastError());
+      }
       break;
   }
   TAM_HIP_CHECK(hipGetLastError());
