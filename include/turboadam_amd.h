@@ -125,11 +125,10 @@ typedef struct TamTensor {
                             /*      *found_inf != 0 (a GradScaler skip).  Given */
                             /*      for one descriptor, given for all (the same */
                             /*      pointer): the launches test descriptor 0.   */
-  uint32_t tail0;           /* [derived] first workgroup of this tensor in pass 0's */
-                            /*      kernel for quarters that are not full        */
+  uint32_t tail0;           /* [derived] first workgroup of this tensor among those */
+                            /*      of pass 0 for quarters outside full units     */
   uint32_t tail_wgs;        /* [derived] its workgroups there: one when a part of */
-                            /*      it lies outside full units (8 blocks), none  */
-                            /*      otherwise or with EF                         */
+                            /*      it lies outside full units (8 blocks), else 0 */
 } TamTensor;
 
 /* Launch summary and workspace layout, filled by tam_prepare(). */
@@ -150,7 +149,7 @@ typedef struct TamStepInfo {
   uint32_t n_ef;           /* tensors with error feedback (a fifth pass runs) */
   uint32_t n_device_step;  /* DEVICE_STEP tensors (pass 0 starts with their prologue) */
   uint64_t off_ef_alpha;   /* EF: previous alpha of each tensor (f32 per tensor) */
-  uint32_t tail_blocks;    /* workgroups of pass 0's kernel for quarters that are not full */
+  uint32_t tail_blocks;    /* workgroups of pass 0 for quarters outside full units */
   uint32_t sel_small;      /* a CoState tensor of at most this many blocks is one workgroup's selection: */
                            /* 32768, or 12288 when some tensor has more than 32768 (slices run then) */
   uint32_t sel_max;        /* blocks of the largest such tensor (0: none) */

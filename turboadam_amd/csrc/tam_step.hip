@@ -15,7 +15,7 @@
 // Per step (tam_multi_tensor_step), four passes:
 //   pass 0  tam_k1_main_<dtype>, or tam_k1_vf32_ / tam_k1_mf32_ (no tensor of the
 //           dtype has 1Q v / every one has 1Q v and fp32 m) and tam_k1_ef_ (error
-//           feedback): full units; tam_k1_tail: the other quarters.  CoState
+//           feedback): CoState
 //           decode + EMA (or fp32 exp_avg EMA), 1Q decode + EMA + stochastic
 //           re-quantisation (or fp32 exp_avg_sq), denominator, decoupled
 //           weight decay, parameter update; per-quarter-tile partials of
@@ -1281,16 +1281,25 @@ __device__ __forceinline__ bool tam_step_skipped(const TamTensor* __restrict__ T
 // ---------------------------------------------------------------------------
 // Pass 0: the fused update
 // ---------------------------------------------------------------------------
+// MODE fixes what a kernel's tensors have in common, so that its registers and
+// its first loads are theirs:
+//   TAM_K1_ANY     flags decide (fp32 moments are loaded when they are needed:
+//                  up front their registers would count against every unit)
+//   TAM_K1_V_F32   fp32 second moment (loaded up front, no 1Q code), either first
+//   TAM_K1_M_F32   fp32 first moment (loaded up front), 1Q second
+//   TAM_K1_EF      CoState with error feedback (the residual is loaded up front)
+enum { TAM_K1_ANY, TAM_K1_V_F32, TAM_K1_M_F32, TAM_K1_EF };
+
 // Per quarter tile: loads, first moment (CoState or fp32), second moment (1Q or
 // fp32), update, store; for CoState tensors the fp64 partial sums of g.g and
 // m.g over the quarter's 4 blocks (pairwise: blocks, then pairs of blocks).
-template <uint32_t DT, bool FULL>
+template <uint32_t DT, bool FULL, int MODE>
 __device__ __forceinline__ void tam_k1_quarter(const TamTensor& d, uint32_t wq, uint32_t lane, float* lutw,
                                                const TamLdsTabs* tabs, uint32_t seed_lo, uint32_t seed_hi,
                                                double2* __restrict__ part) {
   const TamWave W = tam_wave(d, wq, lane, FULL);
-  const bool costate = (d.flags & TAM_FLAG_COSTATE) != 0;
-  const bool compress_v = (d.flags & TAM_FLAG_COMPRESS_V) != 0;
+  const bool costate = MODE == TAM_K1_EF || (MODE != TAM_K1_M_F32 && (d.flags & TAM_FLAG_COSTATE) != 0);
+  const bool compress_v = MODE == TAM_K1_M_F32 || (MODE != TAM_K1_V_F32 && (d.flags & TAM_FLAG_COMPRESS_V) != 0);
   float g[TAM_EPL], p[TAM_EPL], m[TAM_EPL], v[TAM_EPL];
   // every load of the quarter is issued before any result is used
   if (FULL || W.bvalid) {
@@ -1310,7 +1319,12 @@ __device__ __forceinline__ void tam_k1_quarter(const TamTensor& d, uint32_t wq, 
   // ---- first moment ---------------------------------------------------
   if (costate) {
     float ge[TAM_EPL];  // error feedback: the EMA takes g + residual (costate.py:410-416)
-    tam_ef_grad<FULL>(d, W, g, ge);
+    if constexpr (MODE == TAM_K1_EF) {
+      tam_ef_grad<FULL>(d, W, g, ge);
+    } else {
+#pragma unroll
+      for (int i = 0; i < TAM_EPL; ++i) ge[i] = g[i];
+    }
     if (FULL || W.bvalid) tam_costate_m<FULL>(d, W, cs, alpha_prev, g, ge, m);
     float gz[TAM_EPL], mz[TAM_EPL];
 #pragma unroll
@@ -1626,15 +1640,6 @@ __device__ __forceinline__ void tam_vunit_b(const TamTensor& d, uint32_t lane, u
 // the unit's two quarters (part: quarter 2u's {g.g, m.g}, then 2u + 1's).
 // Every load of the unit (but an fp32 parameter's) is issued first and its
 // value pinned, so the unit waits on memory once.
-//
-// MODE fixes what a kernel's tensors have in common, so that its registers and
-// its first loads are theirs:
-//   TAM_K1_ANY     flags decide (fp32 moments are loaded when they are needed:
-//                  up front their registers would count against every unit)
-//   TAM_K1_V_F32   fp32 second moment (loaded up front, no 1Q code), either first
-//   TAM_K1_M_F32   fp32 first moment (loaded up front), 1Q second
-//   TAM_K1_EF      CoState with error feedback (the residual is loaded up front)
-enum { TAM_K1_ANY, TAM_K1_V_F32, TAM_K1_M_F32, TAM_K1_EF };
 template <uint32_t DT, int MODE>
 __device__ __forceinline__ void tam_k1_unit(const TamTensor& d, uint32_t u, uint32_t lane, float* lutw,
                                             const TamLdsTabs* tabs, TamTurn* turn, uint32_t seed_lo,
@@ -1806,14 +1811,25 @@ __device__ __forceinline__ void tam_k1_unit(const TamTensor& d, uint32_t u, uint
   if (compress_v) tam_vunit_b(d, lane, b, e0, v, vx, tabs, seed_lo, seed_hi);
 }
 
+// Workgroups of pass 0 in front of those that stride over the tiles.
+__host__ __device__ __forceinline__ uint32_t tam_tail_grid(uint32_t tails) { return (tails + 7u) & ~7u; }
+
 // Full units (inside the tensor) of one parameter dtype:
 // persistent workgroups of two waves stride over the tiles; wave w takes unit
 // 2(tile - tile0) + w of the tile's tensor (quarters 4(tile - tile0) + 2w and
 // + 1), and the waves never synchronise with each other.  One kernel per
 // dtype and mode holds only that code, so each gets its own register budget.
+//
+// The at most two quarters of a tensor outside full units are a workgroup's of
+// the same launch, a wave per quarter: the first workgroups (tails of them,
+// rounded up to the 8 XCDs; tam_prepare: tail0, tail_wgs) take one tensor each.
+// A launch of their own after this one was a serial chain of 8 us (norms and
+// biases of a GPT-2 block alone: 26.8 us a step with it, 23.0 without) to 15 us
+// (1000 ragged tensors: 341 and 320; a GPT-2 block 71.4 and 60.5).  In front,
+// where they start first, the chain lies beside the units' work.
 template <uint32_t DT, int MODE>
 __device__ __forceinline__ void tam_k1_full_body(const TamTensor* __restrict__ T, int nT, uint32_t total_tiles,
-                                                 uint32_t seed_lo, uint32_t seed_hi,
+                                                 uint32_t tails, uint32_t seed_lo, uint32_t seed_hi,
                                                  double2* __restrict__ partials) {
   if (tam_step_skipped(T)) return;
   // rows of 64 levels, 256-byte aligned (tam_vunit_a forms addresses by or)
@@ -1823,19 +1839,31 @@ __device__ __forceinline__ void tam_k1_full_body(const TamTensor* __restrict__ T
   if constexpr (MODE != TAM_K1_V_F32) tam_lds_tabs_fill(&tabs);
   const uint32_t hw_wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
   const uint32_t wave = hw_wave & 1u;  // within the virtual workgroup
-  const uint32_t stride = gridDim.x * TAM_K1_VWG;
   float* lutw = lut[hw_wave];
+  const uint32_t front = tam_tail_grid(tails);
+  if (blockIdx.x < front) {  // uniform
+    if (blockIdx.x >= tails) return;
+    const TamTensor& d = T[tam_wave_first(nT, [&](int i) { return T[i].tail0 + T[i].tail_wgs > blockIdx.x; })];
+    if (d.dtype != DT || ((d.flags & TAM_FLAG_EF) != 0) != (MODE == TAM_K1_EF)) return;
+    const uint32_t wq = 2u * (uint32_t)(d.n / (8u * TAM_BLOCK_SIZE)) + hw_wave;  // after the full units
+    if (hw_wave < 2u && wq < (d.nb + 3u) / 4u)
+      tam_k1_quarter<DT, false, MODE>(d, wq, lane, lutw, &tabs, seed_lo, seed_hi,
+                                      partials + (uint64_t)d.tile0 * 4u + wq);
+    return;
+  }
+  const uint32_t wg = blockIdx.x - front, wgs = gridDim.x - front;
+  const uint32_t stride = wgs * TAM_K1_VWG;
   // tensor by tensor: the descriptor is read once per tensor, then the wave
   // takes its units of the tensor in grid strides
-  uint32_t tile = tam_tile_slot(blockIdx.x, gridDim.x) * TAM_K1_VWG + (hw_wave >> 1);
+  uint32_t tile = tam_tile_slot(wg, wgs) * TAM_K1_VWG + (hw_wave >> 1);
   int ti = tam_find_tensor(T, nT, tile < total_tiles ? tile : total_tiles - 1u);
   while (tile < total_tiles) {
     ti = tam_advance_tensor(T, nT, ti, tile);
     const TamTensor& d = T[ti];
     const uint32_t end = d.tile0 + d.ntiles;  // the tensor's tiles end here
     if (d.dtype == DT && ((d.flags & TAM_FLAG_EF) != 0) == (MODE == TAM_K1_EF)) {  // uniform
-      // units u < nfull are full; the rest is tam_k1_tail's, and u grows with
-      // the tile
+      // units u < nfull are full; the rest is the first workgroups', and u grows
+      // with the tile
       const uint64_t nfull = d.n / (8u * TAM_BLOCK_SIZE);
       for (; tile < end; tile += stride) {
         const uint32_t u = (tile - d.tile0) * 2u + wave;  // unit within the tensor
@@ -1850,9 +1878,9 @@ __device__ __forceinline__ void tam_k1_full_body(const TamTensor* __restrict__ T
 
 #define TAM_K1_FULL_KERNEL(NAME, DT, MODE, WAVES)                                                               \
   __global__ __launch_bounds__(TAM_K1_BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES))) void NAME(    \
-      const TamTensor* __restrict__ T, int nT, uint32_t total_tiles, uint32_t seed_lo, uint32_t seed_hi,      \
-      double2* __restrict__ partials) {                                                                       \
-    tam_k1_full_body<DT, MODE>(T, nT, total_tiles, seed_lo, seed_hi, partials);                               \
+      const TamTensor* __restrict__ T, int nT, uint32_t total_tiles, uint32_t tails, uint32_t seed_lo,        \
+      uint32_t seed_hi, double2* __restrict__ partials) {                                                     \
+    tam_k1_full_body<DT, MODE>(T, nT, total_tiles, tails, seed_lo, seed_hi, partials);                        \
   }
 #ifndef TAM_K1_WAVES_BF16
 #define TAM_K1_WAVES_BF16 4
@@ -1881,34 +1909,6 @@ TAM_K1_FULL_KERNEL(tam_k1_mf32_f32, TAM_DTYPE_F32, TAM_K1_M_F32, TAM_K1_WAVES_F3
 TAM_K1_FULL_KERNEL(tam_k1_ef_bf16, TAM_DTYPE_BF16, TAM_K1_EF, TAM_K1_WAVES_BF16)
 TAM_K1_FULL_KERNEL(tam_k1_ef_f16, TAM_DTYPE_F16, TAM_K1_EF, TAM_K1_WAVES_F16)
 TAM_K1_FULL_KERNEL(tam_k1_ef_f32, TAM_DTYPE_F32, TAM_K1_EF, TAM_K1_WAVES_F32)
-
-// The at most two quarters of each tensor outside full units, one workgroup per
-// tensor that has any (tam_prepare: tail0, tail_wgs), a wave per quarter.
-__global__ __launch_bounds__(TAM_K1U_WG) void tam_k1_tail(const TamTensor* __restrict__ T, int nT, uint32_t seed_lo,
-                                                      uint32_t seed_hi, double2* __restrict__ partials) {
-  if (tam_step_skipped(T)) return;
-  const TamTensor& d = T[tam_wave_first(nT, [&](int i) { return T[i].tail0 + T[i].tail_wgs > blockIdx.x; })];
-  __shared__ float lut[TAM_K1U_WG / 64][4 * 64];
-  __shared__ TamLdsTabs tabs;
-  tam_lds_tabs_fill(&tabs);
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-  // full units precede: tam_k1_main_<dtype> takes them
-  const uint32_t first = 2u * (uint32_t)(d.n / (8u * TAM_BLOCK_SIZE)), last = (d.nb + 3u) / 4u;
-  for (uint32_t wq = first + wave; wq < last; wq += TAM_K1U_WG / 64) {
-    double2* part = partials + (uint64_t)d.tile0 * 4u + wq;
-    switch (d.dtype) {
-      case TAM_DTYPE_BF16:
-        tam_k1_quarter<TAM_DTYPE_BF16, false>(d, wq, lane, lut[wave], &tabs, seed_lo, seed_hi, part);
-        break;
-      case TAM_DTYPE_F16:
-        tam_k1_quarter<TAM_DTYPE_F16, false>(d, wq, lane, lut[wave], &tabs, seed_lo, seed_hi, part);
-        break;
-      default:
-        tam_k1_quarter<TAM_DTYPE_F32, false>(d, wq, lane, lut[wave], &tabs, seed_lo, seed_hi, part);
-        break;
-    }
-  }
-}
 
 // ---------------------------------------------------------------------------
 // Pass 1: alpha of every CoState tensor (costate.py:37-41)
@@ -2936,7 +2936,8 @@ __device__ __forceinline__ void tam_k4_quarter(const TamTensor& d, uint32_t wq, 
 }
 
 // A full unit of pass 4, 16 elements per lane as in tam_k2_ef: the residual (and
-// an fp32 gradient) in whole lines.
+// an fp32 gradient) in whole lines.  Bound by memory: 375 us for 218M bf16
+// elements (2.27 GB) are 6.0 TB/s, a copy's rate.
 template <uint32_t DT>
 __device__ __forceinline__ void tam_k4_unit(const TamTensor& d, uint32_t u, uint32_t lane, float a_old, float a_new,
                                             char* __restrict__ ws, TamTurn* turn) {
@@ -3901,15 +3902,17 @@ static int tam_launch_pass(int pass, const TamTensor* d_tensors, const TamStepIn
   };
   // pass 0's kernel of a mode and dtype
   const auto k1_launch = [&](int mode, uint32_t dt) -> int {
-    typedef void (*Kernel)(const TamTensor*, int, uint32_t, uint32_t, uint32_t, double2*);
+    typedef void (*Kernel)(const TamTensor*, int, uint32_t, uint32_t, uint32_t, uint32_t, double2*);
     static const Kernel kernels[4][3] = {{tam_k1_main_f32, tam_k1_main_bf16, tam_k1_main_f16},
                                          {tam_k1_vf32_f32, tam_k1_vf32_bf16, tam_k1_vf32_f16},
                                          {tam_k1_mf32_f32, tam_k1_mf32_bf16, tam_k1_mf32_f16},
                                          {tam_k1_ef_f32, tam_k1_ef_bf16, tam_k1_ef_f16}};
     const Kernel k = kernels[mode][dt];
-    hipLaunchKernelGGL(k, dim3(grid_of(TAM_KS_K1 + 3 * mode + (int)dt, (const void*)k, TAM_K1_BLOCK, TAM_K1_VWG)),
-                       dim3(TAM_K1_BLOCK), 0, s, d_tensors, info->n_tensors, info->total_tiles, (uint32_t)seed,
-                       (uint32_t)(seed >> 32), partials);
+    hipLaunchKernelGGL(k,
+                       dim3(grid_of(TAM_KS_K1 + 3 * mode + (int)dt, (const void*)k, TAM_K1_BLOCK, TAM_K1_VWG) +
+                            tam_tail_grid(info->tail_blocks)),
+                       dim3(TAM_K1_BLOCK), 0, s, d_tensors, info->n_tensors, info->total_tiles, info->tail_blocks,
+                       (uint32_t)seed, (uint32_t)(seed >> 32), partials);
     TAM_HIP_CHECK(hipGetLastError());
     return TAM_OK;
   };
@@ -3931,9 +3934,6 @@ static int tam_launch_pass(int pass, const TamTensor* d_tensors, const TamStepIn
           if (rc != TAM_OK) return rc;
         }
       }
-      if (info->tail_blocks)
-        hipLaunchKernelGGL(tam_k1_tail, dim3(info->tail_blocks), dim3(TAM_K1U_WG), 0, s, d_tensors, info->n_tensors,
-                           (uint32_t)seed, (uint32_t)(seed >> 32), partials);
       break;
     case 1:
       hipLaunchKernelGGL(tam_k_alpha_chunks, dim3(info->total_chunks), dim3(TAM_WG), 0, s, d_tensors,

@@ -955,7 +955,9 @@ class TurboAdam(Optimizer):
         self._set_group_fields(f.plan, f.device)
 
     # descriptor lists up to this long go up as kernel arguments (tam_put, 12 to
-    # a launch); longer ones are copied from pinned memory
+    # a launch); longer ones are copied from pinned memory.  Steps of n vectors
+    # of 768, arguments against copy: n = 12 23 and 34 us, 36 34 and 38, 48 38
+    # and 40, 72 49 and 44, 148 88 and 56
     _PUT_MAX = 36
 
     def _submit_fast(self, lib, f) -> None:
