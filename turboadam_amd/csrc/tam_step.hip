@@ -396,9 +396,14 @@ __device__ __forceinline__ void tam_wave_lds_sync() {
 // turns the rows in LDS.  The unit's 256 16-byte chunks q (element 4 q) lie at
 // slot q ^ ((q >> 4) & 3): a wave's 16-byte accesses, by chunk 64 k + lane or by
 // chunk 4 lane + j, then touch every bank once per 16 lanes.
-struct TamTurn {
+//
+// A lane's four slots of the second kind are its first with j xored into address
+// bits 4 and 5, so the array has to start on a multiple of 64 bytes, whatever
+// other LDS a kernel has.
+struct __attribute__((aligned(64))) TamTurn {
   TamW4 slot[256];
 };
+static_assert(alignof(TamTurn) == 64 && sizeof(TamTurn) % 64 == 0, "every row of a TamTurn array starts 64-byte aligned");
 struct TamTurnAt {  // byte addresses of a lane's slots
   uint32_t col, row;
 };
