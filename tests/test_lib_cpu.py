@@ -6,13 +6,14 @@ declares, agrees with the Python struct mirror, and its host-only planning
 import ctypes
 import os
 import re
+import subprocess
 
 import numpy as np
 import pytest
 import torch
 
 from turboadam_amd import _lib
-from turboadam_amd.build import LIB_PATH, REPO_DIR
+from turboadam_amd.build import HIP_FLAGS, HIPCC, LIB_PATH, REPO_DIR, SOURCES
 
 HEADER = os.path.join(REPO_DIR, "include", "turboadam_amd.h")
 
@@ -230,3 +231,13 @@ def test_steady_step_sees_replaced_or_reset_state():
     # the full path compares device addresses of the same tensors
     rows = [_row_tensors(opt.state[p], True) for p in params]
     assert len(_tensor_ptrs(rows)) == 8 + 3 and _tensor_ptrs(rows)[7] == 0  # no error-feedback residual
+
+
+def test_kernels_claim_no_more_alignment_than_their_arrays_have():
+    """A pointer to an element-aligned vector that is passed on as a pointer to the
+    16-byte-aligned one lets the compiler assume an alignment the caller's array
+    does not have; the device compiler reports each such call."""
+    flags = [f for f in HIP_FLAGS if f not in ("-fPIC", "-shared")]
+    res = subprocess.run([HIPCC, *flags, "--cuda-device-only", "-fsyntax-only", "-Werror=align-mismatch", *SOURCES],
+                         capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr[-2000:]

@@ -128,7 +128,9 @@ __device__ __forceinline__ void tam_unpack8(TamW4 w, float* out) {
 
 // The same vectors at element alignment: gfx950 loads and stores global memory at
 // any address, so one instruction moves 16 bytes of a caller's array that is
-// only aligned to its elements.
+// only aligned to its elements.  TAM_GA casts to them: tam_g deduces its type, and
+// a deduced (or template argument) type loses the alignment.
+#define TAM_GA(T, p) ((TAM_GLOBAL T*)(p))
 typedef float TamF4E __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t TamW4E __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t TamW4B __attribute__((ext_vector_type(4), aligned(1)));
@@ -139,7 +141,7 @@ typedef uint16_t TamH1B __attribute__((aligned(1)));
 // 16 consecutive elements of an array of a 16-bit dtype DT as fp32 (all exist).
 template <uint32_t DT>
 __device__ __forceinline__ void tam_ld16(const void* base, uint64_t e0, float* out) {
-  const TAM_GLOBAL TamW4E* b = tam_g((const TamW4E*)((const uint16_t*)base + e0));
+  const TAM_GLOBAL TamW4E* b = TAM_GA(const TamW4E, ((const uint16_t*)base + e0));
   const TamW4 x = b[0], y = b[1];
   tam_unpack8<DT>(x, out);
   tam_unpack8<DT>(y, out + 8);
@@ -152,7 +154,7 @@ __device__ __forceinline__ void tam_ld8(const void* base, uint64_t e0, uint32_t 
   if (DT == TAM_DTYPE_F32) {
     const float* b = (const float*)base + e0;
     if (FULL) {
-      const TamF4 a = tam_g((const TamF4E*)b)[0], c = tam_g((const TamF4E*)b)[1];
+      const TamF4 a = TAM_GA(const TamF4E, b)[0], c = TAM_GA(const TamF4E, b)[1];
       out[0] = a.x; out[1] = a.y; out[2] = a.z; out[3] = a.w;
       out[4] = c.x; out[5] = c.y; out[6] = c.z; out[7] = c.w;
     } else {
@@ -162,7 +164,7 @@ __device__ __forceinline__ void tam_ld8(const void* base, uint64_t e0, uint32_t 
   } else {
     const uint16_t* b = (const uint16_t*)base + e0;
     if (FULL) {
-      tam_unpack8<DT>(tam_g((const TamW4E*)b)[0], out);
+      tam_unpack8<DT>(TAM_GA(const TamW4E, b)[0], out);
     } else {
 #pragma unroll
       for (int i = 0; i < TAM_EPL; ++i) out[i] = (uint32_t)i < nv ? tam_h2f<DT>(tam_g(b)[i]) : 0.0f;
@@ -179,8 +181,8 @@ template <bool FULL>
 __device__ __forceinline__ void tam_st8_f32(float* base, uint64_t e0, uint32_t nv, const float* v) {
   float* b = base + e0;
   if (FULL) {
-    tam_g((TamF4E*)b)[0] = TamF4{v[0], v[1], v[2], v[3]};
-    tam_g((TamF4E*)b)[1] = TamF4{v[4], v[5], v[6], v[7]};
+    TAM_GA(TamF4E, b)[0] = TamF4{v[0], v[1], v[2], v[3]};
+    TAM_GA(TamF4E, b)[1] = TamF4{v[4], v[5], v[6], v[7]};
   } else {
 #pragma unroll
     for (int i = 0; i < TAM_EPL; ++i)
@@ -194,7 +196,7 @@ template <bool FULL>
 __device__ __forceinline__ void tam_st8_bits(void* base, uint64_t e0, uint32_t nv, const uint32_t* pw2) {
   uint16_t* b = (uint16_t*)base + e0;
   if (FULL) {
-    tam_g((TamW4E*)b)[0] = TamW4{pw2[0], pw2[1], pw2[2], pw2[3]};
+    TAM_GA(TamW4E, b)[0] = TamW4{pw2[0], pw2[1], pw2[2], pw2[3]};
   } else {
 #pragma unroll
     for (int i = 0; i < TAM_EPL; ++i)
@@ -425,12 +427,12 @@ __device__ __forceinline__ TAM_LDS TamF4* tam_lds_f4(uint32_t addr) { return (TA
 // fp32 first moment; a gradient that pass 2 still reads is left to the caches.
 template <bool NT = false>
 __device__ __forceinline__ void tam_unit_ld(const float* base, uint64_t e, uint32_t lane, TamF4* w) {
-  const TAM_GLOBAL TamF4E* b = tam_g((const TamF4E*)(base + e)) + lane;
+  const TAM_GLOBAL TamF4E* b = TAM_GA(const TamF4E, (base + e)) + lane;
 #pragma unroll
   for (int k = 0; k < 4; ++k) w[k] = NT ? __builtin_nontemporal_load(b + 64 * k) : b[64 * k];
 }
 __device__ __forceinline__ void tam_unit_st(float* base, uint64_t e, uint32_t lane, const TamF4* w) {
-  TAM_GLOBAL TamF4E* b = tam_g((TamF4E*)(base + e)) + lane;
+  TAM_GLOBAL TamF4E* b = TAM_GA(TamF4E, (base + e)) + lane;
 #pragma unroll
   for (int k = 0; k < 4; ++k) b[64 * k] = w[k];
 }
@@ -1561,9 +1563,9 @@ __device__ __forceinline__ TamVBlk tam_vunit_blk(uint32_t v_bits, uint16_t* v_sc
 // fallback).  Every v of a block that passes the block test lies in
 // [vmin, vmax] with vmin >= 2^-126, where the clamp to 1e-38 (quantize.py:275)
 // leaves it unchanged, so the fast path reads v itself; the exact path clamps.
-// W8: type of the 8-byte index stores (their alignment); with store false
+// BYTES: the 8-byte index stores are aligned to bytes only; with store false
 // (uniform over a block's lanes) nothing is written.
-template <typename W8 = TamW2>
+template <bool BYTES = false>
 __device__ __forceinline__ void tam_vunit_b(const TamTensor& d, uint32_t lane, uint32_t b, uint64_t e0,
                                             const float* v, TamVExt x, const TamLdsTabs* tabs, uint32_t seed_lo,
                                             uint32_t seed_hi, bool store = true) {
@@ -1636,7 +1638,10 @@ __device__ __forceinline__ void tam_vunit_b(const TamTensor& d, uint32_t lane, u
         }
       }
     }
-    if (store) tam_g((W8*)(d.v_idx + e0 + TAM_EPL * h))[0] = TamW2{ow[0], ow[1]};
+    if (store) {
+      if constexpr (BYTES) TAM_GA(TamW2B, d.v_idx + e0 + TAM_EPL * h)[0] = TamW2{ow[0], ow[1]};
+      else tam_g((TamW2*)(d.v_idx + e0 + TAM_EPL * h))[0] = TamW2{ow[0], ow[1]};
+    }
   }
 }
 
@@ -1664,13 +1669,13 @@ __device__ __forceinline__ void tam_k1_unit(const TamTensor& d, uint32_t u, uint
     tam_unit_ld((const float*)d.grad, eu, lane, gf);
   } else {
 #pragma unroll
-    for (int k = 0; k < NW; ++k) gw[k] = tam_g((const TamW4E*)((const char*)d.grad + off))[k];
+    for (int k = 0; k < NW; ++k) gw[k] = TAM_GA(const TamW4E, ((const char*)d.grad + off))[k];
   }
   // an fp32 parameter (16 registers) is loaded just before the update: held
   // from here it would make the kernel spill at 4 waves per SIMD
   if constexpr (DT != TAM_DTYPE_F32) {
 #pragma unroll
-    for (int k = 0; k < NW; ++k) pw[k] = tam_g((const TamW4E*)((const char*)d.param + off))[k];
+    for (int k = 0; k < NW; ++k) pw[k] = TAM_GA(const TamW4E, ((const char*)d.param + off))[k];
   }
   uint32_t label = 0u, amp = 0u, sbytes = 0u;  // sbytes: sign bytes of elements e0..e0+7 (low) and e0+8..e0+15
   float nrm = 0.0f, alpha_prev = 0.0f;
@@ -2221,7 +2226,7 @@ __device__ __forceinline__ TamK2U<F32> tam_k2u_load(const TamTensor& d, uint32_t
   if constexpr (F32) {
     tam_unit_ld<true>((const float*)d.grad, (uint64_t)u * (8u * TAM_BLOCK_SIZE), lane, r.g);
   } else {
-    const TAM_GLOBAL TamW4E* gp = tam_g((const TamW4E*)((const uint16_t*)d.grad + e0));
+    const TAM_GLOBAL TamW4E* gp = TAM_GA(const TamW4E, ((const uint16_t*)d.grad + e0));
 #pragma unroll
     for (int k = 0; k < 2; ++k) r.g[k] = gp[k];
   }
@@ -2301,7 +2306,7 @@ __device__ __forceinline__ void tam_k2_unit(const TamTensor& d, uint32_t u, uint
     const TamStage st = tam_stage(d, ws);
     norms = st.norms;
     amp = st.amp;
-    tam_g((TamH1B*)(st.signs + (e0 >> 3)))[0] = (uint16_t)(sb0 | (sb1 << 8));
+    TAM_GA(TamH1B, (st.signs + (e0 >> 3)))[0] = (uint16_t)(sb0 | (sb1 << 8));
   } else {
     tam_g((uint16_t*)(d.signs + (e0 >> 3)))[0] = (uint16_t)(sb0 | (sb1 << 8));
   }
@@ -2956,7 +2961,7 @@ __device__ __forceinline__ void tam_k4_unit(const TamTensor& d, uint32_t u, uint
   if (has_ef) tam_unit_ld<true>(d.ef_residual, eu, lane, w);
   const uint32_t label = tam_g(st.labels)[b], amp = tam_g(st.amp)[b];  // the staged new encoding
   const float nrm = tam_g(st.norms)[b];
-  const uint32_t bytes = tam_g((const TamH1B*)(st.signs + (e0 >> 3)))[0];
+  const uint32_t bytes = TAM_GA(const TamH1B, (st.signs + (e0 >> 3)))[0];
   tam_compiler_fence();
   float g[TAM_EPU], r[TAM_EPU], ge[TAM_EPU], m[TAM_EPU];
   if constexpr (DT == TAM_DTYPE_F32) {
@@ -3314,7 +3319,7 @@ __global__ __launch_bounds__(TAM_WG) __attribute__((amdgpu_waves_per_eu(4, 4))) 
       const uint64_t e0 = (uint64_t)b * TAM_BLOCK_SIZE + (lane & 7u) * TAM_EPU;
       float gv[TAM_EPU], v[TAM_EPU];
       uint32_t sc = tam_g((const uint32_t*)scales_in)[b];
-      TamW4 iw = tam_g((const TamW4B*)(idx_in + e0))[0];
+      TamW4 iw = TAM_GA(const TamW4B, (idx_in + e0))[0];
       tam_unit_load<DT>(&turn[wave], g, (uint64_t)w * (8u * TAM_BLOCK_SIZE), lane, gv);
       tam_compiler_fence();
       tam_pin(sc);
@@ -3396,7 +3401,7 @@ __device__ __forceinline__ void tam_vunit_floor(uint32_t v_bits, uint64_t e0, co
       }
     }
   }
-  if (store) tam_g((TamW4B*)(idx + e0))[0] = TamW4{ow[0], ow[1], ow[2], ow[3]};
+  if (store) TAM_GA(TamW4B, (idx + e0))[0] = TamW4{ow[0], ow[1], ow[2], ow[3]};
 }
 
 // quantize_logscale_nbits (quantize.py:126-180) of nb blocks of v: per-block fp16
@@ -3449,7 +3454,7 @@ __global__ __launch_bounds__(TAM_WG) void tam_k_quantize(const float* __restrict
     e.nan_seen = e.kmx > 0x7f800000u ? TAM_VEXT_NAN : 0u;
     if (ok) mn = __builtin_elementwise_min(mn, e.nan_seen ? 0u : e.kmn);
     if (STO) {
-      tam_vunit_b<TamW2B>(d, lane, b, e0, x, e, &tabs, seed_lo, seed_hi, ok);
+      tam_vunit_b<true>(d, lane, b, e0, x, e, &tabs, seed_lo, seed_hi, ok);
     } else {
       const TamVBlk q = tam_vunit_blk(bits, scales, lane, b, e, &tabs, ok);
       tam_vunit_floor(bits, e0, x, q, &tabs, idx, ok);
@@ -3568,7 +3573,7 @@ __global__ __launch_bounds__(TAM_WG) void tam_k_v_dequantize(const uint8_t* __re
     uint32_t w[4], high = 0u;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      w[j] = tam_g((const TamW1B*)(idx + e0 + 256u * (uint32_t)j))[0];
+      w[j] = TAM_GA(const TamW1B, (idx + e0 + 256u * (uint32_t)j))[0];
       high |= w[j];
     }
     const bool table = bits < 8u && !__any((high & ~((nbk - 1u) * 0x01010101u)) != 0u);
@@ -3581,7 +3586,7 @@ __global__ __launch_bounds__(TAM_WG) void tam_k_v_dequantize(const uint8_t* __re
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float* t = tab + (2u * (uint32_t)j + (lane >> 5)) * 64u;
-        tam_g((TamF4E*)(out + e0 + 256u * (uint32_t)j))[0] =
+        TAM_GA(TamF4E, (out + e0 + 256u * (uint32_t)j))[0] =
             TamF4{t[w[j] & 0xffu], t[(w[j] >> 8) & 0xffu], t[(w[j] >> 16) & 0xffu], t[w[j] >> 24]};
       }
       tam_wave_lds_sync();  // the next unit rewrites the table
@@ -3590,7 +3595,7 @@ __global__ __launch_bounds__(TAM_WG) void tam_k_v_dequantize(const uint8_t* __re
       for (int j = 0; j < 4; ++j) {
         float lmin, span;
         scale(8u * u + 2u * (uint32_t)j + (lane >> 5), lmin, span);
-        tam_g((TamF4E*)(out + e0 + 256u * (uint32_t)j))[0] =
+        TAM_GA(TamF4E, (out + e0 + 256u * (uint32_t)j))[0] =
             TamF4{value(lmin, span, w[j] & 0xffu), value(lmin, span, (w[j] >> 8) & 0xffu),
                   value(lmin, span, (w[j] >> 16) & 0xffu), value(lmin, span, w[j] >> 24)};
       }
