@@ -229,3 +229,50 @@ def test_steady_step_takes_any_number_and_moved_bias_tensors(lr):
         finals.append([p.detach().cpu() for p in params] + [st["compressed_v"]["indices"].cpu()])
     for a, b in zip(*finals):
         assert torch.equal(a, b)
+
+
+def _bias_run(change, steps=5):
+    """A run of `steps` steps with change(opt, params) before the fourth; the
+    optimizer, its parameters and whether each step was a steady one."""
+    from turboadam_amd import TurboAdam
+
+    dev = torch.device("cuda:0")
+    rng = np.random.default_rng(8)
+    params = [torch.nn.Parameter(torch.from_numpy((rng.standard_normal(n) * 0.02).astype(np.float32)).to(dev))
+              for n in (5000, 300)]
+    for p in params:
+        p.grad = torch.from_numpy((rng.standard_normal(p.numel()) * 1e-3).astype(np.float32)).to(dev)
+    opt = TurboAdam(params, lr=1e-3, philox_seed=3)
+    taken, fast_step = [], opt._fast_step
+    opt._fast_step = lambda: taken.append(fast_step()) or taken[-1]
+    for step in range(steps):
+        if step == 3:
+            change(opt, params)
+        opt.step()
+    return opt, params, taken
+
+
+@pytest.mark.parametrize("how", ["fp64", "replaced", "host"])
+def test_steady_step_writes_the_bias_tensors_that_are_there(how):
+    """The shared bias corrections hold the step's values after a step whatever
+    became of their tensors: cast, moved to the host, or other tensors in their
+    place."""
+    log(f"bias tensors: {how}")
+
+    def change(opt, params):
+        st = opt.state[params[0]]
+        if how == "replaced":
+            for pair in opt._group_step_tensors.values():
+                pair.update({k: torch.zeros_like(t) for k, t in pair.items()})
+            return
+        for k in ("_bc1", "_bc2"):
+            st[k].data = st[k].data.double() if how == "fp64" else st[k].data.cpu()
+
+    opt, params, _ = _bias_run(change)
+    (pair,) = opt._group_step_tensors.values()
+    for k, beta in (("bc1", 0.9), ("bc2", 0.999)):
+        want = 1.0 - beta**5
+        assert pair[k].item() == (want if how == "fp64" else np.float32(want))
+    plain = _bias_run(lambda opt, params: None)[1]
+    for a, b in zip(params, plain):
+        assert torch.equal(a, b)

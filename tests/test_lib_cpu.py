@@ -241,3 +241,22 @@ def test_kernels_claim_no_more_alignment_than_their_arrays_have():
     res = subprocess.run([HIPCC, *flags, "--cuda-device-only", "-fsyntax-only", "-Werror=align-mismatch", *SOURCES],
                          capture_output=True, text=True)
     assert res.returncode == 0, res.stderr[-2000:]
+
+
+def test_bias_addresses_takes_only_what_the_kernel_can_store_to():
+    """The steady step stores the bias corrections through raw addresses: a tensor
+    on the host, one of another dtype or a missing one sends the step to the full
+    path (no address is handed out)."""
+    from turboadam_amd.optimizer import _host
+
+    key = (0, "cuda", 0)
+    out = (ctypes.c_void_p * 2)()
+
+    def taken(m):
+        return _host().bias_addresses(m, [key], 0, ctypes.addressof(out))
+
+    host = {"bc1": torch.zeros(1), "bc2": torch.zeros(1)}
+    for m in ({}, {key: {}}, {key: {"bc1": host["bc1"]}}, {key: {"bc1": 1.0, "bc2": 2.0}}, {key: host},
+              {key: {"bc1": torch.zeros(1, device="meta"), "bc2": torch.zeros(1, device="meta")}}):
+        assert not taken(m)
+    assert not any(out)

@@ -36,7 +36,7 @@ PyObject* item(PyObject* d, PyObject* key) {
 
 struct Keys {
   PyObject *grad, *compressed_v, *indices, *scales, *exp_avg_sq, *exp_avg, *compress_m, *m_mgr, *encoded,
-      *sign_packed, *labels, *block_norms, *alpha, *ef_residual, *step, *lr, *betas, *eps, *weight_decay;
+      *sign_packed, *labels, *block_norms, *alpha, *ef_residual, *step, *lr, *betas, *eps, *weight_decay, *bc1, *bc2;
   Keys() {
     grad = PyUnicode_InternFromString("grad");
     compressed_v = PyUnicode_InternFromString("compressed_v");
@@ -57,6 +57,8 @@ struct Keys {
     betas = PyUnicode_InternFromString("betas");
     eps = PyUnicode_InternFromString("eps");
     weight_decay = PyUnicode_InternFromString("weight_decay");
+    bc1 = PyUnicode_InternFromString("bc1");
+    bc2 = PyUnicode_InternFromString("bc2");
   }
 };
 
@@ -373,6 +375,35 @@ bool steady_groups(py::handle f, uint64_t table_addr, int64_t rows, uint64_t gse
   return true;
 }
 
+// The addresses of the shared bias-correction tensors (map[key]["bc1"] and "bc2"
+// for each key), written to out_addr in order, for kernels that store one float
+// to each.  False, with nothing written, unless every one of them is a
+// one-element fp32 tensor on the HIP device dev_index (the full path's fill_
+// takes any tensor).
+bool bias_addresses(py::handle map, py::handle keys_, int64_t dev_index, uint64_t out_addr) {
+  const Keys& K = keys();
+  PyObject *M = map.ptr(), *L = keys_.ptr();
+  if (!PyDict_Check(M) || !PyList_Check(L)) return false;
+  std::vector<void*> at;
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(L); ++i) {
+    PyObject* pair = PyDict_GetItemWithError(M, PyList_GET_ITEM(L, i));
+    for (PyObject* name : {K.bc1, K.bc2}) {
+      PyObject* o = pair ? item(pair, name) : nullptr;
+      if (!o || !THPVariable_Check(o)) {
+        PyErr_Clear();
+        return false;
+      }
+      const at::Tensor& t = THPVariable_Unpack(o);
+      if (!t.is_cuda() || t.get_device() != dev_index || t.layout() != at::kStrided ||
+          t.scalar_type() != at::kFloat || t.numel() != 1)
+        return false;
+      at.push_back(t.data_ptr());
+    }
+  }
+  for (size_t i = 0; i < at.size(); ++i) ((void**)(uintptr_t)out_addr)[i] = at[i];
+  return true;
+}
+
 // state["step"] += 1 for each state dict (once the step has been launched).
 void advance_steps(py::list states) {
   const Keys& K = keys();
@@ -398,5 +429,7 @@ PYBIND11_MODULE(_tam_host, m) {
   m.def("values_kept", &values_kept, py::arg("map"), py::arg("kept"));
   m.def("steady_groups", &steady_groups, py::arg("f"), py::arg("table_addr"), py::arg("rows"), py::arg("gsel_addr"),
         py::arg("flags_addr"), py::arg("bc_addr"));
+  m.def("bias_addresses", &bias_addresses, py::arg("map"), py::arg("keys"), py::arg("dev_index"),
+        py::arg("out_addr"));
   m.def("states_kept", &states_kept, py::arg("f"));
 }

@@ -251,7 +251,7 @@ class _FastStep:
         self.row_params = [params[i] for i in rows]
         self.ptrs = [p.data_ptr() for p in self.row_params]  # parameter storage the descriptor rows point at
 
-    def bind(self, group_step_tensors) -> None:
+    def bind(self) -> None:
         """What the C++ and library calls of a steady step take: the table as a
         ctypes array, addresses, and the groups' bias-correction sources."""
         plan = self.plan
@@ -264,9 +264,10 @@ class _FastStep:
         self.bc = [(group, src) for _, group, src in self.bc_src]
         self.groups = [(g, index.get((gi, self.device.type, self.device.index), -1)) for g, gi in plan.groups]
         self.bc_values = (ctypes.c_float * max(1, 2 * len(self.bc)))()
-        # the shared bias-correction tensors; their addresses are read at each step
-        self.bc_tensors = [group_step_tensors[key][k] for key, _, _ in self.bc_src for k in ("bc1", "bc2")]
-        self.bc_ptrs = (ctypes.c_void_p * max(1, len(self.bc_tensors)))()
+        # where the shared bias-correction tensors are (TurboAdam._group_step_tensors);
+        # the tensors are checked and their addresses read at each step
+        self.bc_keys = [key for key, _, _ in self.bc_src]
+        self.bc_ptrs = (ctypes.c_void_p * max(1, 2 * len(self.bc)))()
 
 
 class TurboAdam(Optimizer):
@@ -897,12 +898,10 @@ class TurboAdam(Optimizer):
                     src = st
             if src is not None:
                 bc_src.append(((group_idx, device.type, device.index), group, src))
-        if any(key not in self._group_step_tensors for key, _, _ in bc_src):
-            return
         self._fast = _FastStep(self._layout_version, device, params, [p.grad is None for p in params], rows,
                                [it[1] for it in items], [it[0].grad for it in items], [it[0].dtype for it in items],
                                bc_src, plan, self.state)
-        self._fast.bind(self._group_step_tensors)
+        self._fast.bind()
 
     def _fast_state_kept(self, f) -> bool:
         """Whether opt.state still holds f's per-parameter dicts, in order, and
@@ -922,8 +921,11 @@ class TurboAdam(Optimizer):
             return False
         # in C++.  Per row: the same parameters with gradients, their dtypes and
         # storage, each new gradient's checks, the state tensors; then the rows'
-        # gradient pointers and step numbers are written.  Per group: the scalars.
+        # gradient pointers and step numbers are written.  Per group: the shared
+        # bias-correction tensors' checks and addresses, the scalars.
         table, n, gsel, flags = f.addrs
+        if not host.bias_addresses(self._group_step_tensors, f.bc_keys, f.dev_index, ctypes.addressof(f.bc_ptrs)):
+            return False
         if not host.steady_rows(f, table, f.plan.table.itemsize, _GRAD_OFF, _STEP_OFF):
             return False
         if not host.steady_groups(f, table, n, gsel, flags, ctypes.addressof(f.bc_values)):
@@ -971,9 +973,7 @@ class TurboAdam(Optimizer):
         bufs.order_on(stream)
         desc, ws = bufs.desc_buffer(f.nbytes), bufs.workspace(f.info.ws_bytes)
         put = len(f.arr) if len(f.arr) <= self._PUT_MAX else 0
-        for i, t in enumerate(f.bc_tensors):
-            f.bc_ptrs[i] = t.data_ptr()
-        _lib.check(lib.tam_put(f.addrs[0], put, desc.data_ptr(), f.bc_ptrs, f.bc_values, len(f.bc_tensors), raw),
+        _lib.check(lib.tam_put(f.addrs[0], put, desc.data_ptr(), f.bc_ptrs, f.bc_values, 2 * len(f.bc), raw),
                    "tam_put")
         if not put:
             upload = self._uploads.get(f.device)
