@@ -260,3 +260,53 @@ def test_bias_addresses_takes_only_what_the_kernel_can_store_to():
               {key: {"bc1": torch.zeros(1, device="meta"), "bc2": torch.zeros(1, device="meta")}}):
         assert not taken(m)
     assert not any(out)
+
+
+@pytest.mark.parametrize("what", ["exp_avg", "exp_avg_sq", "indices", "scales", "sign_packed", "labels",
+                                  "block_norms", "block scales", "alpha", "residual"])
+@pytest.mark.parametrize("how", ["device", "dtype", "size", "stride"])
+def test_descriptor_rows_refuse_a_state_array_the_kernels_cannot_use(what, how):
+    """A state array on another device, of another dtype, too short or strided
+    raises where the descriptor table is built: the kernels get its address alone.
+    (The table is built on the CPU; nothing is launched.)"""
+    from turboadam_amd.optimizer import TurboAdam
+    from turboadam_amd.oneq import num_blocks
+
+    if (what, how) == ("alpha", "stride"):
+        pytest.skip("one element is contiguous")
+    big, n = what not in ("exp_avg", "exp_avg_sq"), 5000
+    p = torch.nn.Parameter(torch.zeros(n))
+    p.grad = torch.zeros(n)
+    opt = TurboAdam([p], compress_m=big, compress_v=what != "exp_avg_sq", error_feedback=True)
+    st, cpu, nb = opt.state[p], torch.device("cpu"), num_blocks(n)
+    st.update(step=3, _compress_m=big)
+    if what == "exp_avg_sq":
+        st["exp_avg_sq"] = torch.zeros(n)
+    else:
+        st["compressed_v"] = {"indices": torch.zeros(nb * 128, dtype=torch.uint8),
+                              "scales": torch.zeros(nb, 2, dtype=torch.float16), "n_bits": 4}
+    if big:
+        from turboadam_amd.costate import CoStateManager
+
+        mgr = st["m_mgr"] = CoStateManager(error_feedback=True)
+        mgr.allocate(n, cpu)
+        mgr._has_state, mgr._ef_residual = True, torch.zeros(n)
+    else:
+        st["exp_avg"] = torch.zeros(n)
+    holder, key = {"indices": lambda: (st["compressed_v"], "indices"), "scales": lambda: (st["compressed_v"], "scales"),
+                   "alpha": lambda: (mgr.__dict__, "_alpha"), "residual": lambda: (mgr.__dict__, "_ef_residual"),
+                   "block scales": lambda: (mgr._encoded, "scales"), "exp_avg": lambda: (st, "exp_avg"),
+                   "exp_avg_sq": lambda: (st, "exp_avg_sq")}.get(what, lambda: (mgr._encoded, what))()
+    item = (p, st, opt.param_groups[0], 0, 0)
+    assert len(opt._describe(cpu, [item]).table) == 1  # as it should be
+    t = holder[key]
+    if how == "device":
+        holder[key] = t.to("meta")
+    elif how == "dtype":
+        holder[key] = t.to(torch.float64)
+    elif how == "size":
+        holder[key] = t.reshape(-1)[:-1].clone()
+    else:
+        holder[key] = torch.stack([t, t], -1)[..., 0]
+    with pytest.raises(RuntimeError, match="turboadam_amd"):
+        opt._describe(cpu, [item])

@@ -105,6 +105,17 @@ def _tensor_ptrs(rows) -> list:
     return [0 if t is None else t.data_ptr() for row in rows for t in row]
 
 
+def _state_ptr(t, what: str, dtype, numel: int, device) -> int:
+    """Device address of a state array that the kernels read or write as numel
+    contiguous elements of dtype on device; raises where t is anything else."""
+    if not isinstance(t, torch.Tensor) or t.dtype != dtype or t.device != device or t.numel() < numel \
+            or not t.is_contiguous():
+        got = f"{t.dtype} {tuple(t.shape)} on {t.device}" if isinstance(t, torch.Tensor) else type(t).__name__
+        raise RuntimeError(f"turboadam_amd: the state's {what} must be {numel} contiguous {dtype} elements on "
+                           f"{device}, got {got}")
+    return t.data_ptr()
+
+
 class _DeviceBuffers:
     """Per-device descriptor and workspace buffers, grown on demand, and the
     persistent pinned upload buffer of capturable steps."""
@@ -621,20 +632,21 @@ class TurboAdam(Optimizer):
                 if idx.numel() != nb * BLOCK_SIZE or scl.numel() != nb * 2:
                     raise RuntimeError("turboadam_amd: compressed_v does not match the parameter size")
                 flags |= _lib.TAM_FLAG_COMPRESS_V
-                v_idx, v_scales, v_bits = idx.data_ptr(), scl.data_ptr(), cv["n_bits"]
+                v_idx = _state_ptr(idx, "indices", torch.uint8, nb * BLOCK_SIZE, p.device)
+                v_scales, v_bits = _state_ptr(scl, "scales", torch.float16, nb * 2, p.device), cv["n_bits"]
             else:
-                exp_avg_sq = state["exp_avg_sq"].data_ptr()
+                exp_avg_sq = _state_ptr(state["exp_avg_sq"], "exp_avg_sq", torch.float32, n, p.device)
             if state["_compress_m"]:
                 mgr = state["m_mgr"]
                 enc = mgr._encoded
                 flags |= _lib.TAM_FLAG_COSTATE
                 if mgr._has_state:
                     flags |= _lib.TAM_FLAG_HAS_STATE
-                signs = enc["sign_packed"].data_ptr()
-                labels = enc["labels"].data_ptr()
-                norms = enc["block_norms"].data_ptr()
-                amp = enc["scales"].data_ptr()
-                alpha = mgr._alpha.data_ptr()
+                signs = _state_ptr(enc["sign_packed"], "sign_packed", torch.uint8, (n + 7) // 8, p.device)
+                labels = _state_ptr(enc["labels"], "labels", torch.uint8, nb, p.device)
+                norms = _state_ptr(enc["block_norms"], "block_norms", torch.float32, nb, p.device)
+                amp = _state_ptr(enc["scales"], "block scales", torch.float16, nb, p.device)
+                alpha = _state_ptr(mgr._alpha, "alpha", torch.float32, 1, p.device)
                 k_lo, k_hi = mgr.ranks(nb)
                 if mgr._error_feedback:
                     # costate.py:409-437: the residual exists from the tensor's first
@@ -645,9 +657,9 @@ class TurboAdam(Optimizer):
                         self._layout_version += 1
                     else:
                         flags |= _lib.TAM_FLAG_HAS_EF
-                    ef = mgr._ef_residual.data_ptr()
+                    ef = _state_ptr(mgr._ef_residual, "error-feedback residual", torch.float32, n, p.device)
             else:
-                exp_avg = state["exp_avg"].data_ptr()
+                exp_avg = _state_ptr(state["exp_avg"], "exp_avg", torch.float32, n, p.device)
             if capturable:
                 device_step.append((len(rows), p, state, group))
                 step = 0  # filled on the device
