@@ -276,3 +276,47 @@ def test_steady_step_writes_the_bias_tensors_that_are_there(how):
     plain = _bias_run(lambda opt, params: None)[1]
     for a, b in zip(params, plain):
         assert torch.equal(a, b)
+
+
+def test_state_tensors_whose_data_was_replaced_are_followed():
+    """t.data = a copy, for every kind of state array and the error-feedback
+    residual, between steps: the step works on the new storage.  (The old ones
+    stay alive, so a stale descriptor row would update them and show.)"""
+    from turboadam_amd import TurboAdam
+
+    dev = torch.device("cuda:0")
+    sizes, dts = [5000, 300, 4096 + 77], [F32, F32, BF16]
+    for kw in (dict(), dict(error_feedback=True), dict(compress_v=False), dict(compress_m=False)):
+        log(f"state .data replaced, {kw}")
+        rng = np.random.default_rng(54)
+        init = [to_bits((rng.standard_normal(n) * 0.02).astype(np.float32), dt) for n, dt in zip(sizes, dts)]
+        params = [torch.nn.Parameter(to_torch(a, dt, (n,), dev)) for a, dt, n in zip(init, dts, sizes)]
+        opt = TurboAdam(params, philox_seed=23, **kw)
+        oparams = [a.copy() for a in init]
+        orc = O.OracleTurboAdam(oparams, dtypes=dts, seed=23, **kw)
+        taken, fast_step, old = [], opt._fast_step, []
+        opt._fast_step = lambda: taken.append(fast_step()) or taken[-1]
+
+        def move(t):
+            if isinstance(t, torch.Tensor):
+                old.append(t.data)
+                t.data = t.data.clone()
+
+        for step in range(6):
+            if step == 3:
+                for st in opt.state.values():
+                    for t in (st.get("exp_avg"), st.get("exp_avg_sq"), *st.get("compressed_v", {}).values()):
+                        move(t)
+                    mgr = st.get("m_mgr")
+                    if mgr is not None:
+                        for t in (*mgr._encoded.values(), mgr._alpha, mgr._ef_residual):
+                            move(t)
+            gs = [to_bits((rng.standard_normal(n) * 1e-3).astype(np.float32), dt) for n, dt in zip(sizes, dts)]
+            for p, g, dt, n in zip(params, gs, dts, sizes):
+                p.grad = to_torch(g, dt, (n,), dev)
+            opt.step()
+            orc.step(gs)
+            torch.cuda.synchronize()
+            bad = compare_with_oracle(opt, params, orc, oparams, f"step {step + 1}")
+            assert not bad, "\n".join(bad[:20])
+        assert taken == [False, True, True, False, True, True]

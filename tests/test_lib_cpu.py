@@ -310,3 +310,37 @@ def test_descriptor_rows_refuse_a_state_array_the_kernels_cannot_use(what, how):
         holder[key] = torch.stack([t, t], -1)[..., 0]
     with pytest.raises(RuntimeError, match="turboadam_amd"):
         opt._describe(cpu, [item])
+
+
+@pytest.mark.parametrize("what", ["exp_avg", "indices", "labels", "alpha"])
+def test_steady_step_sees_a_state_tensor_whose_data_was_replaced(what):
+    """t.data = t.data.to(...) (offload loops) leaves the object and moves its
+    storage: the kept descriptor row's address is stale then."""
+    from turboadam_amd.costate import CoStateManager
+    from turboadam_amd.optimizer import TurboAdam, _FastStep
+
+    params = [torch.nn.Parameter(torch.zeros(n)) for n in (5000, 300)]
+    opt = TurboAdam(params)
+    for p in params:
+        nb = (p.numel() + 127) // 128
+        st = opt.state[p]
+        st.update(step=3, _compress_m=p.numel() >= 4096,
+                  compressed_v={"indices": torch.zeros(128 * nb, dtype=torch.uint8),
+                                "scales": torch.zeros(2 * nb, dtype=torch.float16)})
+    mgr = opt.state[params[0]]["m_mgr"] = CoStateManager()
+    mgr.allocate(5000, torch.device("cpu"))
+    opt.state[params[1]]["exp_avg"] = torch.zeros(300)
+
+    class Plan:
+        row_cv = [True, True]
+
+    f = _FastStep(0, torch.device("cuda", 0), params, [True, True], [0, 1], [opt.state[p] for p in params],
+                  [None, None], [torch.float32] * 2, [], Plan, opt.state)
+    assert opt._fast_state_kept(f)
+    t = {"exp_avg": opt.state[params[1]]["exp_avg"], "indices": opt.state[params[0]]["compressed_v"]["indices"],
+         "labels": mgr._encoded["labels"], "alpha": mgr._alpha}[what]
+    old = t.data  # stays alive: the new storage is another
+    t.data = old.clone()
+    assert not opt._fast_state_kept(f)
+    t.data = old
+    assert opt._fast_state_kept(f)

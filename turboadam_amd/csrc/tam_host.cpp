@@ -68,8 +68,11 @@ const Keys& keys() {
 }
 
 // Whether the state tensors of one row are, in order, the kept objects at
-// kept[*pos ...] (the order of optimizer._row_tensors); advances *pos.
-bool row_tensors_kept(PyObject* st, bool compress_v, PyObject* kept, Py_ssize_t n_kept, Py_ssize_t* pos) {
+// kept[*pos ...] (the order of optimizer._row_tensors), each still at its kept
+// address in kept_ptrs (a tensor whose .data was replaced is the same object
+// elsewhere); advances *pos.
+bool row_tensors_kept(PyObject* st, bool compress_v, PyObject* kept, PyObject* kept_ptrs, Py_ssize_t n_kept,
+                      Py_ssize_t* pos) {
   const Keys& K = keys();
   PyObject* got[8];
   int n = 0;
@@ -101,29 +104,36 @@ bool row_tensors_kept(PyObject* st, bool compress_v, PyObject* kept, Py_ssize_t 
     got[n++] = item(enc, K.labels);
     got[n++] = item(enc, K.block_norms);
     got[n++] = item(enc, K.scales);
-    got[n++] = a;  // identity only
+    got[n++] = a;
     got[n++] = r;
   } else {
     got[n++] = item(st, K.exp_avg);
   }
   for (int i = 0; i < n; ++i) {
     if (!got[i] || *pos >= n_kept) return false;
-    // None in the kept list stands for a missing error-feedback residual
+    // None in the kept list (address 0) stands for a missing error-feedback residual
     if (PyList_GET_ITEM(kept, *pos) != got[i]) return false;
+    if (got[i] != Py_None) {
+      if (!THPVariable_Check(got[i])) return false;
+      const unsigned long long at = PyLong_AsUnsignedLongLong(PyList_GET_ITEM(kept_ptrs, *pos));
+      if ((uint64_t)(uintptr_t)THPVariable_Unpack(got[i]).const_data_ptr() != at) return false;
+    }
     ++*pos;
   }
   return true;
 }
 
-// Whether every row's state tensors are the kept objects (lists: the rows'
-// state dicts, their compress_v flags, the kept tensors flattened).
-bool all_rows_kept(PyObject* S, PyObject* CV, PyObject* T) {
-  if (!PyList_Check(S) || !PyList_Check(CV) || !PyList_Check(T) || PyList_GET_SIZE(S) != PyList_GET_SIZE(CV))
+// Whether every row's state tensors are the kept objects at their kept addresses
+// (lists: the rows' state dicts, their compress_v flags, the kept tensors
+// flattened, their addresses).
+bool all_rows_kept(PyObject* S, PyObject* CV, PyObject* T, PyObject* TP) {
+  if (!PyList_Check(S) || !PyList_Check(CV) || !PyList_Check(T) || !PyList_Check(TP) ||
+      PyList_GET_SIZE(S) != PyList_GET_SIZE(CV) || PyList_GET_SIZE(T) != PyList_GET_SIZE(TP))
     return false;
   Py_ssize_t pos = 0;
   const Py_ssize_t n_kept = PyList_GET_SIZE(T);
   for (Py_ssize_t j = 0; j < PyList_GET_SIZE(S); ++j) {
-    if (!row_tensors_kept(PyList_GET_ITEM(S, j), PyList_GET_ITEM(CV, j) == Py_True, T, n_kept, &pos)) {
+    if (!row_tensors_kept(PyList_GET_ITEM(S, j), PyList_GET_ITEM(CV, j) == Py_True, T, TP, n_kept, &pos)) {
       PyErr_Clear();
       return false;
     }
@@ -134,10 +144,11 @@ bool all_rows_kept(PyObject* S, PyObject* CV, PyObject* T) {
 }  // namespace
 
 // Whether the rows' state tensors of the kept _FastStep f are still the
-// objects its descriptor rows were built from.
+// objects its descriptor rows were built from, at the same addresses.
 bool states_kept(py::handle f) {
-  py::object states = f.attr("states"), tensors = f.attr("tensors"), row_cv = f.attr("plan").attr("row_cv");
-  return all_rows_kept(states.ptr(), row_cv.ptr(), tensors.ptr());
+  py::object states = f.attr("states"), tensors = f.attr("tensors"), tensor_ptrs = f.attr("tensor_ptrs"),
+             row_cv = f.attr("plan").attr("row_cv");
+  return all_rows_kept(states.ptr(), row_cv.ptr(), tensors.ptr(), tensor_ptrs.ptr());
 }
 
 // The per-row part of a steady step (optimizer.TurboAdam._fast_step), given
@@ -153,7 +164,7 @@ bool steady_rows(py::handle f, uint64_t table_addr, int64_t stride, int64_t grad
   py::object params = f.attr("params"), absent = f.attr("absent"), rows = f.attr("rows"),
              row_params = f.attr("row_params"), ptrs = f.attr("ptrs"), kept_grads = f.attr("grads"),
              pdtypes = f.attr("pcodes"), states = f.attr("states"), tensors = f.attr("tensors"),
-             row_cv = f.attr("plan").attr("row_cv");
+             tensor_ptrs = f.attr("tensor_ptrs"), row_cv = f.attr("plan").attr("row_cv");
   const int64_t dev_index = f.attr("dev_index").cast<int64_t>();
   PyObject* P = params.ptr();
   PyObject* A = absent.ptr();
@@ -173,7 +184,7 @@ bool steady_rows(py::handle f, uint64_t table_addr, int64_t stride, int64_t grad
       PyList_GET_SIZE(KG) != nr || PyList_GET_SIZE(PD) != nr || PyList_GET_SIZE(S) != nr ||
       PyList_GET_SIZE(CV) != nr)
     return false;
-  if (!all_rows_kept(S, CV, T)) return false;
+  if (!all_rows_kept(S, CV, T, tensor_ptrs.ptr())) return false;
   std::vector<PyObject*> gs((size_t)np_, nullptr);  // new references
   auto release = [&]() {
     for (PyObject* g : gs) Py_XDECREF(g);

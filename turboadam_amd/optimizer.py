@@ -238,8 +238,8 @@ class _FastStep:
     A step is not steady either when opt.state no longer holds the kept
     per-parameter dicts in the same order (cleared, an entry replaced or
     removed) or when a row's state tensors (_row_tensors) are not the kept
-    objects; the full path then rebuilds what changed.  A state tensor is
-    recognised by identity here; the full path compares device addresses."""
+    objects at the kept addresses (t.data replaced, as offloading does); the
+    full path then rebuilds what changed."""
 
     def __init__(self, version, device, params, absent, rows, states, grads, pdtypes, bc_src, plan, state_map):
         self.version = version
@@ -247,8 +247,9 @@ class _FastStep:
         # opt.state.clear(), opt.state[p] = {} or a new mapping is not steady
         self.state_map = state_map
         self.state_values = list(state_map.values())
-        # the state tensors of each row (_row_tensors), by identity
+        # the state tensors of each row (_row_tensors) and the addresses the row points at
         self.tensors = [t for st, cv in zip(states, plan.row_cv) for t in _row_tensors(st, cv)]
+        self.tensor_ptrs = _tensor_ptrs([self.tensors])
         self.device = device
         self.dev_index = device.index if device.index is not None else torch.cuda.current_device()
         self.params = params      # every parameter of the optimizer, in order
@@ -917,7 +918,7 @@ class TurboAdam(Optimizer):
 
     def _fast_state_kept(self, f) -> bool:
         """Whether opt.state still holds f's per-parameter dicts, in order, and
-        each descriptor row's state tensors are the objects f kept."""
+        each descriptor row's state tensors are the objects f kept, where they were."""
         return self.state is f.state_map and _host().values_kept(self.state, f.state_values) \
             and _host().states_kept(f)
 
