@@ -344,3 +344,36 @@ def test_steady_step_sees_a_state_tensor_whose_data_was_replaced(what):
     assert not opt._fast_state_kept(f)
     t.data = old
     assert opt._fast_state_kept(f)
+
+
+def _steady_on_cpu(n=300):
+    """A one-parameter _FastStep with fp32 m and v over a real descriptor table, on
+    the CPU: (optimizer, parameter, the call of its per-row checks)."""
+    from turboadam_amd import optimizer as M
+
+    p = torch.nn.Parameter(torch.zeros(n))
+    p.grad = torch.zeros(n)
+    opt = M.TurboAdam([p], compress_v=False)
+    st = opt.state[p]
+    st.update(step=3, _compress_m=False, exp_avg=torch.zeros(n), exp_avg_sq=torch.zeros(n))
+    plan = opt._describe(torch.device("cpu"), [(p, st, opt.param_groups[0], 0, 0)])
+    f = M._FastStep(0, torch.device("cuda", 0), [p], [False], [0], [st], [p.grad], [torch.float32], [], plan,
+                    opt.state)
+    table = plan.table
+    return opt, p, f, lambda: M._host().steady_rows(f, table.ctypes.data, table.itemsize, M._GRAD_OFF, M._STEP_OFF)
+
+
+def test_steady_step_checks_a_gradient_it_has_seen_before():
+    """grad.data = ... changes the storage, dtype or device of the object the last
+    step checked: the checks run on it again.  (Here the kept gradient object lies
+    on the host, where no kernel can read it.)"""
+    _, p, f, steady = _steady_on_cpu()
+    assert f.grads[0] is p.grad and not p.grad.is_cuda
+    assert not steady()
+
+
+def test_gradient_of_another_size_is_refused():
+    opt, p, _, _ = _steady_on_cpu()
+    p.grad.data = torch.zeros(7)
+    with pytest.raises(RuntimeError, match="gradient"):
+        opt._describe(torch.device("cpu"), [(p, opt.state[p], opt.param_groups[0], 0, 0)])

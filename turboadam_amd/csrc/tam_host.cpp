@@ -233,12 +233,11 @@ bool steady_rows(py::handle f, uint64_t table_addr, int64_t stride, int64_t grad
       return false;
     }
     const at::Tensor& gt = THPVariable_Unpack(g);
-    if (g != PyList_GET_ITEM(KG, j)) {  // a new gradient object: the checks of _grad_ptr
-      if (gt.scalar_type() != pt.scalar_type() || gt.layout() != at::kStrided || !gt.is_contiguous() ||
-          !gt.is_cuda() || gt.get_device() != dev_index) {
-        release();
-        return false;
-      }
+    // the checks of _grad_ptr, also for an object seen before (its data may have been replaced)
+    if (gt.scalar_type() != pt.scalar_type() || gt.layout() != at::kStrided || !gt.is_contiguous() ||
+        !gt.is_cuda() || gt.get_device() != dev_index || gt.numel() != pt.numel()) {
+      release();
+      return false;
     }
     gptr[(size_t)j] = (uint64_t)(uintptr_t)gt.data_ptr();
   }
@@ -257,7 +256,7 @@ bool steady_rows(py::handle f, uint64_t table_addr, int64_t stride, int64_t grad
     const uint32_t s1 = (uint32_t)(s + 1);
     std::memcpy(row + step_off, &s1, 4);
   }
-  // f.grads holds this step's gradient objects (checked from now on by identity)
+  // f.grads holds this step's gradient objects until the next step
   for (Py_ssize_t j = 0; j < nr; ++j) {
     PyObject* g = gs[(size_t)PyLong_AsSsize_t(PyList_GET_ITEM(R, j))];
     Py_INCREF(g);

@@ -230,10 +230,10 @@ class _FastStep:
     (TurboAdam._layout_version), every CoState tensor past its first update
     and every error-feedback residual written.  Such a step skips the
     per-parameter walk of _collect: the gradients are gathered by list
-    comprehensions, checked only when a gradient object is new (dtype, layout,
-    contiguity, device), the parameters' storage pointers are compared with the
-    kept descriptor rows (p.data replaced: not steady), and the step numbers
-    and bias corrections come from the kept state dicts.
+    comprehensions and checked (dtype, layout, contiguity, device, size), the
+    parameters' storage pointers are compared with the kept descriptor rows
+    (p.data replaced: not steady), and the step numbers and bias corrections
+    come from the kept state dicts.
 
     A step is not steady either when opt.state no longer holds the kept
     per-parameter dicts in the same order (cleared, an entry replaced or
@@ -256,7 +256,7 @@ class _FastStep:
         self.absent = absent      # [p.grad is None] of the step this was built from
         self.rows = rows          # positions (in params) of the descriptor rows
         self.states = states      # their state dicts
-        self.grads = grads        # the gradient objects last checked, per row
+        self.grads = grads        # the last step's gradient objects, per row (kept alive until the next)
         self.pcodes = [_DTYPES[dt] for dt in pdtypes]  # their TAM_DTYPE_* codes
         self.bc_src = bc_src      # (bc key, group betas, state dict whose step sets the group's bias corrections)
         self.plan = plan
@@ -587,6 +587,8 @@ class TurboAdam(Optimizer):
             raise RuntimeError("turboadam_amd.TurboAdam does not support sparse gradients")
         if g.dtype != p.dtype or g.device != p.device:
             raise RuntimeError("turboadam_amd: gradient dtype/device must match the parameter")
+        if g.numel() != p.numel():
+            raise RuntimeError(f"turboadam_amd: a gradient of {g.numel()} elements for a parameter of {p.numel()}")
         if not g.is_contiguous():
             g = g.contiguous()
             state["_grad_keepalive"] = g
