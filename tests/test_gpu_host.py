@@ -320,3 +320,28 @@ def test_state_tensors_whose_data_was_replaced_are_followed():
             bad = compare_with_oracle(opt, params, orc, oparams, f"step {step + 1}")
             assert not bad, "\n".join(bad[:20])
         assert taken == [False, True, True, False, True, True]
+
+
+@pytest.mark.parametrize("steady", [True, False], ids=["steady", "full"])
+@pytest.mark.parametrize("how", ["transposed", "shorter"])
+def test_parameter_of_another_shape_at_the_same_address_is_refused(how, steady):
+    """p.data = a view of itself keeps the address and changes what lies there: the
+    kept descriptor row no longer describes the parameter."""
+    from turboadam_amd import TurboAdam
+
+    log(f"parameter {how}, {'steady' if steady else 'full'} path")
+    dev = torch.device("cuda:0")
+    p = torch.nn.Parameter(torch.randn(96, 96, device=dev))
+    opt = TurboAdam([p])
+    if not steady:
+        opt._fast_step = lambda: False
+    for _ in range(3):
+        p.grad = torch.randn(96, 96, device=dev)
+        opt.step()
+    p.grad = None
+    p.data = p.data.t() if how == "transposed" else p.data[:50]
+    p.grad = torch.randn(p.shape, device=dev)
+    before = p.detach().clone()
+    with pytest.raises(RuntimeError, match="contiguous" if how == "transposed" else "size"):
+        opt.step()
+    assert torch.equal(p.detach(), before)

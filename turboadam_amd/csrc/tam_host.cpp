@@ -218,10 +218,11 @@ bool steady_rows(py::handle f, uint64_t table_addr, int64_t stride, int64_t grad
       return false;
     }
     const at::Tensor& pt = THPVariable_Unpack(p);
-    // the row was built for this dtype (TAM_DTYPE_F32 / BF16 / F16) and storage
+    // the row was built for this dtype (TAM_DTYPE_F32 / BF16 / F16), size and storage
     const long code = PyLong_AsLong(PyList_GET_ITEM(PD, j));
     const at::ScalarType want = code == 0 ? at::kFloat : code == 1 ? at::kBFloat16 : at::kHalf;
-    if (pt.scalar_type() != want ||
+    if (pt.scalar_type() != want || !pt.is_contiguous() ||
+        (uint64_t)pt.numel() != ((const TamTensor*)(uintptr_t)(table_addr + (uint64_t)j * (uint64_t)stride))->n ||
         (uint64_t)(uintptr_t)pt.data_ptr() != PyLong_AsUnsignedLongLong(PyList_GET_ITEM(PT, j))) {
       PyErr_Clear();
       release();

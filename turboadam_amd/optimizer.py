@@ -185,6 +185,7 @@ class _StepPlan:
         self.key = key
         self.state_ptrs = None  # _tensor_ptrs of the rows' state tensors when the table was built
         self.row_cv = None      # compress_v of each row's group when the table was built
+        self.elements = None    # (numel, dtype) of each row's parameter when the table was built
         self.table = table
         self.gsel = gsel              # group row of each descriptor row
         self.groups = groups          # (group, group_idx) of each group row
@@ -232,8 +233,8 @@ class _FastStep:
     per-parameter walk of _collect: the gradients are gathered by list
     comprehensions and checked (dtype, layout, contiguity, device, size), the
     parameters' storage pointers are compared with the kept descriptor rows
-    (p.data replaced: not steady), and the step numbers and bias corrections
-    come from the kept state dicts.
+    (p.data replaced, or cut or transposed in place: not steady), and the step
+    numbers and bias corrections come from the kept state dicts.
 
     A step is not steady either when opt.state no longer holds the kept
     per-parameter dicts in the same order (cleared, an entry replaced or
@@ -580,9 +581,11 @@ class TurboAdam(Optimizer):
                 bc2_f, inv_bc2, _f32(inv_bc2), _f32(group["eps"]), _f32(-lr), _SQRT_BLOCK_F32)
 
     def _grad_ptr(self, p, state) -> int:
-        """Device address of p's gradient (checked; a contiguous copy of a
-        strided one is kept alive for the step)."""
+        """Device address of p's gradient (checked, as is that p is contiguous; a
+        contiguous copy of a strided gradient is kept alive for the step)."""
         g = p.grad
+        if not p.is_contiguous():
+            raise RuntimeError("turboadam_amd: parameters must be contiguous")
         if g.is_sparse:
             raise RuntimeError("turboadam_amd.TurboAdam does not support sparse gradients")
         if g.dtype != p.dtype or g.device != p.device:
@@ -619,8 +622,6 @@ class TurboAdam(Optimizer):
             code = _DTYPES.get(p.dtype)
             if code is None:
                 raise NotImplementedError(f"turboadam_amd: unsupported parameter dtype {p.dtype}")
-            if not p.is_contiguous():
-                raise RuntimeError("turboadam_amd: parameters must be contiguous")
             gptr = self._grad_ptr(p, state)
             n = p.numel()
             nb = num_blocks(n)
@@ -685,6 +686,7 @@ class TurboAdam(Optimizer):
         plan.static_flags = table["flags"] & np.uint32(
             ~(_lib.TAM_FLAG_HAS_STATE | _lib.TAM_FLAG_HAS_EF | _lib.TAM_FLAG_WD) & 0xFFFFFFFF)
         plan.row_cv = [bool(group["compress_v"]) for _, _, group, _, _ in items]
+        plan.elements = [(it[0].numel(), it[0].dtype) for it in items]
         plan.state_ptrs = _tensor_ptrs(_row_tensors(it[1], cv) for it, cv in zip(items, plan.row_cv))
         return plan
 
@@ -821,8 +823,8 @@ class TurboAdam(Optimizer):
             bufs.order_on(torch.cuda.current_stream(device))
             if self._found_inf is not None:
                 self._skip_ptr = self._skip_flag(device, self._found_inf).data_ptr()
-        # a parameter whose storage was replaced (p.data = ..., a dtype or
-        # device change) needs its descriptor row rebuilt; so does a row whose
+        # a parameter whose storage, size or dtype changed (p.data = ...) needs
+        # its descriptor row rebuilt; so does a row whose
         # state tensors were replaced, and a capturable group whose betas
         # changed (its bias-correction table, _describe_device_step)
         key = (tuple(it[4] for it in items), tuple(it[0].data_ptr() for it in items),
@@ -831,8 +833,8 @@ class TurboAdam(Optimizer):
         if plan is not None and plan.key == (key, self._layout_version):
             try:
                 row_cv = [bool(it[2]["compress_v"]) for it in items]
-                same = row_cv == plan.row_cv and _tensor_ptrs(
-                    _row_tensors(it[1], cv) for it, cv in zip(items, row_cv)) == plan.state_ptrs
+                same = row_cv == plan.row_cv and [(it[0].numel(), it[0].dtype) for it in items] == plan.elements \
+                    and _tensor_ptrs(_row_tensors(it[1], cv) for it, cv in zip(items, row_cv)) == plan.state_ptrs
             except KeyError:
                 same = False
             if not same:
