@@ -127,6 +127,20 @@ def test_compress_partial_block(n, what, stochastic):
     assert np.array_equal(np.isnan(got.view(np.float16)), nan) and np.array_equal(got[~nan], sc_o[~nan])
 
 
+@pytest.mark.parametrize("n", [1, 256, 300])
+def test_compress_of_a_negated_view(n):
+    """A tensor with torch's negative bit (the imaginary part of a conjugate) means
+    the negated values of its memory."""
+    from turboadam_amd import oneq
+
+    log(f"compress a negated view, n={n}")
+    v = torch.rand(n, device=DEV) + 1e-3
+    neg = torch._neg_view(-v)
+    assert neg.is_neg() and torch.equal(neg, v)
+    a, b = oneq.compress_v_logscale(v, 4), oneq.compress_v_logscale(neg, 4)
+    assert torch.equal(a["indices"], b["indices"]) and torch.equal(a["scales"], b["scales"])
+
+
 @pytest.mark.parametrize("bits", [2, 3, 4, 6, 8])
 @pytest.mark.parametrize("n", [1, 128, 1023, 1024, 1025, 1024 * 5 + 77])
 def test_dequantize_units(n, bits):
