@@ -313,6 +313,44 @@ def test_fp32_update_ranges(kw):
                 assert np.array_equal(a[k].view(np.uint32), b[k].view(np.uint32)), (s, i, compress_v)
 
 
+@pytest.mark.parametrize("kw", [dict(), dict(lr=0.0), dict(lr=-1e-3), dict(weight_decay=0.1), dict(lr=1e-30),
+                                dict(compress_m=False), dict(compress_v=False), dict(betas=(0.0, 0.999))])
+def test_fp32_update_of_zero_parameters(kw):
+    """Parameters of +0, -0 and below 2^-40 (pruned, masked, zero-initialised) among
+    ordinary ones, kept there from step to step, with gradients of either zero,
+    tiny, ordinary and large: the sign of a zero result and every last bit."""
+    from turboadam_amd import TurboAdam
+
+    log(f"fp32 update of zero parameters {kw}")
+    rng = np.random.default_rng(9)
+    kw = dict(dict(lr=1e-3), **kw)
+    n = 1024 * 5
+    small = np.float32([0.0, -0.0, 1e-45, -1e-45, 2.0 ** -126, -(2.0 ** -100), 2.0 ** -41, 2.0 ** -40, np.nan])
+    init = (rng.standard_normal(n) * 0.02).astype(np.float32)
+    at = np.concatenate([np.arange(1024, 2048), rng.choice(n, 700, replace=False)])
+    init[at] = rng.choice(small, at.size, p=[0.4, 0.4] + [0.2 / 7] * 7)
+    o_param = init.copy()
+    p = torch.nn.Parameter(_t(init))
+    opt = TurboAdam([p], philox_seed=6, **kw)
+    orc = O.OracleTurboAdam([o_param], dtypes=[O.DT_F32], seed=6, **kw)
+    some = np.float32([0.0, -0.0, 1e-42, 2.0 ** -110, -(2.0 ** -90), 1e-12, -1e-3, 1e3])
+    for s in range(5):
+        g = (rng.standard_normal(n) * 1e-3).astype(np.float32)
+        pick = rng.choice(at, 1500)
+        g[pick] = rng.choice(some, pick.size)
+        g[1024 + 256:1024 + 384] = 0.0  # a block without gradients
+        p.grad = _t(g)
+        opt.step()
+        orc.step([g])
+        a, b = p.detach().cpu().numpy(), o_param.reshape(-1)
+        assert np.array_equal(np.isnan(a), np.isnan(b)), s
+        k = ~np.isnan(b)
+        assert np.array_equal(a[k].view(np.uint32), b[k].view(np.uint32)), s
+        with torch.no_grad():  # pruned again: masked parameters go back to where they were
+            p[_t(at)] = _t(init[at])
+        o_param.reshape(-1)[at] = init[at]
+
+
 # pass 0 has a kernel for each mode (fp32 first moment, fp32 second moment, error feedback, any), pass 2 for
 # error feedback; mixed: tensors of two modes in one dtype
 @pytest.mark.parametrize("offset", [0, 1])

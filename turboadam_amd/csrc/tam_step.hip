@@ -978,9 +978,12 @@ __device__ __forceinline__ void tam_vpath_b(const TamTensor& d, const TamWave& W
 //    which leaves any |p| >= 2^-40 unchanged whatever its last bits.
 // A lane takes these when its q1 are normal (q_ok) and below 2^62, every |p| of
 // its elements is at least 2^-40 and every |u0| below 2^100 (an infinite m or a
-// overflowing quotient fails that); bc1 and eps decide uniformly.  Any other lane
-// takes the compiler's division and square root, and q1 from the reciprocal only
-// when a rounding test proves it (an out-of-range bc2 may put q1 on a tie).
+// overflowing quotient fails that); bc1 and eps decide uniformly.  A smaller |p|
+// (pruned, masked and zero-initialised parameters) is looked at apart: a = +-0
+// adds that zero to p, and p = +-0 takes u where |a| and |u| reach 2^-100 (r1 is
+// exact then, u normal).  Any other lane takes the compiler's division and square
+// root, and q1 from the reciprocal only when a rounding test proves it (an
+// out-of-range bc2 may put q1 on a tie).
 //
 // bf16 / fp16 parameters: a fast sequence u~ = fl(fl(c*m) * r) with
 // r = rcp(fl(s~ + eps)), s~ = sqrt(q) (v_sqrt_f32), q = fl(v * fl(1/bc2)),
@@ -1074,6 +1077,18 @@ __device__ __forceinline__ void tam_update(const TamTensor& d, float* p, const f
           pn[j] = pv + u;
         }
         ok = fast && pmin >= 0x1p-40f && umax < 0x1p100f;
+        if (fast && !ok && umax < 0x1p100f) {  // a p near zero
+          ok = true;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int i = h + j;
+            const float a = d.neg_lr * m[i], pv = wd ? p[i] * d.c_wd : p[i];
+            const bool zero = a == 0.0f, nan = pn[j] != pn[j];
+            const bool full = pv == 0.0f && __builtin_fabsf(a) >= 0x1p-100f && __builtin_fabsf(pn[j]) >= 0x1p-100f;
+            ok = ok && (__builtin_fabsf(pv) >= 0x1p-40f || (zero ? !nan : full));
+            if (zero && !nan) pn[j] = pv + a;
+          }
+        }
       }
       if (!ok) {
 #pragma unroll
