@@ -359,8 +359,7 @@ def _steady_on_cpu(n=300):
     plan = opt._describe(torch.device("cpu"), [(p, st, opt.param_groups[0], 0, 0)])
     f = M._FastStep(0, torch.device("cuda", 0), [p], [False], [0], [st], [p.grad], [torch.float32], [], plan,
                     opt.state)
-    table = plan.table
-    return opt, p, f, lambda: M._host().steady_rows(f, table.ctypes.data, table.itemsize, M._GRAD_OFF, M._STEP_OFF)
+    return opt, p, f, lambda: M._host().steady_rows(f, plan.table.ctypes.data, {}, [], 0)
 
 
 def test_steady_step_checks_a_gradient_it_has_seen_before():

@@ -68,11 +68,8 @@ const Keys& keys() {
 }
 
 // Whether the state tensors of one row are, in order, the kept objects at
-// kept[*pos ...] (the order of optimizer._row_tensors), each still at its kept
-// address in kept_ptrs (a tensor whose .data was replaced is the same object
-// elsewhere); advances *pos.
-bool row_tensors_kept(PyObject* st, bool compress_v, PyObject* kept, PyObject* kept_ptrs, Py_ssize_t n_kept,
-                      Py_ssize_t* pos) {
+// kept[*pos ...] (the order of optimizer._row_tensors); advances *pos.
+bool row_tensors_kept(PyObject* st, bool compress_v, PyObject* kept, Py_ssize_t n_kept, Py_ssize_t* pos) {
   const Keys& K = keys();
   PyObject* got[8];
   int n = 0;
@@ -111,34 +108,70 @@ bool row_tensors_kept(PyObject* st, bool compress_v, PyObject* kept, PyObject* k
   }
   for (int i = 0; i < n; ++i) {
     if (!got[i] || *pos >= n_kept) return false;
-    // None in the kept list (address 0) stands for a missing error-feedback residual
+    // None in the kept list stands for a missing error-feedback residual
     if (PyList_GET_ITEM(kept, *pos) != got[i]) return false;
-    if (got[i] != Py_None) {
-      if (!THPVariable_Check(got[i])) return false;
-      const unsigned long long at = PyLong_AsUnsignedLongLong(PyList_GET_ITEM(kept_ptrs, *pos));
-      if ((uint64_t)(uintptr_t)THPVariable_Unpack(got[i]).const_data_ptr() != at) return false;
-    }
     ++*pos;
   }
   return true;
 }
 
-// Whether every row's state tensors are the kept objects at their kept addresses
-// (lists: the rows' state dicts, their compress_v flags, the kept tensors
-// flattened, their addresses).
-bool all_rows_kept(PyObject* S, PyObject* CV, PyObject* T, PyObject* TP) {
-  if (!PyList_Check(S) || !PyList_Check(CV) || !PyList_Check(T) || !PyList_Check(TP) ||
-      PyList_GET_SIZE(S) != PyList_GET_SIZE(CV) || PyList_GET_SIZE(T) != PyList_GET_SIZE(TP))
+// The address of a tensor's elements, 0 for None.
+uint64_t address_of(PyObject* o) {
+  return o == Py_None ? 0u : (uint64_t)(uintptr_t)THPVariable_Unpack(o).const_data_ptr();
+}
+
+// Whether every row's state tensors are the kept objects (lists: the rows'
+// state dicts, their compress_v flags, the kept tensors flattened) at their kept
+// addresses (one per kept tensor): a tensor whose .data was replaced is the same
+// object elsewhere.  The addresses have a loop of their own: its loads do not
+// wait on one another (1000 tensors' state: 260 us within the walk, 45 here).
+bool all_rows_kept(PyObject* S, PyObject* CV, PyObject* T, const uint64_t* at) {
+  if (!PyList_Check(S) || !PyList_Check(CV) || !PyList_Check(T) || PyList_GET_SIZE(S) != PyList_GET_SIZE(CV))
     return false;
   Py_ssize_t pos = 0;
   const Py_ssize_t n_kept = PyList_GET_SIZE(T);
   for (Py_ssize_t j = 0; j < PyList_GET_SIZE(S); ++j) {
-    if (!row_tensors_kept(PyList_GET_ITEM(S, j), PyList_GET_ITEM(CV, j) == Py_True, T, TP, n_kept, &pos)) {
+    if (!row_tensors_kept(PyList_GET_ITEM(S, j), PyList_GET_ITEM(CV, j) == Py_True, T, n_kept, &pos)) {
       PyErr_Clear();
       return false;
     }
   }
-  return pos == n_kept;
+  if (pos != n_kept) return false;
+  uint64_t moved = 0;
+  for (Py_ssize_t i = 0; i < n_kept; ++i) moved |= address_of(PyList_GET_ITEM(T, i)) ^ at[i];
+  return moved == 0;
+}
+
+// What a steady step reads of the kept _FastStep (its tuple `native`): one
+// attribute lookup for all of it.
+struct Native {
+  PyObject *params;   // list: every parameter
+  PyObject *absent;   // list of bools: it had no gradient
+  PyObject *grads;    // list: the rows' gradients, kept until the next step
+  PyObject *states;   // list: the rows' state dicts
+  PyObject *row_cv;   // list of bools: the rows' compress_v
+  PyObject *tensors;  // list: the rows' state tensors, flattened
+  const uint64_t* tensor_at;  // their addresses
+  const int64_t* rows;        // the rows' positions in params
+  int64_t dev_index;
+};
+bool native_of(py::handle f, py::object* hold, Native* n) {
+  *hold = f.attr("native");
+  PyObject* t = hold->ptr();
+  if (!PyTuple_Check(t) || PyTuple_GET_SIZE(t) != 9) return false;
+  PyObject** lists[6] = {&n->params, &n->absent, &n->grads, &n->states, &n->row_cv, &n->tensors};
+  for (int i = 0; i < 6; ++i) {
+    *lists[i] = PyTuple_GET_ITEM(t, i);
+    if (!PyList_Check(*lists[i])) return false;
+  }
+  n->tensor_at = (const uint64_t*)(uintptr_t)PyLong_AsUnsignedLongLong(PyTuple_GET_ITEM(t, 6));
+  n->rows = (const int64_t*)(uintptr_t)PyLong_AsUnsignedLongLong(PyTuple_GET_ITEM(t, 7));
+  n->dev_index = PyLong_AsLongLong(PyTuple_GET_ITEM(t, 8));
+  if (PyErr_Occurred()) {
+    PyErr_Clear();
+    return false;
+  }
+  return true;
 }
 
 }  // namespace
@@ -146,126 +179,115 @@ bool all_rows_kept(PyObject* S, PyObject* CV, PyObject* T, PyObject* TP) {
 // Whether the rows' state tensors of the kept _FastStep f are still the
 // objects its descriptor rows were built from, at the same addresses.
 bool states_kept(py::handle f) {
-  py::object states = f.attr("states"), tensors = f.attr("tensors"), tensor_ptrs = f.attr("tensor_ptrs"),
-             row_cv = f.attr("plan").attr("row_cv");
-  return all_rows_kept(states.ptr(), row_cv.ptr(), tensors.ptr(), tensor_ptrs.ptr());
+  py::object hold;
+  Native n;
+  return native_of(f, &hold, &n) && all_rows_kept(n.states, n.row_cv, n.tensors, n.tensor_at);
+}
+
+// The addresses of a list of tensors (0 for None), written to out_addr.
+void tensor_addresses(py::list tensors, uint64_t out_addr) {
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(tensors.ptr()); ++i) {
+    PyObject* o = PyList_GET_ITEM(tensors.ptr(), i);
+    if (o != Py_None && !THPVariable_Check(o)) throw py::type_error("tensor_addresses: not a tensor");
+    ((uint64_t*)(uintptr_t)out_addr)[i] = address_of(o);
+  }
+}
+
+// The addresses of the shared bias-correction tensors (map[key]["bc1"] and "bc2"
+// for each key), written to out_addr in order, for kernels that store one float
+// to each.  False, with nothing written, unless every one of them is a
+// one-element fp32 tensor on the HIP device dev_index (the full path's fill_
+// takes any tensor).
+bool bias_addresses(py::handle map, py::handle keys_, int64_t dev_index, uint64_t out_addr) {
+  const Keys& K = keys();
+  PyObject *M = map.ptr(), *L = keys_.ptr();
+  if (!PyDict_Check(M) || !PyList_Check(L)) return false;
+  std::vector<void*> at;
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(L); ++i) {
+    PyObject* pair = PyDict_GetItemWithError(M, PyList_GET_ITEM(L, i));
+    for (PyObject* name : {K.bc1, K.bc2}) {
+      PyObject* o = pair ? item(pair, name) : nullptr;
+      if (!o || !THPVariable_Check(o)) {
+        PyErr_Clear();
+        return false;
+      }
+      const at::Tensor& t = THPVariable_Unpack(o);
+      if (!t.is_cuda() || t.get_device() != dev_index || t.layout() != at::kStrided ||
+          t.scalar_type() != at::kFloat || t.numel() != 1)
+        return false;
+      at.push_back(t.data_ptr());
+    }
+  }
+  for (size_t i = 0; i < at.size(); ++i) ((void**)(uintptr_t)out_addr)[i] = at[i];
+  return true;
 }
 
 // The per-row part of a steady step (optimizer.TurboAdam._fast_step), given
-// the kept _FastStep f and the descriptor table's memory (table_addr, row
-// stride, byte offsets of the uint64 gradient pointer and the uint32 step
-// fields).  On success the gradient pointers and step numbers of every row
-// are written and f.grads holds this step's gradient objects.
-bool steady_rows(py::handle f, uint64_t table_addr, int64_t stride, int64_t grad_off, int64_t step_off) {
+// the kept _FastStep f and the descriptor table's memory: the state tensors,
+// each row's parameter against its descriptor (address, dtype, size, layout),
+// its gradient's checks (those of TurboAdam._grad_ptr, also for an object seen
+// before: its data may have been replaced), and the shared bias-correction
+// tensors (bias_addresses).  On success the gradient pointers and step numbers
+// of every row are written and f.grads holds this step's gradients.
+bool steady_rows(py::handle f, uint64_t table_addr, py::handle bias_map, py::handle bias_keys, uint64_t bias_out) {
   if (PyErr_Occurred()) return false;
   const Keys& K = keys();
-  bool ok = false;
-  // every attribute of f read once (new references, released on return)
-  py::object params = f.attr("params"), absent = f.attr("absent"), rows = f.attr("rows"),
-             row_params = f.attr("row_params"), ptrs = f.attr("ptrs"), kept_grads = f.attr("grads"),
-             pdtypes = f.attr("pcodes"), states = f.attr("states"), tensors = f.attr("tensors"),
-             tensor_ptrs = f.attr("tensor_ptrs"), row_cv = f.attr("plan").attr("row_cv");
-  const int64_t dev_index = f.attr("dev_index").cast<int64_t>();
-  PyObject* P = params.ptr();
-  PyObject* A = absent.ptr();
-  PyObject* R = rows.ptr();
-  PyObject* RP = row_params.ptr();
-  PyObject* PT = ptrs.ptr();
-  PyObject* KG = kept_grads.ptr();
-  PyObject* PD = pdtypes.ptr();
-  PyObject* S = states.ptr();
-  PyObject* T = tensors.ptr();
-  PyObject* CV = row_cv.ptr();
-  if (!PyList_Check(P) || !PyList_Check(A) || !PyList_Check(R) || !PyList_Check(RP) || !PyList_Check(PT) ||
-      !PyList_Check(KG) || !PyList_Check(PD) || !PyList_Check(S) || !PyList_Check(T) || !PyList_Check(CV))
-    return false;
-  const Py_ssize_t np_ = PyList_GET_SIZE(P), nr = PyList_GET_SIZE(R);
-  if (PyList_GET_SIZE(A) != np_ || PyList_GET_SIZE(RP) != nr || PyList_GET_SIZE(PT) != nr ||
-      PyList_GET_SIZE(KG) != nr || PyList_GET_SIZE(PD) != nr || PyList_GET_SIZE(S) != nr ||
-      PyList_GET_SIZE(CV) != nr)
-    return false;
-  if (!all_rows_kept(S, CV, T, tensor_ptrs.ptr())) return false;
-  std::vector<PyObject*> gs((size_t)np_, nullptr);  // new references
-  auto release = [&]() {
-    for (PyObject* g : gs) Py_XDECREF(g);
-  };
+  py::object hold;
+  Native N;
+  if (!native_of(f, &hold, &N)) return false;
+  const Py_ssize_t np_ = PyList_GET_SIZE(N.params), nr = PyList_GET_SIZE(N.states);
+  if (PyList_GET_SIZE(N.absent) != np_ || PyList_GET_SIZE(N.grads) != nr) return false;
+  if (!all_rows_kept(N.states, N.row_cv, N.tensors, N.tensor_at)) return false;
+  if (!bias_addresses(bias_map, bias_keys, N.dev_index, bias_out)) return false;
   // the same parameters have gradients
+  std::vector<at::Tensor> gs((size_t)np_);
   for (Py_ssize_t i = 0; i < np_; ++i) {
-    PyObject* g = PyObject_GetAttr(PyList_GET_ITEM(P, i), K.grad);
-    if (!g) {
-      PyErr_Clear();
-      release();
-      return false;
+    PyObject* p = PyList_GET_ITEM(N.params, i);
+    if (THPVariable_CheckExact(p)) {  // a tensor or parameter: its grad as the attribute gives it
+      gs[(size_t)i] = THPVariable_Unpack(p).grad();
+    } else {
+      py::object g = py::reinterpret_steal<py::object>(PyObject_GetAttr(p, K.grad));
+      if (!g || !(g.is_none() || THPVariable_Check(g.ptr()))) {
+        PyErr_Clear();
+        return false;
+      }
+      if (!g.is_none()) gs[(size_t)i] = THPVariable_Unpack(g.ptr());
     }
-    gs[(size_t)i] = g;
-    if ((g == Py_None) != (PyList_GET_ITEM(A, i) == Py_True)) {
-      release();
-      return false;
-    }
+    if (gs[(size_t)i].defined() == (PyList_GET_ITEM(N.absent, i) == Py_True)) return false;
   }
-  // per row: parameter dtype and storage, gradient object
-  std::vector<uint64_t> gptr((size_t)nr);
+  TamTensor* T = (TamTensor*)(uintptr_t)table_addr;
   for (Py_ssize_t j = 0; j < nr; ++j) {
-    const Py_ssize_t i = PyLong_AsSsize_t(PyList_GET_ITEM(R, j));
-    if (i < 0 || i >= np_) {
+    const int64_t i = N.rows[j];
+    if (i < 0 || i >= np_ || !THPVariable_Check(PyList_GET_ITEM(N.params, i))) return false;
+    const at::Tensor &p = THPVariable_Unpack(PyList_GET_ITEM(N.params, i)), &g = gs[(size_t)i];
+    const uint32_t dt = T[j].dtype;
+    const at::ScalarType want =
+        dt == TAM_DTYPE_F32 ? at::kFloat : dt == TAM_DTYPE_BF16 ? at::kBFloat16 : at::kHalf;
+    if (p.scalar_type() != want || !p.is_contiguous() || (uint64_t)p.numel() != T[j].n ||
+        p.const_data_ptr() != T[j].param)
+      return false;
+    if (!g.defined() || g.scalar_type() != want || g.layout() != at::kStrided || !g.is_cuda() ||
+        g.get_device() != N.dev_index || !g.is_contiguous() || g.numel() != p.numel())
+      return false;
+    PyObject* stp = item(PyList_GET_ITEM(N.states, j), K.step);
+    if (!stp || !PyLong_Check(stp) || PyLong_AsLongLong(stp) < 0) {
       PyErr_Clear();
-      release();
       return false;
     }
-    PyObject* p = PyList_GET_ITEM(RP, j);
-    if (!THPVariable_Check(p)) {
-      release();
-      return false;
-    }
-    const at::Tensor& pt = THPVariable_Unpack(p);
-    // the row was built for this dtype (TAM_DTYPE_F32 / BF16 / F16), size and storage
-    const long code = PyLong_AsLong(PyList_GET_ITEM(PD, j));
-    const at::ScalarType want = code == 0 ? at::kFloat : code == 1 ? at::kBFloat16 : at::kHalf;
-    if (pt.scalar_type() != want || !pt.is_contiguous() ||
-        (uint64_t)pt.numel() != ((const TamTensor*)(uintptr_t)(table_addr + (uint64_t)j * (uint64_t)stride))->n ||
-        (uint64_t)(uintptr_t)pt.data_ptr() != PyLong_AsUnsignedLongLong(PyList_GET_ITEM(PT, j))) {
-      PyErr_Clear();
-      release();
-      return false;
-    }
-    PyObject* g = gs[(size_t)i];
-    if (!THPVariable_Check(g)) {
-      release();
-      return false;
-    }
-    const at::Tensor& gt = THPVariable_Unpack(g);
-    // the checks of _grad_ptr, also for an object seen before (its data may have been replaced)
-    if (gt.scalar_type() != pt.scalar_type() || gt.layout() != at::kStrided || !gt.is_contiguous() ||
-        !gt.is_cuda() || gt.get_device() != dev_index || gt.numel() != pt.numel()) {
-      release();
-      return false;
-    }
-    gptr[(size_t)j] = (uint64_t)(uintptr_t)gt.data_ptr();
   }
   // steady: write the rows' gradient pointers and step numbers
-  char* base = (char*)(uintptr_t)table_addr;
   for (Py_ssize_t j = 0; j < nr; ++j) {
-    PyObject* stp = item(PyList_GET_ITEM(S, j), K.step);
-    const long long s = stp ? PyLong_AsLongLong(stp) : -1;
-    if (!stp || s < 0) {
+    const at::Tensor& g = gs[(size_t)N.rows[j]];
+    T[j].grad = g.const_data_ptr();
+    T[j].step = (uint32_t)(PyLong_AsLongLong(item(PyList_GET_ITEM(N.states, j), K.step)) + 1);
+    PyObject* o = THPVariable_Wrap(g);
+    if (!o) {
       PyErr_Clear();
-      release();
       return false;
     }
-    char* row = base + j * stride;
-    std::memcpy(row + grad_off, &gptr[(size_t)j], 8);
-    const uint32_t s1 = (uint32_t)(s + 1);
-    std::memcpy(row + step_off, &s1, 4);
+    PyList_SetItem(N.grads, j, o);  // steals the new reference
   }
-  // f.grads holds this step's gradient objects until the next step
-  for (Py_ssize_t j = 0; j < nr; ++j) {
-    PyObject* g = gs[(size_t)PyLong_AsSsize_t(PyList_GET_ITEM(R, j))];
-    Py_INCREF(g);
-    PyList_SetItem(KG, j, g);  // steals the new reference
-  }
-  ok = true;
-  release();
-  return ok;
+  return true;
 }
 
 // Whether the dict holds exactly the kept values, in order, by identity.
@@ -386,35 +408,6 @@ bool steady_groups(py::handle f, uint64_t table_addr, int64_t rows, uint64_t gse
   return true;
 }
 
-// The addresses of the shared bias-correction tensors (map[key]["bc1"] and "bc2"
-// for each key), written to out_addr in order, for kernels that store one float
-// to each.  False, with nothing written, unless every one of them is a
-// one-element fp32 tensor on the HIP device dev_index (the full path's fill_
-// takes any tensor).
-bool bias_addresses(py::handle map, py::handle keys_, int64_t dev_index, uint64_t out_addr) {
-  const Keys& K = keys();
-  PyObject *M = map.ptr(), *L = keys_.ptr();
-  if (!PyDict_Check(M) || !PyList_Check(L)) return false;
-  std::vector<void*> at;
-  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(L); ++i) {
-    PyObject* pair = PyDict_GetItemWithError(M, PyList_GET_ITEM(L, i));
-    for (PyObject* name : {K.bc1, K.bc2}) {
-      PyObject* o = pair ? item(pair, name) : nullptr;
-      if (!o || !THPVariable_Check(o)) {
-        PyErr_Clear();
-        return false;
-      }
-      const at::Tensor& t = THPVariable_Unpack(o);
-      if (!t.is_cuda() || t.get_device() != dev_index || t.layout() != at::kStrided ||
-          t.scalar_type() != at::kFloat || t.numel() != 1)
-        return false;
-      at.push_back(t.data_ptr());
-    }
-  }
-  for (size_t i = 0; i < at.size(); ++i) ((void**)(uintptr_t)out_addr)[i] = at[i];
-  return true;
-}
-
 // state["step"] += 1 for each state dict (once the step has been launched).
 void advance_steps(py::list states) {
   const Keys& K = keys();
@@ -434,13 +427,14 @@ void advance_steps(py::list states) {
 
 PYBIND11_MODULE(_tam_host, m) {
   m.doc() = "Host side of a steady TurboAdam step (turboadam_amd.optimizer)";
-  m.def("steady_rows", &steady_rows, py::arg("f"), py::arg("table_addr"), py::arg("stride"), py::arg("grad_off"),
-        py::arg("step_off"));
+  m.def("steady_rows", &steady_rows, py::arg("f"), py::arg("table_addr"), py::arg("bias_map"), py::arg("bias_keys"),
+        py::arg("bias_out"));
   m.def("advance_steps", &advance_steps, py::arg("states"));
   m.def("values_kept", &values_kept, py::arg("map"), py::arg("kept"));
   m.def("steady_groups", &steady_groups, py::arg("f"), py::arg("table_addr"), py::arg("rows"), py::arg("gsel_addr"),
         py::arg("flags_addr"), py::arg("bc_addr"));
   m.def("bias_addresses", &bias_addresses, py::arg("map"), py::arg("keys"), py::arg("dev_index"),
         py::arg("out_addr"));
+  m.def("tensor_addresses", &tensor_addresses, py::arg("tensors"), py::arg("out_addr"));
   m.def("states_kept", &states_kept, py::arg("f"));
 }

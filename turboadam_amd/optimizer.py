@@ -77,11 +77,6 @@ def _host():
     return _host_module
 
 
-# byte offsets of the per-step fields a steady step rewrites in each descriptor row
-_GRAD_OFF = _DESC.fields["grad"][1]
-_STEP_OFF = _DESC.fields["step"][1]
-
-
 def _row_tensors(state, compress_v: bool) -> tuple:
     """The state tensors a descriptor row points at, in a fixed order (None
     where a row has no such array).  A kept descriptor table is valid only
@@ -250,19 +245,21 @@ class _FastStep:
         self.state_values = list(state_map.values())
         # the state tensors of each row (_row_tensors) and the addresses the row points at
         self.tensors = [t for st, cv in zip(states, plan.row_cv) for t in _row_tensors(st, cv)]
-        self.tensor_ptrs = _tensor_ptrs([self.tensors])
+        self.tensor_ptrs = np.empty(len(self.tensors), np.uint64)
+        _host().tensor_addresses(self.tensors, self.tensor_ptrs.ctypes.data)
         self.device = device
         self.dev_index = device.index if device.index is not None else torch.cuda.current_device()
         self.params = params      # every parameter of the optimizer, in order
         self.absent = absent      # [p.grad is None] of the step this was built from
-        self.rows = rows          # positions (in params) of the descriptor rows
+        self.rows = np.asarray(rows, np.int64)  # positions (in params) of the descriptor rows
         self.states = states      # their state dicts
         self.grads = grads        # the last step's gradient objects, per row (kept alive until the next)
-        self.pcodes = [_DTYPES[dt] for dt in pdtypes]  # their TAM_DTYPE_* codes
+        self.pdtypes = pdtypes    # their parameters' dtypes
         self.bc_src = bc_src      # (bc key, group betas, state dict whose step sets the group's bias corrections)
         self.plan = plan
-        self.row_params = [params[i] for i in rows]
-        self.ptrs = [p.data_ptr() for p in self.row_params]  # parameter storage the descriptor rows point at
+        # what the C++ checks read, in the order they take it (tam_host.cpp, Native)
+        self.native = (params, absent, grads, states, plan.row_cv, self.tensors, self.tensor_ptrs.ctypes.data,
+                       self.rows.ctypes.data, self.dev_index)
 
     def bind(self) -> None:
         """What the C++ and library calls of a steady step take: the table as a
@@ -272,7 +269,6 @@ class _FastStep:
         self.arr = (_lib.TamTensor * n).from_buffer(plan.table)
         self.info = _lib.TamStepInfo()
         self.nbytes = ctypes.sizeof(self.arr)
-        self.addrs = (plan.table.ctypes.data, n, plan.gsel.ctypes.data, plan.static_flags.ctypes.data)
         index = {key: i for i, (key, _, _) in enumerate(self.bc_src)}
         self.bc = [(group, src) for _, group, src in self.bc_src]
         self.groups = [(g, index.get((gi, self.device.type, self.device.index), -1)) for g, gi in plan.groups]
@@ -281,6 +277,8 @@ class _FastStep:
         # the tensors are checked and their addresses read at each step
         self.bc_keys = [key for key, _, _ in self.bc_src]
         self.bc_ptrs = (ctypes.c_void_p * max(1, 2 * len(self.bc)))()
+        self.addrs = (plan.table.ctypes.data, n, plan.gsel.ctypes.data, plan.static_flags.ctypes.data,
+                      ctypes.addressof(self.bc_ptrs), ctypes.addressof(self.bc_values))
 
 
 class TurboAdam(Optimizer):
@@ -940,12 +938,10 @@ class TurboAdam(Optimizer):
         # storage, each new gradient's checks, the state tensors; then the rows'
         # gradient pointers and step numbers are written.  Per group: the shared
         # bias-correction tensors' checks and addresses, the scalars.
-        table, n, gsel, flags = f.addrs
-        if not host.bias_addresses(self._group_step_tensors, f.bc_keys, f.dev_index, ctypes.addressof(f.bc_ptrs)):
+        table, n, gsel, flags, bc_ptrs, bc_values = f.addrs
+        if not host.steady_rows(f, table, self._group_step_tensors, f.bc_keys, bc_ptrs):
             return False
-        if not host.steady_rows(f, table, f.plan.table.itemsize, _GRAD_OFF, _STEP_OFF):
-            return False
-        if not host.steady_groups(f, table, n, gsel, flags, ctypes.addressof(f.bc_values)):
+        if not host.steady_groups(f, table, n, gsel, flags, bc_values):
             self._steady_groups(f)
         lib = _lib.load()
         if torch.cuda.current_device() == f.dev_index:
