@@ -45,8 +45,7 @@ def _f32(x: float) -> float:
 # numpy view of the descriptor layout (include/turboadam_amd.h TamTensor)
 _DESC = np.dtype(_lib.TamTensor)
 # the fields gathered per tensor, in the order _describe collects them
-_ROW_FIELDS = ("param", "grad", "v_idx", "v_scales", "exp_avg_sq", "exp_avg", "signs", "labels", "norms", "amp",
-               "alpha", "ef_residual", "n", "dtype", "flags", "v_bits", "tensor_id", "step", "k_lo", "k_hi")
+_ROW_FIELDS = ("param", "grad", "n", "dtype", "flags", "v_bits", "tensor_id", "step", "k_lo", "k_hi")
 # the fields a parameter group shares, in the order _group_fields returns them
 _GROUP_FIELDS = ("c_wd", "beta1", "one_minus_beta1", "beta2", "one_minus_beta2", "bias_correction1",
                  "bias_correction2", "inv_bc2", "inv_bc2_f32", "eps", "neg_lr", "sqrt_block")
@@ -100,15 +99,23 @@ def _tensor_ptrs(rows) -> list:
     return [0 if t is None else t.data_ptr() for row in rows for t in row]
 
 
-def _state_ptr(t, what: str, dtype, numel: int, device) -> int:
-    """Device address of a state array that the kernels read or write as numel
-    contiguous elements of dtype on device; raises where t is anything else."""
-    if not isinstance(t, torch.Tensor) or t.dtype != dtype or t.device != device or t.numel() < numel \
-            or not t.is_contiguous():
+# the state arrays of a descriptor row, as tam_host.cpp's state_addresses takes them
+_STATE_SLOTS = ("v_idx", "v_scales", "exp_avg_sq", "exp_avg", "signs", "labels", "norms", "amp", "alpha",
+                "ef_residual")
+
+
+def _state_addresses(params, tensors) -> np.ndarray:
+    """Device addresses (rows x _STATE_SLOTS) of the rows' state arrays, which the
+    kernels read and write through them alone; raises where an array's dtype,
+    device, size or layout is not what they take."""
+    out = np.empty((len(params), len(_STATE_SLOTS)), np.uint64)
+    bad = _host().state_addresses(params, tensors, out.ctypes.data)
+    if bad >= 0:
+        p, t, slot = params[bad // len(_STATE_SLOTS)], tensors[bad], _STATE_SLOTS[bad % len(_STATE_SLOTS)]
         got = f"{t.dtype} {tuple(t.shape)} on {t.device}" if isinstance(t, torch.Tensor) else type(t).__name__
-        raise RuntimeError(f"turboadam_amd: the state's {what} must be {numel} contiguous {dtype} elements on "
-                           f"{device}, got {got}")
-    return t.data_ptr()
+        raise RuntimeError(f"turboadam_amd: the {slot} array in the state of a parameter of {p.numel()} elements on "
+                           f"{p.device} is not the contiguous array of its dtype, size and device: {got}")
+    return out
 
 
 class _DeviceBuffers:
@@ -603,6 +610,8 @@ class TurboAdam(Optimizer):
         written column by column; the scalars a group shares are computed
         once per group.  The derived fields stay zero for tam_prepare."""
         rows = []
+        params = []
+        arrays = []  # the rows' state arrays, _STATE_SLOTS to a row
         group_rows = []
         groups = {}
         group_list = []
@@ -623,9 +632,8 @@ class TurboAdam(Optimizer):
             gptr = self._grad_ptr(p, state)
             n = p.numel()
             nb = num_blocks(n)
-            v_idx = v_scales = v_bits = exp_avg_sq = exp_avg = 0
-            signs = labels = norms = amp = alpha = ef = 0
-            k_lo = k_hi = 0
+            idx = scl = exp_avg_sq = exp_avg = signs = labels = norms = amp = alpha = ef = None
+            v_bits = k_lo = k_hi = 0
             if compress_v:
                 cv = state["compressed_v"]
                 idx, scl = cv["indices"], cv["scales"]
@@ -634,21 +642,17 @@ class TurboAdam(Optimizer):
                 if idx.numel() != nb * BLOCK_SIZE or scl.numel() != nb * 2:
                     raise RuntimeError("turboadam_amd: compressed_v does not match the parameter size")
                 flags |= _lib.TAM_FLAG_COMPRESS_V
-                v_idx = _state_ptr(idx, "indices", torch.uint8, nb * BLOCK_SIZE, p.device)
-                v_scales, v_bits = _state_ptr(scl, "scales", torch.float16, nb * 2, p.device), cv["n_bits"]
+                v_bits = cv["n_bits"]
             else:
-                exp_avg_sq = _state_ptr(state["exp_avg_sq"], "exp_avg_sq", torch.float32, n, p.device)
+                exp_avg_sq = state["exp_avg_sq"]
             if state["_compress_m"]:
                 mgr = state["m_mgr"]
                 enc = mgr._encoded
                 flags |= _lib.TAM_FLAG_COSTATE
                 if mgr._has_state:
                     flags |= _lib.TAM_FLAG_HAS_STATE
-                signs = _state_ptr(enc["sign_packed"], "sign_packed", torch.uint8, (n + 7) // 8, p.device)
-                labels = _state_ptr(enc["labels"], "labels", torch.uint8, nb, p.device)
-                norms = _state_ptr(enc["block_norms"], "block_norms", torch.float32, nb, p.device)
-                amp = _state_ptr(enc["scales"], "block scales", torch.float16, nb, p.device)
-                alpha = _state_ptr(mgr._alpha, "alpha", torch.float32, 1, p.device)
+                signs, labels, norms, amp = enc["sign_packed"], enc["labels"], enc["block_norms"], enc["scales"]
+                alpha = mgr._alpha
                 k_lo, k_hi = mgr.ranks(nb)
                 if mgr._error_feedback:
                     # costate.py:409-437: the residual exists from the tensor's first
@@ -659,20 +663,23 @@ class TurboAdam(Optimizer):
                         self._layout_version += 1
                     else:
                         flags |= _lib.TAM_FLAG_HAS_EF
-                    ef = _state_ptr(mgr._ef_residual, "error-feedback residual", torch.float32, n, p.device)
+                    ef = mgr._ef_residual
             else:
-                exp_avg = _state_ptr(state["exp_avg"], "exp_avg", torch.float32, n, p.device)
+                exp_avg = state["exp_avg"]
             if capturable:
                 device_step.append((len(rows), p, state, group))
                 step = 0  # filled on the device
             else:
                 step = state["step"] + 1  # the counter advances once the step is launched
-            rows.append((p.data_ptr(), gptr, v_idx, v_scales, exp_avg_sq, exp_avg, signs, labels, norms,
-                         amp, alpha, ef, n, code, flags, v_bits, tid & 0xFFFFFFFF, step & 0xFFFFFFFF, k_lo, k_hi,
+            rows.append((p.data_ptr(), gptr, n, code, flags, v_bits, tid & 0xFFFFFFFF, step & 0xFFFFFFFF, k_lo, k_hi,
                          gk, capturable))
+            params.append(p)
+            arrays += (idx, scl, exp_avg_sq, exp_avg, signs, labels, norms, amp, alpha, ef)
         table = np.zeros(len(rows), dtype=_DESC)
         cols = list(zip(*rows)) if rows else [()] * (len(_ROW_FIELDS) + 2)
         for name, col in zip(_ROW_FIELDS, cols):
+            table[name] = col
+        for name, col in zip(_STATE_SLOTS, _state_addresses(params, arrays).T):
             table[name] = col
         gsel = np.asarray(cols[-2], dtype=np.intp)
         capt = np.asarray(cols[-1], dtype=bool)
