@@ -152,21 +152,21 @@ struct Native {
   PyObject *row_cv;   // list of bools: the rows' compress_v
   PyObject *tensors;  // list: the rows' state tensors, flattened
   const uint64_t* tensor_at;  // their addresses
-  const int64_t* rows;        // the rows' positions in params
+  const int64_t* rows;        // the rows' positions in params (after the addresses in memory)
   int64_t dev_index;
 };
 bool native_of(py::handle f, py::object* hold, Native* n) {
   *hold = f.attr("native");
   PyObject* t = hold->ptr();
-  if (!PyTuple_Check(t) || PyTuple_GET_SIZE(t) != 9) return false;
+  if (!PyTuple_Check(t) || PyTuple_GET_SIZE(t) != 8) return false;
   PyObject** lists[6] = {&n->params, &n->absent, &n->grads, &n->states, &n->row_cv, &n->tensors};
   for (int i = 0; i < 6; ++i) {
     *lists[i] = PyTuple_GET_ITEM(t, i);
     if (!PyList_Check(*lists[i])) return false;
   }
   n->tensor_at = (const uint64_t*)(uintptr_t)PyLong_AsUnsignedLongLong(PyTuple_GET_ITEM(t, 6));
-  n->rows = (const int64_t*)(uintptr_t)PyLong_AsUnsignedLongLong(PyTuple_GET_ITEM(t, 7));
-  n->dev_index = PyLong_AsLongLong(PyTuple_GET_ITEM(t, 8));
+  n->rows = (const int64_t*)n->tensor_at + PyList_GET_SIZE(n->tensors);
+  n->dev_index = PyLong_AsLongLong(PyTuple_GET_ITEM(t, 7));
   if (PyErr_Occurred()) {
     PyErr_Clear();
     return false;
@@ -184,13 +184,30 @@ bool states_kept(py::handle f) {
   return native_of(f, &hold, &n) && all_rows_kept(n.states, n.row_cv, n.tensors, n.tensor_at);
 }
 
-// The addresses of a list of tensors (0 for None), written to out_addr.
-void tensor_addresses(py::list tensors, uint64_t out_addr) {
-  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(tensors.ptr()); ++i) {
+// A numpy array's memory of at least `bytes` (without the format string, which
+// takes numpy longer than the checks below for a table of descriptors).
+void* writable(py::handle array, size_t bytes) {
+  Py_buffer view;
+  if (PyObject_GetBuffer(array.ptr(), &view, PyBUF_WRITABLE) != 0) throw py::error_already_set();
+  void* at = view.buf;
+  const bool fits = (size_t)view.len >= bytes;
+  PyBuffer_Release(&view);
+  if (!fits) throw py::value_error("the array is too short");
+  return at;
+}
+
+// The addresses of a list of tensors (0 for None) and, after them, the integers
+// of a list, written to an array of 8-byte elements; its address.
+uint64_t tensor_addresses(py::list tensors, py::list rows, py::handle out) {
+  const Py_ssize_t n = PyList_GET_SIZE(tensors.ptr()), m = PyList_GET_SIZE(rows.ptr());
+  int64_t* at = (int64_t*)writable(out, 8 * (size_t)(n + m));
+  for (Py_ssize_t i = 0; i < n; ++i) {
     PyObject* o = PyList_GET_ITEM(tensors.ptr(), i);
     if (o != Py_None && !THPVariable_Check(o)) throw py::type_error("tensor_addresses: not a tensor");
-    ((uint64_t*)(uintptr_t)out_addr)[i] = address_of(o);
+    at[i] = (int64_t)address_of(o);
   }
+  for (Py_ssize_t i = 0; i < m; ++i) at[n + i] = py::handle(PyList_GET_ITEM(rows.ptr(), i)).cast<int64_t>();
+  return (uint64_t)(uintptr_t)at;
 }
 
 // The addresses of the shared bias-correction tensors (map[key]["bc1"] and "bc2"
@@ -224,22 +241,24 @@ bool bias_addresses(py::handle map, py::handle keys_, int64_t dev_index, uint64_
 
 // The addresses of the state arrays of descriptor rows, ten to a row in the order
 // of optimizer._STATE_SLOTS (None: the row has no such array, address 0), written
-// to out_addr (ten per row).  Each array must be a contiguous tensor of its slot's
+// to the rows of the table.  Each array must be a contiguous tensor of its slot's
 // dtype on the row's parameter's device, with at least the elements the kernels
 // touch.  Returns -1, or the position in `tensors` of the first that is not.
 // (One call for a table: eight checks per tensor in Python took 2 ms of the
 // first step of 1000 tensors.)
-int64_t state_addresses(py::list params, py::list tensors, uint64_t out_addr) {
+int64_t state_addresses(py::list params, py::list tensors, py::handle table) {
   static const at::ScalarType dtypes[10] = {at::kByte, at::kHalf,  at::kFloat, at::kFloat, at::kByte,
                                             at::kByte, at::kFloat, at::kHalf,  at::kFloat, at::kFloat};
   const Py_ssize_t rows = PyList_GET_SIZE(params.ptr());
   if (PyList_GET_SIZE(tensors.ptr()) != 10 * rows) throw py::value_error("state_addresses: ten arrays to a row");
+  TamTensor* T = (TamTensor*)writable(table, (size_t)rows * sizeof(TamTensor));
   for (Py_ssize_t j = 0; j < rows; ++j) {
     PyObject* po = PyList_GET_ITEM(params.ptr(), j);
     if (!THPVariable_Check(po)) throw py::type_error("state_addresses: not a parameter");
     const at::Tensor& p = THPVariable_Unpack(po);
     const int64_t n = p.numel(), nb = (n + TAM_BLOCK_SIZE - 1) / TAM_BLOCK_SIZE;
     const int64_t need[10] = {nb * TAM_BLOCK_SIZE, 2 * nb, n, n, (n + 7) / 8, nb, nb, nb, 1, n};
+    uint64_t at[10];
     for (int k = 0; k < 10; ++k) {
       PyObject* o = PyList_GET_ITEM(tensors.ptr(), 10 * j + k);
       if (o != Py_None) {
@@ -249,8 +268,19 @@ int64_t state_addresses(py::list params, py::list tensors, uint64_t out_addr) {
             t.numel() < need[k] || !t.is_contiguous())
           return 10 * j + k;
       }
-      ((uint64_t*)(uintptr_t)out_addr)[10 * j + k] = address_of(o);
+      at[k] = address_of(o);
     }
+    TamTensor& t = T[j];
+    t.v_idx = (uint8_t*)at[0];
+    t.v_scales = (uint16_t*)at[1];
+    t.exp_avg_sq = (float*)at[2];
+    t.exp_avg = (float*)at[3];
+    t.signs = (uint8_t*)at[4];
+    t.labels = (uint8_t*)at[5];
+    t.norms = (float*)at[6];
+    t.amp = (uint16_t*)at[7];
+    t.alpha = (float*)at[8];
+    t.ef_residual = (float*)at[9];
   }
   return -1;
 }
@@ -460,7 +490,7 @@ void advance_steps(py::list states) {
 
 PYBIND11_MODULE(_tam_host, m) {
   m.doc() = "Host side of a steady TurboAdam step (turboadam_amd.optimizer)";
-  m.def("state_addresses", &state_addresses, py::arg("params"), py::arg("tensors"), py::arg("out_addr"));
+  m.def("state_addresses", &state_addresses, py::arg("params"), py::arg("tensors"), py::arg("table"));
   m.def("steady_rows", &steady_rows, py::arg("f"), py::arg("table_addr"), py::arg("bias_map"), py::arg("bias_keys"),
         py::arg("bias_out"));
   m.def("advance_steps", &advance_steps, py::arg("states"));
@@ -469,6 +499,6 @@ PYBIND11_MODULE(_tam_host, m) {
         py::arg("flags_addr"), py::arg("bc_addr"));
   m.def("bias_addresses", &bias_addresses, py::arg("map"), py::arg("keys"), py::arg("dev_index"),
         py::arg("out_addr"));
-  m.def("tensor_addresses", &tensor_addresses, py::arg("tensors"), py::arg("out_addr"));
+  m.def("tensor_addresses", &tensor_addresses, py::arg("tensors"), py::arg("rows"), py::arg("out"));
   m.def("states_kept", &states_kept, py::arg("f"));
 }

@@ -104,18 +104,16 @@ _STATE_SLOTS = ("v_idx", "v_scales", "exp_avg_sq", "exp_avg", "signs", "labels",
                 "ef_residual")
 
 
-def _state_addresses(params, tensors) -> np.ndarray:
-    """Device addresses (rows x _STATE_SLOTS) of the rows' state arrays, which the
+def _set_state_addresses(table, params, tensors) -> None:
+    """The addresses of the rows' state arrays (_STATE_SLOTS to a row), which the
     kernels read and write through them alone; raises where an array's dtype,
     device, size or layout is not what they take."""
-    out = np.empty((len(params), len(_STATE_SLOTS)), np.uint64)
-    bad = _host().state_addresses(params, tensors, out.ctypes.data)
+    bad = _host().state_addresses(params, tensors, table)
     if bad >= 0:
         p, t, slot = params[bad // len(_STATE_SLOTS)], tensors[bad], _STATE_SLOTS[bad % len(_STATE_SLOTS)]
         got = f"{t.dtype} {tuple(t.shape)} on {t.device}" if isinstance(t, torch.Tensor) else type(t).__name__
         raise RuntimeError(f"turboadam_amd: the {slot} array in the state of a parameter of {p.numel()} elements on "
                            f"{p.device} is not the contiguous array of its dtype, size and device: {got}")
-    return out
 
 
 class _DeviceBuffers:
@@ -252,21 +250,20 @@ class _FastStep:
         self.state_values = list(state_map.values())
         # the state tensors of each row (_row_tensors) and the addresses the row points at
         self.tensors = [t for st, cv in zip(states, plan.row_cv) for t in _row_tensors(st, cv)]
-        self.tensor_ptrs = np.empty(len(self.tensors), np.uint64)
-        _host().tensor_addresses(self.tensors, self.tensor_ptrs.ctypes.data)
+        # with the positions (in params) of the descriptor rows after them
+        self.at = np.empty(len(self.tensors) + len(rows), np.int64)
+        at = _host().tensor_addresses(self.tensors, rows, self.at)
         self.device = device
         self.dev_index = device.index if device.index is not None else torch.cuda.current_device()
         self.params = params      # every parameter of the optimizer, in order
         self.absent = absent      # [p.grad is None] of the step this was built from
-        self.rows = np.asarray(rows, np.int64)  # positions (in params) of the descriptor rows
         self.states = states      # their state dicts
         self.grads = grads        # the last step's gradient objects, per row (kept alive until the next)
         self.pdtypes = pdtypes    # their parameters' dtypes
         self.bc_src = bc_src      # (bc key, group betas, state dict whose step sets the group's bias corrections)
         self.plan = plan
         # what the C++ checks read, in the order they take it (tam_host.cpp, Native)
-        self.native = (params, absent, grads, states, plan.row_cv, self.tensors, self.tensor_ptrs.ctypes.data,
-                       self.rows.ctypes.data, self.dev_index)
+        self.native = (params, absent, grads, states, plan.row_cv, self.tensors, at, self.dev_index)
 
     def bind(self) -> None:
         """What the C++ and library calls of a steady step take: the table as a
@@ -679,8 +676,7 @@ class TurboAdam(Optimizer):
         cols = list(zip(*rows)) if rows else [()] * (len(_ROW_FIELDS) + 2)
         for name, col in zip(_ROW_FIELDS, cols):
             table[name] = col
-        for name, col in zip(_STATE_SLOTS, _state_addresses(params, arrays).T):
-            table[name] = col
+        _set_state_addresses(table, params, arrays)
         gsel = np.asarray(cols[-2], dtype=np.intp)
         capt = np.asarray(cols[-1], dtype=bool)
         plan = _StepPlan(None, table, gsel, group_list, None, (table["flags"] & _lib.TAM_FLAG_COSTATE) != 0,
