@@ -313,7 +313,8 @@ int tam_v_compress(const float* v, uint64_t n, uint32_t v_bits, int stochastic, 
  * 5 f32->bf16->f32 by the hardware conversion; the raw hardware instructions
  * whose error bounds the certified fast paths assume: 6 v_sqrt_f32,
  * 7 v_rcp_f32, 8 v_log_f32 (log2); and the fp32 update's own operations: 9
- * square root (inputs from 2^-62), 10 reciprocal (inputs up to 2^126)).  No counterpart in the reference: it lets
+ * square root (inputs from 2^-62), 10 reciprocal (inputs up to 2^126), 11 the
+ * quotient in[2i] / in[2i + 1] of n pairs).  No counterpart in the reference: it lets
  * a caller confirm the device math equals the host. */
 int tam_math_eval(int fn, const float* in, float* out, uint64_t n, void* stream);
 

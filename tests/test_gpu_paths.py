@@ -270,6 +270,57 @@ def test_fp32_update_square_root_and_reciprocal_on_every_input():
         assert wrong == 0
 
 
+@pytest.mark.parametrize("what", ["random", "near midpoints", "all ones and powers of two", "range ends"])
+def test_fp32_update_quotient(what):
+    """The fp32 update's own quotient a/x equals the correctly rounded one where it
+    is used: |a| >= 2^-100, x from 2^-32 to 2^80, the quotient from 2^-100 to 2^100."""
+    from turboadam_amd import _lib
+
+    lib, n = _lib.load(), 1 << 24
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(11)
+
+    def ints(lo, hi):
+        return torch.randint(lo, hi, (n,), generator=gen, device=DEV, dtype=torch.int64)
+
+    def power(e):
+        return torch.ldexp(torch.ones((), device=DEV, dtype=torch.float64), e)
+
+    for rnd in range(8):
+        sig_a, sig_x = ints(1 << 23, 1 << 24).double(), ints(1 << 23, 1 << 24).double()
+        exp_x = ints(-32, 80)
+        exp_a = ints(-100, 120)
+        if what == "near midpoints":  # a next to x times a 25-bit odd significand
+            exact = sig_x * (2 * ints(1 << 23, 1 << 24) + 1).double()  # 49 bits
+            a = (exact * 2.0 ** -25).float() if rnd % 2 else exact.float() * 2.0 ** -25
+            step = ints(-2, 3).to(torch.int32)
+            sig_a = (a.view(torch.int32) + step).view(torch.float32).double()
+        elif what == "all ones and powers of two":
+            edge = torch.tensor([1 << 23, (1 << 23) + 1, (1 << 24) - 1, (1 << 24) - 2, 3 << 22], device=DEV).double()
+            sig_x = edge[ints(0, 5)]
+            if rnd % 2:
+                sig_a = edge[ints(0, 5)]
+        elif what == "range ends":
+            ends = torch.tensor([-32, -31, 78, 79], device=DEV)
+            exp_x = ends[ints(0, 4)]
+            exp_a = torch.where(ints(0, 2) == 0, ints(-100, -97), exp_x + ints(-101, -96))
+            if rnd % 2:
+                exp_a = exp_x + ints(96, 101)
+        a = (sig_a * 2.0 ** -23 * power(exp_a)).float()
+        a = torch.where(ints(0, 2) == 0, a, -a)
+        x = (sig_x * 2.0 ** -23 * power(exp_x)).float()
+        q = a.double() / x.double()
+        ok = (a.abs() >= 2.0 ** -100) & torch.isfinite(a) & (q.abs() >= 2.0 ** -100) & (q.abs() < 2.0 ** 100)
+        pairs = torch.stack([a, x], 1)[ok].contiguous()
+        want = q[ok].float()  # 53 bits >= 2 * 24 + 2: the second rounding changes nothing
+        out = torch.empty_like(want)
+        _lib.check(lib.tam_math_eval(11, pairs.data_ptr(), out.data_ptr(), out.numel(), _lib.stream_of(DEV)),
+                   "tam_math_eval")
+        wrong = int((out != want).sum())
+        log(f"quotient, {what}: {out.numel()} pairs, {wrong} wrong")
+        assert out.numel() > n // 20 and wrong == 0
+
+
 @pytest.mark.parametrize("kw", [dict(eps=1e-8), dict(eps=0.0), dict(eps=1e-30), dict(eps=1e4), dict(lr=0.0),
                                 dict(betas=(0.9, 0.5)), dict(betas=(0.0, 0.999), weight_decay=0.1)])
 def test_fp32_update_ranges(kw):

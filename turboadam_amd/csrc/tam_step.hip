@@ -1046,6 +1046,14 @@ __device__ __forceinline__ float tam_rcp_normal(float x) {
   const float y = __builtin_amdgcn_rcpf(x);
   return __builtin_fmaf(__builtin_fmaf(-x, y, 1.0f), y, y);
 }
+// fl(a/x) for |a| >= 2^-100, x as above and a quotient from 2^-100 to 2^100; u0 as
+// above.
+__device__ __forceinline__ float tam_quot_normal(float a, float x, float& u0) {
+  const float y = tam_rcp_normal(x);
+  u0 = a * y;
+  const float u1 = __builtin_fmaf(__builtin_fmaf(-x, u0, a), y, u0);
+  return __builtin_fmaf(__builtin_fmaf(-x, u1, a), y, u1);
+}
 
 template <uint32_t DT>
 __device__ __forceinline__ void tam_update(const TamTensor& d, float* p, const float* m, const float* v,
@@ -1067,10 +1075,8 @@ __device__ __forceinline__ void tam_update(const TamTensor& d, float* p, const f
           const int i = h + j;
           const float s = tam_sqrt_normal((float)((double)v[i] * inv));
           const float t2 = __builtin_fmaf(s, 0x1p-32f, d.eps) * d.bias_correction1;
-          const float a = d.neg_lr * m[i], y = tam_rcp_normal(t2);
-          const float u0 = a * y;
-          const float u1 = __builtin_fmaf(__builtin_fmaf(-t2, u0, a), y, u0);
-          const float u = __builtin_fmaf(__builtin_fmaf(-t2, u1, a), y, u1);
+          float u0;
+          const float u = tam_quot_normal(d.neg_lr * m[i], t2, u0);
           const float pv = wd ? p[i] * d.c_wd : p[i];
           pmin = __builtin_fminf(pmin, __builtin_fabsf(pv));
           umax = __builtin_fmaxf(umax, __builtin_fabsf(u0));  // a NaN stays in u
@@ -3656,7 +3662,7 @@ __global__ __launch_bounds__(256) void tam_k_put(const TamPut a, int n_tensors, 
 __global__ void tam_k_math_eval(int fn, const float* __restrict__ in, float* __restrict__ out, uint64_t n) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const float x = in[i];
+  const float x = in[fn == 11 ? 2u * i : i];
   float y;
   switch (fn) {
     case 0: y = tam_logf(x); break;
@@ -3670,6 +3676,11 @@ __global__ void tam_k_math_eval(int fn, const float* __restrict__ in, float* __r
     case 8: y = __builtin_amdgcn_logf(x); break;
     case 9: y = tam_sqrt_normal(x); break;
     case 10: y = tam_rcp_normal(x); break;
+    case 11: {
+      float u0;
+      y = tam_quot_normal(x, in[2u * i + 1u], u0);
+      break;
+    }
     default: y = x; break;
   }
   out[i] = y;
@@ -4162,7 +4173,7 @@ int tam_philox_uniforms(uint32_t tensor_id, uint32_t step, uint64_t seed, uint64
 int tam_math_eval(int fn, const float* in, float* out, uint64_t n, void* stream) {
   tam_err_buf[0] = 0;
   if (!in || !out) return tam_fail(TAM_E_INVALID, "%snull argument", "");
-  if (fn < 0 || fn > 10) return tam_fail(TAM_E_INVALID, "%sunknown function %ld", "", fn);
+  if (fn < 0 || fn > 11) return tam_fail(TAM_E_INVALID, "%sunknown function %ld", "", fn);
   if (n == 0) return TAM_OK;
   const uint64_t blocks = (n + 255) / 256;
   hipLaunchKernelGGL(tam_k_math_eval, dim3((uint32_t)blocks), dim3(256), 0, (hipStream_t)stream, fn, in, out, n);
