@@ -146,7 +146,13 @@ def _in_form(t: torch.Tensor, dtype, device) -> torch.Tensor:
     return c if c.data_ptr() % 4 == 0 else c.clone()
 
 
-def _decode(encoded: dict, alpha, g: torch.Tensor, n: int, has_state: bool, ema: bool, beta1: float = 0.0):
+def decode_blocks(encoded: dict, alpha, g: torch.Tensor, block_size: int = BLOCK_SIZE,
+                  original_numel: int = None) -> torch.Tensor:
+    """m_hat = alpha*g + s_b*sign (s_b: 0, norm_b/sqrt(128) or the fp16
+    amplitude by label), in fp32 with the shape of g (reference costate.py:261-324)."""
+    _require_gpu(g, "decode_blocks")
+    _require_block_size(block_size)
+    n = g.numel() if original_numel is None else original_numel
     lib = _lib.load()
     dev = g.device
     gf = g.reshape(-1)
@@ -156,35 +162,17 @@ def _decode(encoded: dict, alpha, g: torch.Tensor, n: int, has_state: bool, ema:
     if n != gf.numel():
         raise ValueError(f"decode_blocks: original_numel {n} does not match the gradient's {gf.numel()} elements")
     out = torch.empty(n, dtype=torch.float32, device=dev)
-    ptrs = [0, 0, 0, 0, 0]
-    keep = []
-    if has_state:
-        _check_covers(encoded, n)
-        labels = encoded["labels"].to(device=dev, dtype=torch.uint8).contiguous()
-        signs = encoded["sign_packed"].to(device=dev, dtype=torch.uint8).contiguous()
-        norms = encoded["block_norms"].to(device=dev, dtype=torch.float32).contiguous()
-        amp = encoded["scales"].to(device=dev, dtype=torch.float16).contiguous()
-        a = _scalar_on(alpha, dev)
-        keep = [labels, signs, norms, amp, a]
-        ptrs = [t.data_ptr() for t in keep]
-    b1 = float(torch.tensor(beta1, dtype=torch.float32))
-    ob1 = float(torch.tensor(1.0 - beta1, dtype=torch.float32))
-    with torch.cuda.device(dev):
-        _lib.check(lib.tam_costate_decode(ptrs[0], ptrs[1], ptrs[2], ptrs[3], ptrs[4], gf.data_ptr(),
-                                          _lib.DTYPES[gf.dtype], n, int(has_state), int(ema), b1, ob1,
+    _check_covers(encoded, n)
+    labels = encoded["labels"].to(device=dev, dtype=torch.uint8).contiguous()
+    signs = encoded["sign_packed"].to(device=dev, dtype=torch.uint8).contiguous()
+    norms = encoded["block_norms"].to(device=dev, dtype=torch.float32).contiguous()
+    amp = encoded["scales"].to(device=dev, dtype=torch.float16).contiguous()
+    a = _scalar_on(alpha, dev)
+    with torch.cuda.device(dev):  # a previous state, no EMA
+        _lib.check(lib.tam_costate_decode(labels.data_ptr(), signs.data_ptr(), norms.data_ptr(), amp.data_ptr(),
+                                          a.data_ptr(), gf.data_ptr(), _lib.DTYPES[gf.dtype], n, 1, 0, 0.0, 1.0,
                                           out.data_ptr(), _lib.stream_of(dev)), "tam_costate_decode")
-    del keep
-    return out
-
-
-def decode_blocks(encoded: dict, alpha, g: torch.Tensor, block_size: int = BLOCK_SIZE,
-                  original_numel: int = None) -> torch.Tensor:
-    """m_hat = alpha*g + s_b*sign (s_b: 0, norm_b/sqrt(128) or the fp16
-    amplitude by label), in fp32 with the shape of g (reference costate.py:261-324)."""
-    _require_gpu(g, "decode_blocks")
-    _require_block_size(block_size)
-    n = g.numel() if original_numel is None else original_numel
-    return _decode(encoded, alpha, g, n, True, False).reshape(g.shape)
+    return out.reshape(g.shape)
 
 
 class CoStateManager:

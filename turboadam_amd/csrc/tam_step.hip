@@ -177,17 +177,11 @@ template <bool FULL>
 __device__ __forceinline__ void tam_ld8_f32(const float* base, uint64_t e0, uint32_t nv, float* out) {
   tam_ld8<TAM_DTYPE_F32, FULL>(base, e0, nv, out);
 }
-template <bool FULL>
 __device__ __forceinline__ void tam_st8_f32(float* base, uint64_t e0, uint32_t nv, const float* v) {
   float* b = base + e0;
-  if (FULL) {
-    TAM_GA(TamF4E, b)[0] = TamF4{v[0], v[1], v[2], v[3]};
-    TAM_GA(TamF4E, b)[1] = TamF4{v[4], v[5], v[6], v[7]};
-  } else {
 #pragma unroll
-    for (int i = 0; i < TAM_EPL; ++i)
-      if ((uint32_t)i < nv) tam_g(b)[i] = v[i];
-  }
+  for (int i = 0; i < TAM_EPL; ++i)
+    if ((uint32_t)i < nv) tam_g(b)[i] = v[i];
 }
 
 // 16-bit parameter bit patterns, two per word (element 2k in the low half of
@@ -249,10 +243,6 @@ __device__ __forceinline__ double tam_readlane_d(double v, int l) {
   return tam_u2d(((uint64_t)hi << 32) | lo);
 }
 
-// Balanced pairwise sum of 8 values (adjacent pairing).
-__device__ __forceinline__ double tam_pair8(const double* x) {
-  return ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
-}
 // A lane's partial of a dot product or sum of squares (the reduction contract
 // of the alpha dots and the block norms): the 8 products a[i]*b[i] of fp32
 // values in an fp32 pairwise tree whose first level is fused,
@@ -658,10 +648,9 @@ __device__ __forceinline__ void tam_costate_m(const TamTensor& d, const TamWave&
 struct TamVIn {
   uint32_t sc, iw0, iw1;
 };
-template <bool FULL>
 __device__ __forceinline__ TamVIn tam_v_load(const TamTensor& d, const TamWave& W) {
   TamVIn r = {0u, 0u, 0u};
-  if (FULL || W.bvalid) {
+  if (W.bvalid) {
     r.sc = tam_g((const uint32_t*)d.v_scales)[W.b];
     const TamW2 iw = tam_g((const TamW2*)(d.v_idx + W.e0))[0];
     r.iw0 = iw.x;
@@ -703,7 +692,6 @@ struct TamVExt {
 // First half: decode, EMA, clamp, block extremes.  The parameter update runs
 // between the halves (it needs v, not the new indices), so that p, m and v are
 // no longer live during the re-quantisation.
-template <bool FULL>
 __device__ __forceinline__ TamVExt tam_vpath_a(const TamTensor& d, const TamWave& W, const TamVIn& vin,
                                                const float* g, float* v, float* vc, float* lutw,
                                                const TamLdsTabs* tabs) {
@@ -711,7 +699,7 @@ __device__ __forceinline__ TamVExt tam_vpath_a(const TamTensor& d, const TamWave
   const uint32_t nbk = 1u << bits;
   const float fnb = (float)nbk;
   const float inv_nbk = 1.0f / fnb;  // exact power of two
-  const bool bvalid = FULL || W.bvalid;
+  const bool bvalid = W.bvalid;
   const float lmin0 = tam_f16_to_f32((uint16_t)(vin.sc & 0xffffu));
   const float span0 = tam_f16_to_f32((uint16_t)(vin.sc >> 16)) - lmin0;  // quantize.py:253-255
   const uint32_t iw0 = vin.iw0, iw1 = vin.iw1;
@@ -756,7 +744,7 @@ __device__ __forceinline__ TamVExt tam_vpath_a(const TamTensor& d, const TamWave
     uint32_t xmn = 0xffffffffu, xmx = 0u;
 #pragma unroll
     for (int i = 0; i < TAM_EPL; ++i) {
-      const bool valid = FULL || (uint32_t)i < W.nv;
+      const bool valid = (uint32_t)i < W.nv;
       const float g2 = valid ? g[i] * g[i] : 0.0f;
       v[i] = __builtin_fmaf(d.one_minus_beta2, g2, vo[i] * d.beta2);
       vc[i] = __builtin_fmaxf(v[i], 1e-38f);
@@ -775,7 +763,7 @@ __device__ __forceinline__ TamVExt tam_vpath_a(const TamTensor& d, const TamWave
     uint32_t nan_seen = 0;
 #pragma unroll
     for (int i = 0; i < TAM_EPL; ++i) {
-      const bool valid = FULL || (uint32_t)i < W.nv;
+      const bool valid = (uint32_t)i < W.nv;
       const float g2 = valid ? g[i] * g[i] : 0.0f;
       v[i] = __builtin_fmaf(d.one_minus_beta2, g2, vo[i] * d.beta2);
       vc[i] = v[i] < 1e-38f ? 1e-38f : v[i];
@@ -826,12 +814,11 @@ __device__ __forceinline__ bool tam_q_in_range(const TamTensor& d, const TamVExt
 }
 
 // Second half: logs of the extremes, scales, stochastic re-quantisation.
-template <bool FULL>
 __device__ __forceinline__ void tam_vpath_b(const TamTensor& d, const TamWave& W, const float* vc, TamVExt x,
                                             const TamLdsTabs* tabs, uint32_t seed_lo, uint32_t seed_hi) {
   const uint32_t nbk = 1u << d.v_bits;
   const float fnb = (float)nbk;
-  const bool bvalid = FULL || W.bvalid;
+  const bool bvalid = W.bvalid;
   // extremes of the clamped v (quantize.py:275-280)
   const uint32_t kmn = __builtin_elementwise_max(x.kmn, TAM_BITS_1EM38);
   const uint32_t kmx = __builtin_elementwise_max(x.kmx, TAM_BITS_1EM38);
@@ -850,9 +837,8 @@ __device__ __forceinline__ void tam_vpath_b(const TamTensor& d, const TamWave& W
   }
   // certified stochastic rounding.  K and C from the hardware reciprocal of
   // sp (within 2^-23): K within 2^-22 of ln2*2^bits/sp, C within 2^-22.4 of
-  // -lmin*2^bits/sp.  Partial blocks (c~ = K log2 v + C, per element) take
-  // |log2 v| K 2^-20 and |C| 2^-21 into their bound; full blocks use K with
-  // the ratio form below.
+  // -lmin*2^bits/sp; c~ = K log2 v + C takes |log2 v| K 2^-20 and |C| 2^-21 into
+  // its bound.
   const float rsp = __builtin_amdgcn_rcpf(sp);
   const float K = (0x1.62e430p-1f * fnb) * rsp;
   const float C = (-lmn * fnb) * rsp;
@@ -862,77 +848,26 @@ __device__ __forceinline__ void tam_vpath_b(const TamTensor& d, const TamWave& W
   uint32_t rw[TAM_EPL];
   tam_draws8(W.e0, d.tensor_id, d.step, seed_lo, seed_hi, rw);
   // indices go straight into their bytes (v_cvt_pk_u8_f32 of an integral
-  // value in [0, 255]); partial blocks accept per element (lane masks)
+  // value in [0, 255]); accepted per element (lane masks)
   uint32_t ow[2] = {0u, 0u};
   bool okv[TAM_EPL];
   bool all_ok = true;
-  // Full blocks: every element lies in [vmin, vmax] (normal, no NaN checked
-  // once here), so one bound B serves the block.  With F = 2^bits the exact
-  // path's index is ceil(c - u), c = F fl(fl(l - lmin)/sp), l = fl(ln v).  The
-  // fast path takes c~ = K log2(t) from the hardware log2 of t = fl(v rcp(vmin)),
-  // which lies within 2^-22 of [1, vmax/vmin]: the hardware log's error is
-  // relative to log2 t <= (lmax - lmin)/ln2 rather than to |log2 v|, so the
-  // bound stays small when a block's log span sp is small (as 1Q's repeated
-  // re-quantisation makes it).  |c~ - c| is within:
-  //   F 2^-24 (Lm + |lmin|)/sp   the roundings of l and of lmin to fp32
-  //                              (Lm = max(|lmin|, |lmax|) bounds |l|);
-  //   F 2^-22 / sp               rcp(vmin) (2^-23.3) and the product (2^-24);
-  //   F 2^-21                    the hardware log2 (2^-21 relative; measured 2^-22.6);
-  //   F 2^-20                    the exact path's roundings of l - lmin and of
-  //                              the division, and K's (ln2 in fp32, rcp(sp));
-  //   (F + 2) 2^-21              the fma roundings of values up to F + 3/2,
-  // all times 1 + 2^-16 for the fp32 evaluation of the bound.  When B < 1/4,
-  // |c~| <= F + 1 (c lies in [0, F]).  The fast path evaluates d = fl(c~ + 1/2 - u)
-  // and q = rndne(d), which is ceil(c - u) when d lies farther than B from every
-  // half-integer; t = d - q is exact.  A lane is accepted when max |t| < H =
-  // 1/2 - (B + 2^-22); otherwise its elements are tested one by one in the exact
-  // path below.  Blocks with sp > 64 or vmax >= 2^100 (t or rcp(vmin) out of
-  // range) take the exact path.
-  float H = -1.0f, rmin = 0.0f;
-  if (FULL) {
-    rmin = __builtin_amdgcn_rcpf(tam_u2f(kmn));
-    const float Lm = __builtin_fmaxf(__builtin_fabsf(lmn), __builtin_fabsf(lmx));
-    const float per_sp = __builtin_fmaf(Lm + __builtin_fabsf(lmn), 0x1p-24f, 0x1p-22f);
-    const float flat = __builtin_fmaf(fnb, 0x1p-21f + 0x1p-20f, (fnb + 2.0f) * 0x1p-21f);
-    const float Bb = __builtin_fmaf(fnb * rsp, per_sp, flat) * (1.0f + 0x1p-16f);
-    const bool blk_ok = (tam_u2f(kmn) >= 0x1p-126f) && (tam_u2f(kmx) < 0x1p100f) && !nan_seen && (sp <= 64.0f) &&
-                        (Bb < 0.25f);
-    H = blk_ok ? 0.5f - (Bb + 0x1p-22f) : -1.0f;
-    float tmax = 0.0f;
 #pragma unroll
-    for (int i = 0; i < TAM_EPL; ++i) {
-      const float l2 = __builtin_amdgcn_logf(vc[i] * rmin);
-      const float ct = __builtin_fmaf(l2, K, 0.5f);
-      const float dd = __builtin_fmaf(-(float)rw[i], 0x1p-24f, ct);  // fl(ct - u), u exact
-      const float q = __builtin_rintf(dd);
-      tmax = __builtin_fmaxf(tmax, __builtin_fabsf(dd - q));
-      // the exact path overwrites rejected elements
-      ow[i >> 2] = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_amdgcn_fmed3f(q, 0.0f, fnb - 1.0f), i & 3, ow[i >> 2]);
-    }
-    all_ok = tmax < H;  // false for a NaN bound (then H = -1)
-  } else {
-#pragma unroll
-    for (int i = 0; i < TAM_EPL; ++i) {
-      const float l2 = __builtin_amdgcn_logf(vc[i]);
-      const float ct = __builtin_fmaf(l2, K, C);
-      const float dd = __builtin_fmaf(-(float)rw[i], 0x1p-24f, ct);  // fl(ct - u), u exact
-      const float B = __builtin_fmaf(__builtin_fabsf(l2), KB, __builtin_fmaf(__builtin_fabsf(ct), 0x1p-21f, CB));
-      const float q = __builtin_ceilf(dd);
-      const float r = q - dd;
-      okv[i] = (vc[i] >= 0x1p-126f) && (r >= B) && (1.0f - r > B);  // false for NaN
-      all_ok &= okv[i];
-      ow[i >> 2] = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_amdgcn_fmed3f(q, 0.0f, fnb - 1.0f), i & 3, ow[i >> 2]);
-    }
+  for (int i = 0; i < TAM_EPL; ++i) {
+    const float l2 = __builtin_amdgcn_logf(vc[i]);
+    const float ct = __builtin_fmaf(l2, K, C);
+    const float dd = __builtin_fmaf(-(float)rw[i], 0x1p-24f, ct);  // fl(ct - u), u exact
+    const float B = __builtin_fmaf(__builtin_fabsf(l2), KB, __builtin_fmaf(__builtin_fabsf(ct), 0x1p-21f, CB));
+    const float q = __builtin_ceilf(dd);
+    const float r = q - dd;
+    okv[i] = (vc[i] >= 0x1p-126f) && (r >= B) && (1.0f - r > B);  // false for NaN
+    all_ok &= okv[i];
+    ow[i >> 2] = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_amdgcn_fmed3f(q, 0.0f, fnb - 1.0f), i & 3, ow[i >> 2]);
   }
   if (!all_ok) {
     // exact path: the reference's own sequence with correctly rounded log and division
 #pragma unroll
     for (int i = 0; i < TAM_EPL; ++i) {
-      if (FULL) {  // the element's own test, as in the lane's
-        const float dd = __builtin_fmaf(-(float)rw[i], 0x1p-24f,
-                                        __builtin_fmaf(__builtin_amdgcn_logf(vc[i] * rmin), K, 0.5f));
-        okv[i] = __builtin_fabsf(dd - __builtin_rintf(dd)) < H;
-      }
       if (!okv[i]) {
         const float l = tam_logf_lds(vc[i], tabs);
         const float c = ((l - lmn) / sp) * fnb;  // quantize.py:284-285
@@ -1321,24 +1256,24 @@ enum { TAM_K1_ANY, TAM_K1_V_F32, TAM_K1_M_F32, TAM_K1_EF };
 // Per quarter tile: loads, first moment (CoState or fp32), second moment (1Q or
 // fp32), update, store; for CoState tensors the fp64 partial sums of g.g and
 // m.g over the quarter's 4 blocks (pairwise: blocks, then pairs of blocks).
-template <uint32_t DT, bool FULL, int MODE>
+template <uint32_t DT, int MODE>
 __device__ __forceinline__ void tam_k1_quarter(const TamTensor& d, uint32_t wq, uint32_t lane, float* lutw,
                                                const TamLdsTabs* tabs, uint32_t seed_lo, uint32_t seed_hi,
                                                double2* __restrict__ part) {
-  const TamWave W = tam_wave(d, wq, lane, FULL);
+  const TamWave W = tam_wave(d, wq, lane, false);
   const bool costate = MODE == TAM_K1_EF || (MODE != TAM_K1_M_F32 && (d.flags & TAM_FLAG_COSTATE) != 0);
   const bool compress_v = MODE == TAM_K1_M_F32 || (MODE != TAM_K1_V_F32 && (d.flags & TAM_FLAG_COMPRESS_V) != 0);
   float g[TAM_EPL], p[TAM_EPL], m[TAM_EPL], v[TAM_EPL];
   // every load of the quarter is issued before any result is used
-  if (FULL || W.bvalid) {
-    tam_ld8<DT, FULL>(d.grad, W.e0, W.nv, g);
-    tam_ld8<DT, FULL>(d.param, W.e0, W.nv, p);
+  if (W.bvalid) {
+    tam_ld8<DT, false>(d.grad, W.e0, W.nv, g);
+    tam_ld8<DT, false>(d.param, W.e0, W.nv, p);
   } else {
 #pragma unroll
     for (int i = 0; i < TAM_EPL; ++i) g[i] = p[i] = 0.0f;
   }
-  const TamCsIn cs = costate ? tam_cs_load<FULL>(d, W) : TamCsIn{0u, 0u, 0u, 0.0f};
-  const TamVIn vin = compress_v ? tam_v_load<FULL>(d, W) : TamVIn{0u, 0u, 0u};
+  const TamCsIn cs = costate ? tam_cs_load<false>(d, W) : TamCsIn{0u, 0u, 0u, 0.0f};
+  const TamVIn vin = compress_v ? tam_v_load(d, W) : TamVIn{0u, 0u, 0u};
   const float alpha_prev = (costate && (d.flags & TAM_FLAG_HAS_STATE)) ? tam_g(d.alpha)[0] : 0.0f;
   tam_compiler_fence();
 #pragma unroll
@@ -1348,16 +1283,16 @@ __device__ __forceinline__ void tam_k1_quarter(const TamTensor& d, uint32_t wq, 
   if (costate) {
     float ge[TAM_EPL];  // error feedback: the EMA takes g + residual (costate.py:410-416)
     if constexpr (MODE == TAM_K1_EF) {
-      tam_ef_grad<FULL>(d, W, g, ge);
+      tam_ef_grad<false>(d, W, g, ge);
     } else {
 #pragma unroll
       for (int i = 0; i < TAM_EPL; ++i) ge[i] = g[i];
     }
-    if (FULL || W.bvalid) tam_costate_m<FULL>(d, W, cs, alpha_prev, g, ge, m);
+    if (W.bvalid) tam_costate_m<false>(d, W, cs, alpha_prev, g, ge, m);
     float gz[TAM_EPL], mz[TAM_EPL];
 #pragma unroll
     for (int i = 0; i < TAM_EPL; ++i) {
-      const bool ok = FULL || (W.bvalid && (uint32_t)i < W.nv);
+      const bool ok = W.bvalid && (uint32_t)i < W.nv;
       gz[i] = ok ? g[i] : 0.0f;
       mz[i] = ok ? m[i] : 0.0f;
     }
@@ -1366,40 +1301,40 @@ __device__ __forceinline__ void tam_k1_quarter(const TamTensor& d, uint32_t wq, 
     // pairs; lane 12 stores g.g, lane 13 m.g
     const double t = tam_quarter_sum2((double)tam_lane_dot(gz, gz), (double)tam_lane_dot(mz, gz), lane);
     if (lane - 12u < 2u) tam_g((double*)part)[lane - 12u] = t;
-  } else if (FULL || W.bvalid) {
+  } else if (W.bvalid) {
     // fp32 exp_avg (optimizer.py:113): m = fma(1-b1, g, fl(m*b1))
     float ea[TAM_EPL];
-    tam_ld8_f32<FULL>(d.exp_avg, W.e0, W.nv, ea);
+    tam_ld8_f32<false>(d.exp_avg, W.e0, W.nv, ea);
 #pragma unroll
     for (int i = 0; i < TAM_EPL; ++i) m[i] = __builtin_fmaf(d.one_minus_beta1, g[i], ea[i] * d.beta1);
-    tam_st8_f32<FULL>(d.exp_avg, W.e0, W.nv, m);
+    tam_st8_f32(d.exp_avg, W.e0, W.nv, m);
   }
 
   // ---- second moment --------------------------------------------------
   float vc[TAM_EPL];
   TamVExt vx = {0u, 0u, 0u};
   if (compress_v) {
-    vx = tam_vpath_a<FULL>(d, W, vin, g, v, vc, lutw, tabs);
-  } else if (FULL || W.bvalid) {
+    vx = tam_vpath_a(d, W, vin, g, v, vc, lutw, tabs);
+  } else if (W.bvalid) {
     // fp32 exp_avg_sq (optimizer.py:166): v = fma(fl((1-b2)*g), g, fl(v*b2))
     float es[TAM_EPL];
-    tam_ld8_f32<FULL>(d.exp_avg_sq, W.e0, W.nv, es);
+    tam_ld8_f32<false>(d.exp_avg_sq, W.e0, W.nv, es);
 #pragma unroll
     for (int i = 0; i < TAM_EPL; ++i) v[i] = __builtin_fmaf(d.one_minus_beta2 * g[i], g[i], es[i] * d.beta2);
-    tam_st8_f32<FULL>(d.exp_avg_sq, W.e0, W.nv, v);
+    tam_st8_f32(d.exp_avg_sq, W.e0, W.nv, v);
   }
 
   // ---- parameter update -----------------------------------------------
-  if (FULL || W.bvalid) {
+  if (W.bvalid) {
     uint32_t pw2[TAM_EPL / 2];
-    const bool q_ok = tam_q_in_range<DT>(d, compress_v ? vx : tam_lane_extremes<FULL>(v, W.nv));
+    const bool q_ok = tam_q_in_range<DT>(d, compress_v ? vx : tam_lane_extremes<false>(v, W.nv));
     tam_update<DT>(d, p, m, v, pw2, q_ok);
-    if (DT == TAM_DTYPE_F32) tam_st8_f32<FULL>((float*)d.param, W.e0, W.nv, p);
-    else tam_st8_bits<FULL>(d.param, W.e0, W.nv, pw2);
+    if (DT == TAM_DTYPE_F32) tam_st8_f32((float*)d.param, W.e0, W.nv, p);
+    else tam_st8_bits<false>(d.param, W.e0, W.nv, pw2);
   }
 
   // ---- re-quantisation of v -------------------------------------------
-  if (compress_v) tam_vpath_b<FULL>(d, W, vc, vx, tabs, seed_lo, seed_hi);
+  if (compress_v) tam_vpath_b(d, W, vc, vx, tabs, seed_lo, seed_hi);
 }
 
 // ---------------------------------------------------------------------------
@@ -1545,7 +1480,25 @@ __device__ __forceinline__ TamVExt tam_vunit_a(const TamTensor& d, uint32_t lane
 
 // Logs of a block's extremes, its scales (stored by the first lane of each block
 // when `store`), and the constants of the certified index c~ = K log2(v rmin):
-// |c~ - c| <= Bb on a block with ok (the bound of tam_vpath_b, full blocks).
+// |c~ - c| <= Bb on a block with ok.
+//
+// Every element of the block lies in [vmin, vmax] (normal, no NaN: checked once
+// here), so one bound serves the block.  With F = 2^bits the exact path's c is
+// F fl(fl(l - lmin)/sp), l = fl(ln v).  c~ takes the hardware log2 of
+// t = fl(v rcp(vmin)), which lies within 2^-22 of [1, vmax/vmin]: the hardware
+// log's error is relative to log2 t <= (lmax - lmin)/ln2 rather than to |log2 v|,
+// so the bound stays small when a block's log span sp is small (as 1Q's repeated
+// re-quantisation makes it).  |c~ - c| is within:
+//   F 2^-24 (Lm + |lmin|)/sp   the roundings of l and of lmin to fp32
+//                              (Lm = max(|lmin|, |lmax|) bounds |l|);
+//   F 2^-22 / sp               rcp(vmin) (2^-23.3) and the product (2^-24);
+//   F 2^-21                    the hardware log2 (2^-21 relative; measured 2^-22.6);
+//   F 2^-20                    the exact path's roundings of l - lmin and of
+//                              the division, and K's (ln2 in fp32, rcp(sp));
+//   (F + 2) 2^-21              the fma roundings of values up to F + 3/2,
+// all times 1 + 2^-16 for the fp32 evaluation of the bound.  A block with
+// Bb >= 1/4, sp > 64 or vmax >= 2^100 (t or rcp(vmin) out of range) is not ok and
+// takes the exact path; otherwise |c~| <= F + 1 (c lies in [0, F]).
 struct TamVBlk {
   float lmn, lmx, sp, K, rmin, Bb;
   bool ok;
@@ -1579,9 +1532,10 @@ __device__ __forceinline__ TamVBlk tam_vunit_blk(uint32_t v_bits, uint16_t* v_sc
   return r;
 }
 
-// Scales and certified stochastic re-quantisation of a lane's 16 elements; as
-// tam_vpath_b for a full quarter (same bound, same fast path, same exact
-// fallback).  Every v of a block that passes the block test lies in
+// Scales and certified stochastic re-quantisation of a lane's 16 elements, with
+// the exact path of tam_vpath_b.  The index is ceil(c - u): the fast path takes
+// rndne(d), d = c~ + 1/2 - u, which is that when d lies farther than the bound
+// from every half-integer (d - rndne(d) is exact).  Every v of a block that passes the block test lies in
 // [vmin, vmax] with vmin >= 2^-126, where the clamp to 1e-38 (quantize.py:275)
 // leaves it unchanged, so the fast path reads v itself; the exact path clamps.
 // BYTES: the 8-byte index stores are aligned to bytes only; with store false
@@ -1593,8 +1547,8 @@ __device__ __forceinline__ void tam_vunit_b(const TamTensor& d, uint32_t lane, u
   const TamVBlk q_ = tam_vunit_blk(d.v_bits, d.v_scales, lane, b, x, tabs, store);
   const float fnb = (float)(1u << d.v_bits), lmn = q_.lmn, sp = q_.sp, K = q_.K, rmin = q_.rmin;
   // The fast path subtracts u' = hi 2^-16 + 2^-17 from c~ + 1, hi the high 16
-  // bits of the draw: |u - u'| <= 2^-17.  The quarter path's bound plus 2^-17
-  // covers that, plus 2^-21 the rounding of the larger c~ + 1.
+  // bits of the draw: |u - u'| <= 2^-17.  The block's bound plus 2^-17 covers
+  // that, plus 2^-21 the rounding of the larger c~ + 1.
   const float H = q_.ok ? 0.5f - (q_.Bb + (0x1p-17f + 0x1p-21f)) : -1.0f;
   const uint32_t byte_lsb = d.v_bits < 8u ? 0x01010101u : 0u;  // uniform
   const uint32_t m16 = tam_vconst(0x7fff80u), one = tam_vconst(0x3f800040u);  // 1 + 2^-17
@@ -1878,7 +1832,7 @@ __device__ __forceinline__ void tam_k1_full_body(const TamTensor* __restrict__ T
     if (d.dtype != DT || ((d.flags & TAM_FLAG_EF) != 0) != (MODE == TAM_K1_EF)) return;
     const uint32_t wq = 2u * (uint32_t)(d.n / (8u * TAM_BLOCK_SIZE)) + hw_wave;  // after the full units
     if (hw_wave < 2u && wq < (d.nb + 3u) / 4u)
-      tam_k1_quarter<DT, false, MODE>(d, wq, lane, lutw, &tabs, seed_lo, seed_hi,
+      tam_k1_quarter<DT, MODE>(d, wq, lane, lutw, &tabs, seed_lo, seed_hi,
                                       partials + (uint64_t)d.tile0 * 4u + wq);
     return;
   }
@@ -2920,23 +2874,23 @@ __global__ __launch_bounds__(TAM_SEL_WG) void tam_k_sel_labels(const TamTensor* 
 // after.  The staged encoding then replaces the previous one.  Each quarter
 // reads and writes only its own blocks and sign bytes (the stores follow the
 // residual store, which needs every load).
-template <uint32_t DT, bool FULL>
+template <uint32_t DT>
 __device__ __forceinline__ void tam_k4_quarter(const TamTensor& d, uint32_t wq, uint32_t lane, float a_old,
                                                float a_new, char* __restrict__ ws) {
-  const TamWave W = tam_wave(d, wq, lane, FULL);
-  if (!(FULL || W.bvalid)) return;  // no cross-lane work below
+  const TamWave W = tam_wave(d, wq, lane, false);
+  if (!W.bvalid) return;  // no cross-lane work below
   const bool has_ef = (d.flags & TAM_FLAG_HAS_EF) != 0;
   const TamStage st = tam_stage(d, ws);
   float g[TAM_EPL], ge[TAM_EPL], m[TAM_EPL], r[TAM_EPL];
-  tam_ld8<DT, FULL>(d.grad, W.e0, W.nv, g);
-  const TamCsIn cs = tam_cs_load<FULL>(d, W);
+  tam_ld8<DT, false>(d.grad, W.e0, W.nv, g);
+  const TamCsIn cs = tam_cs_load<false>(d, W);
   TamCsIn cn;  // the staged new encoding of the lane's block
   cn.label = tam_g(st.labels)[W.b];
   cn.nrm = tam_g(st.norms)[W.b];
   cn.amp = tam_g(st.amp)[W.b];
-  cn.byte = (FULL || W.nv > 0) ? tam_g(st.signs)[W.e0 >> 3] : 0u;
+  cn.byte = W.nv > 0 ? tam_g(st.signs)[W.e0 >> 3] : 0u;
   if (has_ef) {
-    tam_ld8_f32<FULL>(d.ef_residual, W.e0, W.nv, r);
+    tam_ld8_f32<false>(d.ef_residual, W.e0, W.nv, r);
   } else {
 #pragma unroll
     for (int i = 0; i < TAM_EPL; ++i) r[i] = 0.0f;
@@ -2944,7 +2898,7 @@ __device__ __forceinline__ void tam_k4_quarter(const TamTensor& d, uint32_t wq, 
   tam_compiler_fence();
 #pragma unroll
   for (int i = 0; i < TAM_EPL; ++i) ge[i] = has_ef ? g[i] + r[i] : g[i];
-  tam_costate_m<FULL>(d, W, cs, a_old, g, ge, m);
+  tam_costate_m<false>(d, W, cs, a_old, g, ge, m);
   const float sph = tam_div_sqrt_block(cn.nrm);
   const float s = cn.label == 1u ? sph : (cn.label == 2u ? tam_f16_to_f32((uint16_t)cn.amp) : 0.0f);
   float rn[TAM_EPL];
@@ -2956,14 +2910,14 @@ __device__ __forceinline__ void tam_k4_quarter(const TamTensor& d, uint32_t wq, 
     const float e = delta - dh;
     rn[i] = has_ef ? d.beta1 * r[i] + d.one_minus_beta1 * e : e;
   }
-  tam_st8_f32<FULL>(d.ef_residual, W.e0, W.nv, rn);
+  tam_st8_f32(d.ef_residual, W.e0, W.nv, rn);
   tam_compiler_fence();
   if (W.l16 == 0) {
     tam_g(d.labels)[W.b] = (uint8_t)cn.label;
     tam_g(d.norms)[W.b] = cn.nrm;
     tam_g(d.amp)[W.b] = (uint16_t)cn.amp;
   }
-  if (FULL || W.nv > 0) tam_g(d.signs)[W.e0 >> 3] = (uint8_t)cn.byte;
+  if (W.nv > 0) tam_g(d.signs)[W.e0 >> 3] = (uint8_t)cn.byte;
 }
 
 // A full unit of pass 4, 16 elements per lane as in tam_k2_ef: the residual (and
@@ -3042,8 +2996,8 @@ __global__ __launch_bounds__(TAM_K1U_WG) void tam_k4_ef(const TamTensor* __restr
     if (tam_unit_full(d, u)) {
       tam_k4_unit<DT>(d, u, lane, ao, an, ws, &turn[wave]);
     } else {
-      tam_k4_quarter<DT, false>(d, 2u * u, lane, ao, an, ws);
-      tam_k4_quarter<DT, false>(d, 2u * u + 1u, lane, ao, an, ws);
+      tam_k4_quarter<DT>(d, 2u * u, lane, ao, an, ws);
+      tam_k4_quarter<DT>(d, 2u * u + 1u, lane, ao, an, ws);
     }
   }
 }
@@ -3113,7 +3067,7 @@ __global__ __launch_bounds__(TAM_WG) void tam_k_decode(const uint8_t* __restrict
       m[i] = has_state ? a * gv[i] + sd : 0.0f;
     }
   }
-  tam_st8_f32<false>(out, W.e0, W.nv, m);
+  tam_st8_f32(out, W.e0, W.nv, m);
 }
 
 // The first launch of CoStateManager.update (costate.py:367-416) on one tensor:
@@ -3179,7 +3133,7 @@ __global__ __launch_bounds__(TAM_WG) void tam_k_costate_m(const TamTensor d, Tam
       const float alpha_prev = has_state ? tam_g(d.alpha)[0] : 0.0f;
       tam_ef_grad<false>(d, W, g, ge);
       tam_costate_m<false>(d, W, cs, alpha_prev, g, ge, m);
-      tam_st8_f32<false>(m_out, W.e0, W.nv, m);
+      tam_st8_f32(m_out, W.e0, W.nv, m);
 #pragma unroll
       for (int i = 0; i < TAM_EPL; ++i)
         if ((uint32_t)i >= W.nv) m[i] = 0.0f;
@@ -3356,12 +3310,12 @@ __global__ __launch_bounds__(TAM_WG) __attribute__((amdgpu_waves_per_eu(4, 4))) 
       tam_ld8<DT, false>(g, W.e0, W.nv, gv);
       d.v_idx = (uint8_t*)idx_in;
       d.v_scales = (uint16_t*)scales_in;
-      const TamVIn vin = tam_v_load<false>(d, W);
-      const TamVExt x = tam_vpath_a<false>(d, W, vin, gv, v, vc, lut[wave], &tabs);
-      if (W.bvalid) tam_st8_f32<false>(v_out, W.e0, W.nv, v);
+      const TamVIn vin = tam_v_load(d, W);
+      const TamVExt x = tam_vpath_a(d, W, vin, gv, v, vc, lut[wave], &tabs);
+      if (W.bvalid) tam_st8_f32(v_out, W.e0, W.nv, v);
       d.v_idx = idx_out;
       d.v_scales = scales_out;
-      tam_vpath_b<false>(d, W, vc, x, &tabs, seed_lo, seed_hi);
+      tam_vpath_b(d, W, vc, x, &tabs, seed_lo, seed_hi);
     }
   }
 }
