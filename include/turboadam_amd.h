@@ -217,7 +217,8 @@ int tam_multi_tensor_step_static(const TamTensor* d_tensors, const TamTensor* h_
  * error-feedback residual and commit of the staged encoding (nothing to do
  * without TAM_FLAG_EF tensors).  Issuing passes 0..4 in order on one stream
  * equals one tam_multi_tensor_step call; callers use it to time the passes one
- * by one.  No counterpart in the reference (its step is not split into passes). */
+ * by one.  Pass 3 works in the memory of pass 0's partial sums: pass 1 is not
+ * repeated after it without pass 0.  No counterpart in the reference (its step is not split into passes). */
 int tam_step_pass(int pass, const TamTensor* d_tensors, const TamStepInfo* info, uint64_t seed,
                   void* workspace, size_t ws_bytes, void* stream);
 

@@ -5,17 +5,18 @@
 // table of the previous step and rewrites only what changes: each row's
 // gradient pointer and step number.  Before it may, it checks that the step is
 // in fact steady: the same parameters have gradients, each parameter still
-// has the storage its row points at, each new gradient object is a dense,
-// contiguous tensor of its parameter's dtype on the step's device, and each
-// row's state tensors are the objects the row was built from.  Doing this per
-// row in Python costs about a microsecond per parameter; here it is a few
-// dictionary lookups and pointer comparisons.
+// has the storage, size and dtype its row was built for, each gradient is a
+// dense, contiguous tensor of its parameter's dtype and size on the step's
+// device, and each row's state tensors are the objects the row was built from,
+// at the same addresses.  Doing this per row in Python costs about a microsecond
+// per parameter; here it is a few dictionary lookups and comparisons.
 //
 // steady_rows() returns False, with nothing written, when any check fails
 // (the optimizer then takes its full path, which validates and raises where
 // something is wrong); steady_groups() writes the fields the parameter groups
 // set (numpy column writes took 20 us a step); advance_steps() adds 1 to each
-// state's step counter once the step has been launched.
+// state's step counter once the step has been launched.  state_addresses() checks
+// the state arrays of a table that is being built.
 #include <torch/extension.h>
 
 #include <cmath>
@@ -301,7 +302,6 @@ bool steady_rows(py::handle f, uint64_t table_addr, py::handle bias_map, py::han
   const Py_ssize_t np_ = PyList_GET_SIZE(N.params), nr = PyList_GET_SIZE(N.states);
   if (PyList_GET_SIZE(N.absent) != np_ || PyList_GET_SIZE(N.grads) != nr) return false;
   if (!all_rows_kept(N.states, N.row_cv, N.tensors, N.tensor_at)) return false;
-  if (!bias_addresses(bias_map, bias_keys, N.dev_index, bias_out)) return false;
   // the same parameters have gradients
   std::vector<at::Tensor> gs((size_t)np_);
   for (Py_ssize_t i = 0; i < np_; ++i) {
@@ -338,6 +338,7 @@ bool steady_rows(py::handle f, uint64_t table_addr, py::handle bias_map, py::han
       return false;
     }
   }
+  if (!bias_addresses(bias_map, bias_keys, N.dev_index, bias_out)) return false;
   // steady: write the rows' gradient pointers and step numbers
   for (Py_ssize_t j = 0; j < nr; ++j) {
     const at::Tensor& g = gs[(size_t)N.rows[j]];

@@ -413,8 +413,9 @@ __device__ __forceinline__ TAM_LDS TamF4* tam_lds_f4(uint32_t addr) { return (TA
 
 // Chunk 64 k + lane of the unit at element e of an fp32 array, k = 0..3.  NT:
 // nontemporal, for what no later pass reads again (the parameter and the
-// moments, the gradient in pass 2): 1127 -> 1053 us for 2^28 elements with an
-// fp32 first moment; a gradient that pass 2 still reads is left to the caches.
+// moments, the gradient in pass 2): pass 0 of 2^28 elements with an fp32 first
+// moment takes 1135 us without and 1075 to 1108 with, pass 2 of a GPT-2-sized
+// fp32 set 129 and 108; a gradient that pass 2 still reads is left to the caches.
 template <bool NT = false>
 __device__ __forceinline__ void tam_unit_ld(const float* base, uint64_t e, uint32_t lane, TamF4* w) {
   const TAM_GLOBAL TamF4E* b = TAM_GA(const TamF4E, (base + e)) + lane;
@@ -474,8 +475,8 @@ __device__ __forceinline__ void tam_unit_store(TamTurn* t, float* base, uint64_t
 // A wave owns 4 consecutive blocks (512 elements) of a tile: lane l holds
 // elements [8*(l%16), 8*(l%16)+8) of block 4*wq + l/16 of its tensor, where wq
 // is the wave's quarter-tile index within the tensor.  `full` quarters lie
-// entirely inside the tensor (and its arrays are 16-byte aligned): no
-// per-element bounds.  Other quarters check every element against n.
+// entirely inside the tensor: no per-element bounds (its parameter and gradient
+// may have any alignment).  Other quarters check every element against n.
 struct TamWave {
   uint32_t lane;  // 0..63
   uint32_t l16;   // lane within the block
@@ -2293,9 +2294,12 @@ __device__ __forceinline__ void tam_k2_unit(const TamTensor& d, uint32_t u, uint
   }
 }
 
-// Pass 2 is bound by memory latency rather than by its arithmetic or
-// bandwidth, so each wave loads the inputs of its next unit before it computes
-// the current one.  Descriptors and the alphas come through scalar loads
+// Pass 2 is bound by its instructions at the clock it holds: an 8B-parameter bf16
+// set takes 4.48 ms (2.04 GHz), 4.45 (2.12 GHz) with every unit's accesses sent to
+// its tensor's first two units (the same instructions, in the caches) and 3.95
+// (2.32 GHz) with the arithmetic left out (its 19 GB at 6 TB/s: 3.2).  So each wave
+// loads the inputs of its next unit before it computes the current one, and the two
+// overlap.  Descriptors and the alphas come through scalar loads
 // (their indices are wave-uniform): no vector-memory wait then covers the
 // loads in flight.  Workgroups of two waves stride over the tiles; wave w takes
 // unit 2(tile - tile0) + w.  tam_k2_encode takes the full units of 16-bit
@@ -2446,8 +2450,8 @@ __global__ __launch_bounds__(TAM_K1U_WG) void tam_k2_ef(const TamTensor* __restr
 // (about 6 us each) run anyway then, and take the tensors between at no cost,
 // where one CU needs 13 us for 18432 keys and 20 for 32768 (6 for 32).
 // The three histograms of a tensor (48 KB) lie in its partial sums, which
-// pass 1 has used up and which are at least 128 KB for a tensor of several
-// slices.
+// pass 1 has used up: one double2 per 4 blocks, at least TAM_SEL_TINY / 4 + 1 of
+// them (16 bytes more than the histograms) for a tensor that is cut into slices.
 #define TAM_SEL_WG 1024
 #define TAM_SEL_SMALL 32768u
 #define TAM_SEL_TINY 12288u
@@ -3973,7 +3977,7 @@ static int tam_launch_pass(int pass, const TamTensor* d_tensors, const TamStepIn
         hipLaunchKernelGGL(tam_k_sel_minmax, dim3(info->total_slices), dim3(TAM_SEL_WG), 0, s, d_tensors,
                            info->n_tensors, ratios, sel, partials, info->sel_small);
         TAM_HIP_CHECK(hipGetLastError());
-        for (int r = 0; r < 3; ++r) {  // 11-bit digits: at most three rounds fix all 32 bits
+        for (int r = 0; r < 3; ++r) {  // 10 + 11 + 11 bits: at most three rounds fix all 32
           hipLaunchKernelGGL(tam_k_sel_hist, dim3(info->total_slices), dim3(TAM_SEL_WG), 0, s, d_tensors,
                              info->n_tensors, ratios, sel, partials, r, info->sel_small);
           TAM_HIP_CHECK(hipGetLastError());
@@ -4054,8 +4058,8 @@ int tam_multi_tensor_step(const TamTensor* d_tensors, const TamTensor* h_tensors
 // hipGetSymbolAddress returns for the current device, looked up once per
 // device on that device's first call and kept in tam_scratch_dev.  Nothing in
 // the array must start at zero: pass 0 writes every partial that pass 1
-// reads, pass 2 every ratio that pass 3 reads, and pass 3 resets its own
-// selection state and histograms first.  Every call on one GPU uses that
+// reads, pass 1 resets the selection state, pass 2 writes every ratio that pass 3
+// reads, and pass 3 clears its histograms first.  Every call on one GPU uses that
 // GPU's one array, so calls that overlap on one GPU (on streams not ordered
 // with each other) race.
 static __device__ __align__(256) char scratch[TAM_STATIC_SCRATCH_BYTES];

@@ -5,9 +5,9 @@ Drop-in for the reference class (davidkny22/turboadam,
 src/turboadam/optimizer.py:19-292): same constructor keywords and
 validation, same step(closure) contract, same per-parameter state keys.
 Behind step() every parameter with a gradient is described in one table and
-updated by four kernel launches per device (libturboadam_amd,
-include/turboadam_amd.h), instead of the reference's per-parameter Python
-loop.  Parameters must live on a HIP device; there is no CPU path.
+updated in four passes per device (libturboadam_amd, include/turboadam_amd.h;
+a few launches whatever the tensor count), instead of the reference's
+per-parameter Python loop.  Parameters must live on a HIP device; there is no CPU path.
 """
 
 import ctypes
@@ -975,7 +975,8 @@ class TurboAdam(Optimizer):
     # descriptor lists up to this long go up as kernel arguments (tam_put, 12 to
     # a launch); longer ones are copied from pinned memory.  Steps of n vectors
     # of 768, arguments against copy: n = 12 23 and 34 us, 36 34 and 38, 48 38
-    # and 40, 72 49 and 44, 148 88 and 56
+    # and 40, 72 49 and 44, 148 88 and 56.  The two cross between 48 and 72; the
+    # line lies at three launches, short of it, where the gain is still 4 us
     _PUT_MAX = 36
 
     def _submit_fast(self, lib, f) -> None:
