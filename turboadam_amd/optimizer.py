@@ -248,11 +248,11 @@ class _FastStep:
         # opt.state.clear(), opt.state[p] = {} or a new mapping is not steady
         self.state_map = state_map
         self.state_values = list(state_map.values())
-        # the state tensors of each row (_row_tensors) and the addresses the row points at
+        # the state tensors of each row (_row_tensors) and where they are (tam_host.cpp, Place)
         self.tensors = [t for st, cv in zip(states, plan.row_cv) for t in _row_tensors(st, cv)]
         # with the positions (in params) of the descriptor rows after them
-        self.at = np.empty(len(self.tensors) + len(rows), np.int64)
-        at = _host().tensor_addresses(self.tensors, rows, self.at)
+        self.at = np.empty(4 * len(self.tensors) + len(rows), np.int64)
+        at = _host().tensor_places(self.tensors, rows, self.at)
         self.device = device
         self.dev_index = device.index if device.index is not None else torch.cuda.current_device()
         self.params = params      # every parameter of the optimizer, in order
