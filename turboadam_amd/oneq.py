@@ -45,7 +45,9 @@ def compress_v_logscale(v: torch.Tensor, n_bits: int = 3, block_size: int = BLOC
     nor (a log of zero) make it infinite.  That value is formed on the device
     (the reference reads min(v) back to the host first), by the pass that
     quantises the whole blocks; a v of whole blocks is read in place."""
-    flat = v.reshape(-1).to(torch.float32).resolve_neg()  # the kernels read its memory
+    flat = v.reshape(-1).to(torch.float32)
+    if flat.is_neg():  # the kernels read its memory
+        flat = flat.resolve_neg()
     count = flat.numel()
     if count % BLOCK_SIZE == 0 or block_size != BLOCK_SIZE:
         indices, scales, _ = quantize_logscale_nbits(flat, n_bits=n_bits, block_size=block_size,
