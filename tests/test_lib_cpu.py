@@ -376,3 +376,34 @@ def test_gradient_of_another_size_is_refused():
     p.grad.data = torch.zeros(7)
     with pytest.raises(RuntimeError, match="gradient"):
         opt._describe(torch.device("cpu"), [(p, opt.state[p], opt.param_groups[0], 0, 0)])
+
+
+def test_group_fields_of_several_groups():
+    """Each row takes its group's scalars, rounded to fp32 once, and the group's
+    weight-decay flag; its other flags stay."""
+    from turboadam_amd.optimizer import TurboAdam
+
+    params = [torch.nn.Parameter(torch.zeros(n)) for n in (5, 300, 7)]
+    opt = TurboAdam([{"params": [params[0], params[2]], "lr": 3e-4, "weight_decay": 0.1},
+                     {"params": [params[1]], "lr": 1e-2, "betas": (0.8, 0.99), "eps": 1e-5}], compress_v=False)
+    items = []
+    for tid, (p, gi) in enumerate([(params[0], 0), (params[1], 1), (params[2], 0)]):
+        n = p.numel()
+        p.grad = torch.zeros(n)
+        opt.state[p].update(step=3, _compress_m=False, exp_avg=torch.zeros(n), exp_avg_sq=torch.zeros(n))
+        items.append((p, opt.state[p], opt.param_groups[gi], gi, tid))
+    dev = torch.device("cpu")
+    opt._bc_values = {(0, "cpu", None): (0.271, 0.003), (1, "cpu", None): (0.5904, 0.0394)}
+    t = opt._describe(dev, items).table
+    f = np.float32
+    for j, (lr, wd, (b1, b2), eps, (c1, c2)) in enumerate([
+            (3e-4, 0.1, (0.9, 0.999), 1e-8, (0.271, 0.003)), (1e-2, 0.0, (0.8, 0.99), 1e-5, (0.5904, 0.0394)),
+            (3e-4, 0.1, (0.9, 0.999), 1e-8, (0.271, 0.003))]):
+        want = dict(c_wd=f(1.0 - lr * wd), beta1=f(b1), one_minus_beta1=f(1.0 - b1), beta2=f(b2),
+                    one_minus_beta2=f(1.0 - b2), bias_correction1=f(c1), bias_correction2=f(c2),
+                    inv_bc2=1.0 / float(f(c2)), inv_bc2_f32=f(1.0 / float(f(c2))), eps=f(eps), neg_lr=f(-lr),
+                    sqrt_block=f(np.sqrt(128.0)))
+        for k, x in want.items():
+            assert t[k][j] == x, (j, k)
+        assert bool(t["flags"][j] & _lib.TAM_FLAG_WD) == (wd != 0.0)
+        assert t["flags"][j] & ~np.uint32(_lib.TAM_FLAG_WD) == 0

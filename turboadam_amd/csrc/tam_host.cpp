@@ -19,6 +19,7 @@
 // the state arrays of a table that is being built.
 #include <torch/extension.h>
 
+#include <array>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -70,12 +71,13 @@ const Keys& keys() {
 
 // Where a tensor's elements were: its implementation, storage, the storage's
 // memory and the offset in it.  None: all zero.
-struct Place {
+struct Place {  // 32 bytes (optimizer._FastStep)
   const at::TensorImpl* impl;
   const c10::StorageImpl* storage;
   const void* data;
   int64_t offset;
 };
+static_assert(sizeof(Place) == 32, "the array's size in _FastStep");
 Place place_of(PyObject* o) {
   if (o == Py_None) return Place{nullptr, nullptr, nullptr, 0};
   const at::TensorImpl* t = THPVariable_Unpack(o).unsafeGetTensorImpl();
@@ -219,8 +221,8 @@ bool states_kept(py::handle f) {
   return native_of(f, &hold, &n) && all_rows_kept(n.states, n.row_cv, n.tensors, n.tensor_at);
 }
 
-// A numpy array's memory of at least `bytes` (without the format string, which
-// takes numpy longer than the checks below for a table of descriptors).
+// An array's memory of at least `bytes` (without the format string, which takes
+// numpy longer than the checks below for a table of descriptors).
 void* writable(py::handle array, size_t bytes) {
   Py_buffer view;
   if (PyObject_GetBuffer(array.ptr(), &view, PyBUF_WRITABLE) != 0) throw py::error_already_set();
@@ -319,6 +321,54 @@ int64_t state_addresses(py::list params, py::list tensors, py::handle table) {
     t.ef_residual = (float*)at[9];
   }
   return -1;
+}
+
+// The addresses of a list of tensors (0 for None).
+py::list tensor_addresses(py::list tensors) {
+  const Py_ssize_t n = PyList_GET_SIZE(tensors.ptr());
+  py::list out(n);
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    PyObject* o = PyList_GET_ITEM(tensors.ptr(), i);
+    if (o != Py_None && !THPVariable_Check(o)) throw py::type_error("tensor_addresses: not a tensor");
+    PyList_SET_ITEM(out.ptr(), i, PyLong_FromUnsignedLongLong(address_of(o)));
+  }
+  return out;
+}
+
+// The fields that parameter groups set in the rows of a descriptor table: for each
+// row j those of group_rows[gsel[j]] (tuples in the order of
+// TurboAdam._group_fields), and the weight-decay flag (wd, a list of bools).
+// (Column by column in numpy this took 70 us of a 12-tensor set's first step.)
+void set_group_fields(py::handle table, py::handle gsel, py::list group_rows, py::list wd) {
+  const size_t groups = group_rows.size();
+  std::vector<std::array<double, 12>> v(groups);
+  for (size_t g = 0; g < groups; ++g) {
+    const py::tuple t = group_rows[g].cast<py::tuple>();
+    if (t.size() != 12) throw py::value_error("set_group_fields: twelve fields to a group");
+    for (size_t k = 0; k < 12; ++k) v[g][k] = t[k].cast<double>();
+  }
+  const Py_ssize_t rows = PyObject_Length(gsel.ptr());
+  if (rows < 0 || wd.size() != groups) throw py::value_error("set_group_fields: lists of different length");
+  TamTensor* T = (TamTensor*)writable(table, (size_t)rows * sizeof(TamTensor));
+  const intptr_t* sel = (const intptr_t*)writable(gsel, (size_t)rows * sizeof(intptr_t));
+  for (Py_ssize_t j = 0; j < rows; ++j) {
+    if (sel[j] < 0 || (size_t)sel[j] >= groups) throw py::value_error("set_group_fields: no such group");
+    const std::array<double, 12>& f = v[(size_t)sel[j]];
+    TamTensor& t = T[j];
+    t.c_wd = (float)f[0];
+    t.beta1 = (float)f[1];
+    t.one_minus_beta1 = (float)f[2];
+    t.beta2 = (float)f[3];
+    t.one_minus_beta2 = (float)f[4];
+    t.bias_correction1 = (float)f[5];
+    t.bias_correction2 = (float)f[6];
+    t.inv_bc2 = f[7];
+    t.inv_bc2_f32 = (float)f[8];
+    t.eps = (float)f[9];
+    t.neg_lr = (float)f[10];
+    t.sqrt_block = (float)f[11];
+    t.flags = (t.flags & ~TAM_FLAG_WD) | (wd[(size_t)sel[j]].cast<bool>() ? TAM_FLAG_WD : 0u);
+  }
 }
 
 // The per-row part of a steady step (optimizer.TurboAdam._fast_step), given
@@ -422,7 +472,7 @@ bool betas_of(PyObject* group, double* b1, double* b2) {
 }  // namespace
 
 // The fields that parameter groups set in the descriptor rows of a steady step
-// (optimizer.TurboAdam._group_fields, _set_group_fields: each scalar a double
+// (optimizer.TurboAdam._group_fields, set_group_fields: each scalar a double
 // rounded to fp32 once) and the rows' flags, given the kept _FastStep f: its
 // `bc` list of (group, state dict whose step sets the group's bias corrections),
 // `groups` list of (group, index into bc or -1) and the addresses of the table,
@@ -526,6 +576,9 @@ void advance_steps(py::list states) {
 
 PYBIND11_MODULE(_tam_host, m) {
   m.doc() = "Host side of a steady TurboAdam step (turboadam_amd.optimizer)";
+  m.def("tensor_addresses", &tensor_addresses, py::arg("tensors"));
+  m.def("set_group_fields", &set_group_fields, py::arg("table"), py::arg("gsel"), py::arg("group_rows"),
+        py::arg("wd"));
   m.def("state_addresses", &state_addresses, py::arg("params"), py::arg("tensors"), py::arg("table"));
   m.def("steady_rows", &steady_rows, py::arg("f"), py::arg("table_addr"), py::arg("bias_map"), py::arg("bias_keys"),
         py::arg("bias_out"));

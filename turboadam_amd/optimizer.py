@@ -46,9 +46,6 @@ def _f32(x: float) -> float:
 _DESC = np.dtype(_lib.TamTensor)
 # the fields gathered per tensor, in the order _describe collects them
 _ROW_FIELDS = ("param", "grad", "n", "dtype", "flags", "v_bits", "tensor_id", "step", "k_lo", "k_hi")
-# the fields a parameter group shares, in the order _group_fields returns them
-_GROUP_FIELDS = ("c_wd", "beta1", "one_minus_beta1", "beta2", "one_minus_beta2", "bias_correction1",
-                 "bias_correction2", "inv_bc2", "inv_bc2_f32", "eps", "neg_lr", "sqrt_block")
 _SQRT_BLOCK_F32 = _f32(math.sqrt(BLOCK_SIZE))
 
 
@@ -96,7 +93,7 @@ def _row_tensors(state, compress_v: bool) -> tuple:
 
 def _tensor_ptrs(rows) -> list:
     """Device addresses of _row_tensors rows, flattened (0 for None)."""
-    return [0 if t is None else t.data_ptr() for row in rows for t in row]
+    return _host().tensor_addresses([t for row in rows for t in row])
 
 
 # the state arrays of a descriptor row, as tam_host.cpp's state_addresses takes them
@@ -251,7 +248,7 @@ class _FastStep:
         # the state tensors of each row (_row_tensors) and where they are (tam_host.cpp, Place)
         self.tensors = [t for st, cv in zip(states, plan.row_cv) for t in _row_tensors(st, cv)]
         # with the positions (in params) of the descriptor rows after them
-        self.at = np.empty(4 * len(self.tensors) + len(rows), np.int64)
+        self.at = bytearray(32 * len(self.tensors) + 8 * len(rows))
         at = _host().tensor_places(self.tensors, rows, self.at)
         self.device = device
         self.dev_index = device.index if device.index is not None else torch.cuda.current_device()
@@ -569,7 +566,8 @@ class TurboAdam(Optimizer):
     # ------------------------------------------------------------------
     def _group_fields(self, group, group_idx, device):
         """The descriptor fields one group shares on one device, each rounded
-        to fp32 once (the kernels' scalars; reference optimizer.py:88-170)."""
+        to fp32 once (the kernels' scalars; reference optimizer.py:88-170), in
+        the order tam_host.cpp's set_group_fields takes them."""
         lr = group["lr"]
         beta1, beta2 = group["betas"]
         wd = group["weight_decay"]
@@ -698,12 +696,8 @@ class TurboAdam(Optimizer):
             group_rows = [self._group_fields(g, gi, device) for g, gi in plan.groups]
         if not group_rows:
             return
-        t = plan.table
-        gvals = np.asarray(group_rows, dtype=np.float64)
-        for j, name in enumerate(_GROUP_FIELDS):
-            t[name] = gvals[plan.gsel, j]
-        wd = np.asarray([_lib.TAM_FLAG_WD if g["weight_decay"] != 0.0 else 0 for g, _ in plan.groups], np.uint32)
-        t["flags"] = (t["flags"] & np.uint32(~_lib.TAM_FLAG_WD & 0xFFFFFFFF)) | wd[plan.gsel]
+        _host().set_group_fields(plan.table, plan.gsel, group_rows,
+                                 [bool(g["weight_decay"] != 0.0) for g, _ in plan.groups])
 
     def _refresh(self, plan, device, items) -> None:
         """Per-step fields of a kept descriptor table: gradient pointers, step
@@ -836,7 +830,7 @@ class TurboAdam(Optimizer):
                 row_cv = [bool(it[2]["compress_v"]) for it in items]
                 same = row_cv == plan.row_cv and [(it[0].numel(), it[0].dtype) for it in items] == plan.elements \
                     and _tensor_ptrs(_row_tensors(it[1], cv) for it, cv in zip(items, row_cv)) == plan.state_ptrs
-            except KeyError:
+            except (KeyError, TypeError):  # an array is gone, or no tensor
                 same = False
             if not same:
                 plan = None
