@@ -407,3 +407,19 @@ def test_group_fields_of_several_groups():
             assert t[k][j] == x, (j, k)
         assert bool(t["flags"][j] & _lib.TAM_FLAG_WD) == (wd != 0.0)
         assert t["flags"][j] & ~np.uint32(_lib.TAM_FLAG_WD) == 0
+
+
+def test_addresses_of_copy_on_write_tensors_are_their_own():
+    """A lazy clone shares its memory until one of the two is written: the addresses
+    the kernels write through, and the steady check, see the array's own memory."""
+    from turboadam_amd import optimizer as M
+
+    opt, p, f, _ = _steady_on_cpu()
+    assert opt._fast_state_kept(f)
+    t = opt.state[p]["exp_avg"]
+    clone = torch._lazy_clone(t)
+    assert not opt._fast_state_kept(f)
+    clone = torch._lazy_clone(opt.state[p]["exp_avg_sq"])
+    row = opt._describe(torch.device("cpu"), [(p, opt.state[p], opt.param_groups[0], 0, 0)]).table[0]
+    assert row["exp_avg_sq"] == opt.state[p]["exp_avg_sq"].data_ptr() != clone.data_ptr()
+    assert M._tensor_ptrs([(t, None)]) == [t.data_ptr(), 0]

@@ -73,7 +73,7 @@ const Keys& keys() {
 // memory and the offset in it.  None: all zero.
 struct Place {  // 32 bytes (optimizer._FastStep)
   const at::TensorImpl* impl;
-  const c10::StorageImpl* storage;
+  c10::StorageImpl* storage;
   const void* data;
   int64_t offset;
 };
@@ -81,8 +81,8 @@ static_assert(sizeof(Place) == 32, "the array's size in _FastStep");
 Place place_of(PyObject* o) {
   if (o == Py_None) return Place{nullptr, nullptr, nullptr, 0};
   const at::TensorImpl* t = THPVariable_Unpack(o).unsafeGetTensorImpl();
-  const c10::StorageImpl* s = t->has_storage() ? t->unsafe_storage().unsafeGetStorageImpl() : nullptr;
-  return Place{t, s, s ? s->data() : nullptr, s ? t->storage_offset() : 0};
+  c10::StorageImpl* s = t->has_storage() ? t->unsafe_storage().unsafeGetStorageImpl() : nullptr;
+  return Place{t, s, s ? s->mutable_data() : nullptr, s ? t->storage_offset() : 0};
 }
 // Whether the tensor is still there.  A kept pointer is followed only once the
 // object above it has been seen to hold it still (nothing keeps them alive).
@@ -90,7 +90,7 @@ bool in_place(PyObject* o, const Place& at) {
   if (o == Py_None) return !at.impl;
   const at::TensorImpl* t = THPVariable_Unpack(o).unsafeGetTensorImpl();
   if (t != at.impl || !t->has_storage() || t->unsafe_storage().unsafeGetStorageImpl() != at.storage) return false;
-  return at.storage->data() == at.data && t->storage_offset() == at.offset;
+  return at.storage->mutable_data() == at.data && t->storage_offset() == at.offset;
 }
 
 // Whether the state tensors of one row are, in order, the kept objects at
@@ -143,9 +143,10 @@ bool row_tensors_kept(PyObject* st, bool compress_v, PyObject* kept, const Place
   return true;
 }
 
-// The address of a tensor's elements, 0 for None.
+// The address of a tensor's elements for writing (a copy-on-write tensor gets its
+// own memory first), 0 for None.
 uint64_t address_of(PyObject* o) {
-  return o == Py_None ? 0u : (uint64_t)(uintptr_t)THPVariable_Unpack(o).const_data_ptr();
+  return o == Py_None ? 0u : (uint64_t)(uintptr_t)THPVariable_Unpack(o).data_ptr();
 }
 
 // Whether every row's state tensors are the kept objects (lists: the rows'
@@ -412,7 +413,7 @@ bool steady_rows(py::handle f, uint64_t table_addr, py::handle bias_map, py::han
     const at::ScalarType want =
         dt == TAM_DTYPE_F32 ? at::kFloat : dt == TAM_DTYPE_BF16 ? at::kBFloat16 : at::kHalf;
     if (p.scalar_type() != want || !p.is_contiguous() || (uint64_t)p.numel() != T[j].n ||
-        p.const_data_ptr() != T[j].param)
+        p.data_ptr() != T[j].param)
       return false;
     if (!g.defined() || g.scalar_type() != want || g.layout() != at::kStrided || !g.is_cuda() ||
         g.get_device() != N.dev_index || !g.is_contiguous() || g.numel() != p.numel())
